@@ -109,17 +109,11 @@ __global__ void k_fill(double *p, std::size_t n, double v) {
 }
 
 // Residual scalars (kokkos_local_energy_reverse.cpp:124-170): a block's input
-// x <- a x + c x0 (x0 the embedding), and the adjoint of the previous block's
-// output g <- a g.
+// x <- a x + c x0 (x0 the embedding).
 __global__ void k_axpby(std::size_t n, double a, double *x, double c, const double *x0) {
   const std::size_t i = std::size_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i < n) x[i] = a * x[i] + c * x0[i];
 }
-__global__ void k_scale(std::size_t n, double a, double *g) {
-  const std::size_t i = std::size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < n) g[i] *= a;
-}
-
 // QK normalisation (kokkos_integrated_block0.cpp:288-328): each head row
 // (32 channels) of q, k, q_ev, k_ev of a node divided by its RMS, eps 1e-6;
 // v untouched.  One thread per (node, row); row r = 4 w + h, w = q, k, q_ev,
@@ -354,7 +348,7 @@ __global__ __launch_bounds__(128) void k_filter_fwd(const int *n_active, const i
     const int lo = c == 0 ? 0 : (c == 1 ? 3 : (c == 2 ? 8 : 15));
     const int hi = c == 0 ? 3 : (c == 1 ? 8 : (c == 2 ? 15 : 24));
     double acc = 0.0;
-    for (int m = lo; m < hi; ++m) {
+    for (int m = lo; ev && m < hi; ++m) {
       const double d = ev[std::size_t(a) * kE + m] - ev[std::size_t(b) * kE + m];
       acc += d * d * A.att_cg[m];
     }
@@ -1914,75 +1908,7 @@ __global__ __launch_bounds__(256) void k_rint_place(const int *n_active, const i
   if (p < *n_active) order[atomicAdd(&cursor[rint_key(pa[2 * p], pr[p], d)], 1)] = p;
 }
 
-// ---------------------------------------------------------------- MFMA node GEMMs
-// out[n][o] = sum_k W[o][k] X[n][k] (+ epilogue), 16 nodes per wavefront as the
-// MFMA column block, output features as rows.  K is read from the node rows in
-// the permuted order k = 16 T + g + 4 v (zero beyond K); W is pre-permuted
-// (permute_mfma) and zero-padded to 16-row tiles and 16-column K chunks.
-// EPI 0: out = acc + bias; 1: out = pre, out2 = silu(pre).  The bias comes in accumulator order
-// (bias_acc) and starts the accumulators.  Output tiles are taken MG at a
-// time; per tile group the operand stream holds, per K chunk, the X chunk and
-// the MG weight fragments.
-template <int EPI, int KT, int MT, int MG>
-__global__ __launch_bounds__(256) void k_gemm(int rows, int K, int O, const double *__restrict__ X, int ldx,
-                                              const double *__restrict__ Wp, const double *__restrict__ biasp,
-                                              double *__restrict__ out, int ldo, double *__restrict__ out2) {
-  // one group of MG output tiles per wavefront (the group is blockIdx.y), so
-  // a few thousand node rows still give every SIMD several wavefronts
-  static_assert(MT % MG == 0, "output tiles must split into equal groups");
-  constexpr int PER_T = 1 + MG, PER_G = KT * PER_T;
-  const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
-  const int w = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (w * 16 >= rows) return;
-  const int grp = blockIdx.y;
-  const int n = w * 16 + j;
-  const bool valid = n < rows;
-  const int nn = valid ? n : rows - 1;
-  const double *xr = X + std::size_t(nn) * ldx;
-  const v4d zero = v4d{0, 0, 0, 0};
-
-  auto load = [&](auto si) -> v4d {
-    constexpr int s = decltype(si)::value, T = s / PER_T, u = s % PER_T;
-    if constexpr (u == 0) {
-      v4d b;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int k = 16 * T + g + 4 * v;
-        b[v] = (16 * T + 16 <= K || k < K) ? xr[k] : 0.0;
-      }
-      return b;
-    } else {
-      return wload(Wp, KT, grp * MG + u - 1, T, lane);
-    }
-  };
-  Stream<PER_G, kFilterPF, decltype(load)> st(load);
-  v4d acc[MG];
-#pragma unroll
-  for (int q = 0; q < MG; ++q) acc[q] = biasp ? tile_load(biasp, grp * MG + q, lane) : zero;
-  st.prime();
-  v4d bT = zero;
-  st.run([&](auto si, const v4d &wv) {
-    constexpr int s = decltype(si)::value, u = s % PER_T;
-    if constexpr (u == 0) {
-      bT = wv;
-    } else {
-      acc[u - 1] = mfma4(wv, bT, acc[u - 1]);
-    }
-  });
-  if (!valid) return;
-#pragma unroll
-  for (int q = 0; q < MG; ++q)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int o = 16 * (grp * MG + q) + g + 4 * r;
-      if (o >= O) continue;
-      const std::size_t io = std::size_t(n) * ldo + o;
-      const double v = acc[q][r];
-      if constexpr (EPI == 0) out[io] = v;
-      if constexpr (EPI == 1) { out[io] = v; out2[io] = silu(v); }
-    }
-}
-
+// ---------------------------------------------------------------- node layers
 // Block-diagonal projections: per head h, the 160 outputs (q k v q_ev k_ev,
 // 32 each) depend on x[h*32 .. h*32+32).  Wp holds, per head, the permuted
 // (160 x 32) matrix; out[n][w*128 + h*32 + o].  Stream per head: the two
@@ -2000,8 +1926,7 @@ __global__ __launch_bounds__(256) void k_qkv_mfma(int rows, const double *__rest
   auto load = [&](auto si) -> v4d {
     constexpr int s = decltype(si)::value;
     if constexpr (s < 2) {
-      return v4d{xr[h * kHW + 16 * s + g], xr[h * kHW + 16 * s + g + 4], xr[h * kHW + 16 * s + g + 8],
-                 xr[h * kHW + 16 * s + g + 12]};
+      return *reinterpret_cast<const v4d *>(xr + h * kHW + 16 * s + 4 * g);
     } else {
       return wload(Wp + std::size_t(h) * 160 * kHW, 2, (s - 2) / 2, (s - 2) % 2, lane);
     }
@@ -2036,58 +1961,6 @@ __global__ __launch_bounds__(256) void k_qkv_mfma(int rows, const double *__rest
   });
 }
 
-// dx[n][h*32 + k] = base[n][.] + sum_{w,o} W[w][h][k][o] g[n][w*128 + h*32 + o];
-// per head the permuted transpose (32 x 160), K read in the permuted order
-// from the 160 gradient entries of that head.  Stream per head and K chunk:
-// the gradient chunk, then the two weight fragments.
-__global__ __launch_bounds__(256) void k_qkv_bwd_mfma(int rows, const double *__restrict__ G,
-                                                      const double *__restrict__ Wtp, const double *__restrict__ base,
-                                                      double *__restrict__ dx) {
-  const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
-  const int w = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (w * 16 >= rows) return;
-  const int n = w * 16 + j;
-  const bool valid = n < rows;
-  const double *gr = G + std::size_t(valid ? n : rows - 1) * 640;
-  const int h = blockIdx.y;  // one head per wavefront
-  constexpr int PER_H = 10 * 3;
-  auto load = [&](auto si) -> v4d {
-    constexpr int s = decltype(si)::value, T = s / 3, u = s % 3;
-    if constexpr (u == 0) {
-      // K entries 16 T + g + 4 v: projection T / 2, channels 32 h + 16 (T % 2)
-      // + g + 4 v, adjacent in the tile-transposed row order (fpos)
-      return *reinterpret_cast<const v4d *>(gr + (T >> 1) * kF + h * kHW + 16 * (T & 1) + 4 * g);
-    } else {
-      return wload(Wtp + std::size_t(h) * kHW * 160, 10, u - 1, T, lane);
-    }
-  };
-  Stream<PER_H, kFilterPF, decltype(load)> st(load);
-  st.prime();
-  const v4d zero = v4d{0, 0, 0, 0};
-  v4d bT = zero, acc[2];
-  st.run([&](auto si, const v4d &wv) {
-    constexpr int s = decltype(si)::value, u = s % 3;
-    if constexpr (s == 0) { acc[0] = zero; acc[1] = zero; }
-    if constexpr (u == 0) bT = wv;
-    else acc[u - 1] = mfma4(wv, bT, acc[u - 1]);
-    if constexpr (s == PER_H - 1) {
-      if (valid) {
-        // base (the attention-residual adjoint) is stored in the
-        // tile-transposed order: channels 16 mt + g + 4 r at 16 mt + 4 g + r
-#pragma unroll
-        for (int mt = 0; mt < 2; ++mt) {
-          const v4d bv = *reinterpret_cast<const v4d *>(base + std::size_t(n) * kF + h * kHW + 16 * mt + 4 * g);
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int c = h * kHW + 16 * mt + g + 4 * r;
-            dx[std::size_t(n) * kF + c] = bv[r] + acc[mt][r];
-          }
-        }
-      }
-    }
-  });
-}
-
 // ---------------------------------------------------------------- attention
 // 16-byte load / store of two adjacent doubles (16-byte aligned)
 __device__ __forceinline__ double2 ld2(const double *p) { return *reinterpret_cast<const double2 *>(p); }
@@ -2097,6 +1970,20 @@ __device__ __forceinline__ void st2(double *p, double a, double b) { *reinterpre
 // equivariant channel off[h] + t of degree h + 1 when t < 2 h + 3, so every
 // per-head sum is a 16-lane group reduction.
 
+
+// The post-attention block's first normalisation of a node row held two
+// channels per lane (biased variance): its normalised values h and 1/sigma
+// (the affine weights are applied where the row is read, k_node_fwd and
+// k_node_bwd).  mode (NormMode): 0 LayerNorm; 1 RMSNorm (no mean removed);
+// 2 none (h = v, is = 1).
+__device__ __forceinline__ void wave_normalise(double v0, double v1, double eps, int mode, double &h0, double &h1,
+                                               double &is) {
+  const double mean = mode == 0 ? wave_sum(v0 + v1) / kF : 0.0;
+  const double d0 = v0 - mean, d1 = v1 - mean;
+  is = mode == 2 ? 1.0 : 1.0 / sqrt(wave_sum(d0 * d0 + d1 * d1) / kF + eps);
+  h0 = d0 * is;
+  h1 = d1 * is;
+}
 
 // Active incidence of this step: entry k of a node's list as active pair
 // index * 2 + side (-1 for a candidate beyond the cutoff) and its partner
@@ -2116,24 +2003,26 @@ __global__ void k_inc_active(int E, const int *inc, const int *cand2act, const i
 // alpha = <q_n, k_o (.) f_p> / avg (per head) and the messages
 // fc alpha v_o (invariant) and fc alpha_ev Y (equivariant, (-1)^l Y when n is
 // the pair's second endpoint).  Lanes: 16 per head, two channels each.
+// Then the residual and its first normalisation (n1hat, 1/sigma), with the
+// whole row in the wavefront.  ev null: zero (block 0).
 // This full form runs with the scalar filter kernels; the MFMA filter forms
 // alpha itself and k_attn_msg does the rest.
 __global__ __launch_bounds__(256) void k_attn_fwd(int N, const int *inc_off, const int *__restrict__ iact,
                                                   const int *__restrict__ iother, const double *__restrict__ x,
                                                   const double *__restrict__ ev, const double *__restrict__ qkv,
                                                   const double *__restrict__ pf, const double *__restrict__ pY,
-                                                  const double *__restrict__ pfc, double inv_avg,
-                                                  double *__restrict__ palpha, double *__restrict__ ainv,
+                                                  const double *__restrict__ pfc, double inv_avg, double eps,
+                                                  int lnmode, double *__restrict__ palpha,
+                                                  double *__restrict__ n1hat, double *__restrict__ n1is,
                                                   double *__restrict__ aev) {
   const int lane = threadIdx.x & 63;
   const int n = xcd_block() * 4 + (threadIdx.x >> 6);
   if (n >= N) return;
   const int h = lane >> 4, t = lane & 15;
   // the lane's two channels sit next to each other in the tile-transposed
-  // rows (filters, q k v): positions 32 h + 2 t and + 1, read as one 16-byte
-  // vector; fpos is its own inverse, so the channels are fpos(position)
-  const int p0 = 32 * h + 2 * t, p1 = p0 + 1;
-  const int c0 = fpos(p0), c1 = fpos(p1);  // c1 = c0 + 4
+  // rows (x, filters, q k v): positions 32 h + 2 t and + 1, read as one
+  // 16-byte vector
+  const int p0 = 32 * h + 2 * t;
   const bool evv = t < 2 * h + 3;
   const int m = evv ? ev_offset(h) + t : 0;
   const double par = slot_parity(h);
@@ -2176,26 +2065,13 @@ __global__ __launch_bounds__(256) void k_attn_fwd(int N, const int *inc_off, con
       }
     }
   });
-  const std::size_t i = std::size_t(n) * kF;
-  ainv[i + c0] = x[i + c0] + acc0;
-  ainv[i + c1] = x[i + c1] + acc1;
-  if (evv) aev[std::size_t(n) * kE + m] = ev[std::size_t(n) * kE + m] + acce;
-}
-
-// LayerNorm over 128 channels held two per lane (biased variance), the
-// lane's two channels having weights w0, w1 and biases b0, b1.
-// mode (NormMode): 0 affine LayerNorm; 1 RMSNorm without scale (no mean
-// removed; the caller passes w = 1, b = 0); 2 none (h = y = v, is = 1)
-__device__ __forceinline__ void wave_layer_norm_pair(double v0, double v1, double w0, double w1, double b0,
-                                                     double b1, double eps, int mode, double &y0, double &y1,
-                                                     double &h0, double &h1, double &is) {
-  const double mean = mode == 0 ? wave_sum(v0 + v1) / kF : 0.0;
-  const double d0 = v0 - mean, d1 = v1 - mean;
-  is = mode == 2 ? 1.0 : 1.0 / sqrt(wave_sum(d0 * d0 + d1 * d1) / kF + eps);
-  h0 = d0 * is;
-  h1 = d1 * is;
-  y0 = h0 * w0 + b0;
-  y1 = h1 * w1 + b1;
+  const std::size_t i = std::size_t(n) * kF + p0;
+  const double2 xv = ld2(x + i);
+  double h0, h1, is;
+  wave_normalise(xv.x + acc0, xv.y + acc1, eps, lnmode, h0, h1, is);
+  st2(n1hat + i, h0, h1);
+  if (lane == 0) n1is[n] = is;
+  if (evv) aev[std::size_t(n) * kE + m] = (ev ? ev[std::size_t(n) * kE + m] : 0.0) + acce;
 }
 
 // Attention forward messages, node-major, with the per-direction logits the
@@ -2206,10 +2082,8 @@ __global__ __launch_bounds__(256) void k_attn_msg(int N, const int *inc_off, con
                                                   const int *__restrict__ iother, const double *__restrict__ x,
                                                   const double *__restrict__ ev, const double *__restrict__ qkv,
                                                   const double *__restrict__ pY, const double *__restrict__ pfc,
-                                                  const double *__restrict__ palpha, const double *__restrict__ lnw,
-                                                  const double *__restrict__ lnb, double eps, int lnmode,
-                                                  double *__restrict__ n1, double *__restrict__ n1hat,
-                                                  double *__restrict__ n1is, double *__restrict__ act,
+                                                  const double *__restrict__ palpha, double eps, int lnmode,
+                                                  double *__restrict__ n1hat, double *__restrict__ n1is,
                                                   double *__restrict__ aev, const int *__restrict__ z,
                                                   const int *__restrict__ cls) {
   const int lane = threadIdx.x & 63;
@@ -2217,7 +2091,6 @@ __global__ __launch_bounds__(256) void k_attn_msg(int N, const int *inc_off, con
   if (n >= N) return;
   const int h = lane >> 4, t = lane & 15;
   const int p0 = 32 * h + 2 * t;
-  const int c0 = fpos(p0), c1 = c0 + 4;
   const bool evv = t < 2 * h + 3;
   const int m = evv ? ev_offset(h) + t : 0;
   const double par = slot_parity(h);
@@ -2239,240 +2112,302 @@ __global__ __launch_bounds__(256) void k_attn_msg(int N, const int *inc_off, con
     acc0 += A.d0; acc1 += A.d1; acce += A.de;
     if (two) { acc0 += B.d0; acc1 += B.d1; acce += B.de; }
   });
-  // the residual, then the post-attention block's LayerNorm 1 and the silu
-  // of it (the MLP input), with the whole node row in this wavefront
-  const std::size_t i = std::size_t(n) * kF;
-  double y0, y1, h0, h1, is;
-  wave_layer_norm_pair(x[i + c0] + acc0, x[i + c1] + acc1, lnw[c0], lnw[c1], lnb[c0], lnb[c1], eps, lnmode, y0, y1,
-                       h0, h1, is);
-  n1[i + c0] = y0;
-  n1[i + c1] = y1;
-  n1hat[i + c0] = h0;
-  n1hat[i + c1] = h1;
+  // the residual and its first normalisation, with the whole node row in
+  // this wavefront
+  const std::size_t i = std::size_t(n) * kF + p0;
+  const double2 xv = ld2(x + i);
+  double h0, h1, is;
+  wave_normalise(xv.x + acc0, xv.y + acc1, eps, lnmode, h0, h1, is);
+  st2(n1hat + i, h0, h1);
   if (lane == 0) n1is[n] = is;
-  act[i + c0] = silu(y0);
-  act[i + c1] = silu(y1);
-  if (evv) aev[std::size_t(n) * kE + m] = ev[std::size_t(n) * kE + m] + acce;
+  if (evv) aev[std::size_t(n) * kE + m] = (ev ? ev[std::size_t(n) * kE + m] : 0.0) + acce;
 }
-
-// LayerNorm over 128 channels held two per lane: channels lane and 64 + lane.
-__device__ __forceinline__ void wave_layer_norm(double v0, double v1, const double *w, const double *b,
-                                                double eps, int mode, int lane, double &y0, double &y1,
-                                                double &h0, double &h1, double &is) {
-  wave_layer_norm_pair(v0, v1, w[lane], w[64 + lane], b[lane], b[64 + lane], eps, mode, y0, y1, h0, h1, is);
-}
-
-// LN1 of the attention residual, and silu of it for the MLP input
-__global__ __launch_bounds__(256) void k_post1(int N, const double *ainv, const double *w, const double *b,
-                                               double eps, int mode, double *n1, double *n1hat, double *n1is,
-                                               double *act) {
-  const int lane = threadIdx.x & 63;
-  const int n = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (n >= N) return;
-  const std::size_t i = std::size_t(n) * kF;
-  double y0, y1, h0, h1, is;
-  wave_layer_norm(ainv[i + lane], ainv[i + 64 + lane], w, b, eps, mode, lane, y0, y1, h0, h1, is);
-  n1[i + lane] = y0; n1[i + 64 + lane] = y1;
-  n1hat[i + lane] = h0; n1hat[i + 64 + lane] = h1;
-  if (lane == 0) n1is[n] = is;
-  act[i + lane] = silu(y0);
-  act[i + 64 + lane] = silu(y1);
-}
-
 
 // The post-attention node chain of one block with every activation in MFMA
 // registers (kokkos_post_attention_block0.cpp:302-333):
+//   n1 = LN1 row (its normalised values n1hat times the affine weights),
 //   hpre = W1 silu(n1) + b1 (kept for the reverse), hid = silu(hpre),
 //   p = n1 + W2 hid + b2,
-//   t = Wint [p, inv(aev)] + bint (132 wide, kept), inv_l = sum_{m in l} aev_m^2 cg_m,
-//   x' = LN2(p + t[0:128]) (statistics kept), ev' = aev (1 + t[128 + slot]).
-// An MFMA output tile (rows 16 mt + 4 r + g of node j in lane j + 16 g,
-// register r) is the B operand of the next layer as it stands, so the layers
-// chain without memory round trips.
+//   t = Wint [p, inv(aev)] + bint (132 wide), inv_l = sum_{m in l} aev_m^2 cg_m,
+//   x' = LN2(p + t[0:128]) (statistics kept), ev' = aev (1 + gate[slot]),
+//   gate l = t[128 + l] (kept),
+// then what reads x' next: the following block's q k v q_ev k_ev rows (TAIL
+// 1), or the heads (TAIL 2; 3 with the C6 head): their hidden layer and the
+// per-atom energy, raw charge and ratios.
+//
+// One workgroup of eight wavefronts per 16 atoms: wavefront w owns output tile
+// w (16 of the 128 features) of every layer, and the layer inputs are
+// exchanged through LDS in MFMA operand order (chunk T of lane l at
+// buf[T][l]).  A tile of the chain is bound by its length (three dependent
+// layers and two row normalisations, each wavefront streaming its own weight
+// fragments from L2), so it is cut as short as the 16 x 16 tiles allow: a
+// wavefront's share is 26 fragments, kNodePF of them in flight.  The gate tile
+// (4 of 16 rows used) is formed from partial products, each wavefront taking
+// its own chunk of p, summed through LDS in wavefront order.  Node rows are
+// in the tile-transposed channel order (fpos), so a chunk is one 32-byte
+// vector per lane.  Two wavefronts per tile, four output tiles each, and the
+// projections, heads and row sums as launches of their own took 570 us per
+// evaluation at 22 atoms, 716 at 99, 1,216 at 3,000, 2,326 for 512 packed
+// molecules and 6.64 ms at 24,000; this form 443, 570, 1,046, 2,126 and 6.50.
 struct NodeChainArgs {
   const double *m1p, *m1bp, *m2p, *m2bp, *intp, *intbp;  // MFMA operand order
-  const double *int_cg, *ln2w, *ln2b, *exp2_256;
+  const double *int_cg, *ln1w, *ln1b, *ln2w, *ln2b;      // 128-wide vectors in fpos order
   double eps;
   int mode2;  // NormMode of the second position (RMSNorm, none: w = 1, b = 0 given)
 };
-// Two wavefronts per 16 atoms (four per block: two 16-atom tiles), so that a
-// 24k-atom system fills the chip: half h of a tile computes the output tiles
-// 4 h .. 4 h + 3 of each layer (and the gate tile 8 in half 0), and the layer inputs are exchanged through LDS in the operand
-// order (chunk T of lane l at buf[tile][T][l]).  LayerNorm 2's row sums are
-// combined across the halves through LDS as well.
-__global__ __launch_bounds__(256) void k_node_fwd(int N, const double *__restrict__ act,
-                                                   const double *__restrict__ n1, const double *__restrict__ aev,
-                                                   NodeChainArgs A, double *__restrict__ hpre,
-                                                   double *__restrict__ tout, double *__restrict__ xout,
-                                                   double *__restrict__ evout, double *__restrict__ pre2hat,
-                                                   double *__restrict__ pre2is) {
-  __shared__ double exp2_lds[256];
-  __shared__ v4d buf[2][8][64];         // one 16-atom tile's layer input, operand order (16 KB per tile)
-  __shared__ double stat[2][2][2][64];  // [tile][half][sum, sum of squares][lane]
-  if (threadIdx.x < 256) exp2_lds[threadIdx.x] = A.exp2_256[threadIdx.x];
-  const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
-  const int wl = threadIdx.x >> 6, tile = wl >> 1, h = wl & 1;
+struct HeadArgs {
+  const double *w1p, *w1tp, *b1p;  // hidden layer (HO x 128), its transpose and bias, MFMA operand order
+  const double *ew2, *qw2, *hkey, *ckey;  // output rows, 128 | 128 | 64 per element (| 64) units, fpos order
+  const double *escale, *eshift, *qemb, *hvshift, *hkey_c, *ckey_c, *cvshift;  // per element
+  double eb2, qb2;
+};
+struct HeadOut {
+  double *hhead;  // hidden pre-activations [N][HO], tiles in fpos order
+  double *eatom, *qraw, *heff, *hir, *c6eff, *c6r;
+};
+// Fragments in flight per wavefront, and wavefronts per SIMD (two workgroups
+// per CU): 6 and 4 measured best over sizes (4 and 4 within 0.3%; 8 and 4
+// spills; 8 or 12 and 2 cost 2% at 12,000 atoms and up).
+constexpr int kNodePF = 6;
+#define NODE_OCCUPANCY __launch_bounds__(512, 4)
+
+// sum over the four lane groups (every lane of a column ends with the total)
+__device__ __forceinline__ double column_sum(double v) {
+  v += __shfl_xor(v, 16, kWave);
+  return v + __shfl_xor(v, 32, kWave);
+}
+// the eight wavefronts' values of one column, in wavefront order
+__device__ __forceinline__ double sum8(const double (*part)[16], int j) {
+  double s = part[0][j];
+#pragma unroll
+  for (int w = 1; w < 8; ++w) s += part[w][j];
+  return s;
+}
+__device__ __forceinline__ double sum8(const double (*part)[64], int lane) {
+  double s = part[0][lane];
+#pragma unroll
+  for (int w = 1; w < 8; ++w) s += part[w][lane];
+  return s;
+}
+// sum over the channels of degree slot g of a row of 24: a_m b_m (cg_m)
+__device__ __forceinline__ double slot_sum(int g, const double *a, const double *b, const double *cg) {
+  const int lo = ev_offset(g), hi = lo + 2 * g + 3;
+  double s = 0.0;
+  for (int m = lo; m < hi; ++m) s += cg ? a[m] * b[m] * cg[m] : a[m] * b[m];
+  return s;
+}
+
+template <int TAIL>
+__global__ NODE_OCCUPANCY void k_node_fwd(int N, const double *__restrict__ n1hat,
+                                                  const double *__restrict__ aev, NodeChainArgs A, HeadArgs H,
+                                                  const double *__restrict__ qkvp, const int *__restrict__ z,
+                                                  double *__restrict__ hpre, double *__restrict__ gates,
+                                                  double *__restrict__ xout, double *__restrict__ evout,
+                                                  double *__restrict__ pre2hat, double *__restrict__ pre2is,
+                                                  double *__restrict__ qkv, HeadOut O) {
+  constexpr int HT = TAIL == 3 ? 24 : 20;  // tiles of the heads' hidden layer
+  __shared__ v4d bufA[8][64], bufB[8][64];
+  __shared__ double gpart[8][64], st1[8][16], st2[8][16];
+  __shared__ double hsum[TAIL >= 2 ? HT : 1][16];
+  const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4, w = threadIdx.x >> 6;
   // every wavefront runs to the end (the barriers); rows beyond N are clamped
-  const int n = blockIdx.x * 32 + tile * 16 + j;
+  const int n = blockIdx.x * 16 + j;
   const bool valid = n < N;
   const std::size_t nn = std::size_t(valid ? n : N - 1);
-  __syncthreads();
-  auto chunk = [&](const double *rows, int T) {
-    const double *r = rows + nn * kF + 16 * T + g;
-    return v4d{r[0], r[4], r[8], r[12]};
-  };
-  // stream: MLP-1 biases (4), per T the act chunk and 4 W1 fragments (40);
-  // MLP-2 biases (4), 8 x 4 W2 fragments (32), the 4 n1 chunks of the
-  // residual; the interaction biases (5: the 5th is the gate tile, used by
-  // half 0 only) and per T (9) 5 fragments
-  constexpr int P1 = 4 + 40, P2 = P1 + 4 + 32 + 4, NS = P2 + 5 + 45;
-  const int o0 = 4 * h;  // first output tile of this half
-  auto tmt = [&](int q) { return q < 4 ? o0 + q : 8; };  // interaction output tile q of this half
+  const int own = 16 * w + 4 * g;  // this lane's four channels of the wavefront's tile, fpos order
+  auto vec = [](const double *p) { return *reinterpret_cast<const v4d *>(p); };
+  // the stream of this wavefront
+  constexpr int L1 = 3, L2 = L1 + 9, G = L2 + 9, L3 = G + 3, LN = L3 + 10, TL = LN + 2;
+  constexpr int NS = TL + (TAIL == 1 ? 10 : TAIL >= 2 ? 27 : 0);
+  const int head = w >> 1;  // TAIL 1: this wavefront's head and half of its ten projection tiles
   auto load = [&](auto si) -> v4d {
     constexpr int s = decltype(si)::value;
-    if constexpr (s < 4) {
-      return tile_load(A.m1bp, o0 + s, lane);
-    } else if constexpr (s < P1) {
-      constexpr int T = (s - 4) / 5, u = (s - 4) % 5;
-      if constexpr (u == 0) return chunk(act, T);
-      else return wload(A.m1p, 8, o0 + u - 1, T, lane);
-    } else if constexpr (s < P1 + 4) {
-      return tile_load(A.m2bp, o0 + s - P1, lane);
-    } else if constexpr (s < P2 - 4) {
-      constexpr int i = s - P1 - 4;
-      return wload(A.m2p, 8, o0 + i % 4, i / 4, lane);
-    } else if constexpr (s < P2) {
-      return chunk(n1, o0 + s - (P2 - 4));
-    } else if constexpr (s < P2 + 5) {
-      return tile_load(A.intbp, tmt(s - P2), lane);
+    if constexpr (s == 0) return vec(n1hat + nn * kF + own);
+    else if constexpr (s == 1) return vec(A.ln1w + own);
+    else if constexpr (s == 2) return vec(A.ln1b + own);
+    else if constexpr (s == L1) return tile_load(A.m1bp, w, lane);
+    else if constexpr (s < L2) return wload(A.m1p, 8, w, s - L1 - 1, lane);
+    else if constexpr (s == L2) return tile_load(A.m2bp, w, lane);
+    else if constexpr (s < G) return wload(A.m2p, 8, w, s - L2 - 1, lane);
+    else if constexpr (s == G) return wload(A.intp, 9, 8, w, lane);
+    else if constexpr (s == G + 1) return wload(A.intp, 9, 8, 8, lane);
+    else if constexpr (s == G + 2) return tile_load(A.intbp, 8, lane);
+    else if constexpr (s == L3) return tile_load(A.intbp, w, lane);
+    else if constexpr (s < LN) return wload(A.intp, 9, w, s - L3 - 1, lane);
+    else if constexpr (s == LN) return vec(A.ln2w + own);
+    else if constexpr (s == LN + 1) return vec(A.ln2b + own);
+    else if constexpr (TAIL == 1) {
+      constexpr int T = (s - TL) / 5, q = (s - TL) % 5;
+      return wload(qkvp + std::size_t(head) * 160 * kHW, 2, 5 * (w & 1) + q, T, lane);
     } else {
-      constexpr int i = s - P2 - 5;
-      return wload(A.intp, 9, tmt(i % 5), i / 5, lane);
+      constexpr int u = (s - TL) / 9, e = (s - TL) % 9;
+      const int t = w + 8 * u < HT ? w + 8 * u : w;  // past the last tile: a valid address, not used
+      if constexpr (e == 0) return tile_load(H.b1p, t, lane);
+      else return wload(H.w1p, 8, t, e - 1, lane);
     }
   };
-  // two operands in flight measured best here (88 against 94 us with four)
-  Stream<NS, 2, decltype(load)> st(load);
+  Stream<NS, kNodePF, decltype(load)> st(load);
   st.prime();
-
-  double inv = 0.0;
-  {
-    const int lo = g == 0 ? 0 : (g == 1 ? 3 : (g == 2 ? 8 : 15));
-    const int hi = g == 0 ? 3 : (g == 1 ? 8 : (g == 2 ? 15 : 24));
-    for (int m = lo; m < hi; ++m) {
-      const double a = aev[nn * kE + m];
-      inv += a * a * A.int_cg[m];
-    }
-  }
-  const v4d inv4 = v4d{inv, 0.0, 0.0, 0.0};
-  v4d acc[5], pb[4], xT;
+  const double inv = slot_sum(g, aev + nn * kE, aev + nn * kE, A.int_cg);
+  const v4d zero = v4d{0.0, 0.0, 0.0, 0.0};
+  v4d n1, lw, p, acc, gp, pb, hh, tacc[5];
+  double mean = 0.0;
   st.run([&](auto si, const v4d &wv) {
     constexpr int s = decltype(si)::value;
-    if constexpr (s < 4) {
-      acc[s] = wv;
-    } else if constexpr (s < P1) {
-      constexpr int u = (s - 4) % 5;
-      if constexpr (u == 0) xT = wv;
-      else acc[u - 1] = mfma4(wv, xT, acc[u - 1]);
-      if constexpr (s == P1 - 1) {
-        // hpre (kept) and silu(hpre) into LDS for both halves
+    if constexpr (s == 0) {
+      n1 = wv;
+    } else if constexpr (s == 1) {
+      lw = wv;
+    } else if constexpr (s == 2) {
+      v4d a;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          v4d hd;
+      for (int r = 0; r < 4; ++r) {
+        n1[r] = n1[r] * lw[r] + wv[r];
+        a[r] = silu(n1[r]);
+      }
+      bufA[w][lane] = a;
+      __syncthreads();
+    } else if constexpr (s == L1 || s == L2 || s == L3) {
+      acc = wv;
+    } else if constexpr (s < L2) {
+      acc = mfma4(wv, bufA[s - L1 - 1][lane], acc);
+      if constexpr (s == L2 - 1) {
+        if (valid) *reinterpret_cast<v4d *>(hpre + nn * kF + own) = acc;
+        v4d a;
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            if (valid) hpre[nn * kF + 16 * (o0 + q) + 4 * r + g] = acc[q][r];
-            hd[r] = silu_tab(acc[q][r], exp2_lds);
-          }
-          buf[tile][o0 + q][lane] = hd;
-        }
+        for (int r = 0; r < 4; ++r) a[r] = silu(acc[r]);
+        bufB[w][lane] = a;
         __syncthreads();
       }
-    } else if constexpr (s < P1 + 4) {
-      acc[s - P1] = wv;
-    } else if constexpr (s < P2 - 4) {
-      constexpr int i = s - P1 - 4;
-      acc[i % 4] = mfma4(wv, buf[tile][i / 4][lane], acc[i % 4]);
-      if constexpr (s == P2 - 5) __syncthreads();  // every half has read the MLP-2 input
-    } else if constexpr (s < P2) {
-      constexpr int q = s - (P2 - 4);
-      pb[q] = acc[q] + wv;  // p = n1 + W2 hid + b2
-      buf[tile][o0 + q][lane] = pb[q];
-      if constexpr (q == 3) __syncthreads();
-    } else if constexpr (s < P2 + 5) {
-      acc[s - P2] = wv;
+    } else if constexpr (s < G) {
+      acc = mfma4(wv, bufB[s - L2 - 1][lane], acc);
+      if constexpr (s == G - 1) {
+        p = n1 + acc;
+        bufA[w][lane] = p;  // every wavefront has read the MLP input (the barrier above)
+      }
+    } else if constexpr (s == G) {
+      gp = mfma4(wv, p, zero);
+    } else if constexpr (s == G + 1) {
+      if (w == 0) gp = mfma(wv[0], inv, gp);
+    } else if constexpr (s == G + 2) {
+      gpart[w][lane] = w == 0 ? gp[0] + wv[0] : gp[0];
+      __syncthreads();
+    } else if constexpr (s < LN - 1) {
+      acc = mfma4(wv, bufA[s - L3 - 1][lane], acc);
+    } else if constexpr (s == LN - 1) {
+      acc = mfma(wv[0], inv, acc);  // the invariants: K rows 128 + g, zero beyond
+      // LayerNorm 2 of p + t over the row, the tiles' sums combined in LDS
+      pb = p + acc;
+      const double sum = column_sum((pb[0] + pb[1]) + (pb[2] + pb[3]));
+      if (g == 0) st1[w][j] = sum;
+      __syncthreads();
+      mean = A.mode2 == 0 ? sum8(st1, j) / kF : 0.0;
+      double var = 0.0;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const double d = pb[r] - mean;
+        var += d * d;
+      }
+      var = column_sum(var);
+      if (g == 0) st2[w][j] = var;
+      __syncthreads();
+      const double is = A.mode2 == 2 ? 1.0 : 1.0 / sqrt(sum8(st2, j) / kF + A.eps);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) hh[r] = (pb[r] - mean) * is;
+      if (valid) {
+        *reinterpret_cast<v4d *>(pre2hat + nn * kF + own) = hh;
+        if (w == 0 && g == 0) pre2is[nn] = is;
+        if (w < 6) {  // ev' = aev (1 + gate[slot]), channel g + 4 w
+          const int m = g + 4 * w;
+          evout[nn * kE + m] = aev[nn * kE + m] * (1.0 + sum8(gpart, j + 16 * degree_slot(m)));
+        } else if (w == 6) {
+          gates[nn * 4 + g] = sum8(gpart, lane);
+        }
+      }
+    } else if constexpr (s == LN) {
+      lw = wv;
+    } else if constexpr (s == LN + 1) {
+      v4d x;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) x[r] = hh[r] * lw[r] + wv[r];
+      if constexpr (TAIL < 2) {
+        if (valid) *reinterpret_cast<v4d *>(xout + nn * kF + own) = x;
+      }
+      if constexpr (TAIL > 0) {
+        bufB[w][lane] = x;  // every wavefront has read the MLP-2 input
+        __syncthreads();
+      }
+    } else if constexpr (TAIL == 1) {
+      constexpr int T = (s - TL) / 5, q = (s - TL) % 5;
+      tacc[q] = mfma4(wv, bufB[2 * head + T][lane], T == 0 ? zero : tacc[q]);
+      if constexpr (T == 1) {
+        // tile mt = 5 (w & 1) + q is projection mt / 2, channels 32 head +
+        // 16 (mt % 2) + [0, 16) of it
+        const int mt = 5 * (w & 1) + q;
+        if (valid)
+          *reinterpret_cast<v4d *>(qkv + nn * 640 + (mt >> 1) * kF + head * kHW + 16 * (mt & 1) + 4 * g) = tacc[q];
+      }
     } else {
-      constexpr int i = s - P2 - 5, T = i / 5, q = i % 5;
-      if (q < 4 || h == 0) {
-        if constexpr (T < 8) acc[q] = mfma4(wv, buf[tile][T][lane], acc[q]);
-        else acc[q] = mfma4(wv, inv4, acc[q]);
+      constexpr int u = (s - TL) / 9, e = (s - TL) % 9;
+      if constexpr (e == 0) acc = wv;
+      else acc = mfma4(wv, bufB[e - 1][lane], acc);
+      if constexpr (e == 8) {
+        const int t = w + 8 * u;
+        if (t < HT) {
+          if (valid) *reinterpret_cast<v4d *>(O.hhead + nn * (16 * HT) + 16 * t + 4 * g) = acc;
+          // the tile's share of its head's output: energy (t < 8), charge
+          // (t < 16), Hirshfeld (t < 20) and C6 logits
+          const int zz = z[nn];
+          const double *row = t < 8 ? H.ew2 + 16 * t
+                                    : (t < 16 ? H.qw2 + 16 * (t - 8)
+                                              : (t < 20 ? H.hkey + zz * kHH + 16 * (t - 16)
+                                                        : H.ckey + zz * kHH + 16 * (t - 20)));
+          const v4d r = vec(row + 4 * g);
+          const double v = (r[0] * silu(acc[0]) + r[1] * silu(acc[1])) + (r[2] * silu(acc[2]) + r[3] * silu(acc[3]));
+          const double sum = column_sum(v);
+          if (g == 0) hsum[t][j] = sum;
+        }
       }
     }
   });
-
-  // interaction output (kept); LayerNorm 2 of p + t over the row, the two
-  // halves' sums combined through LDS
-#pragma unroll
-  for (int q = 0; q < 5; ++q) {
-    if (q == 4 && h != 0) break;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int c = 16 * tmt(q) + 4 * r + g;
-      if (valid && c < kNI) tout[nn * kNI + c] = acc[q][r];
-    }
-  }
-  double sum = 0.0;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    pb[q] += acc[q];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) sum += pb[q][r];
-  }
-  sum += __shfl_xor(sum, 16, kWave);
-  sum += __shfl_xor(sum, 32, kWave);
-  stat[tile][h][0][lane] = sum;
-  __syncthreads();
-  const double mean = A.mode2 == 0 ? (stat[tile][0][0][lane] + stat[tile][1][0][lane]) / kF : 0.0;
-  double var = 0.0;
-#pragma unroll
-  for (int q = 0; q < 4; ++q)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const double d = pb[q][r] - mean;
-      var += d * d;
-    }
-  var += __shfl_xor(var, 16, kWave);
-  var += __shfl_xor(var, 32, kWave);
-  stat[tile][h][1][lane] = var;
-  __syncthreads();
-  const double is = A.mode2 == 2 ? 1.0 : 1.0 / sqrt((stat[tile][0][1][lane] + stat[tile][1][1][lane]) / kF + A.eps);
-  if (valid) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int c = 16 * (o0 + q) + 4 * r + g;
-        const double hh = (pb[q][r] - mean) * is;
-        pre2hat[nn * kF + c] = hh;
-        xout[nn * kF + c] = hh * A.ln2w[c] + A.ln2b[c];
-      }
-    if (h == 0 && g == 0) pre2is[nn] = is;
-  }
-  if (h == 0) {
-    // ev' = aev (1 + gate[slot]); gate l = t[128 + l] in lane j + 16 l of half 0
-    const double gate[4] = {__shfl(acc[4][0], j, kWave), __shfl(acc[4][0], j + 16, kWave),
-                            __shfl(acc[4][0], j + 32, kWave), __shfl(acc[4][0], j + 48, kWave)};
-    if (valid) {
-#pragma unroll
-      for (int k = 0; k < 6; ++k) {
-        const int m = g + 4 * k;
-        evout[nn * kE + m] = aev[nn * kE + m] * (1.0 + pick4(degree_slot(m), gate[0], gate[1], gate[2], gate[3]));
+  if constexpr (TAIL >= 2) {
+    // per-atom energy, raw charge, Hirshfeld (and C6) logit and ratio
+    // (kokkos_output_heads.cpp:108-180,341-451)
+    __syncthreads();
+    if (w == 0 && g < (TAIL == 3 ? 4 : 3) && valid) {
+      const int zz = z[nn];
+      const int t0 = g == 0 ? 0 : (g == 1 ? 8 : (g == 2 ? 16 : 20)), t1 = g == 0 ? 8 : (g == 1 ? 16 : (g == 2 ? 20 : 24));
+      double v = hsum[t0][j];
+      for (int t = t0 + 1; t < t1; ++t) v += hsum[t][j];
+      if (g == 0) {
+        O.eatom[nn] = (v + H.eb2) * H.escale[zz - 1] + H.eshift[zz - 1];
+      } else if (g == 1) {
+        O.qraw[nn] = v + H.qb2 + H.qemb[zz];
+      } else if (g == 2) {
+        // logit q_emb[z] . (W2 a + b2), contracted through the element's row
+        // u[z] = W2^T q_emb[z]; sqrt(64) = 8
+        const double ef = H.hvshift[zz] + (H.hkey_c[zz] + v) / 8.0;
+        O.heff[nn] = ef;
+        O.hir[nn] = fabs(ef);
+      } else {
+        const double ce = H.cvshift[zz] + (H.ckey_c[zz] + v) / 8.0;
+        O.c6eff[nn] = ce;
+        O.c6r[nn] = fabs(ce);
       }
     }
   }
 }
 
-// Reverse of the post-attention node chain, the adjoints in MFMA registers
-// (kokkos_post_attention_reverse.cpp:328-449):
+// Reverse of the node chain, the adjoints in MFMA registers
+// (kokkos_post_attention_reverse.cpp:328-449), starting from the adjoint gx of
+// the block's output x':
+//   SRC 0 (the last block; 2 with the C6 head): the heads' reverse, seeds
+//     energy 1, charge dE/dq - mean, Hirshfeld dE/dh (and dE/dc) through the
+//     hidden layer (kokkos_output_heads.cpp:493-581);
+//   SRC 1: the projections' reverse of the block above, gx = scale (base +
+//     sum_w W_w^T dqkv_w), base its attention-residual adjoint (gainv, which
+//     this kernel then overwrites row by row with its own).
+// Then
 //   LayerNorm 2 reverse: d = LN2^T gx, the adjoint of p and of t[0:128];
 //   t[128 + l] (gates): sum_{m in l} gev_m aev_m; aev: gev (1 + gate);
 //   interaction reverse: gcat = Wint^T gt; p += gcat[0:128];
@@ -2480,246 +2415,190 @@ __global__ __launch_bounds__(256) void k_node_fwd(int N, const double *__restric
 //   MLP reverse: ghid = (W2^T p) silu'(hpre), gact = W1^T ghid;
 //   LayerNorm 1 reverse of g = p + gact silu'(n1): the adjoint of the
 //   attention residual, gainv.
+// Eight wavefronts per 16 atoms as in k_node_fwd.  gev null: zero (the last
+// block's equivariant output is not read).
 struct NodeChainBwdArgs {
   const double *inttp, *m2tp, *m1tp;  // MFMA operand order (transposes)
-  const double *int_cg, *ln1w, *ln2w;
+  const double *int_cg, *ln1w, *ln1b, *ln2w;  // 128-wide vectors in fpos order
   int mode1, mode2;  // NormMode of the two positions: RMSNorm drops the mean term, none both
 };
-// Two wavefronts per 16 atoms (four per block: two 16-atom tiles): half h
-// owns the feature tiles 4 h .. 4 h + 3 of every 128-wide adjoint (and the
-// gate tile 8 in half 0); each layer's input adjoint is exchanged through LDS
-// in the operand order, and the LayerNorm row sums are combined across the
-// halves through LDS.
-__global__ __launch_bounds__(256) void k_node_bwd(int N, const double *__restrict__ gx,
-                                                   const double *__restrict__ gev, const double *__restrict__ t,
-                                                   const double *__restrict__ aev, const double *__restrict__ pre2hat,
-                                                   const double *__restrict__ pre2is, const double *__restrict__ hpre,
-                                                   const double *__restrict__ n1, const double *__restrict__ n1hat,
-                                                   const double *__restrict__ n1is, NodeChainBwdArgs A,
-                                                   double *__restrict__ gainv, double *__restrict__ gaev) {
-  __shared__ v4d buf[2][8][64];         // one tile's layer-input adjoint, operand order (16 KB per tile)
-  __shared__ double stat[2][2][2][64];  // [tile][half][two sums][lane]
-  const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
-  const int wl = threadIdx.x >> 6, tile = wl >> 1, h = wl & 1;
-  const int n = blockIdx.x * 32 + tile * 16 + j;
+struct HeadSeeds {
+  const double *hhead, *qseed, *dh, *heff, *dc, *c6eff;
+};
+template <int SRC>
+__global__ NODE_OCCUPANCY void k_node_bwd(int N, const double *__restrict__ gqkv,
+                                                  const double *__restrict__ qkvtp, double scale, HeadArgs H,
+                                                  HeadSeeds S, const int *__restrict__ z,
+                                                  const double *__restrict__ gev, const double *__restrict__ gates,
+                                                  const double *__restrict__ aev, const double *__restrict__ pre2hat,
+                                                  const double *__restrict__ pre2is, const double *__restrict__ hpre,
+                                                  const double *__restrict__ n1hat, const double *__restrict__ n1is,
+                                                  NodeChainBwdArgs A, double *gainv, double *__restrict__ gaev) {
+  constexpr int HT = SRC == 2 ? 24 : 20;
+  constexpr bool HEADS = SRC != 1;
+  __shared__ v4d buf[HEADS ? HT : 16][64];  // chunks 0..7 and 8..15: the two layer-input buffers
+  __shared__ double gpart[8][64], st[4][8][16];
+  const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4, w = threadIdx.x >> 6;
+  const int n = blockIdx.x * 16 + j;
   const bool valid = n < N;
   const std::size_t nn = std::size_t(valid ? n : N - 1);
-  const int o0 = 4 * h;
-  auto chunk = [&](const double *rows, int T) {
-    const double *r = rows + nn * kF + 16 * T + g;
-    return v4d{r[0], r[4], r[8], r[12]};
-  };
-  auto tmt = [&](int q) { return q < 4 ? o0 + q : 8; };
-  // both halves' two sums of a row, combined (one barrier)
-  auto row_sums = [&](double a, double b, double &ta, double &tb) {
-    a += __shfl_xor(a, 16, kWave);
-    a += __shfl_xor(a, 32, kWave);
-    b += __shfl_xor(b, 16, kWave);
-    b += __shfl_xor(b, 32, kWave);
-    stat[tile][h][0][lane] = a;
-    stat[tile][h][1][lane] = b;
-    __syncthreads();
-    ta = stat[tile][0][0][lane] + stat[tile][1][0][lane];
-    tb = stat[tile][0][1][lane] + stat[tile][1][1][lane];
-  };
-  // stream: the 4 gx and 4 LN2-normalised chunks of this half; Wint^T for
-  // the 5 output tiles (the 5th, the gate tile, for half 0) over 9 K chunks;
-  // W2^T for 4 tiles over 8 chunks and the 4 hpre chunks; W1^T likewise and
-  // the 4 n1 and 4 LN1-normalised chunks
-  constexpr int SA = 8, SB = SA + 45, SD = SB + 32 + 4, NS = SD + 32 + 8;
+  const int own = 16 * w + 4 * g;
+  auto vec = [](const double *p) { return *reinterpret_cast<const v4d *>(p); };
+  const int head = w >> 1;
+  constexpr int X = HEADS ? HT : 21;  // entries of gx
+  constexpr int L3 = X + 2, G = L3, LB = G + 2, L2 = LB + 9, L1 = L2 + 9, LN = L1 + 8, NS = LN + 3;
   auto load = [&](auto si) -> v4d {
     constexpr int s = decltype(si)::value;
-    if constexpr (s < 4) return chunk(gx, o0 + s);
-    else if constexpr (s < SA) return chunk(pre2hat, o0 + s - 4);
-    else if constexpr (s < SB) return wload(A.inttp, 9, tmt((s - SA) % 5), (s - SA) / 5, lane);
-    else if constexpr (s < SD - 4) return wload(A.m2tp, 8, o0 + (s - SB) % 4, (s - SB) / 4, lane);
-    else if constexpr (s < SD) return chunk(hpre, o0 + s - (SD - 4));
-    else if constexpr (s < NS - 8) return wload(A.m1tp, 8, o0 + (s - SD) % 4, (s - SD) / 4, lane);
-    else if constexpr (s < NS - 4) return chunk(n1, o0 + s - (NS - 8));
-    else return chunk(n1hat, o0 + s - (NS - 4));
+    if constexpr (s < X) {
+      if constexpr (HEADS) return wload(H.w1tp, HT, w, s, lane);
+      else if constexpr (s == 20) return vec(gainv + nn * kF + own);
+      else if constexpr ((s & 1) == 0) {
+        // K entries of chunk T: projection T / 2, channels 32 head + 16 (T % 2) + [0, 16)
+        constexpr int T = s / 2;
+        return vec(gqkv + nn * 640 + (T >> 1) * kF + head * kHW + 16 * (T & 1) + 4 * g);
+      } else {
+        return wload(qkvtp + std::size_t(head) * kHW * 160, 10, w & 1, s / 2, lane);
+      }
+    } else if constexpr (s == X) return vec(A.ln2w + own);
+    else if constexpr (s == X + 1) return vec(pre2hat + nn * kF + own);
+    else if constexpr (s == G) return wload(A.inttp, 9, 8, w, lane);
+    else if constexpr (s == G + 1) return wload(A.inttp, 9, 8, 8, lane);
+    else if constexpr (s < L2) return wload(A.inttp, 9, w, s - LB, lane);
+    else if constexpr (s < L1 - 1) return wload(A.m2tp, 8, w, s - L2, lane);
+    else if constexpr (s == L1 - 1) return vec(hpre + nn * kF + own);
+    else if constexpr (s < LN) return wload(A.m1tp, 8, w, s - L1, lane);
+    else if constexpr (s == LN) return vec(n1hat + nn * kF + own);
+    else if constexpr (s == LN + 1) return vec(A.ln1w + own);
+    else return vec(A.ln1b + own);
   };
-  Stream<NS, kFilterPF, decltype(load)> st(load);
-  st.prime();
+  Stream<NS, kNodePF, decltype(load)> stream(load);
+  stream.prime();
 
-  const double *ger = gev + nn * kE, *aer = aev + nn * kE;
-  double ga[6] = {0, 0, 0, 0, 0, 0};
-  if (h == 0) {
-    const double gates[4] = {t[nn * kNI + kF], t[nn * kNI + kF + 1], t[nn * kNI + kF + 2], t[nn * kNI + kF + 3]};
-#pragma unroll
-    for (int k = 0; k < 6; ++k) {
-      const int m = g + 4 * k;
-      ga[k] = ger[m] * (1.0 + pick4(degree_slot(m), gates[0], gates[1], gates[2], gates[3]));
-    }
-  }
-  double gsum = 0.0;
-  {
-    const int lo = g == 0 ? 0 : (g == 1 ? 3 : (g == 2 ? 8 : 15));
-    const int hi = g == 0 ? 3 : (g == 1 ? 8 : (g == 2 ? 15 : 24));
-    for (int m = lo; m < hi; ++m) gsum += ger[m] * aer[m];
-  }
-  const v4d gt8 = v4d{gsum, 0.0, 0.0, 0.0};
+  const double *ger = gev ? gev + nn * kE : nullptr, *aer = aev + nn * kE;
+  const double gsum = ger ? slot_sum(g, ger, aer, nullptr) : 0.0;
   const double is2 = pre2is[nn], is1 = n1is[nn];
-
-  v4d d[4], acc[5], hat[4];
-  double mg = 0.0, mgx = 0.0;
-  st.run([&](auto si, const v4d &wv) {
-    constexpr int s = decltype(si)::value;
-    if constexpr (s < 4) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) d[s][r] = wv[r] * A.ln2w[16 * (o0 + s) + 4 * r + g];
-    } else if constexpr (s < SA) {
-      constexpr int q = s - 4;
-      hat[q] = wv;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        mg += d[q][r];
-        mgx += d[q][r] * wv[r];
-      }
-      if constexpr (q == 3) {
-        // LayerNorm 2 reverse; the adjoint of p and t[0:128] into LDS
-        double tm, tx;
-        row_sums(mg, mgx, tm, tx);
-        tm = A.mode2 == 0 ? tm / kF : 0.0;
-        tx = A.mode2 == 2 ? 0.0 : tx / kF;
-#pragma unroll
-        for (int q2 = 0; q2 < 4; ++q2) {
-#pragma unroll
-          for (int r = 0; r < 4; ++r) d[q2][r] = is2 * (d[q2][r] - tm - hat[q2][r] * tx);
-          buf[tile][o0 + q2][lane] = d[q2];
-        }
-#pragma unroll
-        for (int q2 = 0; q2 < 5; ++q2) acc[q2] = v4d{0.0, 0.0, 0.0, 0.0};
-        __syncthreads();
-      }
-    } else if constexpr (s < SB) {
-      // gcat = Wint^T [d, gate adjoints]
-      constexpr int i = s - SA, T = i / 5, q = i % 5;
-      if (q < 4 || h == 0) {
-        if constexpr (T < 8) acc[q] = mfma4(wv, buf[tile][T][lane], acc[q]);
-        else acc[q] = mfma4(wv, gt8, acc[q]);
-      }
-      if constexpr (s == SB - 1) {
-        // p += gcat[own]; the aev adjoint gains 2 aev cg gcat[128 + slot]
-        if (h == 0) {
-          const double gc[4] = {__shfl(acc[4][0], j, kWave), __shfl(acc[4][0], j + 16, kWave),
-                                __shfl(acc[4][0], j + 32, kWave), __shfl(acc[4][0], j + 48, kWave)};
-#pragma unroll
-          for (int k = 0; k < 6; ++k) {
-            const int m = g + 4 * k;
-            ga[k] += pick4(degree_slot(m), gc[0], gc[1], gc[2], gc[3]) * 2.0 * aer[m] * A.int_cg[m];
-          }
-        }
-        __syncthreads();  // every half has read d
-#pragma unroll
-        for (int q2 = 0; q2 < 4; ++q2) {
-          d[q2] += acc[q2];
-          buf[tile][o0 + q2][lane] = d[q2];
-          acc[q2] = v4d{0.0, 0.0, 0.0, 0.0};
-        }
-        __syncthreads();
-      }
-    } else if constexpr (s < SD - 4) {
-      // W2^T p
-      constexpr int i = s - SB;
-      acc[i % 4] = mfma4(wv, buf[tile][i / 4][lane], acc[i % 4]);
-    } else if constexpr (s < SD) {
-      // ghid = (W2^T p) silu'(hpre), own tiles
-      constexpr int q = s - (SD - 4);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) hat[q][r] = acc[q][r] * silu_prime(wv[r]);
-      if constexpr (q == 3) {
-        __syncthreads();  // every half has read p
-#pragma unroll
-        for (int q2 = 0; q2 < 4; ++q2) {
-          buf[tile][o0 + q2][lane] = hat[q2];
-          acc[q2] = v4d{0.0, 0.0, 0.0, 0.0};
-        }
-        __syncthreads();
-      }
-    } else if constexpr (s < NS - 8) {
-      // gact = W1^T ghid
-      constexpr int i = s - SD;
-      acc[i % 4] = mfma4(wv, buf[tile][i / 4][lane], acc[i % 4]);
-    } else if constexpr (s < NS - 4) {
-      // g = p + gact silu'(n1), then gh = g * w1
-      constexpr int q = s - (NS - 8);
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        acc[q][r] = (d[q][r] + acc[q][r] * silu_prime(wv[r])) * A.ln1w[16 * (o0 + q) + 4 * r + g];
-    } else {
-      hat[s - (NS - 4)] = wv;  // LayerNorm 1 normalised input
+  if constexpr (HEADS) {
+    // the adjoints of the heads' hidden pre-activations, tiles w, w + 8, w + 16
+    const int zz = z[nn];
+    const double es = H.escale[zz - 1], qs = S.qseed[nn];
+    const double ef = S.heff[nn], hs = S.dh[nn] * (ef > 0.0 ? 1.0 : (ef < 0.0 ? -1.0 : 0.0)) / 8.0;
+    double cs = 0.0;
+    if constexpr (SRC == 2) {
+      const double ce = S.c6eff[nn];
+      cs = S.dc[nn] * (ce > 0.0 ? 1.0 : (ce < 0.0 ? -1.0 : 0.0)) / 8.0;
     }
-  });
-
-  // LayerNorm 1 reverse
-  double m1 = 0.0, m1x = 0.0;
 #pragma unroll
-  for (int q = 0; q < 4; ++q)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      m1 += acc[q][r];
-      m1x += acc[q][r] * hat[q][r];
-    }
-  double tm, tx;
-  row_sums(m1, m1x, tm, tx);
-  tm = A.mode1 == 0 ? tm / kF : 0.0;
-  tx = A.mode1 == 2 ? 0.0 : tx / kF;
-  if (valid) {
-    // tile-transposed channel order (fpos): channels 16 T + g + 4 r, r = 0..3,
-    // of this lane are one 32-byte vector at 16 T + 4 g
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
+    for (int u = 0; u < 3; ++u) {
+      const int t = w + 8 * u;
+      if (t >= HT) break;
+      const double *row = u == 0 ? H.ew2 + 16 * t
+                                 : (u == 1 ? H.qw2 + 16 * (t - 8)
+                                           : (t < 20 ? H.hkey + zz * kHH + 16 * (t - 16)
+                                                     : H.ckey + zz * kHH + 16 * (t - 20)));
+      const double seed = u == 0 ? es : (u == 1 ? qs : (t < 20 ? hs : cs));
+      const v4d r = vec(row + 4 * g), pre = vec(S.hhead + nn * (16 * HT) + 16 * t + 4 * g);
       v4d out;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) out[r] = is1 * (acc[q][r] - tm - hat[q][r] * tx);
-      *reinterpret_cast<v4d *>(gainv + nn * kF + 16 * (o0 + q) + 4 * g) = out;
+      for (int q = 0; q < 4; ++q) out[q] = seed * r[q] * silu_prime(pre[q]);
+      buf[t][lane] = out;
     }
-    if (h == 0) {
-#pragma unroll
-      for (int k = 0; k < 6; ++k) gaev[nn * kE + g + 4 * k] = ga[k];
-    }
+    __syncthreads();
   }
+  const v4d zero = v4d{0.0, 0.0, 0.0, 0.0};
+  v4d acc = zero, hold, d, hat, p, gp, n1;
+  stream.run([&](auto si, const v4d &wv) {
+    constexpr int s = decltype(si)::value;
+    if constexpr (s < X) {
+      if constexpr (HEADS) {
+        acc = mfma4(wv, buf[s][lane], acc);
+      } else if constexpr (s == 20) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[r] = scale * (wv[r] + acc[r]);
+      } else if constexpr ((s & 1) == 0) {
+        hold = wv;
+      } else {
+        acc = mfma4(wv, hold, acc);
+      }
+    } else if constexpr (s == X) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) d[r] = acc[r] * wv[r];
+    } else if constexpr (s == X + 1) {
+      // LayerNorm 2 reverse; the adjoint of p and t[0:128] into LDS
+      const double a = column_sum((d[0] + d[1]) + (d[2] + d[3]));
+      const double b = column_sum((d[0] * wv[0] + d[1] * wv[1]) + (d[2] * wv[2] + d[3] * wv[3]));
+      if (g == 0) {
+        st[0][w][j] = a;
+        st[1][w][j] = b;
+      }
+      __syncthreads();
+      const double tm = A.mode2 == 0 ? sum8(st[0], j) / kF : 0.0;
+      const double tx = A.mode2 == 2 ? 0.0 : sum8(st[1], j) / kF;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) d[r] = is2 * (d[r] - tm - wv[r] * tx);
+      buf[w][lane] = d;
+    } else if constexpr (s == G) {
+      gp = mfma4(wv, d, zero);  // this chunk's share of the gate rows of gcat
+    } else if constexpr (s == G + 1) {
+      if (w == 0) gp = mfma(wv[0], gsum, gp);
+      gpart[w][lane] = gp[0];
+      __syncthreads();
+    } else if constexpr (s < L2) {
+      // gcat = Wint^T [d, gate adjoints]
+      if constexpr (s - LB < 8) acc = mfma4(wv, buf[s - LB][lane], s == LB ? zero : acc);
+      else acc = mfma(wv[0], gsum, acc);
+      if constexpr (s == L2 - 1) {
+        p = d + acc;
+        buf[8 + w][lane] = p;
+        __syncthreads();
+      }
+    } else if constexpr (s < L1 - 1) {
+      acc = mfma4(wv, buf[8 + s - L2][lane], s == L2 ? zero : acc);  // W2^T p
+    } else if constexpr (s == L1 - 1) {
+      v4d a;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) a[r] = acc[r] * silu_prime(wv[r]);
+      buf[w][lane] = a;  // every wavefront has read d
+      __syncthreads();
+    } else if constexpr (s < LN) {
+      acc = mfma4(wv, buf[s - L1][lane], s == L1 ? zero : acc);  // W1^T ghid
+    } else if constexpr (s == LN) {
+      hat = wv;
+    } else if constexpr (s == LN + 1) {
+      hold = wv;
+    } else {
+      // g = p + gact silu'(n1), then LayerNorm 1 reverse
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        n1[r] = hat[r] * hold[r] + wv[r];
+        acc[r] = (p[r] + acc[r] * silu_prime(n1[r])) * hold[r];
+      }
+      const double a = column_sum((acc[0] + acc[1]) + (acc[2] + acc[3]));
+      const double b = column_sum((acc[0] * hat[0] + acc[1] * hat[1]) + (acc[2] * hat[2] + acc[3] * hat[3]));
+      if (g == 0) {
+        st[2][w][j] = a;
+        st[3][w][j] = b;
+      }
+      __syncthreads();
+      const double tm = A.mode1 == 0 ? sum8(st[2], j) / kF : 0.0;
+      const double tx = A.mode1 == 2 ? 0.0 : sum8(st[3], j) / kF;
+      if (valid) {
+        v4d out;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) out[r] = is1 * (acc[r] - tm - hat[r] * tx);
+        *reinterpret_cast<v4d *>(gainv + nn * kF + own) = out;
+        if (w < 6) {
+          // aev: gev (1 + gate) + 2 aev cg gcat[128 + slot], channel g + 4 w
+          const int m = g + 4 * w, sl = degree_slot(m);
+          const double gc = sum8(gpart, j + 16 * sl);
+          const double e = ger ? ger[m] * (1.0 + gates[nn * 4 + sl]) : 0.0;
+          gaev[nn * kE + m] = e + gc * 2.0 * aer[m] * A.int_cg[m];
+        }
+      }
+    }
+  });
 }
 
 // ---------------------------------------------------------------- heads
-struct HeadArgs {
-  const double *ew2, *qw2, *escale, *eshift, *qemb, *hqemb, *hvshift, *hkey_bwd, *hkey_c;
-  double eb2, qb2;
-  const double *ckey_bwd, *ckey_c, *cvshift;  // C6 ratio head (null: none); its hidden units at 320
-  int ho;                                     // head activation row width (320, or 384 with the C6 head)
-};
-
-// energy, raw charge, Hirshfeld key and ratio (kokkos_output_heads.cpp:137-176,341-451)
-// (and, with the C6 head, its logit and ratio: the same form as Hirshfeld's,
-// kokkos_output_heads.cpp:108-180)
-__global__ __launch_bounds__(256) void k_heads(int N, const int *z, const double *act, HeadArgs H,
-                                               double *eatom, double *qraw, double *heff, double *hir,
-                                               double *c6eff, double *c6r) {
-  const int lane = threadIdx.x & 63;
-  const int n = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (n >= N) return;
-  const double *a = act + std::size_t(n) * H.ho;
-  const int zz = z[n];
-  const double e = wave_sum(H.ew2[lane] * a[lane] + H.ew2[64 + lane] * a[64 + lane]);
-  const double q = wave_sum(H.qw2[lane] * a[128 + lane] + H.qw2[64 + lane] * a[192 + lane]);
-  // Hirshfeld logit q_emb[z] . (W2 a + b2), contracted through the element's
-  // row u[z] = W2^T q_emb[z]
-  const double qk = H.hkey_c[zz] + wave_sum(H.hkey_bwd[zz * kHH + lane] * a[256 + lane]);
-  const double ck = H.ckey_bwd ? H.ckey_c[zz] + wave_sum(H.ckey_bwd[zz * kHH + lane] * a[320 + lane]) : 0.0;
-  if (lane == 0) {
-    eatom[n] = (e + H.eb2) * H.escale[zz - 1] + H.eshift[zz - 1];
-    qraw[n] = q + H.qb2 + H.qemb[zz];
-    const double ef = H.hvshift[zz] + qk / 8.0;  // sqrt(64)
-    heff[n] = ef;
-    hir[n] = fabs(ef);
-    if (H.ckey_bwd) {
-      const double ce = H.cvshift[zz] + ck / 8.0;
-      c6eff[n] = ce;
-      c6r[n] = fabs(ce);
-    }
-  }
-}
-
 // per-image mean removal: out = in + (target - sum_image(in)) / count  (sign = +1)
 // or out = in - mean_image(in) (target ignored, sign = -1).  One block per image.
 __global__ __launch_bounds__(1024) void k_image_center(const std::int64_t *img_off, const double *target,
@@ -2737,35 +2616,6 @@ __global__ __launch_bounds__(1024) void k_image_center(const std::int64_t *img_o
   const double cnt = double(hi - lo);
   const double shift = mode == 0 ? (target[blockIdx.x] - part[0]) / cnt : -part[0] / cnt;
   for (std::int64_t i = lo + threadIdx.x; i < hi; i += 1024) out[i] = in[i] + shift;
-}
-
-// seeds -> d/d(x_final): energy 1, charge (dE/dq - mean), Hirshfeld dE/dh
-// (and dE/dc of the C6 head into its hidden units)
-__global__ __launch_bounds__(256) void k_heads_bwd(int N, const int *z, const double *pre, const double *qseed,
-                                                   const double *dh, const double *heff, const double *dc,
-                                                   const double *c6eff, HeadArgs H, double *ghead) {
-  const int lane = threadIdx.x & 63;
-  const int n = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (n >= N) return;
-  const double *pr = pre + std::size_t(n) * H.ho;
-  double *g = ghead + std::size_t(n) * H.ho;
-  const int zz = z[n];
-  const double sc = H.escale[zz - 1];
-  g[lane] = sc * H.ew2[lane] * silu_prime(pr[lane]);
-  g[64 + lane] = sc * H.ew2[64 + lane] * silu_prime(pr[64 + lane]);
-  const double qs = qseed[n];
-  g[128 + lane] = qs * H.qw2[lane] * silu_prime(pr[128 + lane]);
-  g[192 + lane] = qs * H.qw2[64 + lane] * silu_prime(pr[192 + lane]);
-  const double ef = heff[n];
-  const double sg = ef > 0.0 ? 1.0 : (ef < 0.0 ? -1.0 : 0.0);
-  const double hs = dh[n] * sg / 8.0;
-  // ghh[i] = sum_j hw2[j][i] gk[j] with gk[j] = hs * hqemb[z][j] = hs * u[z][i]
-  g[256 + lane] = hs * H.hkey_bwd[zz * kHH + lane] * silu_prime(pr[256 + lane]);
-  if (H.ckey_bwd) {
-    const double ce = c6eff[n];
-    const double cs = dc[n] * (ce > 0.0 ? 1.0 : (ce < 0.0 ? -1.0 : 0.0)) / 8.0;
-    g[320 + lane] = cs * H.ckey_bwd[zz * kHH + lane] * silu_prime(pr[320 + lane]);
-  }
 }
 
 // ---------------------------------------------------------------- long range
@@ -3381,6 +3231,14 @@ std::vector<double> bias_acc(const std::vector<double> &b, std::size_t M) {
   return p;
 }
 
+// Rows of 128 (64) channels in the tile-transposed order of the node rows
+// (fpos: a 4 x 4 transpose inside each run of 16).
+static std::vector<double> tile_order(const std::vector<double> &v) {
+  std::vector<double> t(v.size());
+  for (std::size_t i = 0; i < v.size(); ++i) t[(i & ~std::size_t(127)) + fpos(int(i & 127))] = v[i];
+  return t;
+}
+
 std::vector<double> permute_mfma(const std::vector<double> &w, std::size_t M, std::size_t K) {
   const std::size_t MT = (M + 15) / 16;
   if (K == 4) {
@@ -3540,24 +3398,18 @@ Evaluator::Evaluator(std::shared_ptr<Model> model, int device) : model_(std::mov
     // the same kernels with w = 1, b = 0
     const std::vector<double> ones(F, 1.0), zeros(F, 0.0);
     const bool ln1 = a.norm1 == NormMode::Layer, ln2 = a.norm2 == NormMode::Layer;
-    B.ln1w = up(ln1 ? m.f64(p + "layer_norm_inv_1.weight", {F}) : ones);
-    B.ln1b = up(ln1 ? m.f64(p + "layer_norm_inv_1.bias", {F}) : zeros);
-    B.ln2w = up(ln2 ? m.f64(p + "layer_norm_inv_2.weight", {F}) : ones);
-    B.ln2b = up(ln2 ? m.f64(p + "layer_norm_inv_2.bias", {F}) : zeros);
+    B.ln1w = up(ln1 ? tile_order(m.f64(p + "layer_norm_inv_1.weight", {F})) : ones);
+    B.ln1b = up(ln1 ? tile_order(m.f64(p + "layer_norm_inv_1.bias", {F})) : zeros);
+    B.ln2w = up(ln2 ? tile_order(m.f64(p + "layer_norm_inv_2.weight", {F})) : ones);
+    B.ln2b = up(ln2 ? tile_order(m.f64(p + "layer_norm_inv_2.bias", {F})) : zeros);
     const auto m1 = m.f64(p + "mlp_1.1.weight", {F, F}), m2 = m.f64(p + "mlp_1.3.weight", {F, F});
-    B.m1w = up(m1); B.m1t = up(transpose(m1, F, F));
-    B.m2w = up(m2); B.m2t = up(transpose(m2, F, F));
     B.m1p = up(permute_mfma(m1, F, F)); B.m2p = up(permute_mfma(m2, F, F));
     B.m1tp = up(permute_mfma(transpose(m1, F, F), F, F)); B.m2tp = up(permute_mfma(transpose(m2, F, F), F, F));
-    B.m1b = up(m.f64(p + "mlp_1.1.bias", {F}));
-    B.m2b = up(m.f64(p + "mlp_1.3.bias", {F}));
     B.m1bp = up(bias_acc(m.f64(p + "mlp_1.1.bias", {F}), F));
     B.m2bp = up(bias_acc(m.f64(p + "mlp_1.3.bias", {F}), F));
     const auto iw = m.f64(p + "interaction_block.linear_layer.weight", {NI, NI});
-    B.intw = up(iw); B.intt = up(transpose(iw, NI, NI));
     B.intp = up(permute_mfma(iw, NI, NI));
     B.inttp = up(permute_mfma(transpose(iw, NI, NI), NI, NI));
-    B.intb = up(m.f64(p + "interaction_block.linear_layer.bias", {NI}));
     B.intbp = up(bias_acc(m.f64(p + "interaction_block.linear_layer.bias", {NI}), NI));
   }
   // block 0's radial hidden layers as piecewise polynomials (radial tables),
@@ -3660,17 +3512,14 @@ Evaluator::Evaluator(std::shared_ptr<Model> model, int device) : model_(std::mov
     }
     const int HO = c6_ ? 384 : 320;
     hw_.ho = HO;
-    hw_.w1 = up(w1);
-    hw_.w1t = up(transpose(w1, HO, F));
     hw_.w1p = up(permute_mfma(w1, HO, F));
     hw_.w1tp = up(permute_mfma(transpose(w1, HO, F), F, HO));
-    hw_.b1 = up(b1);
     hw_.b1p = up(bias_acc(b1, HO));
-    hw_.ew2 = up(m.f64(e + "final_layer.weight", {1, F}));
+    hw_.ew2 = up(tile_order(m.f64(e + "final_layer.weight", {1, F})));
     hw_.eb2 = m.f64(e + "final_layer.bias", {1})[0];
     hw_.escale = up(m.f64(e + "energy_scales.weight", {1, 118}));
     hw_.eshift = up(m.f64(e + "energy_shifts", {118}));
-    hw_.qw2 = up(m.f64(q + "transform_inv_features.2.weight", {1, F}));
+    hw_.qw2 = up(tile_order(m.f64(q + "transform_inv_features.2.weight", {1, F})));
     hw_.qb2 = m.f64(q + "transform_inv_features.2.bias", {1})[0];
     hw_.qemb = up(m.f64(q + "atomic_embedding.weight", {100, 1}));
     // reverse of a ratio head's key layer seeded by the element's query:
@@ -3690,12 +3539,11 @@ Evaluator::Evaluator(std::shared_ptr<Model> model, int device) : model_(std::mov
         }
         for (std::size_t j = 0; j < HH; ++j) c[zz] += qe[zz * HH + j] * b2[j];
       }
-      kbwd = up(u);
+      kbwd = up(tile_order(u));
       kc = up(c);
       vsh = up(m.f64(pre + "v_shift_embedding.weight", {100, 1}));
-      return qe;
     };
-    hw_.hqemb = up(ratio_head(h, hw_.hkey_bwd, hw_.hkey_c, hw_.hvshift));
+    ratio_head(h, hw_.hkey_bwd, hw_.hkey_c, hw_.hvshift);
     hw_.ckey_bwd = hw_.ckey_c = hw_.cvshift = nullptr;
     if (c6_) ratio_head(c6h, hw_.ckey_bwd, hw_.ckey_c, hw_.cvshift);
     const auto bb = m.f64("model.radial_embedding.radial_basis_fn.b", {R});
@@ -3754,15 +3602,15 @@ Evaluator::Evaluator(std::shared_ptr<Model> model, int device) : model_(std::mov
   lr_.inv_w_disp = 1.0 / (lr_.cutoff - lr_.cuton_disp);
 
   z_ = buf("z"); x0_ = buf("x0"); img_of_node_ = buf("img"); img_off_ = buf("img_off"); img_q_ = buf("img_q");
-  xs_ = buf("xs"); evs_ = buf("evs"); qkv_ = buf("qkv"); aev_ = buf("aev"); n1_ = buf("n1");
-  n1hat_ = buf("n1hat"); n1is_ = buf("n1is"); hpre_ = buf("hpre"); tout_ = buf("tout");
-  pre2hat_ = buf("pre2hat"); pre2is_ = buf("pre2is"); ainv_ = buf("ainv"); act_ = buf("act");
+  xs_ = buf("xs"); evs_ = buf("evs"); qkv_ = buf("qkv"); aev_ = buf("aev"); 
+  n1hat_ = buf("n1hat"); n1is_ = buf("n1is"); hpre_ = buf("hpre"); gates_ = buf("gates");
+  pre2hat_ = buf("pre2hat"); pre2is_ = buf("pre2is"); 
   hhead_ = buf("hhead");
   heff_ = buf("heff"); eatom_ = buf("eatom"); qraw_ = buf("qraw"); q_ = buf("q"); hir_ = buf("hir");
   qseed_ = buf("qseed"); elr_ = buf("elr"); dq_ = buf("dq"); dh_ = buf("dh"); flr_ = buf("flr");
-  vlr_ = buf("vlr"); elr_parts_ = buf("elr_parts"); ezbl_ = buf("ezbl"); gx_ = buf("gx");
+  vlr_ = buf("vlr"); elr_parts_ = buf("elr_parts"); ezbl_ = buf("ezbl"); 
   gev_ = buf("gev"); gainv_ = buf("gainv"); gaev_ = buf("gaev"); gqkv_ = buf("gqkv");
-  ghead_ = buf("ghead"); fout_ = buf("fout"); etot_ = buf("etot"); red_ = buf("red");
+  fout_ = buf("fout"); etot_ = buf("etot"); red_ = buf("red");
   qkis_ = buf("qkis"); c6eff_ = buf("c6eff"); c6r_ = buf("c6r"); dc_ = buf("dc");
   owner_ = buf("owner"); sr_rows_ = buf("sr_rows"); sr_nodes_ = buf("sr_nodes");
   sr_inc_off_ = buf("sr_inc_off"); sr_inc_ = buf("sr_inc"); lr_rows_ = buf("lr_rows");
@@ -3831,8 +3679,9 @@ void Evaluator::set_system(const std::vector<std::int32_t> &z, const std::vector
     const double inv = 1.0 / model_->arch().embedding_scale;
     for (std::int64_t i = lo; i < hi; ++i) {
       img[i] = int(k);
+      // (the v1 kernels keep their node rows in the tile-transposed order)
       for (int c = 0; c < F; ++c)
-        x0[std::size_t(i) * F + c] = (emb_w_[c * 118 + (z[i] - 1)] + tab[(z[i] - 1) * F + c]) * inv;
+        x0[std::size_t(i) * F + (gen_ ? c : fpos(c))] = (emb_w_[c * 118 + (z[i] - 1)] + tab[(z[i] - 1) * F + c]) * inv;
     }
   }
   n_ = n;
@@ -4005,15 +3854,12 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
   double *evs = nullptr;
   double *qkv = nullptr;
   double *aev = nullptr;
-  double *n1 = nullptr;
   double *n1hat = nullptr;
   double *n1is = nullptr;
   double *hpre = nullptr;
-  double *tout = nullptr;
+  double *gates = nullptr;
   double *pre2hat = nullptr;
   double *pre2is = nullptr;
-  double *ainv = nullptr;
-  double *act = nullptr;
   double *hhead = nullptr;
   double *heff = nullptr;
   double *eatom = nullptr;
@@ -4028,12 +3874,10 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
   double *vlr = nullptr;
   double *parts = nullptr;
   double *ezbl = nullptr;
-  double *gx = nullptr;
   double *gev = nullptr;
   double *gainv = nullptr;
   double *gaev = nullptr;
   double *gqkv = nullptr;
-  double *ghead = nullptr;
   double *fo = nullptr;
   double *etot = nullptr;
   double *red = nullptr;
@@ -4081,22 +3925,17 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
     evs = take<double>(evs_, (L + 1) * Nz * kE);
     qkv = take<double>(qkv_, L * Nz * 640);
     aev = take<double>(aev_, L * Nz * kE);
-    n1 = take<double>(n1_, L * Nz * kF);
     n1hat = take<double>(n1hat_, L * Nz * kF);
     n1is = take<double>(n1is_, L * Nz);
     hpre = take<double>(hpre_, L * Nz * kF);
-    tout = take<double>(tout_, L * Nz * kNI);
+    gates = take<double>(gates_, L * Nz * 4);
     pre2hat = take<double>(pre2hat_, L * Nz * kF);
     pre2is = take<double>(pre2is_, L * Nz);
-    ainv = take<double>(ainv_, Nz * kF);
-    act = take<double>(act_, Nz * HO); // MLP input (128 wide) and head activations (HO)
     hhead = take<double>(hhead_, Nz * HO);
-    gx = take<double>(gx_, Nz * kF);
     gev = take<double>(gev_, Nz * kE);
     gainv = take<double>(gainv_, Nz * kF);
     gaev = take<double>(gaev_, Nz * kE);
     gqkv = take<double>(gqkv_, Nz * 640);
-    ghead = take<double>(ghead_, Nz * HO);
     qkis = qk_norm_ ? take<double>(qkis_, L * Nz * 16) : nullptr;
     ps = take<double>(ps_, L * 4 * Pa);
     // filter rows of every block for the scalar cross-check path; of blocks
@@ -4197,7 +4036,6 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
     carve_used_ = 0;
   }
   carve_all();
-  double *hact = act;
   const int *sr_rows = static_cast<const int *>(sr_rows_->p);
   const int *sr_nodes = static_cast<const int *>(sr_nodes_->p);
   const int *sr_off = static_cast<const int *>(sr_inc_off_->p);
@@ -4227,25 +4065,6 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
   };
   auto fill = [&](double *p, std::size_t cnt) {
     if (cnt) hipLaunchKernelGGL(k_fill, dim3(unsigned((cnt + 255) / 256)), dim3(256), 0, s, p, cnt, 0.0);
-  };
-  // node GEMM shapes (K, O) of the heads: 128->320 and its reverse 320->128;
-  // output tiles per wavefront: MT / MG groups run as separate wavefronts
-#ifndef SO3LR_MG8
-#define SO3LR_MG8 4
-#endif
-  auto gemm = [&](int epi, int rows, int K, int O, const double *X, int ldx, const double *Wp, const double *bias,
-                  double *out, int ldo, double *out2) {
-    const dim3 grid(unsigned(ceil_div(rows, 64)));
-#define SO3LR_GEMM(E, KT, MT, MG)                                                                             \
-  if (epi == E && (K + 15) / 16 == KT && (O + 15) / 16 == MT) {                                              \
-    hipLaunchKernelGGL((k_gemm<E, KT, MT, MG>), dim3(grid.x, MT / MG), dim3(256), 0, s, rows, K, O, X, ldx, Wp, \
-                       bias, out, ldo, out2);                                                                 \
-    return;                                                                                                   \
-  }
-    SO3LR_GEMM(0, 20, 8, SO3LR_MG8) SO3LR_GEMM(1, 8, 20, 4)
-    SO3LR_GEMM(0, 24, 8, SO3LR_MG8) SO3LR_GEMM(1, 8, 24, 4)  // with the C6 head (384 hidden units)
-#undef SO3LR_GEMM
-    throw std::logic_error("SO3LR: internal error, no node GEMM for this shape");
   };
   const unsigned gN64 = unsigned(std::max(1, ceil_div(N, 64)));
 
@@ -4350,12 +4169,20 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
     hipLaunchKernelGGL(k_image_center, dim3(unsigned(n_images_)), dim3(1024), 0, s, img_off, img_q, dq, qseed, 1);
     gen_->reverse(G);
   } else {
-  HIP_CHECK(hipMemcpyAsync(xs, x0, Nz * kF * sizeof(double), hipMemcpyDeviceToDevice, s));
   const unsigned gNF = unsigned((Nz * kF + 255) / 256);
+  const unsigned gN16 = unsigned(ceil_div(N, 16));  // 16 atoms per node-chain block
   // residual scalars: block b's input is resid[b] x + x0[b] x0, x the block
-  // below's output (block 0: the embedding itself)
-  if (!resid_.empty()) hipLaunchKernelGGL(k_axpby, dim3(gNF), dim3(256), 0, s, Nz * kF, resid_[0], xs, x0l_[0], x0);
-  fill(evs, Nz * kE);
+  // below's output (block 0: the embedding itself); its projections are a
+  // launch of their own then
+  const bool scaled = !resid_.empty();
+  if (scaled) {
+    HIP_CHECK(hipMemcpyAsync(xs, x0, Nz * kF * sizeof(double), hipMemcpyDeviceToDevice, s));
+    hipLaunchKernelGGL(k_axpby, dim3(gNF), dim3(256), 0, s, Nz * kF, resid_[0], xs, x0l_[0], x0);
+  }
+  const HeadArgs H{hw_.w1p, hw_.w1tp, hw_.b1p, hw_.ew2, hw_.qw2, hw_.hkey_bwd, hw_.ckey_bwd, hw_.escale, hw_.eshift,
+                   hw_.qemb, hw_.hvshift, hw_.hkey_c, hw_.ckey_c, hw_.cvshift, hw_.eb2, hw_.qb2};
+  const HeadOut HO_{hhead, eatom, qraw, heff, hir, c6eff, c6r};
+  const HeadSeeds HS{hhead, qseed, dh, heff, dc, c6eff};
   const double inv_avg = 1.0 / avg_;
   const unsigned gP = unsigned(PA);
   const unsigned gP64 = unsigned(std::max(1, ceil_div(PA, 64)));  // 64 pairs per MFMA block
@@ -4368,10 +4195,11 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
   // --- interaction blocks, forward ---
   for (int b = 0; b < L; ++b) {
     const BlockWeights &B = bw_[b];
-    double *xb = xs + b * Nz * kF, *evb = evs + b * Nz * kE;
+    // block 0's input is the embedding, ev = 0
+    const double *xb = b == 0 && !scaled ? x0 : xs + b * Nz * kF, *evb = b == 0 ? nullptr : evs + b * Nz * kE;
     double *qb = qkv + b * Nz * 640, *aevb = aev + b * Nz * kE;
-    double *n1b = n1 + b * Nz * kF, *n1hb = n1hat + b * Nz * kF, *n1ib = n1is + b * Nz;
-    double *hpb = hpre + b * Nz * kF, *tb = tout + b * Nz * kNI;
+    double *n1hb = n1hat + b * Nz * kF, *n1ib = n1is + b * Nz;
+    double *hpb = hpre + b * Nz * kF, *gtb = gates + b * Nz * 4;
     double *p2h = pre2hat + b * Nz * kF, *p2i = pre2is + b * Nz;
     double *psb = ps + b * 4 * Pa, *pab = palpha + b * 16 * Pa;
     double *pfb = scalar ? pf + b * 256 * Pa : (b > 0 ? pf + (b - 1) * 256 * Pa : nullptr);
@@ -4424,7 +4252,8 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
         hipLaunchKernelGGL(k_cls_place, gsort, dim3(256), 0, s, nact, pa, z, lut, C, ccur, cord);
       }
     } else {
-      hipLaunchKernelGGL(k_qkv_mfma, dim3(gN64, kHeads), dim3(256), 0, s, int(N), xb, B.qkvp, qb);
+      if (b == 0 || scaled)  // the other blocks' rows come from the node chain below them
+        hipLaunchKernelGGL(k_qkv_mfma, dim3(gN64, kHeads), dim3(256), 0, s, int(N), xb, B.qkvp, qb);
       if (qk_norm_)
         hipLaunchKernelGGL(k_qk_norm, dim3(unsigned(ceil_div(16 * N, 256))), dim3(256), 0, s, int(N), qb,
                            qkis + b * Nz * 16);
@@ -4454,46 +4283,41 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
     timed("attn_fwd", 1, [&] {
       if (scalar)
         hipLaunchKernelGGL(k_attn_fwd, dim3(gN4), dim3(256), 0, s, int(N), sr_off, iact, iother, xb, evb, qb,
-                           pfb, pY, pfc, inv_avg, pab, ainv, aevb);
+                           pfb, pY, pfc, inv_avg, ln_eps_, norm1_, pab, n1hb, n1ib, aevb);
       else
         hipLaunchKernelGGL(k_attn_msg, dim3(gN4), dim3(256), 0, s, int(N), sr_off, iact, iother, xb, evb,
-                           blk0 && use_cls ? cqkv : qb, pY, pfc, pab, B.ln1w, B.ln1b, ln_eps_, norm1_, n1b, n1hb,
-                           n1ib, act, aevb, z, blk0 && use_cls ? static_cast<const int *>(cls_lut_->p) : nullptr);
+                           blk0 && use_cls ? cqkv : qb, pY, pfc, pab, ln_eps_, norm1_, n1hb, n1ib, aevb, z, blk0 && use_cls ? static_cast<const int *>(cls_lut_->p) : nullptr);
     });
-    if (scalar)  // the MFMA path's k_attn_msg has done LayerNorm 1 already
-      hipLaunchKernelGGL(k_post1, dim3(gN4), dim3(256), 0, s, int(N), ainv, B.ln1w, B.ln1b, ln_eps_, norm1_, n1b,
-                         n1hb, n1ib, act);
-    // the post-attention node chain in one kernel (MLP, interaction, LayerNorm 2, ev gate)
-    const NodeChainArgs NC{B.m1p, B.m1bp, B.m2p, B.m2bp, B.intp, B.intbp, B.int_cg, B.ln2w, B.ln2b, hw_.exp2_256,
+    // the post-attention node chain in one kernel (MLP, interaction,
+    // LayerNorm 2, ev gate), then the next block's projections or the heads
+    const NodeChainArgs NC{B.m1p, B.m1bp, B.m2p, B.m2bp, B.intp, B.intbp, B.int_cg, B.ln1w, B.ln1b, B.ln2w, B.ln2b,
                            ln_eps_, norm2_};
-    hipLaunchKernelGGL(k_node_fwd, dim3(unsigned(ceil_div(N, 32))), dim3(256), 0, s, int(N), act, n1b, aevb, NC, hpb, tb,
-                       xs + (b + 1) * Nz * kF, evs + (b + 1) * Nz * kE, p2h, p2i);
-    if (!resid_.empty() && b + 1 < L)
+#define SO3LR_NODE_FWD(TAIL)                                                                                        \
+  hipLaunchKernelGGL(k_node_fwd<TAIL>, dim3(gN16), dim3(512), 0, s, int(N), n1hb, aevb, NC, H,                      \
+                     b + 1 < L ? bw_[b + 1].qkvp : nullptr, z, hpb, gtb, xs + (b + 1) * Nz * kF,                     \
+                     evs + (b + 1) * Nz * kE, p2h, p2i, b + 1 < L ? qkv + (b + 1) * Nz * 640 : nullptr, HO_)
+    if (b + 1 < L && scaled) SO3LR_NODE_FWD(0);
+    else if (b + 1 < L) SO3LR_NODE_FWD(1);
+    else if (c6_) SO3LR_NODE_FWD(3);
+    else SO3LR_NODE_FWD(2);
+#undef SO3LR_NODE_FWD
+    if (scaled && b + 1 < L)
       hipLaunchKernelGGL(k_axpby, dim3(gNF), dim3(256), 0, s, Nz * kF, resid_[b + 1], xs + (b + 1) * Nz * kF,
                          x0l_[b + 1], x0);
   }
 
-  // --- heads, charge correction, long range ---
-  HeadArgs H{hw_.ew2, hw_.qw2, hw_.escale, hw_.eshift, hw_.qemb, hw_.hqemb, hw_.hvshift,
-             hw_.hkey_bwd, hw_.hkey_c, hw_.eb2, hw_.qb2, hw_.ckey_bwd, hw_.ckey_c, hw_.cvshift, hw_.ho};
-  const double *xf = xs + L * Nz * kF;
-  gemm(1, int(N), kF, int(HO), xf, kF, hw_.w1p, hw_.b1p, hhead, int(HO), hact);
-  hipLaunchKernelGGL(k_heads, dim3(gN4), dim3(256), 0, s, int(N), z, hact, H, eatom, qraw, heff, hir, c6eff, c6r);
+  // --- charge correction, long range (the heads ran in the last node chain) ---
   hipLaunchKernelGGL(k_image_center, dim3(unsigned(n_images_)), dim3(1024), 0, s, img_off, img_q, qraw, q, 0);
   long_range();
   hipLaunchKernelGGL(k_image_center, dim3(unsigned(n_images_)), dim3(1024), 0, s, img_off, img_q, dq, qseed, 1);
-  hipLaunchKernelGGL(k_heads_bwd, dim3(gN4), dim3(256), 0, s, int(N), z, hhead, qseed, dh, heff, dc, c6eff, H,
-                     ghead);
-  gemm(0, int(N), int(HO), kF, ghead, int(HO), hw_.w1tp, nullptr, gx, kF, nullptr);
-  fill(gev, Nz * kE);
 
   // --- interaction blocks, reverse ---
   for (int b = L - 1; b >= 0; --b) {
     const BlockWeights &B = bw_[b];
     double *evb = evs + b * Nz * kE;
     double *qb = qkv + b * Nz * 640, *aevb = aev + b * Nz * kE;
-    double *n1b = n1 + b * Nz * kF, *n1hb = n1hat + b * Nz * kF, *n1ib = n1is + b * Nz;
-    double *hpb = hpre + b * Nz * kF, *tb = tout + b * Nz * kNI;
+    double *n1hb = n1hat + b * Nz * kF, *n1ib = n1is + b * Nz;
+    double *hpb = hpre + b * Nz * kF, *gtb = gates + b * Nz * 4;
     double *p2h = pre2hat + b * Nz * kF, *p2i = pre2is + b * Nz;
     double *psb = ps + b * 4 * Pa, *pab = palpha + b * 16 * Pa;
     double *pfb = scalar ? pf + b * 256 * Pa : (b > 0 ? pf + (b - 1) * 256 * Pa : nullptr);
@@ -4503,10 +4327,18 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
       A.fe0[k] = B.fe0[k]; A.feb0[k] = B.feb0[k]; A.fe1t[k] = B.fe1t[k]; A.feb1[k] = B.feb1[k];
     }
     A.att_cg = B.att_cg; A.rbf_b = hw_.rbf_b; A.rbf_k = hw_.rbf_k; A.rbf_kr = hw_.rbf_kr; A.gamma = gamma_;
-    // the post-attention node chain in reverse in one kernel: gainv, gaev
-    const NodeChainBwdArgs NB{B.inttp, B.m2tp, B.m1tp, B.int_cg, B.ln1w, B.ln2w, norm1_, norm2_};
-    hipLaunchKernelGGL(k_node_bwd, dim3(unsigned(ceil_div(N, 32))), dim3(256), 0, s, int(N), gx, gev, tb, aevb, p2h,
-                       p2i, hpb, n1b, n1hb, n1ib, NB, gainv, gaev);
+    // the post-attention node chain in reverse in one kernel (gainv, gaev),
+    // from the heads' reverse or from the projections' reverse of the block
+    // above (with its residual scalar)
+    const NodeChainBwdArgs NB{B.inttp, B.m2tp, B.m1tp, B.int_cg, B.ln1w, B.ln1b, B.ln2w, norm1_, norm2_};
+#define SO3LR_NODE_BWD(SRC)                                                                                        \
+  hipLaunchKernelGGL(k_node_bwd<SRC>, dim3(gN16), dim3(512), 0, s, int(N), gqkv,                                    \
+                     b + 1 < L ? bw_[b + 1].qkvtp : nullptr, b + 1 < L && scaled ? resid_[b + 1] : 1.0, H, HS, z,    \
+                     b + 1 < L ? gev : nullptr, gtb, aevb, p2h, p2i, hpb, n1hb, n1ib, NB, gainv, gaev)
+    if (b + 1 < L) SO3LR_NODE_BWD(1);
+    else if (c6_) SO3LR_NODE_BWD(2);
+    else SO3LR_NODE_BWD(0);
+#undef SO3LR_NODE_BWD
     if (scalar) {
       // scalar cross-check path: the attention reverse writes the pair
       // adjoints (df, dE/dfc, dE/dY) and the scalar filter reverse reads them
@@ -4582,9 +4414,6 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
       if (qk_norm_)  // through the QK normalisation to the raw projections
         hipLaunchKernelGGL(k_qk_norm_bwd, dim3(unsigned(ceil_div(16 * N, 256))), dim3(256), 0, s, int(N), qb,
                            qkis + b * Nz * 16, gqkv);
-      hipLaunchKernelGGL(k_qkv_bwd_mfma, dim3(gN64, kHeads), dim3(256), 0, s, int(N), gqkv, B.qkvtp, gainv, gx);
-      // residual scalars: the adjoint of the block below's output
-      if (!resid_.empty()) hipLaunchKernelGGL(k_scale, dim3(gNF), dim3(256), 0, s, Nz * kF, resid_[b], gx);
       hipLaunchKernelGGL(k_ev_bwd, dim3(gN4), dim3(256), 0, s, int(N), sr_off, iact, iother, evb, B.att_cg, ds,
                          gaev, gev);
     }

@@ -56,10 +56,7 @@ struct BlockWeights {
   const double *fe1[2], *feb1[2];       // spherical layer 1 (128, 32), (128)
   const double *fe1t[2];                // its transpose
   const double *att_cg, *int_cg;        // (24)
-  const double *ln1w, *ln1b, *ln2w, *ln2b;
-  const double *m1t, *m1b, *m2t, *m2b;  // MLP weights transposed (in, out)
-  const double *m1w, *m2w;              // (out, in) for the reverse
-  const double *intt, *intb, *intw;     // interaction (132x132): transposed and (out, in)
+  const double *ln1w, *ln1b, *ln2w, *ln2b;  // (128) in the tile-transposed order of the node rows
   // MFMA operand order of the filter weights (see permute_mfma in evaluator.hip)
   const double *w0p[2], *w1p[2], *e0p[2], *e1p[2];     // forward
   const double *w1tp[2], *w0tp[2], *e1tp[2], *e0tp[2];  // reverse (transposes)
@@ -83,16 +80,13 @@ struct HeadWeights {
   int ho = 320;              // first-layer width: energy 128 | charge 128 | Hirshfeld 64 (| C6 64)
   const double *w1p, *w1tp;  // MFMA operand order: (ho x 128) and its transpose
   const double *b1p;         // first-layer bias (ho) in accumulator order
-  const double *w1t;    // (128, 320): energy | charge | Hirshfeld first layers, transposed
-  const double *w1;     // (320, 128)
-  const double *b1;     // (320)
-  const double *ew2, *qw2;  // (128)
+  const double *ew2, *qw2;  // (128), tile-transposed order
   double eb2, qb2;
   const double *escale, *eshift;  // (118)
   const double *qemb;             // (100)
-  const double *hkey_bwd;         // (100, 64): u[z][i] = sum_j hw2[j][i] hqemb[z][j]
-  const double *hkey_c;           // (100): hqemb[z] . hb2
-  const double *hqemb, *hvshift;  // (100, 64), (100)
+  const double *hkey_bwd;  // (100, 64): u[z][i] = sum_j hw2[j][i] hqemb[z][j], tile-transposed order
+  const double *hkey_c;    // (100): hqemb[z] . hb2
+  const double *hvshift;   // (100)
   const double *ckey_bwd, *ckey_c, *cvshift;  // the C6 ratio head's, as hkey_bwd, hkey_c, hvshift (or null)
   const double *rbf_b, *rbf_k, *rbf_kr;  // (32) each
   const double *rbf_e;                   // (32) Bernstein recurrence factors (FilterMfma::rbf_e)
@@ -232,11 +226,10 @@ class Evaluator {
 
   // node-sized device buffers (named members so the kernels' arguments read clearly)
   Buffer *z_, *x0_, *img_of_node_, *img_off_, *img_q_;
-  Buffer *xs_, *evs_, *qkv_, *aev_, *n1_, *n1hat_, *n1is_, *hpre_, *tout_, *pre2hat_, *pre2is_;
-  Buffer *ainv_, *act_;
+  Buffer *xs_, *evs_, *qkv_, *aev_, *n1hat_, *n1is_, *hpre_, *gates_, *pre2hat_, *pre2is_;
   Buffer *hhead_, *heff_, *eatom_, *qraw_, *q_, *hir_, *qseed_;
   Buffer *elr_, *dq_, *dh_, *flr_, *vlr_, *elr_parts_, *ezbl_;
-  Buffer *gx_, *gev_, *gainv_, *gaev_, *gqkv_, *ghead_;
+  Buffer *gev_, *gainv_, *gaev_, *gqkv_;
   Buffer *qkis_, *c6eff_, *c6r_, *dc_;  // QK normalisation 1/rms; C6 head logit, ratio, dE/dratio
   Buffer *fout_, *etot_, *red_, *red_part_;
   // pair-sized buffers

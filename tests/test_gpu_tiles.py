@@ -1,0 +1,27 @@
+"""HIP path vs the CPU oracle at the sizes where the kernels' work is cut: atom
+counts at and beside the edges of their 16-atom tiles, on the scalar and the
+fused filter kernels of the shipped model and on the generic widths.  Bars as
+in test_gpu_edges.py: energy 1e-10 relative, forces and virial 1e-9.
+"""
+import numpy as np
+import pytest
+
+from test_gpu_edges import _both_paths, model, orc  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+def _cluster(n, seed=3):
+    """n H and O atoms on a jittered 1.7 A lattice, every pair of neighbours
+    inside the short-range cutoff."""
+    rng = np.random.default_rng([seed, n])
+    g = int(np.ceil(n ** (1 / 3) - 1e-9))
+    sites = np.array([[i, j, k] for i in range(g) for j in range(g) for k in range(g)], float)[:n]
+    z = rng.choice([1, 8], size=n, p=[0.6, 0.4])
+    return z, 1.7 * sites + rng.uniform(-0.2, 0.2, (n, 3)), 1.0 + float((z == 1).sum() % 2)
+
+
+@pytest.mark.parametrize("n", [2, 15, 16, 17, 33, 65])
+def test_atom_tiles(orc, model, n):  # noqa: F811
+    z, x, m = _cluster(n)
+    _both_paths(z, x, 0.0, m, orc, model)
