@@ -12,6 +12,7 @@
 // (-1)^l Y(v/r).  Node sums are gathers over a CSR incidence list.
 #include "evaluator.hpp"
 #include "mfma_ops.hpp"
+#include "node_chain.hpp"
 #include "radial_table.hpp"
 
 #include <algorithm>
@@ -1908,59 +1909,6 @@ __global__ __launch_bounds__(256) void k_rint_place(const int *n_active, const i
   if (p < *n_active) order[atomicAdd(&cursor[rint_key(pa[2 * p], pr[p], d)], 1)] = p;
 }
 
-// ---------------------------------------------------------------- node layers
-// Block-diagonal projections: per head h, the 160 outputs (q k v q_ev k_ev,
-// 32 each) depend on x[h*32 .. h*32+32).  Wp holds, per head, the permuted
-// (160 x 32) matrix; out[n][w*128 + h*32 + o].  Stream per head: the two
-// input chunks, then the 10 x 2 weight fragments (tile-major).
-__global__ __launch_bounds__(256) void k_qkv_mfma(int rows, const double *__restrict__ X,
-                                                  const double *__restrict__ Wp, double *__restrict__ out) {
-  const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
-  const int w = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (w * 16 >= rows) return;
-  const int n = w * 16 + j;
-  const bool valid = n < rows;
-  const double *xr = X + std::size_t(valid ? n : rows - 1) * kF;
-  const int h = blockIdx.y;  // one head per wavefront
-  constexpr int PER_H = 2 + 20;
-  auto load = [&](auto si) -> v4d {
-    constexpr int s = decltype(si)::value;
-    if constexpr (s < 2) {
-      return *reinterpret_cast<const v4d *>(xr + h * kHW + 16 * s + 4 * g);
-    } else {
-      return wload(Wp + std::size_t(h) * 160 * kHW, 2, (s - 2) / 2, (s - 2) % 2, lane);
-    }
-  };
-  Stream<PER_H, kFilterPF, decltype(load)> st(load);
-  st.prime();
-  const v4d zero = v4d{0, 0, 0, 0};
-  v4d b[2] = {zero, zero}, acc[10];
-  st.run([&](auto si, const v4d &wv) {
-    constexpr int s = decltype(si)::value;
-    if constexpr (s < 2) {
-      b[s] = wv;
-      if constexpr (s == 0) {
-#pragma unroll
-        for (int mt = 0; mt < 10; ++mt) acc[mt] = zero;
-      }
-    } else {
-      constexpr int mt = (s - 2) / 2, T = (s - 2) % 2;
-      acc[mt] = mfma4(wv, b[T], acc[mt]);
-    }
-    if constexpr (s == PER_H - 1) {
-      if (valid) {
-        // tile mt is projection mt / 2, channels 32 h + 16 (mt % 2) + [0, 16):
-        // one 16-channel tile of the row, stored in the tile-transposed order
-        // (fpos), so each lane writes its four values as one vector
-        double *row = out + std::size_t(n) * 640 + h * kHW + 4 * g;
-#pragma unroll
-        for (int mt = 0; mt < 10; ++mt)
-          *reinterpret_cast<v4d *>(row + (mt >> 1) * kF + 16 * (mt & 1)) = acc[mt];
-      }
-    }
-  });
-}
-
 // ---------------------------------------------------------------- attention
 // 16-byte load / store of two adjacent doubles (16-byte aligned)
 __device__ __forceinline__ double2 ld2(const double *p) { return *reinterpret_cast<const double2 *>(p); }
@@ -2123,482 +2071,7 @@ __global__ __launch_bounds__(256) void k_attn_msg(int N, const int *inc_off, con
   if (evv) aev[std::size_t(n) * kE + m] = (ev ? ev[std::size_t(n) * kE + m] : 0.0) + acce;
 }
 
-// The post-attention node chain of one block with every activation in MFMA
-// registers (kokkos_post_attention_block0.cpp:302-333):
-//   n1 = LN1 row (its normalised values n1hat times the affine weights),
-//   hpre = W1 silu(n1) + b1 (kept for the reverse), hid = silu(hpre),
-//   p = n1 + W2 hid + b2,
-//   t = Wint [p, inv(aev)] + bint (132 wide), inv_l = sum_{m in l} aev_m^2 cg_m,
-//   x' = LN2(p + t[0:128]) (statistics kept), ev' = aev (1 + gate[slot]),
-//   gate l = t[128 + l] (kept),
-// then what reads x' next: the following block's q k v q_ev k_ev rows (TAIL
-// 1), or the heads (TAIL 2; 3 with the C6 head): their hidden layer and the
-// per-atom energy, raw charge and ratios.
-//
-// One workgroup of eight wavefronts per 16 atoms: wavefront w owns output tile
-// w (16 of the 128 features) of every layer, and the layer inputs are
-// exchanged through LDS in MFMA operand order (chunk T of lane l at
-// buf[T][l]).  A tile of the chain is bound by its length (three dependent
-// layers and two row normalisations, each wavefront streaming its own weight
-// fragments from L2), so it is cut as short as the 16 x 16 tiles allow: a
-// wavefront's share is 26 fragments, kNodePF of them in flight.  The gate tile
-// (4 of 16 rows used) is formed from partial products, each wavefront taking
-// its own chunk of p, summed through LDS in wavefront order.  Node rows are
-// in the tile-transposed channel order (fpos), so a chunk is one 32-byte
-// vector per lane.  Two wavefronts per tile, four output tiles each, and the
-// projections, heads and row sums as launches of their own took 570 us per
-// evaluation at 22 atoms, 716 at 99, 1,216 at 3,000, 2,326 for 512 packed
-// molecules and 6.64 ms at 24,000; this form 443, 570, 1,046, 2,126 and 6.50.
-struct NodeChainArgs {
-  const double *m1p, *m1bp, *m2p, *m2bp, *intp, *intbp;  // MFMA operand order
-  const double *int_cg, *ln1w, *ln1b, *ln2w, *ln2b;      // 128-wide vectors in fpos order
-  double eps;
-  int mode2;  // NormMode of the second position (RMSNorm, none: w = 1, b = 0 given)
-};
-struct HeadArgs {
-  const double *w1p, *w1tp, *b1p;  // hidden layer (HO x 128), its transpose and bias, MFMA operand order
-  const double *ew2, *qw2, *hkey, *ckey;  // output rows, 128 | 128 | 64 per element (| 64) units, fpos order
-  const double *escale, *eshift, *qemb, *hvshift, *hkey_c, *ckey_c, *cvshift;  // per element
-  double eb2, qb2;
-};
-struct HeadOut {
-  double *hhead;  // hidden pre-activations [N][HO], tiles in fpos order
-  double *eatom, *qraw, *heff, *hir, *c6eff, *c6r;
-};
-// Fragments in flight per wavefront, and wavefronts per SIMD (two workgroups
-// per CU): 6 and 4 measured best over sizes (4 and 4 within 0.3%; 8 and 4
-// spills; 8 or 12 and 2 cost 2% at 12,000 atoms and up).
-constexpr int kNodePF = 6;
-#define NODE_OCCUPANCY __launch_bounds__(512, 4)
-
-// sum over the four lane groups (every lane of a column ends with the total)
-__device__ __forceinline__ double column_sum(double v) {
-  v += __shfl_xor(v, 16, kWave);
-  return v + __shfl_xor(v, 32, kWave);
-}
-// the eight wavefronts' values of one column, in wavefront order
-__device__ __forceinline__ double sum8(const double (*part)[16], int j) {
-  double s = part[0][j];
-#pragma unroll
-  for (int w = 1; w < 8; ++w) s += part[w][j];
-  return s;
-}
-__device__ __forceinline__ double sum8(const double (*part)[64], int lane) {
-  double s = part[0][lane];
-#pragma unroll
-  for (int w = 1; w < 8; ++w) s += part[w][lane];
-  return s;
-}
-// sum over the channels of degree slot g of a row of 24: a_m b_m (cg_m)
-__device__ __forceinline__ double slot_sum(int g, const double *a, const double *b, const double *cg) {
-  const int lo = ev_offset(g), hi = lo + 2 * g + 3;
-  double s = 0.0;
-  for (int m = lo; m < hi; ++m) s += cg ? a[m] * b[m] * cg[m] : a[m] * b[m];
-  return s;
-}
-
-template <int TAIL>
-__global__ NODE_OCCUPANCY void k_node_fwd(int N, const double *__restrict__ n1hat,
-                                                  const double *__restrict__ aev, NodeChainArgs A, HeadArgs H,
-                                                  const double *__restrict__ qkvp, const int *__restrict__ z,
-                                                  double *__restrict__ hpre, double *__restrict__ gates,
-                                                  double *__restrict__ xout, double *__restrict__ evout,
-                                                  double *__restrict__ pre2hat, double *__restrict__ pre2is,
-                                                  double *__restrict__ qkv, HeadOut O) {
-  constexpr int HT = TAIL == 3 ? 24 : 20;  // tiles of the heads' hidden layer
-  __shared__ v4d bufA[8][64], bufB[8][64];
-  __shared__ double gpart[8][64], st1[8][16], st2[8][16];
-  __shared__ double hsum[TAIL >= 2 ? HT : 1][16];
-  const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4, w = threadIdx.x >> 6;
-  // every wavefront runs to the end (the barriers); rows beyond N are clamped
-  const int n = blockIdx.x * 16 + j;
-  const bool valid = n < N;
-  const std::size_t nn = std::size_t(valid ? n : N - 1);
-  const int own = 16 * w + 4 * g;  // this lane's four channels of the wavefront's tile, fpos order
-  auto vec = [](const double *p) { return *reinterpret_cast<const v4d *>(p); };
-  // the stream of this wavefront
-  constexpr int L1 = 3, L2 = L1 + 9, G = L2 + 9, L3 = G + 3, LN = L3 + 10, TL = LN + 2;
-  constexpr int NS = TL + (TAIL == 1 ? 10 : TAIL >= 2 ? 27 : 0);
-  const int head = w >> 1;  // TAIL 1: this wavefront's head and half of its ten projection tiles
-  auto load = [&](auto si) -> v4d {
-    constexpr int s = decltype(si)::value;
-    if constexpr (s == 0) return vec(n1hat + nn * kF + own);
-    else if constexpr (s == 1) return vec(A.ln1w + own);
-    else if constexpr (s == 2) return vec(A.ln1b + own);
-    else if constexpr (s == L1) return tile_load(A.m1bp, w, lane);
-    else if constexpr (s < L2) return wload(A.m1p, 8, w, s - L1 - 1, lane);
-    else if constexpr (s == L2) return tile_load(A.m2bp, w, lane);
-    else if constexpr (s < G) return wload(A.m2p, 8, w, s - L2 - 1, lane);
-    else if constexpr (s == G) return wload(A.intp, 9, 8, w, lane);
-    else if constexpr (s == G + 1) return wload(A.intp, 9, 8, 8, lane);
-    else if constexpr (s == G + 2) return tile_load(A.intbp, 8, lane);
-    else if constexpr (s == L3) return tile_load(A.intbp, w, lane);
-    else if constexpr (s < LN) return wload(A.intp, 9, w, s - L3 - 1, lane);
-    else if constexpr (s == LN) return vec(A.ln2w + own);
-    else if constexpr (s == LN + 1) return vec(A.ln2b + own);
-    else if constexpr (TAIL == 1) {
-      constexpr int T = (s - TL) / 5, q = (s - TL) % 5;
-      return wload(qkvp + std::size_t(head) * 160 * kHW, 2, 5 * (w & 1) + q, T, lane);
-    } else {
-      constexpr int u = (s - TL) / 9, e = (s - TL) % 9;
-      const int t = w + 8 * u < HT ? w + 8 * u : w;  // past the last tile: a valid address, not used
-      if constexpr (e == 0) return tile_load(H.b1p, t, lane);
-      else return wload(H.w1p, 8, t, e - 1, lane);
-    }
-  };
-  Stream<NS, kNodePF, decltype(load)> st(load);
-  st.prime();
-  const double inv = slot_sum(g, aev + nn * kE, aev + nn * kE, A.int_cg);
-  const v4d zero = v4d{0.0, 0.0, 0.0, 0.0};
-  v4d n1, lw, p, acc, gp, pb, hh, tacc[5];
-  double mean = 0.0;
-  st.run([&](auto si, const v4d &wv) {
-    constexpr int s = decltype(si)::value;
-    if constexpr (s == 0) {
-      n1 = wv;
-    } else if constexpr (s == 1) {
-      lw = wv;
-    } else if constexpr (s == 2) {
-      v4d a;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        n1[r] = n1[r] * lw[r] + wv[r];
-        a[r] = silu(n1[r]);
-      }
-      bufA[w][lane] = a;
-      __syncthreads();
-    } else if constexpr (s == L1 || s == L2 || s == L3) {
-      acc = wv;
-    } else if constexpr (s < L2) {
-      acc = mfma4(wv, bufA[s - L1 - 1][lane], acc);
-      if constexpr (s == L2 - 1) {
-        if (valid) *reinterpret_cast<v4d *>(hpre + nn * kF + own) = acc;
-        v4d a;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) a[r] = silu(acc[r]);
-        bufB[w][lane] = a;
-        __syncthreads();
-      }
-    } else if constexpr (s < G) {
-      acc = mfma4(wv, bufB[s - L2 - 1][lane], acc);
-      if constexpr (s == G - 1) {
-        p = n1 + acc;
-        bufA[w][lane] = p;  // every wavefront has read the MLP input (the barrier above)
-      }
-    } else if constexpr (s == G) {
-      gp = mfma4(wv, p, zero);
-    } else if constexpr (s == G + 1) {
-      if (w == 0) gp = mfma(wv[0], inv, gp);
-    } else if constexpr (s == G + 2) {
-      gpart[w][lane] = w == 0 ? gp[0] + wv[0] : gp[0];
-      __syncthreads();
-    } else if constexpr (s < LN - 1) {
-      acc = mfma4(wv, bufA[s - L3 - 1][lane], acc);
-    } else if constexpr (s == LN - 1) {
-      acc = mfma(wv[0], inv, acc);  // the invariants: K rows 128 + g, zero beyond
-      // LayerNorm 2 of p + t over the row, the tiles' sums combined in LDS
-      pb = p + acc;
-      const double sum = column_sum((pb[0] + pb[1]) + (pb[2] + pb[3]));
-      if (g == 0) st1[w][j] = sum;
-      __syncthreads();
-      mean = A.mode2 == 0 ? sum8(st1, j) / kF : 0.0;
-      double var = 0.0;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const double d = pb[r] - mean;
-        var += d * d;
-      }
-      var = column_sum(var);
-      if (g == 0) st2[w][j] = var;
-      __syncthreads();
-      const double is = A.mode2 == 2 ? 1.0 : 1.0 / sqrt(sum8(st2, j) / kF + A.eps);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) hh[r] = (pb[r] - mean) * is;
-      if (valid) {
-        *reinterpret_cast<v4d *>(pre2hat + nn * kF + own) = hh;
-        if (w == 0 && g == 0) pre2is[nn] = is;
-        if (w < 6) {  // ev' = aev (1 + gate[slot]), channel g + 4 w
-          const int m = g + 4 * w;
-          evout[nn * kE + m] = aev[nn * kE + m] * (1.0 + sum8(gpart, j + 16 * degree_slot(m)));
-        } else if (w == 6) {
-          gates[nn * 4 + g] = sum8(gpart, lane);
-        }
-      }
-    } else if constexpr (s == LN) {
-      lw = wv;
-    } else if constexpr (s == LN + 1) {
-      v4d x;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) x[r] = hh[r] * lw[r] + wv[r];
-      if constexpr (TAIL < 2) {
-        if (valid) *reinterpret_cast<v4d *>(xout + nn * kF + own) = x;
-      }
-      if constexpr (TAIL > 0) {
-        bufB[w][lane] = x;  // every wavefront has read the MLP-2 input
-        __syncthreads();
-      }
-    } else if constexpr (TAIL == 1) {
-      constexpr int T = (s - TL) / 5, q = (s - TL) % 5;
-      tacc[q] = mfma4(wv, bufB[2 * head + T][lane], T == 0 ? zero : tacc[q]);
-      if constexpr (T == 1) {
-        // tile mt = 5 (w & 1) + q is projection mt / 2, channels 32 head +
-        // 16 (mt % 2) + [0, 16) of it
-        const int mt = 5 * (w & 1) + q;
-        if (valid)
-          *reinterpret_cast<v4d *>(qkv + nn * 640 + (mt >> 1) * kF + head * kHW + 16 * (mt & 1) + 4 * g) = tacc[q];
-      }
-    } else {
-      constexpr int u = (s - TL) / 9, e = (s - TL) % 9;
-      if constexpr (e == 0) acc = wv;
-      else acc = mfma4(wv, bufB[e - 1][lane], acc);
-      if constexpr (e == 8) {
-        const int t = w + 8 * u;
-        if (t < HT) {
-          if (valid) *reinterpret_cast<v4d *>(O.hhead + nn * (16 * HT) + 16 * t + 4 * g) = acc;
-          // the tile's share of its head's output: energy (t < 8), charge
-          // (t < 16), Hirshfeld (t < 20) and C6 logits
-          const int zz = z[nn];
-          const double *row = t < 8 ? H.ew2 + 16 * t
-                                    : (t < 16 ? H.qw2 + 16 * (t - 8)
-                                              : (t < 20 ? H.hkey + zz * kHH + 16 * (t - 16)
-                                                        : H.ckey + zz * kHH + 16 * (t - 20)));
-          const v4d r = vec(row + 4 * g);
-          const double v = (r[0] * silu(acc[0]) + r[1] * silu(acc[1])) + (r[2] * silu(acc[2]) + r[3] * silu(acc[3]));
-          const double sum = column_sum(v);
-          if (g == 0) hsum[t][j] = sum;
-        }
-      }
-    }
-  });
-  if constexpr (TAIL >= 2) {
-    // per-atom energy, raw charge, Hirshfeld (and C6) logit and ratio
-    // (kokkos_output_heads.cpp:108-180,341-451)
-    __syncthreads();
-    if (w == 0 && g < (TAIL == 3 ? 4 : 3) && valid) {
-      const int zz = z[nn];
-      const int t0 = g == 0 ? 0 : (g == 1 ? 8 : (g == 2 ? 16 : 20)), t1 = g == 0 ? 8 : (g == 1 ? 16 : (g == 2 ? 20 : 24));
-      double v = hsum[t0][j];
-      for (int t = t0 + 1; t < t1; ++t) v += hsum[t][j];
-      if (g == 0) {
-        O.eatom[nn] = (v + H.eb2) * H.escale[zz - 1] + H.eshift[zz - 1];
-      } else if (g == 1) {
-        O.qraw[nn] = v + H.qb2 + H.qemb[zz];
-      } else if (g == 2) {
-        // logit q_emb[z] . (W2 a + b2), contracted through the element's row
-        // u[z] = W2^T q_emb[z]; sqrt(64) = 8
-        const double ef = H.hvshift[zz] + (H.hkey_c[zz] + v) / 8.0;
-        O.heff[nn] = ef;
-        O.hir[nn] = fabs(ef);
-      } else {
-        const double ce = H.cvshift[zz] + (H.ckey_c[zz] + v) / 8.0;
-        O.c6eff[nn] = ce;
-        O.c6r[nn] = fabs(ce);
-      }
-    }
-  }
-}
-
-// Reverse of the node chain, the adjoints in MFMA registers
-// (kokkos_post_attention_reverse.cpp:328-449), starting from the adjoint gx of
-// the block's output x':
-//   SRC 0 (the last block; 2 with the C6 head): the heads' reverse, seeds
-//     energy 1, charge dE/dq - mean, Hirshfeld dE/dh (and dE/dc) through the
-//     hidden layer (kokkos_output_heads.cpp:493-581);
-//   SRC 1: the projections' reverse of the block above, gx = scale (base +
-//     sum_w W_w^T dqkv_w), base its attention-residual adjoint (gainv, which
-//     this kernel then overwrites row by row with its own).
-// Then
-//   LayerNorm 2 reverse: d = LN2^T gx, the adjoint of p and of t[0:128];
-//   t[128 + l] (gates): sum_{m in l} gev_m aev_m; aev: gev (1 + gate);
-//   interaction reverse: gcat = Wint^T gt; p += gcat[0:128];
-//   aev += 2 aev cg gcat[128 + slot];
-//   MLP reverse: ghid = (W2^T p) silu'(hpre), gact = W1^T ghid;
-//   LayerNorm 1 reverse of g = p + gact silu'(n1): the adjoint of the
-//   attention residual, gainv.
-// Eight wavefronts per 16 atoms as in k_node_fwd.  gev null: zero (the last
-// block's equivariant output is not read).
-struct NodeChainBwdArgs {
-  const double *inttp, *m2tp, *m1tp;  // MFMA operand order (transposes)
-  const double *int_cg, *ln1w, *ln1b, *ln2w;  // 128-wide vectors in fpos order
-  int mode1, mode2;  // NormMode of the two positions: RMSNorm drops the mean term, none both
-};
-struct HeadSeeds {
-  const double *hhead, *qseed, *dh, *heff, *dc, *c6eff;
-};
-template <int SRC>
-__global__ NODE_OCCUPANCY void k_node_bwd(int N, const double *__restrict__ gqkv,
-                                                  const double *__restrict__ qkvtp, double scale, HeadArgs H,
-                                                  HeadSeeds S, const int *__restrict__ z,
-                                                  const double *__restrict__ gev, const double *__restrict__ gates,
-                                                  const double *__restrict__ aev, const double *__restrict__ pre2hat,
-                                                  const double *__restrict__ pre2is, const double *__restrict__ hpre,
-                                                  const double *__restrict__ n1hat, const double *__restrict__ n1is,
-                                                  NodeChainBwdArgs A, double *gainv, double *__restrict__ gaev) {
-  constexpr int HT = SRC == 2 ? 24 : 20;
-  constexpr bool HEADS = SRC != 1;
-  __shared__ v4d buf[HEADS ? HT : 16][64];  // chunks 0..7 and 8..15: the two layer-input buffers
-  __shared__ double gpart[8][64], st[4][8][16];
-  const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4, w = threadIdx.x >> 6;
-  const int n = blockIdx.x * 16 + j;
-  const bool valid = n < N;
-  const std::size_t nn = std::size_t(valid ? n : N - 1);
-  const int own = 16 * w + 4 * g;
-  auto vec = [](const double *p) { return *reinterpret_cast<const v4d *>(p); };
-  const int head = w >> 1;
-  constexpr int X = HEADS ? HT : 21;  // entries of gx
-  constexpr int L3 = X + 2, G = L3, LB = G + 2, L2 = LB + 9, L1 = L2 + 9, LN = L1 + 8, NS = LN + 3;
-  auto load = [&](auto si) -> v4d {
-    constexpr int s = decltype(si)::value;
-    if constexpr (s < X) {
-      if constexpr (HEADS) return wload(H.w1tp, HT, w, s, lane);
-      else if constexpr (s == 20) return vec(gainv + nn * kF + own);
-      else if constexpr ((s & 1) == 0) {
-        // K entries of chunk T: projection T / 2, channels 32 head + 16 (T % 2) + [0, 16)
-        constexpr int T = s / 2;
-        return vec(gqkv + nn * 640 + (T >> 1) * kF + head * kHW + 16 * (T & 1) + 4 * g);
-      } else {
-        return wload(qkvtp + std::size_t(head) * kHW * 160, 10, w & 1, s / 2, lane);
-      }
-    } else if constexpr (s == X) return vec(A.ln2w + own);
-    else if constexpr (s == X + 1) return vec(pre2hat + nn * kF + own);
-    else if constexpr (s == G) return wload(A.inttp, 9, 8, w, lane);
-    else if constexpr (s == G + 1) return wload(A.inttp, 9, 8, 8, lane);
-    else if constexpr (s < L2) return wload(A.inttp, 9, w, s - LB, lane);
-    else if constexpr (s < L1 - 1) return wload(A.m2tp, 8, w, s - L2, lane);
-    else if constexpr (s == L1 - 1) return vec(hpre + nn * kF + own);
-    else if constexpr (s < LN) return wload(A.m1tp, 8, w, s - L1, lane);
-    else if constexpr (s == LN) return vec(n1hat + nn * kF + own);
-    else if constexpr (s == LN + 1) return vec(A.ln1w + own);
-    else return vec(A.ln1b + own);
-  };
-  Stream<NS, kNodePF, decltype(load)> stream(load);
-  stream.prime();
-
-  const double *ger = gev ? gev + nn * kE : nullptr, *aer = aev + nn * kE;
-  const double gsum = ger ? slot_sum(g, ger, aer, nullptr) : 0.0;
-  const double is2 = pre2is[nn], is1 = n1is[nn];
-  if constexpr (HEADS) {
-    // the adjoints of the heads' hidden pre-activations, tiles w, w + 8, w + 16
-    const int zz = z[nn];
-    const double es = H.escale[zz - 1], qs = S.qseed[nn];
-    const double ef = S.heff[nn], hs = S.dh[nn] * (ef > 0.0 ? 1.0 : (ef < 0.0 ? -1.0 : 0.0)) / 8.0;
-    double cs = 0.0;
-    if constexpr (SRC == 2) {
-      const double ce = S.c6eff[nn];
-      cs = S.dc[nn] * (ce > 0.0 ? 1.0 : (ce < 0.0 ? -1.0 : 0.0)) / 8.0;
-    }
-#pragma unroll
-    for (int u = 0; u < 3; ++u) {
-      const int t = w + 8 * u;
-      if (t >= HT) break;
-      const double *row = u == 0 ? H.ew2 + 16 * t
-                                 : (u == 1 ? H.qw2 + 16 * (t - 8)
-                                           : (t < 20 ? H.hkey + zz * kHH + 16 * (t - 16)
-                                                     : H.ckey + zz * kHH + 16 * (t - 20)));
-      const double seed = u == 0 ? es : (u == 1 ? qs : (t < 20 ? hs : cs));
-      const v4d r = vec(row + 4 * g), pre = vec(S.hhead + nn * (16 * HT) + 16 * t + 4 * g);
-      v4d out;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) out[q] = seed * r[q] * silu_prime(pre[q]);
-      buf[t][lane] = out;
-    }
-    __syncthreads();
-  }
-  const v4d zero = v4d{0.0, 0.0, 0.0, 0.0};
-  v4d acc = zero, hold, d, hat, p, gp, n1;
-  stream.run([&](auto si, const v4d &wv) {
-    constexpr int s = decltype(si)::value;
-    if constexpr (s < X) {
-      if constexpr (HEADS) {
-        acc = mfma4(wv, buf[s][lane], acc);
-      } else if constexpr (s == 20) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) acc[r] = scale * (wv[r] + acc[r]);
-      } else if constexpr ((s & 1) == 0) {
-        hold = wv;
-      } else {
-        acc = mfma4(wv, hold, acc);
-      }
-    } else if constexpr (s == X) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) d[r] = acc[r] * wv[r];
-    } else if constexpr (s == X + 1) {
-      // LayerNorm 2 reverse; the adjoint of p and t[0:128] into LDS
-      const double a = column_sum((d[0] + d[1]) + (d[2] + d[3]));
-      const double b = column_sum((d[0] * wv[0] + d[1] * wv[1]) + (d[2] * wv[2] + d[3] * wv[3]));
-      if (g == 0) {
-        st[0][w][j] = a;
-        st[1][w][j] = b;
-      }
-      __syncthreads();
-      const double tm = A.mode2 == 0 ? sum8(st[0], j) / kF : 0.0;
-      const double tx = A.mode2 == 2 ? 0.0 : sum8(st[1], j) / kF;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) d[r] = is2 * (d[r] - tm - wv[r] * tx);
-      buf[w][lane] = d;
-    } else if constexpr (s == G) {
-      gp = mfma4(wv, d, zero);  // this chunk's share of the gate rows of gcat
-    } else if constexpr (s == G + 1) {
-      if (w == 0) gp = mfma(wv[0], gsum, gp);
-      gpart[w][lane] = gp[0];
-      __syncthreads();
-    } else if constexpr (s < L2) {
-      // gcat = Wint^T [d, gate adjoints]
-      if constexpr (s - LB < 8) acc = mfma4(wv, buf[s - LB][lane], s == LB ? zero : acc);
-      else acc = mfma(wv[0], gsum, acc);
-      if constexpr (s == L2 - 1) {
-        p = d + acc;
-        buf[8 + w][lane] = p;
-        __syncthreads();
-      }
-    } else if constexpr (s < L1 - 1) {
-      acc = mfma4(wv, buf[8 + s - L2][lane], s == L2 ? zero : acc);  // W2^T p
-    } else if constexpr (s == L1 - 1) {
-      v4d a;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) a[r] = acc[r] * silu_prime(wv[r]);
-      buf[w][lane] = a;  // every wavefront has read d
-      __syncthreads();
-    } else if constexpr (s < LN) {
-      acc = mfma4(wv, buf[s - L1][lane], s == L1 ? zero : acc);  // W1^T ghid
-    } else if constexpr (s == LN) {
-      hat = wv;
-    } else if constexpr (s == LN + 1) {
-      hold = wv;
-    } else {
-      // g = p + gact silu'(n1), then LayerNorm 1 reverse
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        n1[r] = hat[r] * hold[r] + wv[r];
-        acc[r] = (p[r] + acc[r] * silu_prime(n1[r])) * hold[r];
-      }
-      const double a = column_sum((acc[0] + acc[1]) + (acc[2] + acc[3]));
-      const double b = column_sum((acc[0] * hat[0] + acc[1] * hat[1]) + (acc[2] * hat[2] + acc[3] * hat[3]));
-      if (g == 0) {
-        st[2][w][j] = a;
-        st[3][w][j] = b;
-      }
-      __syncthreads();
-      const double tm = A.mode1 == 0 ? sum8(st[2], j) / kF : 0.0;
-      const double tx = A.mode1 == 2 ? 0.0 : sum8(st[3], j) / kF;
-      if (valid) {
-        v4d out;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) out[r] = is1 * (acc[r] - tm - hat[r] * tx);
-        *reinterpret_cast<v4d *>(gainv + nn * kF + own) = out;
-        if (w < 6) {
-          // aev: gev (1 + gate) + 2 aev cg gcat[128 + slot], channel g + 4 w
-          const int m = g + 4 * w, sl = degree_slot(m);
-          const double gc = sum8(gpart, j + 16 * sl);
-          const double e = ger ? ger[m] * (1.0 + gates[nn * 4 + sl]) : 0.0;
-          gaev[nn * kE + m] = e + gc * 2.0 * aer[m] * A.int_cg[m];
-        }
-      }
-    }
-  });
-}
-
-// ---------------------------------------------------------------- heads
+// ---------------------------------------------------------------- charges
 // per-image mean removal: out = in + (target - sum_image(in)) / count  (sign = +1)
 // or out = in - mean_image(in) (target ignored, sign = -1).  One block per image.
 __global__ __launch_bounds__(1024) void k_image_center(const std::int64_t *img_off, const double *target,
@@ -3233,7 +2706,7 @@ std::vector<double> bias_acc(const std::vector<double> &b, std::size_t M) {
 
 // Rows of 128 (64) channels in the tile-transposed order of the node rows
 // (fpos: a 4 x 4 transpose inside each run of 16).
-static std::vector<double> tile_order(const std::vector<double> &v) {
+std::vector<double> tile_order(const std::vector<double> &v) {
   std::vector<double> t(v.size());
   for (std::size_t i = 0; i < v.size(); ++i) t[(i & ~std::size_t(127)) + fpos(int(i & 127))] = v[i];
   return t;
@@ -4179,7 +3652,7 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
     HIP_CHECK(hipMemcpyAsync(xs, x0, Nz * kF * sizeof(double), hipMemcpyDeviceToDevice, s));
     hipLaunchKernelGGL(k_axpby, dim3(gNF), dim3(256), 0, s, Nz * kF, resid_[0], xs, x0l_[0], x0);
   }
-  const HeadArgs H{hw_.w1p, hw_.w1tp, hw_.b1p, hw_.ew2, hw_.qw2, hw_.hkey_bwd, hw_.ckey_bwd, hw_.escale, hw_.eshift,
+  const HeadArgs H{hw_.ho / 16, kF / 16, hw_.w1p, hw_.w1tp, hw_.b1p, hw_.ew2, hw_.qw2, hw_.hkey_bwd, hw_.ckey_bwd, hw_.escale, hw_.eshift,
                    hw_.qemb, hw_.hvshift, hw_.hkey_c, hw_.ckey_c, hw_.cvshift, hw_.eb2, hw_.qb2};
   const HeadOut HO_{hhead, eatom, qraw, heff, hir, c6eff, c6r};
   const HeadSeeds HS{hhead, qseed, dh, heff, dc, c6eff};
@@ -4232,7 +3705,7 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
       hipLaunchKernelGGL(k_class_reps, dim3(unsigned(ceil_div(std::max<std::int64_t>(N, C * C), 256))), dim3(256), 0, s,
                          int(N), z, lut, perm, static_cast<const int *>(cls_rep0_->p), crep, C * C, chist);
       hipLaunchKernelGGL(k_class_rows, dim3(unsigned(ceil_div(C * kF, 256))), dim3(256), 0, s, C, crep, xb, cxr);
-      hipLaunchKernelGGL(k_qkv_mfma, dim3(1, kHeads), dim3(256), 0, s, C, cxr, B.qkvp, cqkv);
+      hipLaunchKernelGGL(k_qkv_mfma<true>, dim3(1, kHeads), dim3(256), 0, s, C, kF, cxr, B.qkvp, cqkv);
       if (qk_norm_)
         hipLaunchKernelGGL(k_qk_norm, dim3(unsigned(ceil_div(16 * C, 256))), dim3(256), 0, s, C, cqkv, cqis);
       if (!use_rad || rad_stale_)  // with the radial tables filled, nothing reads these
@@ -4253,7 +3726,7 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
       }
     } else {
       if (b == 0 || scaled)  // the other blocks' rows come from the node chain below them
-        hipLaunchKernelGGL(k_qkv_mfma, dim3(gN64, kHeads), dim3(256), 0, s, int(N), xb, B.qkvp, qb);
+        hipLaunchKernelGGL(k_qkv_mfma<true>, dim3(gN64, kHeads), dim3(256), 0, s, int(N), kF, xb, B.qkvp, qb);
       if (qk_norm_)
         hipLaunchKernelGGL(k_qk_norm, dim3(unsigned(ceil_div(16 * N, 256))), dim3(256), 0, s, int(N), qb,
                            qkis + b * Nz * 16);
@@ -4292,14 +3765,15 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
     // LayerNorm 2, ev gate), then the next block's projections or the heads
     const NodeChainArgs NC{B.m1p, B.m1bp, B.m2p, B.m2bp, B.intp, B.intbp, B.int_cg, B.ln1w, B.ln1b, B.ln2w, B.ln2b,
                            ln_eps_, norm2_};
-#define SO3LR_NODE_FWD(TAIL)                                                                                        \
-  hipLaunchKernelGGL(k_node_fwd<TAIL>, dim3(gN16), dim3(512), 0, s, int(N), n1hb, aevb, NC, H,                      \
-                     b + 1 < L ? bw_[b + 1].qkvp : nullptr, z, hpb, gtb, xs + (b + 1) * Nz * kF,                     \
-                     evs + (b + 1) * Nz * kE, p2h, p2i, b + 1 < L ? qkv + (b + 1) * Nz * 640 : nullptr, HO_)
-    if (b + 1 < L && scaled) SO3LR_NODE_FWD(0);
-    else if (b + 1 < L) SO3LR_NODE_FWD(1);
-    else if (c6_) SO3LR_NODE_FWD(3);
-    else SO3LR_NODE_FWD(2);
+    const NodeFwdArgs NF{int(N), n1hb, aevb, NC, H, b + 1 < L ? bw_[b + 1].qkvp : nullptr, z, hpb, gtb,
+                         xs + (b + 1) * Nz * kF, evs + (b + 1) * Nz * kE, p2h, p2i,
+                         b + 1 < L ? qkv + (b + 1) * Nz * 640 : nullptr, HO_};
+#define SO3LR_NODE_FWD(TAIL, HTC) \
+  hipLaunchKernelGGL((k_node_fwd<8, true, TAIL, HTC, SlotsV1>), dim3(gN16), dim3(512), 0, s, NF, SlotsV1{})
+    if (b + 1 < L && scaled) SO3LR_NODE_FWD(0, 0);
+    else if (b + 1 < L) SO3LR_NODE_FWD(1, 0);
+    else if (c6_) SO3LR_NODE_FWD(2, 24);
+    else SO3LR_NODE_FWD(2, 20);
 #undef SO3LR_NODE_FWD
     if (scaled && b + 1 < L)
       hipLaunchKernelGGL(k_axpby, dim3(gNF), dim3(256), 0, s, Nz * kF, resid_[b + 1], xs + (b + 1) * Nz * kF,
@@ -4331,13 +3805,14 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
     // from the heads' reverse or from the projections' reverse of the block
     // above (with its residual scalar)
     const NodeChainBwdArgs NB{B.inttp, B.m2tp, B.m1tp, B.int_cg, B.ln1w, B.ln1b, B.ln2w, norm1_, norm2_};
-#define SO3LR_NODE_BWD(SRC)                                                                                        \
-  hipLaunchKernelGGL(k_node_bwd<SRC>, dim3(gN16), dim3(512), 0, s, int(N), gqkv,                                    \
-                     b + 1 < L ? bw_[b + 1].qkvtp : nullptr, b + 1 < L && scaled ? resid_[b + 1] : 1.0, H, HS, z,    \
-                     b + 1 < L ? gev : nullptr, gtb, aevb, p2h, p2i, hpb, n1hb, n1ib, NB, gainv, gaev)
-    if (b + 1 < L) SO3LR_NODE_BWD(1);
-    else if (c6_) SO3LR_NODE_BWD(2);
-    else SO3LR_NODE_BWD(0);
+    const NodeBwdArgs NR{int(N), gqkv, b + 1 < L ? bw_[b + 1].qkvtp : nullptr,
+                         b + 1 < L && scaled ? resid_[b + 1] : 1.0, H, HS, z, b + 1 < L ? gev : nullptr, gtb, aevb,
+                         p2h, p2i, hpb, n1hb, n1ib, NB, gainv, gaev};
+#define SO3LR_NODE_BWD(SRC, HTC) \
+  hipLaunchKernelGGL((k_node_bwd<8, true, SRC, HTC, SlotsV1>), dim3(gN16), dim3(512), 0, s, NR, SlotsV1{})
+    if (b + 1 < L) SO3LR_NODE_BWD(1, 0);
+    else if (c6_) SO3LR_NODE_BWD(0, 24);
+    else SO3LR_NODE_BWD(0, 20);
 #undef SO3LR_NODE_BWD
     if (scalar) {
       // scalar cross-check path: the attention reverse writes the pair

@@ -41,10 +41,13 @@ struct TopologyError : std::runtime_error {
 // Host-side weight layouts of the fp64 MFMA kernels (evaluator.hip): the
 // transpose of a rows x cols row-major matrix; a bias of length M in MFMA
 // accumulator order (a D tile starts from it); an M x K row-major matrix in
-// MFMA A-operand order, 16-row tiles by 16-wide K chunks.
+// MFMA A-operand order, 16-row tiles by 16-wide K chunks; rows of 128 or 64
+// channels in the tile-transposed order (a 4 x 4 transpose inside each run of
+// 16, fpos in evaluator.hip).
 std::vector<double> transpose(const std::vector<double> &w, std::size_t rows, std::size_t cols);
 std::vector<double> bias_acc(const std::vector<double> &b, std::size_t M);
 std::vector<double> permute_mfma(const std::vector<double> &w, std::size_t M, std::size_t K);
+std::vector<double> tile_order(const std::vector<double> &v);
 
 // Device weight pointers for one interaction block.
 struct BlockWeights {

@@ -14,6 +14,7 @@
 #include "generic.hpp"
 #include "evaluator.hpp"
 #include "mfma_ops.hpp"
+#include "node_chain.hpp"
 
 #include <algorithm>
 #include <array>
@@ -41,173 +42,6 @@ __device__ __forceinline__ double gsilu_prime(double x) {
 __device__ __forceinline__ double wsum(double v) {
   for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
   return __shfl(v, 0, 64);
-}
-
-// ------------------------------------------------------------------ GEMM
-// Y (rows x O, leading dimension ldy) = epilogue(X (rows x K, ldx) op(W) + bias)
-// with op(W) = W^T for W (O x K) row-major (the model file's (out, in)
-// layout) or, WKO, W itself for W (K x O) row-major (the adjoint of a layer:
-// X W).  rows = min(*rows_dev, rows) when rows_dev is given (the active-pair
-// count on the device).
-enum { EPI_STORE = 0, EPI_SILU, EPI_ACCUM, EPI_ADD, EPI_DSILU, EPI_DSILU_ADD };
-struct GemmArgs {
-  int rows;
-  const int *rows_dev;
-  int K, O;
-  const double *X;
-  int ldx;
-  const double *W;
-  const double *bias;
-  double *Y;
-  int ldy;
-  double *Y2;         // EPI_SILU: the pre-activation as well (may be null)
-  int ldy2;
-  const double *aux;  // EPI_DSILU*: silu' of aux
-  int ldaux;
-  const double *res;  // EPI_ADD, EPI_DSILU_ADD: added
-  int ldres;
-  // batches (grid z = nby * nbx, z = zy * nbx + zx): X, Y and res move by
-  // zy * (..)0 + zx * (..)1 elements, W by z * wbs
-  int nbx;
-  long xbs0, xbs1, ybs0, ybs1, rbs0, rbs1, wbs;
-  int ldw;  // WKO: the weight's row length (its full output width); 0: O
-};
-
-typedef double gv4d __attribute__((ext_vector_type(4)));
-
-// 64 x BN output tiles (BN = 32 NT, up to 320 columns: a filter or node
-// layer's whole output row in one workgroup, so X is read once) on fp64 MFMA
-// 16x16x4: four wavefronts in 2 x 2, each 32 rows x BN/2 columns (2 x NT
-// MFMA tiles).
-// D[i][j] += sum_k A[i][k] B[k][j] with A[i][k] = X[row i][k] (lane l gives
-// i = l % 16, k = l / 16) and B[k][j] = op(W)[k][col j] (lane l gives
-// k = l / 16, j = l % 16); lane l holds D[l / 16 + 4 r][l % 16] in register
-// r, so sixteen lanes write sixteen adjacent columns of one row.  K runs in
-// chunks of 16 through LDS; the next chunk's global loads are issued before
-// the current chunk's MFMAs.
-#ifndef SO3LR_GEMM_WAVES
-#define SO3LR_GEMM_WAVES 3
-#endif
-template <int EPI, bool WKO, int NT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SO3LR_GEMM_WAVES))) void g_gemm(GemmArgs A) {
-  constexpr int BN = 32 * NT;      // output columns per workgroup (NT MFMA column tiles per wavefront)
-  constexpr int WPT = BN / 16;     // W chunk values per thread (BN x 16 / 256)
-  __shared__ double xs[64][17];
-  __shared__ double ws[BN][17];
-  const int rows = A.rows_dev ? min(*A.rows_dev, A.rows) : A.rows;
-  // With several column blocks the grid's x is a multiple of 8 and the
-  // blocks are taken in dispatch order, (row block, column block) such that
-  // the column blocks of one row block run one after another on one XCD
-  // (dispatch goes round-robin over the 8 XCDs): the later ones read that
-  // row block's X from the XCD's L2, not HBM.
-  int rb = blockIdx.x, cb = blockIdx.y;
-  if (gridDim.y > 1) {
-    const unsigned lin = blockIdx.y * gridDim.x + blockIdx.x, k = lin >> 3;
-    rb = int((k / gridDim.y) * 8 + (lin & 7));
-    cb = int(k % gridDim.y);
-  }
-  const int row0 = rb * 64, col0 = cb * BN;
-  if (row0 >= rows) return;  // uniform over the block
-  {
-    const long zx = long(blockIdx.z) % A.nbx, zy = long(blockIdx.z) / A.nbx;
-    A.X += zy * A.xbs0 + zx * A.xbs1;
-    A.Y += zy * A.ybs0 + zx * A.ybs1;
-    if (A.res) A.res += zy * A.rbs0 + zx * A.rbs1;
-    A.W += long(blockIdx.z) * A.wbs;
-  }
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int wr0 = (wv >> 1) * 32, wc0 = (wv & 1) * (BN / 2);
-  const int li = lane & 15, lk = lane >> 4;
-  double xreg[4], wreg[WPT];
-  auto fetch = [&](int k0) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int idx = tid + 256 * q, kk = idx & 15, rr = idx >> 4;
-      const int row = row0 + rr, k = k0 + kk;
-      xreg[q] = (row < rows && k < A.K) ? A.X[std::size_t(row) * A.ldx + k] : 0.0;
-    }
-#pragma unroll
-    for (int q = 0; q < WPT; ++q) {
-      const int idx = tid + 256 * q;
-      if (WKO) {
-        const int cc = idx % BN, kk = idx / BN, col = col0 + cc, k = k0 + kk;
-        wreg[q] = (col < A.O && k < A.K) ? A.W[std::size_t(k) * (A.ldw ? A.ldw : A.O) + col] : 0.0;
-      } else {
-        const int kk = idx & 15, cc = idx >> 4, col = col0 + cc, k = k0 + kk;
-        wreg[q] = (col < A.O && k < A.K) ? A.W[std::size_t(col) * A.K + k] : 0.0;
-      }
-    }
-  };
-  auto stash = [&] {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int idx = tid + 256 * q;
-      xs[idx >> 4][idx & 15] = xreg[q];
-    }
-#pragma unroll
-    for (int q = 0; q < WPT; ++q) {
-      const int idx = tid + 256 * q;
-      if (WKO) ws[idx % BN][idx / BN] = wreg[q];
-      else ws[idx >> 4][idx & 15] = wreg[q];
-    }
-  };
-  gv4d acc[2][NT];
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < NT; ++b) acc[a][b] = gv4d{0.0, 0.0, 0.0, 0.0};
-  fetch(0);
-  stash();
-  __syncthreads();
-  for (int k0 = 0; k0 < A.K; k0 += 16) {
-    const bool more = k0 + 16 < A.K;
-    if (more) fetch(k0 + 16);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int kk = lk + 4 * v;
-      double av[2], bv[NT];
-#pragma unroll
-      for (int a = 0; a < 2; ++a) av[a] = xs[wr0 + 16 * a + li][kk];
-#pragma unroll
-      for (int b = 0; b < NT; ++b) bv[b] = ws[wc0 + 16 * b + li][kk];
-#pragma unroll
-      for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < NT; ++b) acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[a], bv[b], acc[a][b], 0, 0, 0);
-    }
-    __syncthreads();
-    if (more) {
-      stash();
-      __syncthreads();
-    }
-  }
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < NT; ++b)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = row0 + wr0 + 16 * a + lk + 4 * r;
-        const int col = col0 + wc0 + 16 * b + li;
-        if (row >= rows || col >= A.O) continue;
-        const double dot = acc[a][b][r];
-        const double pre = dot + (A.bias ? A.bias[col] : 0.0);
-        double *y = A.Y + std::size_t(row) * A.ldy + col;
-        if (EPI == EPI_STORE) {
-          *y = pre;
-        } else if (EPI == EPI_SILU) {
-          if (A.Y2) A.Y2[std::size_t(row) * A.ldy2 + col] = pre;
-          *y = gsilu(pre);
-        } else if (EPI == EPI_ACCUM) {
-          *y += pre;
-        } else if (EPI == EPI_ADD) {
-          *y = pre + A.res[std::size_t(row) * A.ldres + col];
-        } else if (EPI == EPI_DSILU) {
-          *y = dot * gsilu_prime(A.aux[std::size_t(row) * A.ldaux + col]);
-        } else {
-          *y = A.res[std::size_t(row) * A.ldres + col] + dot * gsilu_prime(A.aux[std::size_t(row) * A.ldaux + col]);
-        }
-      }
 }
 
 // ------------------------------------------------------------- node kernels
@@ -244,21 +78,13 @@ __global__ void g_axpby(std::size_t n, double a, double *x, double c, const doub
   const std::size_t i = std::size_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i < n) x[i] = a * x[i] + c * x0[i];
 }
-__global__ void g_scale(std::size_t n, double a, double *g) {
-  const std::size_t i = std::size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < n) g[i] *= a;
-}
-__global__ void g_fill(double *p, std::size_t n) {
-  const std::size_t i = std::size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0.0;
-}
 
-// The normalisation of one node row held 4 channels per lane (c = lane + 64 j,
-// j < F / 64; kokkos_post_attention_block0.cpp:97-162): mode 0 affine
-// LayerNorm (biased variance), 1 RMSNorm without scale (w = 1, b = 0
-// given), 2 none.  h = normalised row, y = h w + b, is = 1 / sigma.
-__device__ __forceinline__ void g_norm_row(int F, int mode, const double *v, const double *w, const double *b,
-                                           double eps, int lane, double *y, double *h, double &is) {
+// The first normalisation of one node row held F / 64 channels per lane
+// (kokkos_post_attention_block0.cpp:97-162): mode 0 LayerNorm (biased
+// variance), 1 RMSNorm (no mean removed), 2 none; h = normalised row,
+// is = 1 / sigma (the affine weights are applied where the row is read,
+// node_chain.hpp).
+__device__ __forceinline__ void g_norm_row(int F, int mode, const double *v, double eps, double *h, double &is) {
   const int J = F >> 6;
   double s = 0.0;
   for (int j = 0; j < J; ++j) s += v[j];
@@ -266,29 +92,16 @@ __device__ __forceinline__ void g_norm_row(int F, int mode, const double *v, con
   double q = 0.0;
   for (int j = 0; j < J; ++j) q += (v[j] - mean) * (v[j] - mean);
   is = mode == 2 ? 1.0 : 1.0 / sqrt(wsum(q) / F + eps);
-  for (int j = 0; j < J; ++j) {
-    const int c = lane + 64 * j;
-    h[j] = (v[j] - mean) * is;
-    y[j] = mode == 2 ? v[j] : h[j] * w[c] + b[c];
-  }
+  for (int j = 0; j < J; ++j) h[j] = (v[j] - mean) * is;
 }
-// Its adjoint: gx given gy, the normalised row h and 1 / sigma.
-__device__ __forceinline__ void g_norm_row_bwd(int F, int mode, const double *gy, const double *w,
-                                               const double *h, double is, int lane, double *gx) {
-  const int J = F >> 6;
-  if (mode == 2) {
-    for (int j = 0; j < J; ++j) gx[j] = gy[j];
-    return;
-  }
-  double gh[4], a = 0.0, bsum = 0.0;
-  for (int j = 0; j < J; ++j) {
-    gh[j] = mode == 0 ? gy[j] * w[lane + 64 * j] : gy[j];
-    a += gh[j];
-    bsum += gh[j] * h[j];
-  }
-  const double mg = mode == 0 ? wsum(a) / F : 0.0, mgx = wsum(bsum) / F;
-  for (int j = 0; j < J; ++j) gx[j] = is * (gh[j] - mg - h[j] * mgx);
-}
+
+// The degree slots of a model, for the node-chain kernels.
+struct SlotsG {
+  GDims d;
+  __device__ __forceinline__ int E() const { return d.E; }
+  __device__ __forceinline__ int off(int s) const { return d.off[s]; }
+  __device__ __forceinline__ int slot(int m) const { return d.slot[m]; }
+};
 
 // Dispatch block b (round-robin over the 8 XCDs) to logical block: each XCD
 // takes a contiguous run of the `active` blocks, so consecutive pairs or
@@ -305,17 +118,15 @@ __device__ __forceinline__ int g_xcd_block(int active) {
 // Attention messages, node-major (kokkos_integrated_block0.cpp:330-385):
 // node n receives from each incident pair's partner o the invariant message
 // fc alpha v_o and the equivariant fc alpha_ev Y (parity of the direction),
-// then the residual and the first normalisation (and silu of it, the MLP
-// input).  One wavefront per node.
+// then the residual and the first normalisation.  ev null: zero (block 0).
+// One wavefront per node.
 __global__ __launch_bounds__(256) void g_attn_msg(GDims d, int N, const int *__restrict__ inc_off,
                                                   const int *__restrict__ iact, const int *__restrict__ iother,
                                                   const double *__restrict__ x, const double *__restrict__ ev,
                                                   const double *__restrict__ qkv, const double *__restrict__ pY,
                                                   const double *__restrict__ pfc, const double *__restrict__ palpha,
-                                                  const double *__restrict__ lnw, const double *__restrict__ lnb,
-                                                  double eps, int mode, double *__restrict__ n1,
-                                                  double *__restrict__ n1hat, double *__restrict__ n1is,
-                                                  double *__restrict__ act, double *__restrict__ aev) {
+                                                  double eps, int mode, double *__restrict__ n1hat,
+                                                  double *__restrict__ n1is, double *__restrict__ aev) {
   const int lane = threadIdx.x & 63;
   const int blk = g_xcd_block((N + 3) / 4);
   if (blk < 0) return;
@@ -373,191 +184,15 @@ __global__ __launch_bounds__(256) void g_attn_msg(GDims d, int N, const int *__r
     add(A);
     if (two) add(B);
   });
-  double v[4], y[4], h[4], is;
+  double v[4], h[4], is;
   for (int j = 0; j < J; ++j) v[j] = x[std::size_t(n) * F + lane + 64 * j] + di[j];
-  g_norm_row(F, mode, v, lnw, lnb, eps, lane, y, h, is);
-  for (int j = 0; j < J; ++j) {
-    const std::size_t i = std::size_t(n) * F + lane + 64 * j;
-    n1[i] = y[j];
-    n1hat[i] = h[j];
-    act[i] = gsilu(y[j]);
-  }
+  g_norm_row(F, mode, v, eps, h, is);
+  for (int j = 0; j < J; ++j) n1hat[std::size_t(n) * F + lane + 64 * j] = h[j];
   if (lane == 0) n1is[n] = is;
   for (int j = 0; j < 2; ++j) {
     const int c = lane + 64 * j;
-    if (c < E) aev[std::size_t(n) * E + c] = ev[std::size_t(n) * E + c] + de[j];
+    if (c < E) aev[std::size_t(n) * E + c] = (ev ? ev[std::size_t(n) * E + c] : 0.0) + de[j];
   }
-}
-
-// Interaction input: cat[n][F + s] = sum_{c in slot s} aev_c^2 cg_c
-// (kokkos_post_attention_block0.cpp:302-333).
-__global__ void g_cat_inv(GDims d, int N, const double *__restrict__ aev, const double *__restrict__ cg,
-                          double *__restrict__ cat) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= N * d.NH) return;
-  const int n = t / d.NH, s = t % d.NH;
-  double acc = 0.0;
-  for (int c = d.off[s]; c < d.off[s + 1]; ++c) {
-    const double a = aev[std::size_t(n) * d.E + c];
-    acc += a * a * cg[c];
-  }
-  cat[std::size_t(n) * d.NI + d.F + s] = acc;
-}
-
-// Block output: x' = norm2(p + t[0:F]), ev' = aev (1 + t[F + slot]).
-__global__ __launch_bounds__(256) void g_node_post(GDims d, int N, const double *__restrict__ cat,
-                                                   const double *__restrict__ tout, const double *__restrict__ aev,
-                                                   const double *__restrict__ lnw, const double *__restrict__ lnb,
-                                                   double eps, int mode, double *__restrict__ xout,
-                                                   double *__restrict__ evout, double *__restrict__ pre2hat,
-                                                   double *__restrict__ pre2is) {
-  const int lane = threadIdx.x & 63;
-  const int n = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (n >= N) return;
-  const int F = d.F, J = F >> 6;
-  const std::size_t r = std::size_t(n) * d.NI;
-  double v[4], y[4], h[4], is;
-  for (int j = 0; j < J; ++j) v[j] = cat[r + lane + 64 * j] + tout[r + lane + 64 * j];
-  g_norm_row(F, mode, v, lnw, lnb, eps, lane, y, h, is);
-  for (int j = 0; j < J; ++j) {
-    const std::size_t i = std::size_t(n) * F + lane + 64 * j;
-    xout[i] = y[j];
-    pre2hat[i] = h[j];
-  }
-  if (lane == 0) pre2is[n] = is;
-  for (int j = 0; j < 2; ++j) {
-    const int c = lane + 64 * j;
-    if (c < d.E) evout[std::size_t(n) * d.E + c] = aev[std::size_t(n) * d.E + c] * (1.0 + tout[r + F + d.slot[c]]);
-  }
-}
-
-// Output heads from their hidden activations (kokkos_output_heads.cpp:137-176):
-// energy (HK), charge (HK), Hirshfeld and C6 ratio keys (64 each).
-__global__ __launch_bounds__(256) void g_heads(GDims d, int N, const int *__restrict__ z, const double *__restrict__ hact,
-                                               const double *__restrict__ hkey, GHeads H, double *__restrict__ eatom,
-                                               double *__restrict__ qraw, double *__restrict__ heff,
-                                               double *__restrict__ hir, double *__restrict__ c6eff,
-                                               double *__restrict__ c6r) {
-  const int lane = threadIdx.x & 63;
-  const int n = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (n >= N) return;
-  const double *a = hact + std::size_t(n) * d.HO;
-  double e = 0.0, q = 0.0;
-  for (int c = lane; c < d.HK; c += 64) {
-    e += H.ew2[c] * a[c];
-    q += H.qw2[c] * a[d.HK + c];
-  }
-  e = wsum(e);
-  q = wsum(q);
-  const int zz = z[n];
-  const double hk = wsum(H.hqemb[zz * 64 + lane] * hkey[std::size_t(n) * 128 + lane]);
-  const double ck = d.c6 ? wsum(H.cqemb[zz * 64 + lane] * hkey[std::size_t(n) * 128 + 64 + lane]) : 0.0;
-  if (lane == 0) {
-    eatom[n] = (e + H.eb2) * H.escale[zz - 1] + H.eshift[zz - 1];
-    qraw[n] = q + H.qb2 + H.qemb[zz];
-    const double hv = H.hvshift[zz] + hk / 8.0;  // q . k / sqrt(64)
-    heff[n] = hv;
-    hir[n] = fabs(hv);
-    if (d.c6) {
-      const double cv = H.cvshift[zz] + ck / 8.0;
-      c6eff[n] = cv;
-      c6r[n] = fabs(cv);
-    }
-  }
-}
-
-// Heads in reverse to the adjoint of their hidden pre-activations
-// (kokkos_output_heads.cpp:182-220): energy seed 1, charge seed qseed,
-// Hirshfeld dE/dh, C6 dE/dc.
-__global__ __launch_bounds__(256) void g_heads_bwd(GDims d, int N, const int *__restrict__ z,
-                                                   const double *__restrict__ hpre, const double *__restrict__ qseed,
-                                                   const double *__restrict__ dh, const double *__restrict__ heff,
-                                                   const double *__restrict__ dc, const double *__restrict__ c6eff,
-                                                   GHeads H, double *__restrict__ ghead) {
-  const int lane = threadIdx.x & 63;
-  const int n = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (n >= N) return;
-  const int zz = z[n], HK = d.HK;
-  const double *pre = hpre + std::size_t(n) * d.HO;
-  double *g = ghead + std::size_t(n) * d.HO;
-  const double es = H.escale[zz - 1], qs = qseed[n];
-  for (int c = lane; c < HK; c += 64) {
-    g[c] = es * H.ew2[c] * gsilu_prime(pre[c]);
-    g[HK + c] = qs * H.qw2[c] * gsilu_prime(pre[HK + c]);
-  }
-  auto ratio = [&](double seed, double logit, const double *qemb, const double *w2, int at) {
-    const double sg = logit > 0.0 ? 1.0 : (logit < 0.0 ? -1.0 : 0.0);
-    const double s = seed * sg / 8.0;
-    double acc = 0.0;  // sum_j W2[j][lane] q_emb[z][j] s
-    for (int j = 0; j < 64; ++j) acc += w2[j * 64 + lane] * (s * qemb[zz * 64 + j]);
-    g[at + lane] = acc * gsilu_prime(pre[at + lane]);
-  };
-  ratio(dh[n], heff[n], H.hqemb, H.hw2, 2 * HK);
-  if (d.c6) ratio(dc[n], c6eff[n], H.cqemb, H.cw2, 2 * HK + 64);
-}
-
-// Reverse of the second normalisation and the ev gate (kokkos_post_attention_reverse.cpp):
-// gt[0:F] = dnorm2, gt[F + s] = sum_{c in s} gev_c aev_c, ga = gev (1 + t[F + slot]).
-__global__ __launch_bounds__(256) void g_ln2_bwd(GDims d, int N, const double *__restrict__ gx,
-                                                 const double *__restrict__ gev, const double *__restrict__ tout,
-                                                 const double *__restrict__ aev, const double *__restrict__ pre2hat,
-                                                 const double *__restrict__ pre2is, const double *__restrict__ lnw,
-                                                 int mode, double *__restrict__ gt, double *__restrict__ ga) {
-  const int lane = threadIdx.x & 63;
-  const int n = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (n >= N) return;
-  const int F = d.F, J = F >> 6;
-  double gy[4], h[4], gxo[4];
-  for (int j = 0; j < J; ++j) {
-    gy[j] = gx[std::size_t(n) * F + lane + 64 * j];
-    h[j] = pre2hat[std::size_t(n) * F + lane + 64 * j];
-  }
-  g_norm_row_bwd(F, mode, gy, lnw, h, pre2is[n], lane, gxo);
-  const std::size_t r = std::size_t(n) * d.NI;
-  for (int j = 0; j < J; ++j) gt[r + lane + 64 * j] = gxo[j];
-  if (lane < d.NH) {
-    double acc = 0.0;
-    for (int c = d.off[lane]; c < d.off[lane + 1]; ++c) acc += gev[std::size_t(n) * d.E + c] * aev[std::size_t(n) * d.E + c];
-    gt[r + F + lane] = acc;
-  }
-  for (int j = 0; j < 2; ++j) {
-    const int c = lane + 64 * j;
-    if (c < d.E) ga[std::size_t(n) * d.E + c] = gev[std::size_t(n) * d.E + c] * (1.0 + tout[r + F + d.slot[c]]);
-  }
-}
-
-// gp = gt[0:F] + gcat[0:F]; ga += gcat[F + slot] 2 aev cg.
-__global__ void g_cat_bwd(GDims d, int N, const double *__restrict__ gt, const double *__restrict__ gcat,
-                          const double *__restrict__ aev, const double *__restrict__ cg, double *__restrict__ gp,
-                          double *__restrict__ ga) {
-  const std::size_t t = std::size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int W = d.F + d.E;
-  if (t >= std::size_t(N) * W) return;
-  const int n = int(t / W), c = int(t % W);
-  const std::size_t r = std::size_t(n) * d.NI;
-  if (c < d.F) {
-    gp[std::size_t(n) * d.F + c] = gt[r + c] + gcat[r + c];
-  } else {
-    const int m = c - d.F;
-    const std::size_t i = std::size_t(n) * d.E + m;
-    ga[i] += gcat[r + d.F + d.slot[m]] * 2.0 * aev[i] * cg[m];
-  }
-}
-
-__global__ __launch_bounds__(256) void g_ln1_bwd(int F, int N, const double *__restrict__ gn1,
-                                                 const double *__restrict__ lnw, const double *__restrict__ n1hat,
-                                                 const double *__restrict__ n1is, int mode, double *__restrict__ gainv) {
-  const int lane = threadIdx.x & 63;
-  const int n = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (n >= N) return;
-  const int J = F >> 6;
-  double gy[4], h[4], go[4];
-  for (int j = 0; j < J; ++j) {
-    gy[j] = gn1[std::size_t(n) * F + lane + 64 * j];
-    h[j] = n1hat[std::size_t(n) * F + lane + 64 * j];
-  }
-  g_norm_row_bwd(F, mode, gy, lnw, h, n1is[n], lane, go);
-  for (int j = 0; j < J; ++j) gainv[std::size_t(n) * F + lane + 64 * j] = go[j];
 }
 
 // The attention reverse's node gathers (kokkos_attention_scatter_reverse.cpp:280-500):
@@ -670,15 +305,15 @@ __global__ void g_rbf(int R, const int *nact, int cap, const double *__restrict_
 }
 
 // Equivariant invariants per slot: s = sum_{c in slot} (ev_a - ev_b)^2 cg
-// (kokkos_integrated_block0.cpp:166-195).
+// (kokkos_integrated_block0.cpp:166-195).  ev null: zero (block 0).
 __global__ void g_pair_inv(GDims d, const int *nact, int cap, const int *__restrict__ pa,
                            const double *__restrict__ ev, const double *__restrict__ cg, double *__restrict__ ps) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   const int p = t / d.NH, s = t % d.NH;
   if (p >= min(*nact, cap)) return;
-  const double *ea = ev + std::size_t(pa[2 * p]) * d.E, *eb = ev + std::size_t(pa[2 * p + 1]) * d.E;
   double acc = 0.0;
-  for (int c = d.off[s]; c < d.off[s + 1]; ++c) {
+  for (int c = d.off[s]; ev && c < d.off[s + 1]; ++c) {
+    const double *ea = ev + std::size_t(pa[2 * p]) * d.E, *eb = ev + std::size_t(pa[2 * p + 1]) * d.E;
     const double x = ea[c] - eb[c];
     acc += x * x * cg[c];
   }
@@ -1638,84 +1273,21 @@ unsigned blocks_for(std::size_t n, int per) { return unsigned((n + std::size_t(p
 // ------------------------------------------------------------------ host side
 namespace {
 enum Buf {
-  XS = 0, EVS, QKV, QKIS, AEV, N1, N1HAT, N1IS, HPRE, TOUT, PRE2HAT, PRE2IS,
-  ACT, HID, CAT, HACT, HHPRE, HKEY, GHEAD,
-  GX, GEV, GT, GCAT, GA, GP, GHID, GN1, GAINV, GQKV,
+  XS = 0, EVS, QKV, QKIS, AEV, N1HAT, N1IS, HPRE, GATES, PRE2HAT, PRE2IS, HHEAD,
+  GEV, GA, GAINV, GQKV,
   RBF, PS, PF, PALPHA, PSC, DFC, DS, CLS_M, CLS_B,
   NBUF
 };
 static_assert(NBUF <= GenericPath::kBuffers, "generic path buffer table");
 
-#ifndef SO3LR_GEMM_MAX_NT
-#define SO3LR_GEMM_MAX_NT 4
-#endif
-constexpr int kGemmMaxNT = SO3LR_GEMM_MAX_NT;
-
-template <int EPI, bool WKO>
-void gemm(hipStream_t s, int rows, const int *rows_dev, int K, int O, const double *X, int ldx, const double *W,
-          const double *bias, double *Y, int ldy, const double *aux = nullptr, int ldaux = 0,
-          const double *res = nullptr, int ldres = 0, double *Y2 = nullptr, int ldy2 = 0) {
-  if (rows <= 0) return;
-  GemmArgs A{rows, rows_dev, K, O, X, ldx, W, bias, Y, ldy, Y2, ldy2, aux, ldaux, res, ldres,
-             1, 0, 0, 0, 0, 0, 0, 0, 0};
-  // column blocks of 32 kGemmMaxNT columns, and the rest (O not a multiple
-  // of that, e.g. 320 = 2 x 128 + 64) as a launch of its own on the columns
-  // left, so no block computes padded columns; NT = 32-column tiles per
-  // wavefront
-  const int cmax = 32 * kGemmMaxNT;
-  const dim3 gr(blocks_for(std::size_t(rows), 64));
-  auto launch = [&](GemmArgs B, int nb, int tiles) {
-    const dim3 grid(nb > 1 ? (gr.x + 7) / 8 * 8 : gr.x, unsigned(nb));
-#define G_GEMM_NT(NT)                                                              \
-  if (tiles <= NT) {                                                               \
-    hipLaunchKernelGGL((g_gemm<EPI, WKO, NT>), grid, dim3(256), 0, s, B);          \
-    return;                                                                        \
-  }
-    G_GEMM_NT(2) G_GEMM_NT(4) G_GEMM_NT(6) G_GEMM_NT(8) G_GEMM_NT(10)
-#undef G_GEMM_NT
-    throw std::logic_error("SO3LR: generic GEMM with more than 320 columns per block");
-  };
-  const int full = O / cmax, rest = O - full * cmax;
-  if (full == 0 || rest == 0) {
-    const int nb = (O + cmax - 1) / cmax, cols = (O + nb - 1) / nb;
-    launch(A, nb, (cols + 31) / 32);
-    return;
-  }
-  GemmArgs M = A;
-  M.O = full * cmax;
-  if (WKO) M.ldw = O;
-  launch(M, full, kGemmMaxNT);
-  GemmArgs R = A;
-  const int c0 = full * cmax;
-  R.O = rest;
-  if (WKO) {
-    R.W = W + c0;
-    R.ldw = O;
-  } else {
-    R.W = W + std::size_t(c0) * K;
-  }
-  if (bias) R.bias = bias + c0;
-  R.Y = Y + c0;
-  if (Y2) R.Y2 = Y2 + c0;
-  if (aux) R.aux = aux + c0;
-  if (res) R.res = res + c0;
-  launch(R, 1, (rest + 31) / 32);
-}
-// Per-head 32 x 32 projections as one batched launch (O = K = 32).
-template <int EPI, bool WKO>
-void gemm_heads(hipStream_t s, int rows, int nby, int nbx, const double *X, int ldx, long xbs0, long xbs1,
-                const double *W, long wbs, double *Y, int ldy, long ybs0, long ybs1, const double *res = nullptr,
-                int ldres = 0, long rbs0 = 0, long rbs1 = 0) {
-  if (rows <= 0) return;
-  GemmArgs A{rows, nullptr, 32, 32, X, ldx, W, nullptr, Y, ldy, nullptr, 0, nullptr, 0, res, ldres,
-             nbx, xbs0, xbs1, ybs0, ybs1, rbs0, rbs1, wbs, 0};
-  hipLaunchKernelGGL((g_gemm<EPI, WKO, 2>), dim3(blocks_for(std::size_t(rows), 64), 1, unsigned(nby * nbx)),
-                     dim3(256), 0, s, A);
-}
 }  // namespace
 
 namespace {
 bool cls_on(const GContext &c) { return c.cls_C > 0; }
+HeadArgs head_args(const GDims &d, const GHeads &H) {
+  return HeadArgs{d.HT, d.HKT, H.w1p, H.w1tp, H.b1p, H.ew2, H.qw2, H.hkey, H.ckey, H.escale, H.eshift, H.qemb,
+                  H.hvshift, H.hkey_c, H.ckey_c, H.cvshift, H.eb2, H.qb2};
+}
 
 // Slots of block 0's element-pair order, at most: every nonempty bucket
 // padded by fewer than kB0Pad
@@ -2087,7 +1659,8 @@ GenericPath::GenericPath(const Model &m, const std::function<const double *(cons
   d.HK = a.head_hidden;
   d.NI = a.F + a.heads;
   d.c6 = a.c6_head ? 1 : 0;
-  d.HO = 2 * d.HK + 64 + (d.c6 ? 64 : 0);
+  d.HKT = (d.HK + 15) / 16;
+  d.HT = 2 * d.HKT + 4 + (d.c6 ? 4 : 0);
   if ((d.F != 128 && d.F != 256) || d.NH * 32 != d.F)
     throw std::logic_error("SO3LR: generic path given widths other than F = 128 or 256 in heads of 32");
   int off = 0;
@@ -2121,7 +1694,21 @@ GenericPath::GenericPath(const Model &m, const std::function<const double *(cons
       const auto w = m.f64(at + nm, {NH, 32, 32});
       qkv.insert(qkv.end(), w.begin(), w.end());
     }
-    B.wqkv = up(qkv);
+    {
+      // per head the (160 x 32) projections as MFMA operands, and their transposes
+      std::vector<double> fwdp, bwdp;
+      for (std::size_t h = 0; h < NH; ++h) {
+        std::vector<double> Mh(160 * 32);  // [w*32 + o][k] = W[w][h][k][o]
+        for (std::size_t w = 0; w < 5; ++w)
+          for (std::size_t k = 0; k < 32; ++k)
+            for (std::size_t o = 0; o < 32; ++o) Mh[(w * 32 + o) * 32 + k] = qkv[((w * NH + h) * 32 + k) * 32 + o];
+        const auto pf = permute_mfma(Mh, 160, 32), pb = permute_mfma(transpose(Mh, 160, 32), 32, 160);
+        fwdp.insert(fwdp.end(), pf.begin(), pf.end());
+        bwdp.insert(bwdp.end(), pb.begin(), pb.end());
+      }
+      B.qkvp = up(fwdp);
+      B.qkvtp = up(bwdp);
+    }
     for (int k = 0; k < 2; ++k) {
       // the transformer-level filter nets (kokkos_integrated_block0.cpp:507-512)
       const std::string f = p + (k == 0 ? "filter_net_inv." : "filter_net_ev.");
@@ -2181,42 +1768,64 @@ GenericPath::GenericPath(const Model &m, const std::function<const double *(cons
     B.ln1b = up(ln1 ? m.f64(p + "layer_norm_inv_1.bias", {F}) : zeros);
     B.ln2w = up(ln2 ? m.f64(p + "layer_norm_inv_2.weight", {F}) : ones);
     B.ln2b = up(ln2 ? m.f64(p + "layer_norm_inv_2.bias", {F}) : zeros);
-    B.m1 = up(m.f64(p + "mlp_1.1.weight", {F, F}));
-    B.m1b = up(m.f64(p + "mlp_1.1.bias", {F}));
-    B.m2 = up(m.f64(p + "mlp_1.3.weight", {F, F}));
-    B.m2b = up(m.f64(p + "mlp_1.3.bias", {F}));
-    B.wi = up(m.f64(p + "interaction_block.linear_layer.weight", {NI, NI}));
-    B.bi = up(m.f64(p + "interaction_block.linear_layer.bias", {NI}));
+    const auto m1 = m.f64(p + "mlp_1.1.weight", {F, F}), m2 = m.f64(p + "mlp_1.3.weight", {F, F}),
+               wi = m.f64(p + "interaction_block.linear_layer.weight", {NI, NI});
+    B.m1p = up(permute_mfma(m1, F, F));
+    B.m2p = up(permute_mfma(m2, F, F));
+    B.intp = up(permute_mfma(wi, NI, NI));
+    B.m1tp = up(permute_mfma(transpose(m1, F, F), F, F));
+    B.m2tp = up(permute_mfma(transpose(m2, F, F), F, F));
+    B.inttp = up(permute_mfma(transpose(wi, NI, NI), NI, NI));
+    B.m1bp = up(bias_acc(m.f64(p + "mlp_1.1.bias", {F}), F));
+    B.m2bp = up(bias_acc(m.f64(p + "mlp_1.3.bias", {F}), F));
+    B.intbp = up(bias_acc(m.f64(p + "interaction_block.linear_layer.bias", {NI}), NI));
   }
   const std::string e = "model.atomic_energy_output_block.", q = "model.partial_charges_output_block.",
                     h = "model.hirshfeld_output_block.", c6h = "model.c6_ratios_output_block.";
-  std::vector<double> w1 = m.f64(e + "layers.0.weight", {HK, F});
-  std::vector<double> b1 = m.f64(e + "layers.0.bias", {HK});
-  auto append = [](std::vector<double> &dst, const std::vector<double> &src) { dst.insert(dst.end(), src.begin(), src.end()); };
-  append(w1, m.f64(q + "transform_inv_features.0.weight", {HK, F}));
-  append(b1, m.f64(q + "transform_inv_features.0.bias", {HK}));
-  append(w1, m.f64(h + "transform_features.0.weight", {HH, F}));
-  append(b1, m.f64(h + "transform_features.0.bias", {HH}));
-  if (d.c6) {
-    append(w1, m.f64(c6h + "transform_features.0.weight", {HH, F}));
-    append(b1, m.f64(c6h + "transform_features.0.bias", {HH}));
-  }
-  hw_.w1 = up(w1);
-  hw_.b1 = up(b1);
-  hw_.hw2 = up(m.f64(h + "transform_features.2.weight", {HH, HH}));
-  hw_.hb2 = up(m.f64(h + "transform_features.2.bias", {HH}));
-  hw_.hqemb = up(m.f64(h + "q_embedding.weight", {100, HH}));
-  hw_.hvshift = up(m.f64(h + "v_shift_embedding.weight", {100, 1}));
-  hw_.cw2 = hw_.cb2 = hw_.cqemb = hw_.cvshift = nullptr;
-  if (d.c6) {
-    hw_.cw2 = up(m.f64(c6h + "transform_features.2.weight", {HH, HH}));
-    hw_.cb2 = up(m.f64(c6h + "transform_features.2.bias", {HH}));
-    hw_.cqemb = up(m.f64(c6h + "q_embedding.weight", {100, HH}));
-    hw_.cvshift = up(m.f64(c6h + "v_shift_embedding.weight", {100, 1}));
-  }
-  hw_.ew2 = up(m.f64(e + "final_layer.weight", {1, HK}));
+  // the heads' hidden layers stacked, energy and charge units padded with
+  // zero rows to whole tiles (their activations are then 0, and so are the
+  // padded output weights)
+  const std::size_t HP = 16 * std::size_t(d.HKT), HT = 16 * std::size_t(d.HT);
+  std::vector<double> w1(HT * F, 0.0), b1(HT, 0.0);
+  auto place = [&](const std::string &pre, std::size_t rows, std::size_t at) {
+    const auto w = m.f64(pre + ".weight", {rows, F}), bias = m.f64(pre + ".bias", {rows});
+    std::copy(w.begin(), w.end(), w1.begin() + std::ptrdiff_t(at * F));
+    std::copy(bias.begin(), bias.end(), b1.begin() + std::ptrdiff_t(at));
+  };
+  place(e + "layers.0", HK, 0);
+  place(q + "transform_inv_features.0", HK, HP);
+  place(h + "transform_features.0", HH, 2 * HP);
+  if (d.c6) place(c6h + "transform_features.0", HH, 2 * HP + HH);
+  hw_.w1p = up(permute_mfma(w1, HT, F));
+  hw_.w1tp = up(permute_mfma(transpose(w1, HT, F), F, HT));
+  hw_.b1p = up(bias_acc(b1, HT));
+  auto padded = [&](std::vector<double> v) {
+    v.resize(HP, 0.0);
+    return up(tile_order(v));
+  };
+  // a ratio head's logit q_emb[z] . (W2 a + b2) contracted to u[z] . a + c[z],
+  // u[z] = W2^T q_emb[z] (the reverse needs u[z] as well)
+  auto ratio_head = [&](const std::string &pre, const double *&key, const double *&kc, const double *&vsh) {
+    const auto w2 = m.f64(pre + "transform_features.2.weight", {HH, HH});
+    const auto qe = m.f64(pre + "q_embedding.weight", {100, HH});
+    const auto b2 = m.f64(pre + "transform_features.2.bias", {HH});
+    std::vector<double> u(100 * HH, 0.0), c(100, 0.0);
+    for (std::size_t zz = 0; zz < 100; ++zz)
+      for (std::size_t jj = 0; jj < HH; ++jj) {
+        const double qv = qe[zz * HH + jj];
+        for (std::size_t i = 0; i < HH; ++i) u[zz * HH + i] += w2[jj * HH + i] * qv;
+        c[zz] += qv * b2[jj];
+      }
+    key = up(tile_order(u));
+    kc = up(c);
+    vsh = up(m.f64(pre + "v_shift_embedding.weight", {100, 1}));
+  };
+  ratio_head(h, hw_.hkey, hw_.hkey_c, hw_.hvshift);
+  hw_.ckey = hw_.ckey_c = hw_.cvshift = nullptr;
+  if (d.c6) ratio_head(c6h, hw_.ckey, hw_.ckey_c, hw_.cvshift);
+  hw_.ew2 = padded(m.f64(e + "final_layer.weight", {1, HK}));
   hw_.eb2 = m.f64(e + "final_layer.bias", {1})[0];
-  hw_.qw2 = up(m.f64(q + "transform_inv_features.2.weight", {1, HK}));
+  hw_.qw2 = padded(m.f64(q + "transform_inv_features.2.weight", {1, HK}));
   hw_.qb2 = m.f64(q + "transform_inv_features.2.bias", {1})[0];
   hw_.escale = up(m.f64(e + "energy_scales.weight", {1, 118}));
   hw_.eshift = up(m.f64(e + "energy_shifts", {118}));
@@ -2317,13 +1926,11 @@ GenericPath::GenericPath(const Model &m, const std::function<const double *(cons
 
 void GenericPath::carve(int N, int cap, int C, const std::function<double *(int, std::size_t)> &take) {
   const std::size_t n = std::size_t(N), P = std::size_t(std::max(cap, 1)), L = std::size_t(layers_);
-  const std::size_t F = std::size_t(d_.F), E = std::size_t(d_.E), NH = std::size_t(d_.NH), NI = std::size_t(d_.NI),
-                    R = std::size_t(d_.R), HO = std::size_t(d_.HO);
+  const std::size_t F = std::size_t(d_.F), E = std::size_t(d_.E), NH = std::size_t(d_.NH), R = std::size_t(d_.R);
   const std::size_t sizes[NBUF] = {
-      (L + 1) * n * F, (L + 1) * n * E, L * n * 5 * F, L * n * 4 * NH, L * n * E, L * n * F, L * n * F, L * n,
-      L * n * F, L * n * NI, L * n * F, L * n,
-      n * F, n * F, n * NI, n * HO, n * HO, n * 128, n * HO,
-      n * F, n * E, n * NI, n * NI, n * E, n * F, n * F, n * F, n * F, n * 5 * F,
+      (L + 1) * n * F, (L + 1) * n * E, L * n * 5 * F, L * n * 4 * NH, L * n * E, L * n * F, L * n,
+      L * n * F, L * n * NH, L * n * F, L * n, n * 16 * std::size_t(d_.HT),
+      n * E, n * E, n * F, n * 5 * F,
       // the pairs' basis rows, s, filter rows (none for block 0 on the
       // element-pair tables), logits, the logits' adjoints, dE/dfc, dE/ds
       P * R, L * P * NH, (L - (C > 0 ? 1 : 0)) * P * 2 * F, L * P * 4 * NH, P * 4 * NH, P, P * NH,
@@ -2343,16 +1950,17 @@ double *GenericPath::pf_rows(const GContext &c, int b) const {
 void GenericPath::forward(const GContext &c) {
   const GDims &d = d_;
   const hipStream_t s = c.s;
-  const int N = c.N, cap = c.cap, F = d.F, E = d.E, NH = d.NH, NI = d.NI, R = d.R, FH = d.FH;
+  const int N = c.N, cap = c.cap, F = d.F, E = d.E, NH = d.NH, R = d.R, FH = d.FH;
   const std::size_t n = std::size_t(N), P = std::size_t(std::max(cap, 1));
-  const unsigned g4 = blocks_for(n, 4), g4x = (g4 + 7) / 8 * 8;  // g4x: g_xcd_block's grids
+  const unsigned g4x = (blocks_for(n, 4) + 7) / 8 * 8;  // g_xcd_block's grids
   const unsigned gP = blocks_for(P, 256);
   double *xs = b_[XS], *evs = b_[EVS];
-  G_CHECK(hipMemcpyAsync(xs, c.x0, n * F * sizeof(double), hipMemcpyDeviceToDevice, s));
-  if (!c.resid->empty())
+  const bool scaled = !c.resid->empty();
+  if (scaled) {
+    G_CHECK(hipMemcpyAsync(xs, c.x0, n * F * sizeof(double), hipMemcpyDeviceToDevice, s));
     hipLaunchKernelGGL(g_axpby, dim3(blocks_for(n * F, 256)), dim3(256), 0, s, n * F, (*c.resid)[0], xs,
                        (*c.x0l)[0], c.x0);
-  hipLaunchKernelGGL(g_fill, dim3(blocks_for(n * E, 256)), dim3(256), 0, s, evs, n * E);
+  }
   // the basis rows, read by the full filter chains only: not when every
   // block runs on its radial tables
   if (!(c.rint_order && cls_on(c) && c.rad_tab))
@@ -2360,15 +1968,18 @@ void GenericPath::forward(const GContext &c) {
                        hw_.rbf_kr, b_[RBF]);
   for (int b = 0; b < layers_; ++b) {
     const GBlock &B = bw_[b];
-    double *xb = xs + b * n * F, *evb = evs + b * n * E;
+    // block 0's input is the embedding, ev = 0
+    const double *xb = b == 0 && !scaled ? c.x0 : xs + b * n * F, *evb = b == 0 ? nullptr : evs + b * n * E;
     double *qb = b_[QKV] + b * n * 5 * F, *aevb = b_[AEV] + b * n * E;
-    double *n1b = b_[N1] + b * n * F, *n1hb = b_[N1HAT] + b * n * F, *n1ib = b_[N1IS] + b * n;
-    double *hpb = b_[HPRE] + b * n * F, *tb = b_[TOUT] + b * n * NI;
+    double *n1hb = b_[N1HAT] + b * n * F, *n1ib = b_[N1IS] + b * n;
+    double *hpb = b_[HPRE] + b * n * F, *gtb = b_[GATES] + b * n * NH;
     double *p2h = b_[PRE2HAT] + b * n * F, *p2i = b_[PRE2IS] + b * n;
     double *psb = b_[PS] + b * P * NH, *pfb = pf_rows(c, b), *pab = b_[PALPHA] + b * P * 4 * NH;
     // q k v q_ev k_ev per head: out[w][h*32 + o] = sum_k x[h*32 + k] W[w][h][k][o]
-    // (kokkos_integrated_block0.cpp:257-287), batch z = w NH + h
-    gemm_heads<EPI_STORE, true>(s, N, 5, NH, xb, F, 0, 32, B.wqkv, 1024, qb, 5 * F, F, 32);
+    // (kokkos_integrated_block0.cpp:257-287); the other blocks' rows come from
+    // the node chain below them
+    if (b == 0 || scaled)
+      hipLaunchKernelGGL(k_qkv_mfma<false>, dim3(blocks_for(n, 64), unsigned(NH)), dim3(256), 0, s, N, F, xb, B.qkvp, qb);
     if (c.qk_norm)
       hipLaunchKernelGGL(g_qk_norm, dim3(blocks_for(n * 4 * NH, 256)), dim3(256), 0, s, N, F, NH, qb,
                          b_[QKIS] + b * n * 4 * NH);
@@ -2418,60 +2029,71 @@ void GenericPath::forward(const GContext &c) {
     }
     }
     hipLaunchKernelGGL(g_attn_msg, dim3(g4x), dim3(256), 0, s, d, N, c.inc_off, c.iact, c.iother, xb, evb, qb, c.pY,
-                       c.pfc, pab, B.ln1w, B.ln1b, c.ln_eps, c.norm1, n1b, n1hb, n1ib, b_[ACT], aevb);
-    // post-attention node chain (kokkos_post_attention_block0.cpp:165-300)
-    gemm<EPI_SILU, false>(s, N, nullptr, F, F, b_[ACT], F, B.m1, B.m1b, b_[HID], F, nullptr, 0, nullptr, 0, hpb, F);
-    gemm<EPI_ADD, false>(s, N, nullptr, F, F, b_[HID], F, B.m2, B.m2b, b_[CAT], NI, nullptr, 0, n1b, F);
-    hipLaunchKernelGGL(g_cat_inv, dim3(blocks_for(n * NH, 256)), dim3(256), 0, s, d, N, aevb, B.int_cg, b_[CAT]);
-    gemm<EPI_STORE, false>(s, N, nullptr, NI, NI, b_[CAT], NI, B.wi, B.bi, tb, NI);
-    hipLaunchKernelGGL(g_node_post, dim3(g4), dim3(256), 0, s, d, N, b_[CAT], tb, aevb, B.ln2w, B.ln2b, c.ln_eps,
-                       c.norm2, xs + (b + 1) * n * F, evs + (b + 1) * n * E, p2h, p2i);
-    if (!c.resid->empty() && b + 1 < layers_)
+                       c.pfc, pab, c.ln_eps, c.norm1, n1hb, n1ib, aevb);
+    // the post-attention node chain (kokkos_post_attention_block0.cpp:165-300),
+    // then the next block's projections or the heads
+    const bool last = b + 1 == layers_;
+    const NodeFwdArgs A{N, n1hb, aevb,
+                        {B.m1p, B.m1bp, B.m2p, B.m2bp, B.intp, B.intbp, B.int_cg, B.ln1w, B.ln1b, B.ln2w, B.ln2b,
+                         c.ln_eps, c.norm2},
+                        head_args(d, hw_), last ? nullptr : bw_[b + 1].qkvp, c.z, hpb, gtb, xs + (b + 1) * n * F,
+                        evs + (b + 1) * n * E, p2h, p2i, last ? nullptr : b_[QKV] + (b + 1) * n * 5 * F,
+                        {b_[HHEAD], c.eatom, c.qraw, c.heff, c.hir, c.c6eff, c.c6r}};
+    const unsigned g16 = blocks_for(n, 16);
+#define G_NODE_FWD(NT, TAIL) \
+  hipLaunchKernelGGL((k_node_fwd<NT, false, TAIL, 0, SlotsG>), dim3(g16), dim3(64 * NT), 0, s, A, SlotsG{d})
+    if (F == 128) {
+      if (last) G_NODE_FWD(8, 2);
+      else if (scaled) G_NODE_FWD(8, 0);
+      else G_NODE_FWD(8, 1);
+    } else {
+      if (last) G_NODE_FWD(16, 2);
+      else if (scaled) G_NODE_FWD(16, 0);
+      else G_NODE_FWD(16, 1);
+    }
+#undef G_NODE_FWD
+    if (scaled && !last)
       hipLaunchKernelGGL(g_axpby, dim3(blocks_for(n * F, 256)), dim3(256), 0, s, n * F, (*c.resid)[b + 1],
                          xs + (b + 1) * n * F, (*c.x0l)[b + 1], c.x0);
   }
-  // output heads (kokkos_output_heads.cpp:137-176)
-  const double *xf = xs + std::size_t(layers_) * n * F;
-  gemm<EPI_SILU, false>(s, N, nullptr, F, d.HO, xf, F, hw_.w1, hw_.b1, b_[HACT], d.HO, nullptr, 0, nullptr, 0,
-                        b_[HHPRE], d.HO);
-  gemm<EPI_STORE, false>(s, N, nullptr, 64, 64, b_[HACT] + 2 * d.HK, d.HO, hw_.hw2, hw_.hb2, b_[HKEY], 128);
-  if (d.c6)
-    gemm<EPI_STORE, false>(s, N, nullptr, 64, 64, b_[HACT] + 2 * d.HK + 64, d.HO, hw_.cw2, hw_.cb2, b_[HKEY] + 64,
-                           128);
-  hipLaunchKernelGGL(g_heads, dim3(g4), dim3(256), 0, s, d, N, c.z, b_[HACT], b_[HKEY], hw_, c.eatom, c.qraw,
-                     c.heff, c.hir, c.c6eff, c.c6r);
   G_CHECK(hipGetLastError());
 }
 
 void GenericPath::reverse(const GContext &c) {
   const GDims &d = d_;
   const hipStream_t s = c.s;
-  const int N = c.N, cap = c.cap, F = d.F, E = d.E, NH = d.NH, NI = d.NI, R = d.R;
+  const int N = c.N, cap = c.cap, F = d.F, E = d.E, NH = d.NH, R = d.R;
   const std::size_t n = std::size_t(N), P = std::size_t(std::max(cap, 1));
-  const unsigned g4 = blocks_for(n, 4), g4x = (g4 + 7) / 8 * 8;  // g4x: g_xcd_block's grids
-  // heads in reverse to dE/dx of the last block's output
-  hipLaunchKernelGGL(g_heads_bwd, dim3(g4), dim3(256), 0, s, d, N, c.z, b_[HHPRE], c.qseed, c.dh, c.heff, c.dc,
-                     c.c6eff, hw_, b_[GHEAD]);
-  gemm<EPI_STORE, true>(s, N, nullptr, d.HO, F, b_[GHEAD], d.HO, hw_.w1, nullptr, b_[GX], F);
-  hipLaunchKernelGGL(g_fill, dim3(blocks_for(n * E, 256)), dim3(256), 0, s, b_[GEV], n * E);
-  double *gx = b_[GX], *gev = b_[GEV];
+  const unsigned g4x = (blocks_for(n, 4) + 7) / 8 * 8;  // g_xcd_block's grids
+  double *gev = b_[GEV];
   for (int b = layers_ - 1; b >= 0; --b) {
     const GBlock &B = bw_[b];
     const double *evb = b_[EVS] + b * n * E;
     double *qb = b_[QKV] + b * n * 5 * F, *aevb = b_[AEV] + b * n * E;
-    double *n1b = b_[N1] + b * n * F, *n1hb = b_[N1HAT] + b * n * F, *n1ib = b_[N1IS] + b * n;
-    double *hpb = b_[HPRE] + b * n * F, *tb = b_[TOUT] + b * n * NI;
+    double *n1hb = b_[N1HAT] + b * n * F, *n1ib = b_[N1IS] + b * n;
+    double *hpb = b_[HPRE] + b * n * F, *gtb = b_[GATES] + b * n * NH;
     double *p2h = b_[PRE2HAT] + b * n * F, *p2i = b_[PRE2IS] + b * n;
     double *psb = b_[PS] + b * P * NH, *pfb = pf_rows(c, b), *pab = b_[PALPHA] + b * P * 4 * NH;
-    // post-attention chain in reverse (kokkos_post_attention_reverse.cpp:107-449)
-    hipLaunchKernelGGL(g_ln2_bwd, dim3(g4), dim3(256), 0, s, d, N, gx, gev, tb, aevb, p2h, p2i, B.ln2w, c.norm2,
-                       b_[GT], b_[GA]);
-    gemm<EPI_STORE, true>(s, N, nullptr, NI, NI, b_[GT], NI, B.wi, nullptr, b_[GCAT], NI);
-    hipLaunchKernelGGL(g_cat_bwd, dim3(blocks_for(n * (F + E), 256)), dim3(256), 0, s, d, N, b_[GT], b_[GCAT], aevb,
-                       B.int_cg, b_[GP], b_[GA]);
-    gemm<EPI_DSILU, true>(s, N, nullptr, F, F, b_[GP], F, B.m2, nullptr, b_[GHID], F, hpb, F);
-    gemm<EPI_DSILU_ADD, true>(s, N, nullptr, F, F, b_[GHID], F, B.m1, nullptr, b_[GN1], F, n1b, F, b_[GP], F);
-    hipLaunchKernelGGL(g_ln1_bwd, dim3(g4), dim3(256), 0, s, F, N, b_[GN1], B.ln1w, n1hb, n1ib, c.norm1, b_[GAINV]);
+    // the post-attention chain in reverse (kokkos_post_attention_reverse.cpp:107-449),
+    // from the heads' reverse or from the projections' reverse of the block above
+    const bool last = b + 1 == layers_;
+    const NodeBwdArgs A{N, b_[GQKV], last ? nullptr : bw_[b + 1].qkvtp,
+                        !last && !c.resid->empty() ? (*c.resid)[std::size_t(b + 1)] : 1.0, head_args(d, hw_),
+                        {b_[HHEAD], c.qseed, c.dh, c.heff, c.dc, c.c6eff}, c.z, last ? nullptr : gev, gtb, aevb, p2h,
+                        p2i, hpb, n1hb, n1ib,
+                        {B.inttp, B.m2tp, B.m1tp, B.int_cg, B.ln1w, B.ln1b, B.ln2w, c.norm1, c.norm2}, b_[GAINV],
+                        b_[GA]};
+    const unsigned g16 = blocks_for(n, 16);
+#define G_NODE_BWD(NT, SRC) \
+  hipLaunchKernelGGL((k_node_bwd<NT, false, SRC, 0, SlotsG>), dim3(g16), dim3(64 * NT), 0, s, A, SlotsG{d})
+    if (F == 128) {
+      if (last) G_NODE_BWD(8, 0);
+      else G_NODE_BWD(8, 1);
+    } else {
+      if (last) G_NODE_BWD(16, 0);
+      else G_NODE_BWD(16, 1);
+    }
+#undef G_NODE_BWD
     // attention reverse per pair (kokkos_attention_scatter_reverse.cpp:280-500)
     const bool tables = b == 0 && cls_on(c);
     section(c, "generic_attn_bwd_pairs", [&] {
@@ -2530,17 +2152,6 @@ void GenericPath::reverse(const GContext &c) {
       if (c.qk_norm)
         hipLaunchKernelGGL(g_qk_norm_bwd, dim3(blocks_for(n * 4 * NH, 256)), dim3(256), 0, s, N, F, NH, qb,
                            b_[QKIS] + b * n * 4 * NH, b_[GQKV]);
-      // gx = gainv + sum_w gqkv[w] W[w]^T per head, batch z = h
-      for (int w = 0; w < 5; ++w) {
-        if (w == 0)
-          gemm_heads<EPI_ADD, false>(s, N, 1, NH, b_[GQKV], 5 * F, 0, 32, B.wqkv, 1024, gx, F, 0, 32, b_[GAINV], F,
-                                     0, 32);
-        else
-          gemm_heads<EPI_ACCUM, false>(s, N, 1, NH, b_[GQKV] + w * F, 5 * F, 0, 32, B.wqkv + std::size_t(w) * NH * 1024,
-                                       1024, gx, F, 0, 32);
-      }
-      if (!c.resid->empty())
-        hipLaunchKernelGGL(g_scale, dim3(blocks_for(n * F, 256)), dim3(256), 0, s, n * F, (*c.resid)[b], gx);
       hipLaunchKernelGGL(g_ev_bwd, dim3(g4x), dim3(256), 0, s, d, N, c.inc_off, c.iact, c.iother, evb, B.att_cg,
                          b_[DS], b_[GA], gev);
     }

@@ -11,8 +11,8 @@
 // {a, b} with both directions carried per pair, node sums as gathers over the
 // node-major incidence, no atomics.  The filters over pairs are fused fp64
 // MFMA kernels that keep each pair's hidden row in registers (block 0 of a
-// one-image system through its element-pair tables); the node-side dense
-// layers are one LDS-tiled fp64 GEMM with fused epilogues; the rest are
+// one-image system through its element-pair tables); the node-side layers of
+// a block are one fused MFMA kernel each way (node_chain.hpp); the rest are
 // node- or pair-major kernels in natural channel order.
 #pragma once
 
@@ -34,7 +34,8 @@ constexpr int kGMaxE = 72;  // equivariant channels, at most (8 slots of l = 4)
 // harmonic sh[c] (l = 1..4 in order, 2l + 1 each: the 24 values of a pair's
 // harmonics row) and belongs to slot slot[c].
 struct GDims {
-  int F, NH, E, R, FH, HK, NI, HO;  // HO: energy HK | charge HK | Hirshfeld 64 (| C6 64)
+  int F, NH, E, R, FH, HK, NI;
+  int HKT, HT;  // 16-unit tiles of the energy (charge) head and of all heads: 2 HKT + 4 Hirshfeld (+ 4 C6)
   int c6;
   signed char slot[kGMaxE], sh[kGMaxE];
   signed char off[9];
@@ -45,7 +46,7 @@ struct GDims {
 
 // Device weights of one interaction block, in the model file's layouts.
 struct GBlock {
-  const double *wqkv;  // (5, NH, 32, 32): q k v q_ev k_ev, (head, in, out)
+  const double *qkvp, *qkvtp;  // per head (160 x 32): q k v q_ev k_ev, and its transpose, MFMA operand order
   const double *w0[2], *b0[2], *w1[2], *b1[2];    // radial layers (F, R) (F) (F, F) (F)
   const double *e0[2], *eb0[2], *e1[2], *eb1[2];  // spherical layers (FH, NH) (FH) (F, FH) (F)
   // both output layers side by side, (F, F + FH): [W1 | E1], and b1 + eb1,
@@ -64,20 +65,19 @@ struct GBlock {
   const double *rdr;
   const double *att_cg, *int_cg;                  // (E)
   const double *ln1w, *ln1b, *ln2w, *ln2b;        // (F); RMSNorm and none: 1 and 0
-  const double *m1, *m1b, *m2, *m2b;              // (F, F) (F)
-  const double *wi, *bi;                          // (NI, NI) (NI)
+  // the node layers, MFMA operand order, their transposes, biases in accumulator order
+  const double *m1p, *m2p, *intp, *m1tp, *m2tp, *inttp, *m1bp, *m2bp, *intbp;
 };
 
 struct GHeads {
-  const double *w1, *b1;      // (HO, F) (HO): the first layers of all heads
-  const double *hw2, *hb2;    // Hirshfeld key layer (64, 64) (64)
-  const double *cw2, *cb2;    // C6 ratio head key layer (or null)
-  const double *ew2, *qw2;    // (HK)
+  const double *w1p, *w1tp, *b1p;  // the first layers of all heads (16 HT x F), MFMA operand order
+  const double *ew2, *qw2;         // (16 HKT), tile-transposed order
   double eb2, qb2;
-  const double *escale, *eshift;  // (118)
-  const double *qemb;             // (100)
-  const double *hqemb, *hvshift;  // (100, 64) (100)
-  const double *cqemb, *cvshift;  // C6 head's (or null)
+  const double *hkey, *hkey_c;     // Hirshfeld (100, 64): W2^T q_emb[z], tile-transposed; (100): q_emb[z] . b2
+  const double *ckey, *ckey_c;     // C6 ratio head's (or null)
+  const double *escale, *eshift;   // (118)
+  const double *qemb;              // (100)
+  const double *hvshift, *cvshift; // (100)
   const double *rbf_b, *rbf_k, *rbf_kr;  // (R)
   const double *exp2_256;                // 2^(j/256), j < 256 (exp_tab)
 };

@@ -1,11 +1,14 @@
 """HIP path vs the CPU oracle at the sizes where the kernels' work is cut: atom
 counts at and beside the edges of their 16-atom tiles, on the scalar and the
-fused filter kernels of the shipped model and on the generic widths.  Bars as
-in test_gpu_edges.py: energy 1e-10 relative, forces and virial 1e-9.
+fused filter kernels of the shipped model and on the generic widths; head
+widths that leave a part of a 16-unit tile.  Bars as in test_gpu_edges.py:
+energy 1e-10 relative, forces and virial 1e-9.
 """
 import numpy as np
 import pytest
 
+import support
+from oracle.oracle import Oracle
 from test_gpu_edges import _both_paths, model, orc  # noqa: F401
 
 pytestmark = pytest.mark.gpu
@@ -25,3 +28,12 @@ def _cluster(n, seed=3):
 def test_atom_tiles(orc, model, n):  # noqa: F811
     z, x, m = _cluster(n)
     _both_paths(z, x, 0.0, m, orc, model)
+
+
+@pytest.mark.parametrize("width", [129, 200])
+def test_head_width_remainder(tmp_path, width):
+    """Energy and charge heads whose width is no multiple of 16 (the generic
+    kernels pad their last tile)."""
+    path = support.head_width_model(tmp_path / "heads.so3lr", width, live=True)
+    z, x, m = _cluster(17)
+    _both_paths(z, x, 0.0, m, Oracle(path), path)
