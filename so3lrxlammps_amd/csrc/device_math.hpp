@@ -171,7 +171,7 @@ __device__ __forceinline__ void zbl_directed(const ZblParams &P, double zi, doub
                                              double &energy, double &grad) {
   energy = 0.0;
   grad = 0.0;
-  if (!(r > 0.0) || r > P.rc * (1.0 + 1e-12)) return;
+  if (!(r > 0.0) || r > P.rc * (1.0 + 1e-12) || r >= P.switch_off) return;  // the switch is 0 from switch_off on
   const double xn = r / P.rc, x2 = xn * xn, x3 = x2 * xn;
   const double fc = r < P.rc ? 1.0 - 10.0 * x3 + 15.0 * x3 * xn - 6.0 * x3 * x2 : 0.0;
   const double dfc = r < P.rc ? (-30.0 * x2 + 60.0 * x3 - 30.0 * x3 * xn) / P.rc : 0.0;

@@ -66,7 +66,10 @@ char *scratch_on_device(int device) {
 }
 
 constexpr int kWave = 64;
-constexpr int kCompactPerBlock = 1024;  // candidates per compaction block (256 threads x 4)
+constexpr int kCompactPerBlock = 256;  // candidates per compaction block, one per thread
+// up to this many compaction blocks, every block sums the counts before its
+// own; more go through k_scan_counts
+constexpr int kPrefixBlocks = 1024;
 
 // DPP lane permute of a double within the 16-lane rows of a wavefront (two
 // 32-bit moves).  CTRL: 0xB1 quad_perm(1,0,3,2), 0x4E quad_perm(2,3,0,1),
@@ -102,11 +105,6 @@ __device__ __forceinline__ double wave_sum(double v) {
 }
 __device__ __forceinline__ double pick4(int s, double a, double b, double c, double d) {
   return s == 0 ? a : (s == 1 ? b : (s == 2 ? c : d));
-}
-
-__global__ void k_fill(double *p, std::size_t n, double v) {
-  const std::size_t i = std::size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = v;
 }
 
 // Residual scalars (kokkos_local_energy_reverse.cpp:124-170): a block's input
@@ -166,12 +164,20 @@ struct RowsPos {
     dz = x[3 * ra + 2] - x[3 * rb + 2];
   }
 };
+// (PERM: positions in the caller's atom order, node n at perm[n])
+template <bool PERM>
 struct ShiftPos {
   const double *x;
   const int *nodes, *codes;
   double lx, ly, lz;
+  const int *perm;
   __device__ __forceinline__ void vec(int c, double &dx, double &dy, double &dz) const {
-    const int a = nodes[2 * c], b = nodes[2 * c + 1], code = codes[c];
+    int a = nodes[2 * c], b = nodes[2 * c + 1];
+    const int code = codes[c];
+    if constexpr (PERM) {
+      a = perm[a];
+      b = perm[b];
+    }
     dx = x[3 * a] - x[3 * b] - (code / 9 - 1) * lx;
     dy = x[3 * a + 1] - x[3 * b + 1] - ((code / 3) % 3 - 1) * ly;
     dz = x[3 * a + 2] - x[3 * b + 2] - (code % 3 - 1) * lz;
@@ -185,104 +191,155 @@ __device__ __forceinline__ bool sr_active(const Pos &pos, int c, double rc2, dou
   return r2 > 0.0 && r2 < rc2;
 }
 
+// Active candidates per block of kCompactPerBlock; in the same launch, what
+// the evaluation needs before its first pair: positions gathered into node
+// order (xn, with perm) and the bucket counters cleared.
+struct CountExtras {
+  int n3, nkeys;       // 3 N values of xn (0: none); counters
+  const double *xin;
+  const int *perm;
+  double *xn;
+  int *hist;
+};
 template <class Pos>
-__global__ __launch_bounds__(256) void k_sr_count(int P, Pos pos, double rc2, int *blk_count) {
-  __shared__ int part[256];
-  const int base = blockIdx.x * kCompactPerBlock + threadIdx.x * 4;
-  int cnt = 0;
-  for (int j = 0; j < 4; ++j) {
-    const int c = base + j;
-    double dx, dy, dz;
-    if (c < P && sr_active(pos, c, rc2, dx, dy, dz)) ++cnt;
-  }
-  part[threadIdx.x] = cnt;
+__global__ __launch_bounds__(256) void k_sr_count(int P, Pos pos, double rc2, int *blk_count, CountExtras X) {
+  __shared__ int part[4];
+  const int c = blockIdx.x * kCompactPerBlock + threadIdx.x;
+  const int stride = gridDim.x * 256;
+  for (int i = c; i < X.n3; i += stride) X.xn[i] = X.xin[3 * X.perm[i / 3] + i % 3];
+  for (int i = c; i < X.nkeys; i += stride) X.hist[i] = 0;
+  double dx, dy, dz;
+  const bool in = c < P && sr_active(pos, c, rc2, dx, dy, dz);
+  const unsigned long long m = __ballot(in);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = __popcll(m);
   __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (int(threadIdx.x) < s) part[threadIdx.x] += part[threadIdx.x + s];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) blk_count[blockIdx.x] = part[0];
+  if (threadIdx.x == 0) blk_count[blockIdx.x] = (part[0] + part[1]) + (part[2] + part[3]);
 }
 
-// exclusive scan of per-block counts in place; the total to *n_total and,
-// clamped to the capacity of the active-pair buffers, to *n_active
+// exclusive scan of per-block counts in place (one block, a run of counts per
+// thread); the total to *n_total and, clamped to the capacity of the
+// active-pair buffers, to *n_active
 __global__ __launch_bounds__(1024) void k_scan_counts(int nblk, int *cnt, int *n_active, int cap, int *n_total) {
-  __shared__ int buf[1024];
-  __shared__ int carry;
-  if (threadIdx.x == 0) carry = 0;
+  __shared__ int v[1024];
+  const int t = threadIdx.x, per = (nblk + 1023) / 1024, k0 = min(nblk, t * per), k1 = min(nblk, k0 + per);
+  int own = 0;
+  for (int k = k0; k < k1; ++k) own += cnt[k];
+  v[t] = own;
   __syncthreads();
-  for (int start = 0; start < nblk; start += 1024) {
-    const int i = start + threadIdx.x;
-    const int v = i < nblk ? cnt[i] : 0;
-    buf[threadIdx.x] = v;
+  for (int o = 1; o < 1024; o <<= 1) {
+    const int add = t >= o ? v[t - o] : 0;
     __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {
-      const int t = int(threadIdx.x) >= off ? buf[threadIdx.x - off] : 0;
-      __syncthreads();
-      buf[threadIdx.x] += t;
-      __syncthreads();
-    }
-    if (i < nblk) cnt[i] = carry + buf[threadIdx.x] - v;
-    __syncthreads();
-    if (threadIdx.x == 1023) carry += buf[1023];
+    v[t] += add;
     __syncthreads();
   }
-  if (threadIdx.x == 0) {
-    *n_active = carry < cap ? carry : cap;
-    if (n_total) *n_total = carry;
+  int run = v[t] - own;
+  for (int k = k0; k < k1; ++k) {
+    const int c = cnt[k];
+    cnt[k] = run;
+    run += c;
+  }
+  if (t == 1023) {
+    *n_active = v[t] < cap ? v[t] : cap;
+    if (n_total) *n_total = v[t];
   }
 }
 
-template <class Pos>
+// Bucket of a pair for the blocks after 0's radial tables: (spatial block of
+// kRintAtoms nodes of its first endpoint, interval of r).
+__device__ __forceinline__ int rint_key(int a, double r, const RadialDomain &d) {
+  double t;
+  bool inside;
+  return (a / kRintAtoms) * kBlockIntervals + radial_locate(r, d, t, inside);
+}
+// The pairs of one workgroup lie in few spatial blocks (candidates in node
+// order): counters of kRintWindow spatial blocks in LDS, one global atomic per
+// key and workgroup; keys outside the window go to the global counters.  One
+// global atomic per pair, in kernels of their own, took 36 + 56 us at 24,000
+// atoms and 23 + 24 at 3,000, where the keys are few; the counts now ride in
+// k_sr_compact and the placement in k_inc_active (12 -> 14 us at 24,000).  The
+// ranks follow the pair order within a workgroup, so a bucket's pairs are
+// nearly ordered: the reverse filter reads its pair records in 528 against
+// 571 us.
+constexpr int kRintWindow = 4, kRintLocal = kRintWindow * kBlockIntervals;
+
+// Active pairs in candidate order with their geometry.  blk: the blocks'
+// counts (PREFIX: this block sums those before its own, the last block writes
+// the totals) or their scanned offsets.  hist: bucket counts of the pairs
+// (null: none).  A workgroup's active candidates are moved to its first
+// lanes before the geometry, so no lane idles on a candidate beyond the
+// cutoff.  Four candidates per thread with the geometry where a candidate was
+// found took 69 us at 24,000 atoms and 22 at 99; this form 41 and 10.
+template <class Pos, bool PREFIX>
 __global__ __launch_bounds__(256) void k_sr_compact(
-    int P, Pos pos, const int *nodes, double rc2, const int *blk_off, int cap,
+    int P, Pos pos, const int *nodes, double rc2, const int *blk, int cap,
     const int *z, ZblParams zp, int *cand2act, int *pa, double *pv, double *pr, double *pY,
-    double *pfc, double *pzbl) {
-  __shared__ int part[256];
-  const int base = blockIdx.x * kCompactPerBlock + threadIdx.x * 4;
-  int flags = 0, cnt = 0;
-  for (int j = 0; j < 4; ++j) {
-    const int c = base + j;
-    double dx, dy, dz;
-    if (c < P && sr_active(pos, c, rc2, dx, dy, dz)) { flags |= 1 << j; ++cnt; }
+    double *pfc, double *pzbl, double *dr, int *n_active, int *n_total, RadialDomain dom, int *hist) {
+  __shared__ int part[4], psum[4], cand[256], lcnt[kRintLocal], window;
+  __shared__ double vx[256], vy[256], vz[256];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int c = blockIdx.x * kCompactPerBlock + tid;
+  double dx = 0, dy = 0, dz = 0;
+  const bool in = c < P && sr_active(pos, c, rc2, dx, dy, dz);
+  const unsigned long long m = __ballot(in);
+  if (lane == 0) part[wv] = __popcll(m);
+  if constexpr (PREFIX) {
+    int before = 0;
+    for (int k = tid; k < int(blockIdx.x); k += 256) before += blk[k];
+    for (int o = 32; o >= 1; o >>= 1) before += __shfl_xor(before, o, kWave);
+    if (lane == 0) psum[wv] = before;
   }
-  part[threadIdx.x] = cnt;
+  if (hist && tid < kRintLocal) lcnt[tid] = 0;
   __syncthreads();
-  for (int off = 1; off < 256; off <<= 1) {
-    const int t = int(threadIdx.x) >= off ? part[threadIdx.x - off] : 0;
-    __syncthreads();
-    part[threadIdx.x] += t;
-    __syncthreads();
+  const int base = PREFIX ? (psum[0] + psum[1]) + (psum[2] + psum[3]) : blk[blockIdx.x];
+  const int count = (part[0] + part[1]) + (part[2] + part[3]);
+  if (PREFIX && blockIdx.x + 1 == gridDim.x && tid == 0) {
+    const int total = base + count;
+    *n_active = total < cap ? total : cap;
+    *n_total = total;
   }
-  int at = blk_off[blockIdx.x] + part[threadIdx.x] - cnt;
-  const double rc = sqrt(rc2);
-  for (int j = 0; j < 4; ++j) {
-    const int c = base + j;
-    if (c >= P) break;
-    if (!(flags & (1 << j))) { cand2act[c] = -1; continue; }
-    double dx, dy, dz;
-    sr_active(pos, c, rc2, dx, dy, dz);
-    const int p = at++;
-    if (p >= cap) {  // beyond the active-pair buffers: the host grows them and evaluates again
-      cand2act[c] = -1;
-      continue;
-    }
-    cand2act[c] = p;
-    const int na = nodes[2 * c], nb = nodes[2 * c + 1];
+  int rank = __popcll(m & (lane ? (~0ull >> (64 - lane)) : 0ull));
+  for (int k = 0; k < wv; ++k) rank += part[k];
+  // beyond the active-pair buffers: the host grows them and evaluates again
+  if (c < P) cand2act[c] = in && base + rank < cap ? base + rank : -1;
+  if (in) {
+    cand[rank] = c;
+    vx[rank] = dx;
+    vy[rank] = dy;
+    vz[rank] = dz;
+    if (rank == 0) window = nodes[2 * c] / kRintAtoms;
+  }
+  __syncthreads();
+  const int p = base + tid;
+  if (tid < count && p < cap) {
+    const int na = nodes[2 * cand[tid]], nb = nodes[2 * cand[tid] + 1];
+    dx = vx[tid];
+    dy = vy[tid];
+    dz = vz[tid];
     pa[2 * p] = na;
     pa[2 * p + 1] = nb;
     pv[3 * p] = dx; pv[3 * p + 1] = dy; pv[3 * p + 2] = dz;
     const double r = sqrt(dx * dx + dy * dy + dz * dz);
     pr[p] = r;
+    dr[p] = 0.0;
+    if (hist) {
+      const int key = rint_key(na, r, dom), local = key - window * kBlockIntervals;
+      if (local >= 0 && local < kRintLocal) atomicAdd(&lcnt[local], 1);
+      else atomicAdd(&hist[key], 1);
+    }
     const double inv = r > 1e-14 ? 1.0 / r : 0.0;
     const double ux = dx * inv, uy = dy * inv, uz = dz * inv;
-    for (int m = 0; m < kE; ++m) pY[kE * p + m] = sh_component(m, ux, uy, uz);
-    const double t = r / rc, t3 = t * t * t;
+#pragma unroll
+    for (int q = 0; q < kE; ++q) pY[kE * std::size_t(p) + q] = sh_component(q, ux, uy, uz);
+    const double rc = sqrt(rc2), t = r / rc, t3 = t * t * t;
     pfc[p] = r < rc ? 1.0 - 10.0 * t3 + 15.0 * t3 * t - 6.0 * t3 * t * t : 0.0;
     double e, g;
     zbl_directed(zp, double(z[na]), double(z[nb]), r, e, g);
     pzbl[2 * p] = e;
     pzbl[2 * p + 1] = g;
+  }
+  if (hist) {
+    __syncthreads();
+    if (tid < kRintLocal && lcnt[tid]) atomicAdd(&hist[window * kBlockIntervals + tid], lcnt[tid]);
   }
 }
 
@@ -1861,29 +1918,18 @@ __global__ __launch_bounds__(256) void k_radial_bwd(const int *n_active, const i
 // MFMA products over a wavefront's 16 pairs, which therefore lie in one
 // interval.  The active pairs are bucketed by (spatial block of kRintAtoms
 // nodes of their first endpoint, interval), each bucket padded to a multiple
-// of 16 slots (-1 in the padding): counts (k_rint_count), bucket starts (k_rint_scan),
-// placement (k_rint_place).  The nodes are in spatial order, so a block's
+// of 16 slots (-1 in the padding): counts (k_sr_compact), bucket starts
+// (k_rint_scan), placement (k_inc_active).  The nodes are in spatial order, so a block's
 // buckets, run one after another on one XCD, read one region's node rows
 // from L2.  Within a bucket the order depends on the atomics' timing; each
 // pair's results go to its own rows, so the results do not.
-__device__ __forceinline__ int rint_key(int a, double r, const RadialDomain &d) {
-  double t;
-  bool inside;
-  return (a / kRintAtoms) * kBlockIntervals + radial_locate(r, d, t, inside);
-}
+// The counts are taken by k_sr_compact.
 
-// one active pair per thread: hist[key] += 1
-__global__ __launch_bounds__(256) void k_rint_count(const int *n_active, const int *pa, const double *pr,
-                                                    RadialDomain d, int *hist) {
-  const int p = blockIdx.x * 256 + threadIdx.x;
-  if (p < *n_active) atomicAdd(&hist[rint_key(pa[2 * p], pr[p], d)], 1);
-}
-
-// bucket starts, each bucket padded to a multiple of 16 slots, into cursor;
-// the slots' end into *total (one block: a run of keys per thread)
-__global__ __launch_bounds__(1024) void k_rint_scan(int nkeys, const int *hist, int *cursor, int *total) {
+// bucket starts, each bucket padded to a multiple of 16 slots, into start and
+// cursor; the slots' end into *total (one block: a run of keys per thread)
+__global__ __launch_bounds__(1024) void k_rint_scan(int nkeys, const int *hist, int *start, int *cursor, int *total) {
   __shared__ int v[1024];
-  const int t = threadIdx.x, per = (nkeys + 1023) / 1024, k0 = t * per, k1 = min(nkeys, k0 + per);
+  const int t = threadIdx.x, per = (nkeys + 1023) / 1024, k0 = min(nkeys, t * per), k1 = min(nkeys, k0 + per);
   int own = 0;
   for (int k = k0; k < k1; ++k) own += (hist[k] + 15) / 16 * 16;
   v[t] = own;
@@ -1896,17 +1942,57 @@ __global__ __launch_bounds__(1024) void k_rint_scan(int nkeys, const int *hist, 
   }
   int run = v[t] - own;
   for (int k = k0; k < k1; ++k) {
-    cursor[k] = run;
+    start[k] = cursor[k] = run;
     run += (hist[k] + 15) / 16 * 16;
   }
   if (t == 1023) *total = v[t];
 }
 
-// one active pair per thread: its slot from its bucket's cursor
-__global__ __launch_bounds__(256) void k_rint_place(const int *n_active, const int *pa, const double *pr,
-                                                    RadialDomain d, int *cursor, int *order) {
-  const int p = blockIdx.x * 256 + threadIdx.x;
-  if (p < *n_active) order[atomicAdd(&cursor[rint_key(pa[2 * p], pr[p], d)], 1)] = p;
+// Active incidence of this step: entry k of a node's list as active pair
+// index * 2 + side (-1 for a candidate beyond the cutoff) and its partner
+// node, so the node-major kernels read their pairs with one coalesced load
+// per 64 entries instead of a chain of dependent lookups.  With order given,
+// the same launch places the pairs in their buckets (a workgroup's pairs
+// ranked in LDS, one global atomic per key and workgroup) and writes the
+// padding of every bucket.
+struct PlaceArgs {
+  const int *n_active;
+  const double *pr;
+  RadialDomain dom;
+  int nkeys;
+  const int *hist, *start;
+  int *cursor, *order;  // order null: incidence only
+};
+__global__ __launch_bounds__(256) void k_inc_active(int E, const int *inc, const int *cand2act, const int *pa,
+                                                    int *iact, int *iother, PlaceArgs R) {
+  __shared__ int lcnt[kRintLocal], lbase[kRintLocal];
+  const int t = blockIdx.x * 256 + threadIdx.x;
+  if (t < E) {
+    const int e = inc[t];
+    const int p = cand2act[e >> 1];
+    iact[t] = p < 0 ? -1 : (p << 1 | (e & 1));
+    iother[t] = p < 0 ? 0 : pa[2 * p + 1 - (e & 1)];
+  }
+  if (!R.order) return;
+  if (t < R.nkeys)
+    for (int q = R.start[t] + R.hist[t], end = R.start[t] + (R.hist[t] + 15) / 16 * 16; q < end; ++q) R.order[q] = -1;
+  const int nact = *R.n_active;
+  if (int(blockIdx.x) * 256 >= nact) return;  // the whole block
+  if (threadIdx.x < kRintLocal) lcnt[threadIdx.x] = 0;
+  __syncthreads();
+  const int window = pa[2 * (int(blockIdx.x) * 256)] / kRintAtoms * kBlockIntervals;
+  int key = -1, local = -1, rank = 0;
+  if (t < nact) {
+    key = rint_key(pa[2 * t], R.pr[t], R.dom);
+    local = key - window;
+    if (local < 0 || local >= kRintLocal) local = -1;
+    if (local >= 0) rank = atomicAdd(&lcnt[local], 1);
+  }
+  __syncthreads();
+  if (threadIdx.x < kRintLocal && lcnt[threadIdx.x])
+    lbase[threadIdx.x] = atomicAdd(&R.cursor[window + threadIdx.x], lcnt[threadIdx.x]);
+  __syncthreads();
+  if (key >= 0) R.order[local >= 0 ? lbase[local] + rank : atomicAdd(&R.cursor[key], 1)] = t;
 }
 
 // ---------------------------------------------------------------- attention
@@ -1931,19 +2017,6 @@ __device__ __forceinline__ void wave_normalise(double v0, double v1, double eps,
   is = mode == 2 ? 1.0 : 1.0 / sqrt(wave_sum(d0 * d0 + d1 * d1) / kF + eps);
   h0 = d0 * is;
   h1 = d1 * is;
-}
-
-// Active incidence of this step: entry k of a node's list as active pair
-// index * 2 + side (-1 for a candidate beyond the cutoff) and its partner
-// node, so the node-major kernels read their pairs with one coalesced load
-// per 64 entries instead of a chain of dependent lookups.
-__global__ void k_inc_active(int E, const int *inc, const int *cand2act, const int *pa, int *iact, int *iother) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= E) return;
-  const int e = inc[k];
-  const int p = cand2act[e >> 1];
-  iact[k] = p < 0 ? -1 : (p << 1 | (e & 1));
-  iother[k] = p < 0 ? 0 : pa[2 * p + 1 - (e & 1)];
 }
 
 // Attention forward, node-major (kokkos_integrated_block0.cpp:330-385): for
@@ -2521,11 +2594,6 @@ __global__ void k_fill_int(int *p, int n, int v) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
 }
-// the active-pair count next to the reduced energy and virial, for one read-back
-__global__ void k_copy_count(const int *n_active, double *dst) {
-  if (threadIdx.x == 0) dst[0] = double(*n_active);
-}
-
 // xn[n] = x[perm[n]] (positions into node order)
 __global__ void k_gather_pos(int N, const int *perm, const double *x, double *xn) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
@@ -2597,23 +2665,22 @@ __global__ __launch_bounds__(256) void k_vatom(int N, const int *inc_off, const 
 // one block then sums the partials in block order.
 constexpr int kReduceBlocks = 240;
 
-__device__ __forceinline__ void block_sum9(double *acc, double *sh, double *dst) {
+// 256 threads' nine sums: wavefront sums, then the four wavefronts in order
+__device__ __forceinline__ void block_sum9(const double *acc, double (*sh)[9], double *dst) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+#pragma unroll
   for (int c = 0; c < 9; ++c) {
-    sh[threadIdx.x] = acc[c];
-    __syncthreads();
-    for (int st = 128; st > 0; st >>= 1) {
-      if (int(threadIdx.x) < st) sh[threadIdx.x] += sh[threadIdx.x + st];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) dst[c] = sh[0];
-    __syncthreads();
+    const double v = wave_sum(acc[c]);
+    if (lane == c) sh[wv][c] = v;
   }
+  __syncthreads();
+  if (threadIdx.x < 9) dst[threadIdx.x] = ((sh[0][threadIdx.x] + sh[1][threadIdx.x]) + sh[2][threadIdx.x]) + sh[3][threadIdx.x];
 }
 
 __global__ __launch_bounds__(256) void k_reduce_part(int N, const int *n_active, const double *etot,
                                                      const double *pv, const double *pg, const double *vlr,
                                                      const double *parts, double *partial) {
-  __shared__ double sh[256];
+  __shared__ double sh[4][9];
   double acc[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
   const int B = gridDim.x, b = blockIdx.x;
   const int nper = (N + B - 1) / B, n0 = b * nper, n1 = min(N, n0 + nper);
@@ -2635,11 +2702,14 @@ __global__ __launch_bounds__(256) void k_reduce_part(int N, const int *n_active,
   block_sum9(acc, sh, partial + 9 * std::size_t(b));
 }
 
-__global__ __launch_bounds__(256) void k_reduce_final(int B, const double *partial, double *red) {
-  __shared__ double sh[256];
+// the totals, with the number of pairs found (*n_total) after them, straight
+// into the host's pinned result block
+__global__ __launch_bounds__(256) void k_reduce_final(int B, const double *partial, const int *n_total, double *host) {
+  __shared__ double sh[4][9];
   double acc[9];
   for (int c = 0; c < 9; ++c) acc[c] = int(threadIdx.x) < B ? partial[9 * threadIdx.x + c] : 0.0;
-  block_sum9(acc, sh, red);
+  block_sum9(acc, sh, host);
+  if (threadIdx.x == 9) host[9] = double(*n_total);
 }
 
 int ceil_div(std::int64_t a, std::int64_t b) { return int((a + b - 1) / b); }
@@ -3083,7 +3153,7 @@ Evaluator::Evaluator(std::shared_ptr<Model> model, int device) : model_(std::mov
   qseed_ = buf("qseed"); elr_ = buf("elr"); dq_ = buf("dq"); dh_ = buf("dh"); flr_ = buf("flr");
   vlr_ = buf("vlr"); elr_parts_ = buf("elr_parts"); ezbl_ = buf("ezbl"); 
   gev_ = buf("gev"); gainv_ = buf("gainv"); gaev_ = buf("gaev"); gqkv_ = buf("gqkv");
-  fout_ = buf("fout"); etot_ = buf("etot"); red_ = buf("red");
+  fout_ = buf("fout"); etot_ = buf("etot"); 
   qkis_ = buf("qkis"); c6eff_ = buf("c6eff"); c6r_ = buf("c6r"); dc_ = buf("dc");
   owner_ = buf("owner"); sr_rows_ = buf("sr_rows"); sr_nodes_ = buf("sr_nodes");
   sr_inc_off_ = buf("sr_inc_off"); sr_inc_ = buf("sr_inc"); lr_rows_ = buf("lr_rows");
@@ -3189,7 +3259,7 @@ void Evaluator::set_system(const std::vector<std::int32_t> &z, const std::vector
   }
   // block 0's radial tables: sized here (no allocation in the evaluation),
   // filled by the next evaluation
-  rad_stale_ = true;
+  rad_stale_ = cls_stale_ = true;
   const std::size_t rad_rec = gen_ ? (gen_->radial_ok() ? gen_->radial_record() : 0) : (radial_ok_ ? kRadRecord : 0);
   if (rad_rec && n_cls_ > 0)
     (void)ensure<double>(rad_tab_, 2 * std::size_t(n_cls_) * (n_cls_ + 1) / 2 * kRadialIntervals * rad_rec);
@@ -3301,12 +3371,12 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
       hipLaunchKernelGGL(k_gather_pos, dim3(unsigned((3 * Nz + 255) / 256)), dim3(256), 0, s, int(N), perm, x_in,
                          const_cast<double *>(x));
     if (shift_mode_) {
-      const ShiftPos pos{x, static_cast<const int *>(sr_nodes_->p), static_cast<const int *>(sr_code_->p),
-                         box_len_[0], box_len_[1], box_len_[2]};
-      hipLaunchKernelGGL(k_sr_count<ShiftPos>, dim3(nblk), dim3(256), 0, s, int(P), pos, rc2, cnt);
+      const ShiftPos<false> pos{x, static_cast<const int *>(sr_nodes_->p), static_cast<const int *>(sr_code_->p),
+                                box_len_[0], box_len_[1], box_len_[2], nullptr};
+      hipLaunchKernelGGL(k_sr_count<ShiftPos<false>>, dim3(nblk), dim3(256), 0, s, int(P), pos, rc2, cnt, CountExtras{});
     } else {
       const RowsPos pos{x, static_cast<const int *>(sr_rows_->p)};
-      hipLaunchKernelGGL(k_sr_count<RowsPos>, dim3(nblk), dim3(256), 0, s, int(P), pos, rc2, cnt);
+      hipLaunchKernelGGL(k_sr_count<RowsPos>, dim3(nblk), dim3(256), 0, s, int(P), pos, rc2, cnt, CountExtras{});
     }
     hipLaunchKernelGGL(k_scan_counts, dim3(1), dim3(1024), 0, s, nblk, cnt, cnt + nblk, 0x7fffffff, cnt + nblk + 1);
     int total = 0;
@@ -3353,7 +3423,6 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
   double *gqkv = nullptr;
   double *fo = nullptr;
   double *etot = nullptr;
-  double *red = nullptr;
   int *blk = nullptr;
   int *nact = nullptr;
   int *c2a = nullptr;
@@ -3422,8 +3491,8 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
     psc = scalar ? nullptr : take<double>(psc_, 16 * Pa);
     ds = take<double>(ds_, 4 * Pa);
     if (use_rt) {
-      // counts, bucket cursors and the slots' end; the bucket order
-      rhist = take<int>(rint_hist_, 2 * std::size_t(rkeys) + 1);
+      // counts, bucket starts and cursors, and the slots' end; the bucket order
+      rhist = take<int>(rint_hist_, 3 * std::size_t(rkeys) + 1);
       rord = take<int>(rint_order_, Pa + 16 * std::size_t(rkeys));
     }
     if (use_cls) {
@@ -3443,7 +3512,7 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
       gen_->carve(int(N), int(PA), gen_cls ? n_cls_ : 0,
                   [&](int i, std::size_t cnt) { return take<double>(gbuf_[i], cnt); });
       if (use_grt) {
-        rhist = take<int>(rint_hist_, 2 * std::size_t(rkeys) + 1);
+        rhist = take<int>(rint_hist_, 3 * std::size_t(rkeys) + 1);
         rord = take<int>(rint_order_, Pa + 16 * std::size_t(rkeys));
       }
       if (gen_cls) {
@@ -3473,7 +3542,6 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
     dc = c6_ ? take<double>(dc_, Nz) : nullptr;
     fo = f_out ? f_out : take<double>(fout_, Nz * 3);
     etot = eatom_out ? eatom_out : take<double>(etot_, Nz);
-    red = take<double>(red_, 16);
     blk = take<int>(blk_count_, nblk);
     nact = take<int>(n_active_, 2);  // [0] active pairs kept, [1] active pairs found
     c2a = take<int>(cand2act_, Pz);
@@ -3536,39 +3604,60 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
     HIP_CHECK(hipEventRecord(pd.b, s));
     pending.push_back(pd);
   };
-  auto fill = [&](double *p, std::size_t cnt) {
-    if (cnt) hipLaunchKernelGGL(k_fill, dim3(unsigned((cnt + 255) / 256)), dim3(256), 0, s, p, cnt, 0.0);
-  };
   const unsigned gN64 = unsigned(std::max(1, ceil_div(N, 64)));
 
   // Everything from here to the read-back is one sequence on stream s: run
   // directly, or captured once into a graph and replayed.
   auto enqueue = [&] {
-  if (gather_pos)
-    hipLaunchKernelGGL(k_gather_pos, dim3(unsigned((3 * Nz + 255) / 256)), dim3(256), 0, s, int(N), perm, x_in,
-                       const_cast<double *>(x));
-  // --- active short-range pairs, geometry, ZBL ---
+  // --- active short-range pairs, geometry, ZBL, and their bucket order for
+  // the blocks after 0's radial tables ---
   const int cap = int(PA);
+  const bool buckets = use_rt || use_grt;
+  const RadialDomain bdom = use_rt ? rbl_dom_ : (use_grt ? gen_->rbl_domain() : RadialDomain{});
+  int *rstart = rhist ? rhist + rkeys : nullptr, *rcursor = rhist ? rhist + 2 * rkeys : nullptr;
+  int *rslots = rhist ? rhist + 3 * rkeys : nullptr;
+  auto active_pairs = [&](auto count_pos, auto pos) {
+    using CountPos = decltype(count_pos);
+    using Pos = decltype(pos);
+    const CountExtras X{gather_pos ? int(3 * N) : 0, buckets ? rkeys : 0, x_in, perm, const_cast<double *>(x), rhist};
+    hipLaunchKernelGGL(k_sr_count<CountPos>, dim3(nblk), dim3(256), 0, s, int(P), count_pos, rc2, blk, X);
+#define SO3LR_COMPACT(PREFIX)                                                                                       \
+  hipLaunchKernelGGL((k_sr_compact<Pos, PREFIX>), dim3(nblk), dim3(256), 0, s, int(P), pos, sr_nodes, rc2, blk, cap, \
+                     z, zbl_, c2a, pa, pv, pr, pY, pfc, pzbl, dr, nact, nact + 1, bdom, buckets ? rhist : nullptr)
+    if (nblk <= kPrefixBlocks) {
+      SO3LR_COMPACT(true);
+    } else {
+      hipLaunchKernelGGL(k_scan_counts, dim3(1), dim3(1024), 0, s, nblk, blk, nact, cap, nact + 1);
+      SO3LR_COMPACT(false);
+    }
+#undef SO3LR_COMPACT
+  };
   if (P > 0 && !shift_mode_) {
-    const RowsPos pos{x, sr_rows};
-    hipLaunchKernelGGL(k_sr_count<RowsPos>, dim3(nblk), dim3(256), 0, s, int(P), pos, rc2, blk);
-    hipLaunchKernelGGL(k_scan_counts, dim3(1), dim3(1024), 0, s, nblk, blk, nact, cap, nact + 1);
-    hipLaunchKernelGGL(k_sr_compact<RowsPos>, dim3(nblk), dim3(256), 0, s, int(P), pos, sr_nodes, rc2, blk, cap, z,
-                       zbl_, c2a, pa, pv, pr, pY, pfc, pzbl);
+    active_pairs(RowsPos{x, sr_rows}, RowsPos{x, sr_rows});
   } else if (P > 0) {
-    const ShiftPos pos{x, sr_nodes, static_cast<const int *>(sr_code_->p), box_len_[0], box_len_[1], box_len_[2]};
-    hipLaunchKernelGGL(k_sr_count<ShiftPos>, dim3(nblk), dim3(256), 0, s, int(P), pos, rc2, blk);
-    hipLaunchKernelGGL(k_scan_counts, dim3(1), dim3(1024), 0, s, nblk, blk, nact, cap, nact + 1);
-    hipLaunchKernelGGL(k_sr_compact<ShiftPos>, dim3(nblk), dim3(256), 0, s, int(P), pos, sr_nodes, rc2, blk, cap, z,
-                       zbl_, c2a, pa, pv, pr, pY, pfc, pzbl);
+    const int *codes = static_cast<const int *>(sr_code_->p);
+    const ShiftPos<false> pos{x, sr_nodes, codes, box_len_[0], box_len_[1], box_len_[2], nullptr};
+    if (gather_pos)  // the counts run on the caller's order while the same launch gathers x
+      active_pairs(ShiftPos<true>{x_in, sr_nodes, codes, box_len_[0], box_len_[1], box_len_[2], perm}, pos);
+    else
+      active_pairs(pos, pos);
   } else {
+    if (gather_pos)
+      hipLaunchKernelGGL(k_gather_pos, dim3(unsigned((3 * Nz + 255) / 256)), dim3(256), 0, s, int(N), perm, x_in,
+                         const_cast<double *>(x));
     hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, s, nact, 2, 0);  // no memset nodes in graphs
+    if (buckets) hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, s, rslots, 1, 0);
   }
-  // active incidence of this step (2 entries per candidate pair)
-  if (P > 0)
-    hipLaunchKernelGGL(k_inc_active, dim3(unsigned((2 * Pz + 255) / 256)), dim3(256), 0, s, int(2 * P), sr_inc, c2a,
-                       pa, iact, iother);
-  fill(dr, Pa);
+  // active incidence of this step (2 entries per candidate pair), and the
+  // placement of the pairs in bucket order
+  if (P > 0) {
+    if (buckets)
+      hipLaunchKernelGGL(k_rint_scan, dim3(1), dim3(1024), 0, s, rkeys, rhist, rstart, rcursor, rslots);
+    const std::int64_t threads = std::max<std::int64_t>(2 * P, buckets ? rkeys : 0);
+    const PlaceArgs R{nact, pr, bdom, rkeys, rhist, rstart, rcursor, buckets ? rord : nullptr};
+    hipLaunchKernelGGL(k_inc_active, dim3(unsigned(ceil_div(threads, 256))), dim3(256), 0, s, int(2 * P), sr_inc, c2a,
+                       pa, iact, iother, R);
+  }
   // erf(r / sigma) by the polynomial of erf_lean when r / sigma stays within [0, 3]
   const bool lean_erf = lr_.cutoff * lr_.inv_sigma <= 3.0;
   auto long_range = [&] { timed("long_range", 1, [&] {
@@ -3606,8 +3695,9 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
       G.cls_rep = crep;
       G.cls_order = cord;
       G.cls_slots = cslots;
-      hipLaunchKernelGGL(k_class_reps, dim3(unsigned(ceil_div(std::max<std::int64_t>(N, C * C), 256))), dim3(256), 0, s,
-                         int(N), z, G.cls_lut, perm, static_cast<const int *>(cls_rep0_->p), crep, C * C, chist);
+      if (!gen_->radial_ok() || rad_stale_)  // with the radial tables filled, nothing reads these
+        hipLaunchKernelGGL(k_class_reps, dim3(unsigned(ceil_div(std::max<std::int64_t>(N, C * C), 256))), dim3(256), 0,
+                           s, int(N), z, G.cls_lut, perm, static_cast<const int *>(cls_rep0_->p), crep, C * C, chist);
       if (gen_->radial_ok()) {
         // block 0 through the radial tables (filled once after set_system), in pair order
         G.rad_tab = static_cast<double *>(rad_tab_->p);
@@ -3623,18 +3713,10 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
       }
     }
     if (use_grt) {
-      // the blocks after 0 on their radial tables: the active pairs in bucket order
-      const int slots_max = PA + 16 * rkeys;
-      const RadialDomain &dom = gen_->rbl_domain();
-      const dim3 gpair(unsigned(std::max(1, ceil_div(PA, 256))));
-      hipLaunchKernelGGL(k_fill_int, dim3(unsigned(ceil_div(rkeys, 256))), dim3(256), 0, s, rhist, rkeys, 0);
-      hipLaunchKernelGGL(k_fill_int, dim3(unsigned(ceil_div(slots_max, 256))), dim3(256), 0, s, rord, slots_max, -1);
-      hipLaunchKernelGGL(k_rint_count, gpair, dim3(256), 0, s, nact, pa, pr, dom, rhist);
-      hipLaunchKernelGGL(k_rint_scan, dim3(1), dim3(1024), 0, s, rkeys, rhist, rhist + rkeys, rhist + 2 * rkeys);
-      hipLaunchKernelGGL(k_rint_place, gpair, dim3(256), 0, s, nact, pa, pr, dom, rhist + rkeys, rord);
+      // the blocks after 0 on their radial tables
       G.rint_order = rord;
-      G.rint_slots = rhist + 2 * rkeys;
-      G.rint_max = slots_max;
+      G.rint_slots = rslots;
+      G.rint_max = int(PA) + 16 * rkeys;
     }
     gen_->forward(G);
     hipLaunchKernelGGL(k_image_center, dim3(unsigned(n_images_)), dim3(1024), 0, s, img_off, img_q, qraw, q, 0);
@@ -3663,7 +3745,6 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
   // slots of the bucket order: every bucket padded by fewer than 16
   const int rslots_max = PA + 16 * rkeys;
   const unsigned gR = unsigned(ceil_div(rslots_max, 64));  // 16 slots per wavefront
-  const int *rslots = rhist ? rhist + 2 * rkeys : nullptr;
 
   // --- interaction blocks, forward ---
   for (int b = 0; b < L; ++b) {
@@ -3683,31 +3764,26 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
     }
     A.att_cg = B.att_cg; A.rbf_b = hw_.rbf_b; A.rbf_k = hw_.rbf_k; A.rbf_kr = hw_.rbf_kr; A.gamma = gamma_;
     const FilterMfma FM = filter_mfma(B, hw_, gamma_);
-    if (use_rt && b == 1) {
-      // the active pairs in bucket order, for every block after 0 and the reverse
-      const dim3 gpair(unsigned(std::max(1, ceil_div(PA, 256))));
-      hipLaunchKernelGGL(k_fill_int, dim3(unsigned(ceil_div(rkeys, 256))), dim3(256), 0, s, rhist, rkeys, 0);
-      hipLaunchKernelGGL(k_fill_int, dim3(unsigned(ceil_div(rslots_max, 256))), dim3(256), 0, s, rord, rslots_max, -1);
-      hipLaunchKernelGGL(k_rint_count, gpair, dim3(256), 0, s, nact, pa, pr, rbl_dom_, rhist);
-      hipLaunchKernelGGL(k_rint_scan, dim3(1), dim3(1024), 0, s, rkeys, rhist, rhist + rkeys, rhist + 2 * rkeys);
-      hipLaunchKernelGGL(k_rint_place, gpair, dim3(256), 0, s, nact, pa, pr, rbl_dom_, rhist + rkeys, rord);
-    }
     // the MFMA filter also forms the attention logits of both directions
     // from the filter tiles it holds; the scalar cross-check path leaves them
     // to the full attention kernel
     // block 0 runs cheaper instantiations (ev = 0): timed under their own names
     const bool blk0 = b == 0 && !scalar;
     if (blk0 && use_cls) {
-      // block 0's q k v rows of the element classes only, the element-pair
-      // tables from them, and the active pairs in element-pair order (used
-      // again by the reverse)
+      // block 0's q k v rows of the element classes only and the element-pair
+      // tables from them; both depend on the system alone, so with the radial
+      // tables the rows are formed once after set_system (in the scratch
+      // array, which keeps nothing, by every call)
       const int *lut = static_cast<const int *>(cls_lut_->p);
-      hipLaunchKernelGGL(k_class_reps, dim3(unsigned(ceil_div(std::max<std::int64_t>(N, C * C), 256))), dim3(256), 0, s,
-                         int(N), z, lut, perm, static_cast<const int *>(cls_rep0_->p), crep, C * C, chist);
-      hipLaunchKernelGGL(k_class_rows, dim3(unsigned(ceil_div(C * kF, 256))), dim3(256), 0, s, C, crep, xb, cxr);
-      hipLaunchKernelGGL(k_qkv_mfma<true>, dim3(1, kHeads), dim3(256), 0, s, C, kF, cxr, B.qkvp, cqkv);
-      if (qk_norm_)
-        hipLaunchKernelGGL(k_qk_norm, dim3(unsigned(ceil_div(16 * C, 256))), dim3(256), 0, s, C, cqkv, cqis);
+      if (!use_rad || from_scratch || cls_stale_) {
+        hipLaunchKernelGGL(k_class_reps, dim3(unsigned(ceil_div(std::max<std::int64_t>(N, C * C), 256))), dim3(256), 0,
+                           s, int(N), z, lut, perm, static_cast<const int *>(cls_rep0_->p), crep, C * C, chist);
+        hipLaunchKernelGGL(k_class_rows, dim3(unsigned(ceil_div(C * kF, 256))), dim3(256), 0, s, C, crep, xb, cxr);
+        hipLaunchKernelGGL(k_qkv_mfma<true>, dim3(1, kHeads), dim3(256), 0, s, C, kF, cxr, B.qkvp, cqkv);
+        if (qk_norm_)
+          hipLaunchKernelGGL(k_qk_norm, dim3(unsigned(ceil_div(16 * C, 256))), dim3(256), 0, s, C, cqkv, cqis);
+        if (!from_scratch) cls_stale_ = false;
+      }
       if (!use_rad || rad_stale_)  // with the radial tables filled, nothing reads these
         hipLaunchKernelGGL(k_class_tables, dim3(unsigned(C * C), 8), dim3(128), 0, s, C, cqkv, B.fw1[0], B.fw1[1],
                            B.ob10[0], B.ob10[1], cmt, cc0);
@@ -3903,10 +3979,8 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
                      perm, fo, ezbl, etot);
   hipLaunchKernelGGL(k_reduce_part, dim3(kReduceBlocks), dim3(256), 0, s, int(N), nact, etot, pv, pg, vlr, parts,
                      partial);
-  hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(256), 0, s, kReduceBlocks, partial, red);
-  hipLaunchKernelGGL(k_copy_count, dim3(1), dim3(64), 0, s, nact + 1, red + 9);  // the pairs found
+  hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(256), 0, s, kReduceBlocks, partial, nact + 1, host_out_);
   HIP_CHECK(hipGetLastError());
-  HIP_CHECK(hipMemcpyAsync(host_out_, red, 10 * sizeof(double), hipMemcpyDeviceToHost, s));
   };  // enqueue
 
   const GraphKey key{x_in, fo, etot, flags, {box_len_[0], box_len_[1], box_len_[2]}, s, topo_version_,

@@ -234,7 +234,7 @@ class Evaluator {
   Buffer *elr_, *dq_, *dh_, *flr_, *vlr_, *elr_parts_, *ezbl_;
   Buffer *gev_, *gainv_, *gaev_, *gqkv_;
   Buffer *qkis_, *c6eff_, *c6r_, *dc_;  // QK normalisation 1/rms; C6 head logit, ratio, dE/dratio
-  Buffer *fout_, *etot_, *red_, *red_part_;
+  Buffer *fout_, *etot_, *red_part_;
   // pair-sized buffers
   Buffer *owner_, *sr_rows_, *sr_nodes_, *sr_inc_off_, *sr_inc_, *lr_rows_, *lr_nodes_,
       *lr_inc_off_, *lr_inc_, *blk_count_, *n_active_, *cand2act_;
@@ -298,7 +298,8 @@ class Evaluator {
   // MFMA kernels.  rad_tab_ holds the element pairs' value and slope tables,
   // sized by set_system and filled by the first evaluation after it
   // (rad_stale_).
-  bool radial_tables_ = true, radial_ok_ = false, rad_stale_ = true;
+  // cls_stale_: the classes' rows (cls_rows_) are still to be formed for this system.
+  bool radial_tables_ = true, radial_ok_ = false, rad_stale_ = true, cls_stale_ = true;
   // the blocks after 0 on their radial tables (BlockWeights::rrow, rdr): every
   // such block's both radial branches fit to the bound; their pairs in
   // buckets of (spatial block, interval), each padded to a multiple of 16
