@@ -343,19 +343,7 @@ __global__ __launch_bounds__(256) void k_sr_compact(
   }
 }
 
-// Workgroups go to the 8 XCDs round-robin (block b on XCD b % 8).  Remapped
-// so that each XCD walks one contiguous range of logical blocks: with nodes
-// in spatial order, the neighbour rows a range gathers stay in its XCD's L2.
-// A bijection of [0, gridDim.x) whatever the grid size.
-__device__ __forceinline__ int xcd_block() {
-#ifdef SO3LR_NO_XCD_MAP
-  return blockIdx.x;
-#endif
-  const int G = gridDim.x, b = blockIdx.x;
-  const int per = G >> 3, rem = G & 7, xcd = b & 7, i = b >> 3;
-  return xcd * per + (xcd < rem ? xcd : rem) + i;
-}
-// The same for a grid sized for an upper bound of the work: only the first A
+// xcd_block for a grid sized for an upper bound of the work: only the first A
 // logical blocks have work (A <= gridDim.x, known on the device only), and
 // they are spread evenly over the XCDs; -1 for a block with none.
 __device__ __forceinline__ int xcd_block_active(int A) {
@@ -2099,7 +2087,8 @@ __global__ __launch_bounds__(256) void k_attn_fwd(int N, const int *inc_off, con
 // forward MFMA filter computed (same lane layout as k_attn_fwd): for node n
 // and every incident active pair, fc alpha v_o (invariant) and fc alpha_ev Y
 // (equivariant, (-1)^l Y when n is the pair's second endpoint).
-__global__ __launch_bounds__(256) void k_attn_msg(int N, const int *inc_off, const int *__restrict__ iact,
+template <int W>
+__global__ __launch_bounds__(NodeShare<W>::kBlock) void k_attn_msg(int N, const int *inc_off, const int *__restrict__ iact,
                                                   const int *__restrict__ iother, const double *__restrict__ x,
                                                   const double *__restrict__ ev, const double *__restrict__ qkv,
                                                   const double *__restrict__ pY, const double *__restrict__ pfc,
@@ -2108,14 +2097,16 @@ __global__ __launch_bounds__(256) void k_attn_msg(int N, const int *inc_off, con
                                                   double *__restrict__ aev, const int *__restrict__ z,
                                                   const int *__restrict__ cls) {
   const int lane = threadIdx.x & 63;
-  const int n = xcd_block() * 4 + (threadIdx.x >> 6);
-  if (n >= N) return;
+  __shared__ double lds[W > 1 ? NodeShare<W>::kBlock * 3 : 1];
+  const NodeShare<W> S(N, inc_off);
+  const int n = S.n;
+  if (W == 1 && !S.on) return;
   const int h = lane >> 4, t = lane & 15;
   const int p0 = 32 * h + 2 * t;
   const bool evv = t < 2 * h + 3;
   const int m = evv ? ev_offset(h) + t : 0;
   const double par = slot_parity(h);
-  double acc0 = 0.0, acc1 = 0.0, acce = 0.0;
+  double acc[3] = {0.0, 0.0, 0.0};
   struct Terms { double d0, d1, de; };
   auto terms = [&](int e, int o) {
     const int p = e >> 1, side = e & 1;
@@ -2127,21 +2118,23 @@ __global__ __launch_bounds__(256) void k_attn_msg(int N, const int *inc_off, con
     const double y = pY[kE * std::size_t(p) + m] * (side == 0 ? 1.0 : par);
     return Terms{fc * ai * vv.x, fc * ai * vv.y, fc * ae * y};
   };
-  for_active_pairs(inc_off[n], inc_off[n + 1], iact, iother, lane, [&](int e1, int o1, int e2, int o2, bool two) {
+  for_active_pairs(S.beg, S.end, iact, iother, lane, [&](int e1, int o1, int e2, int o2, bool two) {
     const Terms A = terms(e1, o1);
     const Terms B = terms(e2, o2);
-    acc0 += A.d0; acc1 += A.d1; acce += A.de;
-    if (two) { acc0 += B.d0; acc1 += B.d1; acce += B.de; }
+    acc[0] += A.d0; acc[1] += A.d1; acc[2] += A.de;
+    if (two) { acc[0] += B.d0; acc[1] += B.d1; acc[2] += B.de; }
   });
+  share_sum<W>(lds, acc);
+  if (!S.on || !S.first) return;
   // the residual and its first normalisation, with the whole node row in
   // this wavefront
   const std::size_t i = std::size_t(n) * kF + p0;
   const double2 xv = ld2(x + i);
   double h0, h1, is;
-  wave_normalise(xv.x + acc0, xv.y + acc1, eps, lnmode, h0, h1, is);
+  wave_normalise(xv.x + acc[0], xv.y + acc[1], eps, lnmode, h0, h1, is);
   st2(n1hat + i, h0, h1);
   if (lane == 0) n1is[n] = is;
-  if (evv) aev[std::size_t(n) * kE + m] = (ev ? ev[std::size_t(n) * kE + m] : 0.0) + acce;
+  if (evv) aev[std::size_t(n) * kE + m] = (ev ? ev[std::size_t(n) * kE + m] : 0.0) + acc[2];
 }
 
 // ---------------------------------------------------------------- charges
@@ -2464,8 +2457,8 @@ __global__ __launch_bounds__(256) void k_attn_bwd(int N, const int *inc_off, con
 // (32 bytes, psc + 16 p + 4 h), dE/dfc and dE/dY (FIRST, the first block of
 // the reverse pass, writes dE/dY without reading it).  Lane layout as in
 // k_attn_fwd; gainv in the tile-transposed order.
-template <bool FIRST>
-__global__ __launch_bounds__(256) void k_attn_bwd_nodes(int N, const int *inc_off, const int *__restrict__ iact,
+template <bool FIRST, int W>
+__global__ __launch_bounds__(NodeShare<W>::kBlock) void k_attn_bwd_nodes(int N, const int *inc_off, const int *__restrict__ iact,
                                                         const int *__restrict__ iother, const double *__restrict__ qkv,
                                                         const double *__restrict__ pf, const double *__restrict__ pY,
                                                         const double *__restrict__ pfc,
@@ -2475,8 +2468,10 @@ __global__ __launch_bounds__(256) void k_attn_bwd_nodes(int N, const int *inc_of
                                                         double *__restrict__ gqkv, double *__restrict__ psc,
                                                         double *__restrict__ pdfc, double *__restrict__ dY) {
   const int lane = threadIdx.x & 63;
-  const int n = xcd_block() * 4 + (threadIdx.x >> 6);
-  if (n >= N) return;
+  __shared__ double lds[W > 1 ? NodeShare<W>::kBlock * 10 : 1];
+  const NodeShare<W> S(N, inc_off);
+  const int n = S.n;
+  if (W == 1 && !S.on) return;
   const int h = lane >> 4, t = lane & 15;
   const int p0 = 32 * h + 2 * t;
   const bool evv = t < 2 * h + 3;
@@ -2486,7 +2481,7 @@ __global__ __launch_bounds__(256) void k_attn_bwd_nodes(int N, const int *inc_of
   const double2 mvv = ld2(me + 256 + p0);
   const double2 mgv = ld2(gainv + std::size_t(n) * kF + p0);
   const double mge = evv ? gaev[std::size_t(n) * kE + m] : 0.0;
-  double dq0 = 0, dq1 = 0, dk0 = 0, dk1 = 0, dv0 = 0, dv1 = 0, dqe0 = 0, dqe1 = 0, dke0 = 0, dke1 = 0;
+  double d[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};  // dq, dk, dv, dq_ev, dk_ev, two channels each
   auto visit = [&](int e, int o) {
     const int p = e >> 1, side = e & 1;
     const double *ot = qkv + std::size_t(o) * 640;
@@ -2511,11 +2506,11 @@ __global__ __launch_bounds__(256) void k_attn_bwd_nodes(int N, const int *inc_of
     const double coe = group_sum(oge * y_o);
     const double sin_ = fc * ci * inv_avg, sine = fc * ce * inv_avg;
     const double sout = fc * co * inv_avg, soute = fc * coe * inv_avg;
-    dq0 += sin_ * okv.x * fiv.x; dq1 += sin_ * okv.y * fiv.y;
-    dqe0 += sine * okev.x * fev.x; dqe1 += sine * okev.y * fev.y;
-    dk0 += sout * oqv.x * fiv.x; dk1 += sout * oqv.y * fiv.y;
-    dke0 += soute * oqev.x * fev.x; dke1 += soute * oqev.y * fev.y;
-    dv0 += fc * aout_i * ogv.x; dv1 += fc * aout_i * ogv.y;
+    d[0] += sin_ * okv.x * fiv.x; d[1] += sin_ * okv.y * fiv.y;
+    d[6] += sine * okev.x * fev.x; d[7] += sine * okev.y * fev.y;
+    d[2] += sout * oqv.x * fiv.x; d[3] += sout * oqv.y * fiv.y;
+    d[8] += soute * oqev.x * fev.x; d[9] += soute * oqev.y * fev.y;
+    d[4] += fc * aout_i * ogv.x; d[5] += fc * aout_i * ogv.y;
     // the pair's terms, once per pair (its side-0 endpoint; side is uniform
     // across the wavefront): every head's sums appear in that head's 16 lanes
     if (side == 0) {
@@ -2530,37 +2525,40 @@ __global__ __launch_bounds__(256) void k_attn_bwd_nodes(int N, const int *inc_of
       }
     }
   };
-  for_active_pairs(inc_off[n], inc_off[n + 1], iact, iother, lane, [&](int e1, int o1, int e2, int o2, bool two) {
+  for_active_pairs(S.beg, S.end, iact, iother, lane, [&](int e1, int o1, int e2, int o2, bool two) {
     visit(e1, o1);
     if (two) visit(e2, o2);
   });
-  double *gq = gqkv + std::size_t(n) * 640;
-  st2(gq + p0, dq0, dq1);
-  st2(gq + 128 + p0, dk0, dk1);
-  st2(gq + 256 + p0, dv0, dv1);
-  st2(gq + 384 + p0, dqe0, dqe1);
-  st2(gq + 512 + p0, dke0, dke1);
+  share_sum<W>(lds, d);
+  if (!S.on || !S.first) return;
+  double *gq = gqkv + std::size_t(n) * 640 + p0;
+#pragma unroll
+  for (int k = 0; k < 5; ++k) st2(gq + 128 * k, d[2 * k], d[2 * k + 1]);
 }
 
 // g_ev_in = g_aev + sum_pairs 2 (ev_n - ev_o) cg ds[slot]
-__global__ __launch_bounds__(256) void k_ev_bwd(int N, const int *inc_off, const int *__restrict__ iact,
+template <int W>
+__global__ __launch_bounds__(NodeShare<W>::kBlock) void k_ev_bwd(int N, const int *inc_off, const int *__restrict__ iact,
                                                 const int *__restrict__ iother, const double *__restrict__ ev,
                                                 const double *__restrict__ cg, const double *__restrict__ ds,
                                                 const double *__restrict__ gaev, double *__restrict__ gev) {
   const int lane = threadIdx.x & 63;
-  const int n = xcd_block() * 4 + (threadIdx.x >> 6);
-  if (n >= N) return;
+  __shared__ double lds[W > 1 ? NodeShare<W>::kBlock : 1];
+  const NodeShare<W> S(N, inc_off);
+  const int n = S.n;
+  if (W == 1 && !S.on) return;
   const int c = lane < kE ? lane : 0;
   const int slot = degree_slot(c);
   const double en = ev[std::size_t(n) * kE + c];
-  double acc = gaev[std::size_t(n) * kE + c];
+  double acc[1] = {S.first ? gaev[std::size_t(n) * kE + c] : 0.0};
   auto term = [&](int e, int o) { return 2.0 * (en - ev[std::size_t(o) * kE + c]) * cg[c] * ds[4 * std::size_t(e >> 1) + slot]; };
-  for_active_pairs(inc_off[n], inc_off[n + 1], iact, iother, lane, [&](int e1, int o1, int e2, int o2, bool two) {
+  for_active_pairs(S.beg, S.end, iact, iother, lane, [&](int e1, int o1, int e2, int o2, bool two) {
     const double a = term(e1, o1), b = term(e2, o2);
-    acc += a;
-    if (two) acc += b;
+    acc[0] += a;
+    if (two) acc[0] += b;
   });
-  if (lane < kE) gev[std::size_t(n) * kE + lane] = acc;
+  share_sum<W>(lds, acc);
+  if (S.on && S.first && lane < kE) gev[std::size_t(n) * kE + lane] = acc[0];
 }
 
 // ---------------------------------------------------------------- geometry
@@ -3591,6 +3589,9 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
   const double *img_q = static_cast<const double *>(img_q_->p);
 
   const int gN4 = ceil_div(N, 4);
+  // wavefronts per node of the node-major pair kernels (NodeShare)
+  auto by_split = [&](auto &&launch) { by_node_share(int(N), launch); };
+  auto node_grid = [&](auto w) { return dim3(unsigned(ceil_div(N, NodeShare<decltype(w)::value>::kNodes))); };
   // per-launch HIP events for the measured kernels; units: 0 = active pairs, 1 = nodes
   struct Pending { const char *name; hipEvent_t a, b; int unit_kind; };
   std::vector<Pending> pending;
@@ -3834,8 +3835,12 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
         hipLaunchKernelGGL(k_attn_fwd, dim3(gN4), dim3(256), 0, s, int(N), sr_off, iact, iother, xb, evb, qb,
                            pfb, pY, pfc, inv_avg, ln_eps_, norm1_, pab, n1hb, n1ib, aevb);
       else
-        hipLaunchKernelGGL(k_attn_msg, dim3(gN4), dim3(256), 0, s, int(N), sr_off, iact, iother, xb, evb,
-                           blk0 && use_cls ? cqkv : qb, pY, pfc, pab, ln_eps_, norm1_, n1hb, n1ib, aevb, z, blk0 && use_cls ? static_cast<const int *>(cls_lut_->p) : nullptr);
+        by_split([&](auto w) {
+          constexpr int W = decltype(w)::value;
+          hipLaunchKernelGGL(k_attn_msg<W>, node_grid(w), dim3(NodeShare<W>::kBlock), 0, s, int(N), sr_off, iact, iother,
+                             xb, evb, blk0 && use_cls ? cqkv : qb, pY, pfc, pab, ln_eps_, norm1_, n1hb, n1ib, aevb, z,
+                             blk0 && use_cls ? static_cast<const int *>(cls_lut_->p) : nullptr);
+        });
     });
     // the post-attention node chain in one kernel (MLP, interaction,
     // LayerNorm 2, ev gate), then the next block's projections or the heads
@@ -3914,12 +3919,12 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
       const bool first = b == L - 1;
       if (b > 0)
         timed("attn_bwd", 1, [&] {
-          if (first)
-            hipLaunchKernelGGL(k_attn_bwd_nodes<true>, dim3(gN4), dim3(256), 0, s, int(N), sr_off, iact, iother, qb,
-                               pfb, pY, pfc, pab, gainv, gaev, inv_avg, gqkv, psc, dfc, dY);
-          else
-            hipLaunchKernelGGL(k_attn_bwd_nodes<false>, dim3(gN4), dim3(256), 0, s, int(N), sr_off, iact, iother, qb,
-                               pfb, pY, pfc, pab, gainv, gaev, inv_avg, gqkv, psc, dfc, dY);
+          by_split([&](auto w) {
+            constexpr int W = decltype(w)::value;
+            hipLaunchKernelGGL((first ? k_attn_bwd_nodes<true, W> : k_attn_bwd_nodes<false, W>), node_grid(w),
+                               dim3(NodeShare<W>::kBlock), 0, s, int(N), sr_off, iact, iother, qb, pfb, pY, pfc, pab,
+                               gainv, gaev, inv_avg, gqkv, psc, dfc, dY);
+          });
         });
       const FilterMfma FM = filter_mfma(B, hw_, gamma_);
       if (b == 0 && use_cls) {
@@ -3965,8 +3970,11 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
       if (qk_norm_)  // through the QK normalisation to the raw projections
         hipLaunchKernelGGL(k_qk_norm_bwd, dim3(unsigned(ceil_div(16 * N, 256))), dim3(256), 0, s, int(N), qb,
                            qkis + b * Nz * 16, gqkv);
-      hipLaunchKernelGGL(k_ev_bwd, dim3(gN4), dim3(256), 0, s, int(N), sr_off, iact, iother, evb, B.att_cg, ds,
-                         gaev, gev);
+      by_split([&](auto w) {
+        constexpr int W = decltype(w)::value;
+        hipLaunchKernelGGL(k_ev_bwd<W>, node_grid(w), dim3(NodeShare<W>::kBlock), 0, s, int(N), sr_off, iact, iother,
+                           evb, B.att_cg, ds, gaev, gev);
+      });
     }
   }
 

@@ -119,8 +119,9 @@ __device__ __forceinline__ int g_xcd_block(int active) {
 // node n receives from each incident pair's partner o the invariant message
 // fc alpha v_o and the equivariant fc alpha_ev Y (parity of the direction),
 // then the residual and the first normalisation.  ev null: zero (block 0).
-// One wavefront per node.
-__global__ __launch_bounds__(256) void g_attn_msg(GDims d, int N, const int *__restrict__ inc_off,
+// NodeShare: wavefronts per node.
+template <int W>
+__global__ __launch_bounds__(NodeShare<W>::kBlock) void g_attn_msg(GDims d, int N, const int *__restrict__ inc_off,
                                                   const int *__restrict__ iact, const int *__restrict__ iother,
                                                   const double *__restrict__ x, const double *__restrict__ ev,
                                                   const double *__restrict__ qkv, const double *__restrict__ pY,
@@ -128,12 +129,12 @@ __global__ __launch_bounds__(256) void g_attn_msg(GDims d, int N, const int *__r
                                                   double eps, int mode, double *__restrict__ n1hat,
                                                   double *__restrict__ n1is, double *__restrict__ aev) {
   const int lane = threadIdx.x & 63;
-  const int blk = g_xcd_block((N + 3) / 4);
-  if (blk < 0) return;
-  const int n = blk * 4 + (threadIdx.x >> 6);
-  if (n >= N) return;
+  __shared__ double lds[W > 1 ? NodeShare<W>::kBlock * 6 : 1];
+  const NodeShare<W> S(N, inc_off);
+  const int n = S.n;
+  if (W == 1 && !S.on) return;
   const int F = d.F, NH = d.NH, E = d.E, J = F >> 6;
-  double di[4] = {0, 0, 0, 0}, de[2] = {0, 0};
+  double sum[6] = {0, 0, 0, 0, 0, 0};  // four invariant channels, two equivariant
   // this lane's channels: invariant c = lane + 64 j (head c / 32), and
   // equivariant c = lane + 64 j below E (slot, harmonic, parity)
   int sl[2] = {0, 0}, sh[2] = {0, 0};
@@ -174,24 +175,26 @@ __global__ __launch_bounds__(256) void g_attn_msg(GDims d, int N, const int *__r
   auto add = [&](const Terms &T) {
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-      if (j < J) di[j] += T.fc * T.a[j] * T.v[j];
+      if (j < J) sum[j] += T.fc * T.a[j] * T.v[j];
 #pragma unroll
     for (int j = 0; j < 2; ++j)
-      if (lane + 64 * j < E) de[j] += T.fc * T.ae[j] * T.y[j];
+      if (lane + 64 * j < E) sum[4 + j] += T.fc * T.ae[j] * T.y[j];
   };
-  for_active_pairs(inc_off[n], inc_off[n + 1], iact, iother, lane, [&](int e1, int o1, int e2, int o2, bool two) {
+  for_active_pairs(S.beg, S.end, iact, iother, lane, [&](int e1, int o1, int e2, int o2, bool two) {
     const Terms A = load(e1, o1), B = load(e2, o2);
     add(A);
     if (two) add(B);
   });
+  share_sum<W>(lds, sum);
+  if (!S.on || !S.first) return;
   double v[4], h[4], is;
-  for (int j = 0; j < J; ++j) v[j] = x[std::size_t(n) * F + lane + 64 * j] + di[j];
+  for (int j = 0; j < J; ++j) v[j] = x[std::size_t(n) * F + lane + 64 * j] + sum[j];
   g_norm_row(F, mode, v, eps, h, is);
   for (int j = 0; j < J; ++j) n1hat[std::size_t(n) * F + lane + 64 * j] = h[j];
   if (lane == 0) n1is[n] = is;
   for (int j = 0; j < 2; ++j) {
     const int c = lane + 64 * j;
-    if (c < E) aev[std::size_t(n) * E + c] = (ev ? ev[std::size_t(n) * E + c] : 0.0) + de[j];
+    if (c < E) aev[std::size_t(n) * E + c] = (ev ? ev[std::size_t(n) * E + c] : 0.0) + sum[4 + j];
   }
 }
 
@@ -264,30 +267,43 @@ __global__ __launch_bounds__(256) void g_attn_bwd_node(GDims d, int N, const int
 
 // gev = ga + sum over incident pairs of 2 (ev_n - ev_o) cg ds[slot]: the
 // edge invariants' adjoint (kokkos_block2_attention_input_reverse.cpp:144-196).
-__global__ __launch_bounds__(256) void g_ev_bwd(GDims d, int N, const int *__restrict__ inc_off,
-                                                const int *__restrict__ iact, const int *__restrict__ iother,
-                                                const double *__restrict__ ev, const double *__restrict__ cg,
-                                                const double *__restrict__ ds, const double *__restrict__ ga,
-                                                double *__restrict__ gev) {
+template <int W>
+__global__ __launch_bounds__(NodeShare<W>::kBlock) void g_ev_bwd(
+    GDims d, int N, const int *__restrict__ inc_off, const int *__restrict__ iact, const int *__restrict__ iother,
+    const double *__restrict__ ev, const double *__restrict__ cg, const double *__restrict__ ds,
+    const double *__restrict__ ga, double *__restrict__ gev) {
+  __shared__ double lds[W > 1 ? NodeShare<W>::kBlock * 2 : 1];
   const int lane = threadIdx.x & 63;
-  const int blk = g_xcd_block((N + 3) / 4);
-  if (blk < 0) return;
-  const int n = blk * 4 + (threadIdx.x >> 6);
-  if (n >= N) return;
+  const NodeShare<W> S(N, inc_off);
+  const int n = S.n;
+  if (W == 1 && !S.on) return;
   const int E = d.E;
+  // this lane's channels lane and 64 + lane (past E: channel 0, not written)
+  int c[2], sl[2];
+  double en[2], w[2], acc[2];
+#pragma unroll
   for (int j = 0; j < 2; ++j) {
-    const int c = lane + 64 * j;
-    if (c >= E) continue;
-    const int sl = d.slot[c];
-    const double en = ev[std::size_t(n) * E + c];
-    double acc = ga[std::size_t(n) * E + c];
-    for (int k = inc_off[n]; k < inc_off[n + 1]; ++k) {
-      const int e = iact[k];
-      if (e < 0) continue;
-      acc += 2.0 * (en - ev[std::size_t(iother[k]) * E + c]) * cg[c] * ds[std::size_t(e >> 1) * d.NH + sl];
-    }
-    gev[std::size_t(n) * E + c] = acc;
+    c[j] = lane + 64 * j < E ? lane + 64 * j : 0;
+    sl[j] = d.slot[c[j]];
+    en[j] = ev[std::size_t(n) * E + c[j]];
+    w[j] = 2.0 * cg[c[j]];
+    acc[j] = S.first ? ga[std::size_t(n) * E + c[j]] : 0.0;
   }
+  auto add = [&](int e, int o) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      if (j == 0 || E > 64)
+        acc[j] += (en[j] - ev[std::size_t(o) * E + c[j]]) * w[j] * ds[std::size_t(e >> 1) * d.NH + sl[j]];
+  };
+  for_active_pairs(S.beg, S.end, iact, iother, lane, [&](int e1, int o1, int e2, int o2, bool two) {
+    add(e1, o1);
+    if (two) add(e2, o2);
+  });
+  share_sum<W>(lds, acc);
+  if (!S.on || !S.first) return;
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+    if (lane + 64 * j < E) gev[std::size_t(n) * E + lane + 64 * j] = acc[j];
 }
 
 // ------------------------------------------------------------- pair kernels
@@ -1952,7 +1968,6 @@ void GenericPath::forward(const GContext &c) {
   const hipStream_t s = c.s;
   const int N = c.N, cap = c.cap, F = d.F, E = d.E, NH = d.NH, R = d.R, FH = d.FH;
   const std::size_t n = std::size_t(N), P = std::size_t(std::max(cap, 1));
-  const unsigned g4x = (blocks_for(n, 4) + 7) / 8 * 8;  // g_xcd_block's grids
   const unsigned gP = blocks_for(P, 256);
   double *xs = b_[XS], *evs = b_[EVS];
   const bool scaled = !c.resid->empty();
@@ -2028,8 +2043,12 @@ void GenericPath::forward(const GContext &c) {
     });
     }
     }
-    hipLaunchKernelGGL(g_attn_msg, dim3(g4x), dim3(256), 0, s, d, N, c.inc_off, c.iact, c.iother, xb, evb, qb, c.pY,
-                       c.pfc, pab, c.ln_eps, c.norm1, n1hb, n1ib, aevb);
+    by_node_share(N, [&](auto w) {
+      constexpr int W = decltype(w)::value;
+      hipLaunchKernelGGL(g_attn_msg<W>, dim3(blocks_for(n, NodeShare<W>::kNodes)), dim3(NodeShare<W>::kBlock), 0, s, d,
+                         N, c.inc_off, c.iact, c.iother, xb, evb, qb, c.pY, c.pfc, pab, c.ln_eps, c.norm1, n1hb, n1ib,
+                         aevb);
+    });
     // the post-attention node chain (kokkos_post_attention_block0.cpp:165-300),
     // then the next block's projections or the heads
     const bool last = b + 1 == layers_;
@@ -2064,7 +2083,6 @@ void GenericPath::reverse(const GContext &c) {
   const hipStream_t s = c.s;
   const int N = c.N, cap = c.cap, F = d.F, E = d.E, NH = d.NH, R = d.R;
   const std::size_t n = std::size_t(N), P = std::size_t(std::max(cap, 1));
-  const unsigned g4x = (blocks_for(n, 4) + 7) / 8 * 8;  // g_xcd_block's grids
   double *gev = b_[GEV];
   for (int b = layers_ - 1; b >= 0; --b) {
     const GBlock &B = bw_[b];
@@ -2152,8 +2170,11 @@ void GenericPath::reverse(const GContext &c) {
       if (c.qk_norm)
         hipLaunchKernelGGL(g_qk_norm_bwd, dim3(blocks_for(n * 4 * NH, 256)), dim3(256), 0, s, N, F, NH, qb,
                            b_[QKIS] + b * n * 4 * NH, b_[GQKV]);
-      hipLaunchKernelGGL(g_ev_bwd, dim3(g4x), dim3(256), 0, s, d, N, c.inc_off, c.iact, c.iother, evb, B.att_cg,
-                         b_[DS], b_[GA], gev);
+      by_node_share(N, [&](auto w) {
+        constexpr int W = decltype(w)::value;
+        hipLaunchKernelGGL(g_ev_bwd<W>, dim3(blocks_for(n, NodeShare<W>::kNodes)), dim3(NodeShare<W>::kBlock), 0, s, d,
+                           N, c.inc_off, c.iact, c.iother, evb, B.att_cg, b_[DS], b_[GA], gev);
+      });
     }
   }
   G_CHECK(hipGetLastError());

@@ -4,6 +4,8 @@
 // reverse.  F = 16 NT features (NT = 8 or 16), NT / 2 heads and degree slots.
 #pragma once
 
+#include <type_traits>
+
 #include "device_math.hpp"
 #include "mfma_ops.hpp"
 #include "model.hpp"
@@ -30,6 +32,70 @@ __device__ __forceinline__ void row_store(double *row, int t, int g, const v4d &
     r[4] = v[1];
     r[8] = v[2];
     r[12] = v[3];
+  }
+}
+
+// Workgroups go to the 8 XCDs round-robin (block b on XCD b % 8).  Remapped
+// so that each XCD walks one contiguous range of logical blocks: with nodes
+// in spatial order, the neighbour rows a range gathers stay in its XCD's L2.
+// A bijection of [0, gridDim.x) whatever the grid size.
+__device__ __forceinline__ int xcd_block() {
+#ifdef SO3LR_NO_XCD_MAP
+  return blockIdx.x;
+#endif
+  const int G = gridDim.x, b = blockIdx.x;
+  const int per = G >> 3, rem = G & 7, xcd = b & 7, i = b >> 3;
+  return xcd * per + (xcd < rem ? xcd : rem) + i;
+}
+// A node's wavefronts in the node-major kernels: W wavefronts share a node's
+// incidence list in W runs, and the first adds the others' sums in run order.
+// One wavefront per node reads its list serially (about 1 us per pair of
+// partners, latency alone); with few nodes the chip is idle beside it, so the
+// list is cut in 8 below kShare8 nodes and in 4 below kShare4.  Measured (us
+// per evaluation at 1 / 2 / 4 / 8 wavefronts): 99 atoms 515 / 439 / 391 / 373,
+// 375 atoms 502 / 438 / 409 / 397, 750 atoms 571 / 503 / 462 / 468, 1,764
+// atoms 769 / 727 / 717 / 732, 3,000 atoms 929 / 958 / 931 / 961.
+constexpr int kShare8 = 500, kShare4 = 2400;
+template <class Launch>
+void by_node_share(int N, Launch &&launch) {
+  if (N < kShare8) launch(std::integral_constant<int, 8>{});
+  else if (N < kShare4) launch(std::integral_constant<int, 4>{});
+  else launch(std::integral_constant<int, 1>{});
+}
+template <int W>
+struct NodeShare {
+  static constexpr int kBlock = W > 4 ? 64 * W : 256, kNodes = kBlock / 64 / W;
+  int n, beg, end;
+  bool on, first;  // n < N; this wavefront writes the node's results
+  __device__ __forceinline__ NodeShare(int N, const int *__restrict__ off) {
+    const int wv = threadIdx.x >> 6, part = wv % W;
+    n = xcd_block() * kNodes + wv / W;
+    on = n < N;
+    first = part == 0;
+    if (on) {
+      const int b = off[n], len = off[n + 1] - b;
+      beg = b + len * part / W;
+      end = b + len * (part + 1) / W;
+    } else {
+      beg = end = n = 0;
+    }
+  }
+};
+// v[0..M) summed over the node's wavefronts, in the first of them (every
+// wavefront of the block calls this; lds: kBlock * M doubles)
+template <int W, int M>
+__device__ __forceinline__ void share_sum(double *lds, double (&v)[M]) {
+  if constexpr (W > 1) {
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+#pragma unroll
+    for (int k = 0; k < M; ++k) lds[(wv * M + k) * 64 + lane] = v[k];
+    __syncthreads();
+    if (wv % W == 0) {
+#pragma unroll
+      for (int q = 1; q < W; ++q)
+#pragma unroll
+        for (int k = 0; k < M; ++k) v[k] += lds[((wv + q) * M + k) * 64 + lane];
+    }
   }
 }
 

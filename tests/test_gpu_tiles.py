@@ -14,19 +14,28 @@ from test_gpu_edges import _both_paths, model, orc  # noqa: F401
 pytestmark = pytest.mark.gpu
 
 
-def _cluster(n, seed=3):
-    """n H and O atoms on a jittered 1.7 A lattice, every pair of neighbours
-    inside the short-range cutoff."""
+def _cluster(n, seed=3, spacing=1.7):
+    """n H and O atoms on a jittered lattice, every pair of neighbours inside
+    the short-range cutoff."""
     rng = np.random.default_rng([seed, n])
     g = int(np.ceil(n ** (1 / 3) - 1e-9))
     sites = np.array([[i, j, k] for i in range(g) for j in range(g) for k in range(g)], float)[:n]
     z = rng.choice([1, 8], size=n, p=[0.6, 0.4])
-    return z, 1.7 * sites + rng.uniform(-0.2, 0.2, (n, 3)), 1.0 + float((z == 1).sum() % 2)
+    return z, spacing * sites + rng.uniform(-0.2, 0.2, (n, 3)), 1.0 + float((z == 1).sum() % 2)
 
 
 @pytest.mark.parametrize("n", [2, 15, 16, 17, 33, 65])
 def test_atom_tiles(orc, model, n):  # noqa: F811
     z, x, m = _cluster(n)
+    _both_paths(z, x, 0.0, m, orc, model)
+
+
+@pytest.mark.parametrize("n", [499, 500, 2399, 2400])
+def test_node_shares(orc, model, n):  # noqa: F811
+    """Both sides of the atom counts at which 8, 4 and 1 wavefronts share a
+    node's incidence list; nodes with fewer partners than wavefronts are at
+    the cluster's corners."""
+    z, x, m = _cluster(n, spacing=2.8)
     _both_paths(z, x, 0.0, m, orc, model)
 
 
