@@ -777,17 +777,30 @@ __global__ __launch_bounds__(256) FILTER_FWD_OCCUPANCY void k_filter_fwd_mfma(co
 // logits of both directions to palpha as in k_filter_fwd_mfma.  Measured
 // as two passes (the rows in bucket order, the logits in pair order) it
 // took 0.79 against 0.70 ms.
+//
+// SPLIT, below kFewPairs pairs: eight wavefronts per 16 slots, one per filter
+// and head (two output tiles each, the spherical hidden layer formed by
+// each).  One wavefront walks 134 dependent operands for its 16 pairs, and
+// few pairs leave most SIMDs without one; with more, the hidden layer's
+// seven further copies cost more than the shorter walk gives.  Whole
+// evaluations without / with this kernel and k_filter_bwd_split (us, by pairs
+// with their margin): 22 atoms 316 / 284, 2,200 pairs 372 / 323, 4,700 394 /
+// 366, 6,200 396 / 374, 6,900 451 / 430, 10,300 420 / 431, 11,200 428 / 443.
+constexpr int kFewPairs = 8500;
 #ifndef SO3LR_RT_FWD_PF
 #define SO3LR_RT_FWD_PF 6
 #endif
-__global__ __launch_bounds__(256) FILTER_FWD_OCCUPANCY void k_radial_fwd_rows(
+template <bool SPLIT>
+__global__ __launch_bounds__(SPLIT ? 512 : 256) FILTER_FWD_OCCUPANCY void k_radial_fwd_rows(
     const int *n_slots, const int *order, const int *pa, const double *pr, const double *__restrict__ ev,
     const double *__restrict__ qkv, const double *__restrict__ rtab, RadialDomain rd, double inv_avg, FilterMfma A,
     double *ps, double *pf, double *palpha) {
   SO3LR_EXP2_TABLE(A)
   const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
-  const int blk = xcd_block_active((*n_slots + 63) / 64);
-  const int wave = blk < 0 ? -1 : blk * 4 + (threadIdx.x >> 6);
+  const int blk = xcd_block_active(SPLIT ? (*n_slots + 15) / 16 : (*n_slots + 63) / 64);
+  const int sub = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  const int wave = blk < 0 ? -1 : (SPLIT ? blk : blk * 4 + sub);
+  const int which0 = SPLIT ? sub >> 2 : 0, mt0 = SPLIT ? 2 * (sub & 3) : 0;
   int p, ri;
   bool inside;
   v4d tp[2];
@@ -797,23 +810,25 @@ __global__ __launch_bounds__(256) FILTER_FWD_OCCUPANCY void k_radial_fwd_rows(
   const int a = pa[2 * pp], b = pa[2 * pp + 1];
   const double *qa = qkv + std::size_t(a) * 640 + 4 * g, *qb = qkv + std::size_t(b) * 640 + 4 * g;
   const double *coef = rtab + std::size_t(ri) * 2 * 16 * 256;
-  constexpr int TS = 3, PT = 8, NF = TS + 8 * PT;
+  constexpr int TS = 3, PT = 8, NF = TS + (SPLIT ? 2 : 8) * PT;
   auto load = [&](auto si) -> v4d {
-    constexpr int S = decltype(si)::value, which = S / NF, s = S % NF;
-    if constexpr (s < 2) return tile_load(A.eb0p[which], s, lane);
-    else if constexpr (s == 2) return tile_load(A.e0pk[which], 0, lane);
+    constexpr int S = decltype(si)::value, s = S % NF;
+    const int which = which0 + S / NF;
+    if constexpr (s < 2) return tile_load(which ? A.eb0p[1] : A.eb0p[0], s, lane);
+    else if constexpr (s == 2) return tile_load(which ? A.e0pk[1] : A.e0pk[0], 0, lane);
     else {
-      constexpr int mt = (s - TS) / PT, u = (s - TS) % PT;
-      constexpr int qoff = which ? 384 : 0, koff = which ? 512 : 128;
+      constexpr int u = (s - TS) % PT;
+      const int mt = mt0 + (s - TS) / PT;
+      const int qoff = which ? 384 : 0, koff = which ? 512 : 128;
       if constexpr (u < 2) return wload(coef + which * 16 * 256, 2, mt, u, lane);
       else if constexpr (u == 2) return *reinterpret_cast<const v4d *>(qa + qoff + 16 * mt);
       else if constexpr (u == 3) return *reinterpret_cast<const v4d *>(qb + koff + 16 * mt);
       else if constexpr (u == 4) return *reinterpret_cast<const v4d *>(qb + qoff + 16 * mt);
       else if constexpr (u == 5) return *reinterpret_cast<const v4d *>(qa + koff + 16 * mt);
-      else return wload(A.e1p[which], 2, mt, u - 6, lane);
+      else return wload(which ? A.e1p[1] : A.e1p[0], 2, mt, u - 6, lane);
     }
   };
-  Stream<2 * NF, SO3LR_RT_FWD_PF, decltype(load)> st(load);
+  Stream<(SPLIT ? 1 : 2) * NF, SO3LR_RT_FWD_PF, decltype(load)> st(load);
   st.prime();
   // equivariant invariant of degree slot g, all loads in flight at once
   double sg = 0.0;
@@ -832,14 +847,15 @@ __global__ __launch_bounds__(256) FILTER_FWD_OCCUPANCY void k_radial_fwd_rows(
       const double d = va[k] - vb[k];
       sg += k < n ? d * d * A.att_cg[lo + k] : 0.0;
     }
-    if (valid) ps[4 * std::size_t(p) + g] = sg;
+    if (valid && (!SPLIT || sub == 0)) ps[4 * std::size_t(p) + g] = sg;
   }
   v4d *const rowv = reinterpret_cast<v4d *>(pf + 256 * std::size_t(pp) + 4 * g);
   const v4d zero = v4d{0.0, 0.0, 0.0, 0.0};
   v4d h2[2], o, qv, qk0, qk1;
   double t0 = 0.0, t1 = 0.0;
   st.run([&](auto si, const v4d &w) {
-    constexpr int S = decltype(si)::value, which = S / NF, s = S % NF;
+    constexpr int S = decltype(si)::value, s = S % NF;
+    const int which = which0 + S / NF;
     if constexpr (s < 2) {
       h2[s] = w;
     } else if constexpr (s == 2) {
@@ -850,7 +866,8 @@ __global__ __launch_bounds__(256) FILTER_FWD_OCCUPANCY void k_radial_fwd_rows(
         for (int r = 0; r < 4; ++r) h2[t][r] = silu_tab_wide(h2[t][r], exp2_lds);
       }
     } else {
-      constexpr int mt = (s - TS) / PT, u = (s - TS) % PT;
+      constexpr int u = (s - TS) % PT;
+      const int mt = mt0 + (s - TS) / PT;
       if constexpr (u == 0) {
         o = mfma4(w, tp[0], zero);
       } else if constexpr (u == 1) {
@@ -867,12 +884,12 @@ __global__ __launch_bounds__(256) FILTER_FWD_OCCUPANCY void k_radial_fwd_rows(
           if (valid) __builtin_nontemporal_store(o, rowv + which * 32 + 4 * mt);
           t0 += ((qk0[0] * o[0] + qk0[1] * o[1]) + qk0[2] * o[2]) + qk0[3] * o[3];
           t1 += ((qk1[0] * o[0] + qk1[1] * o[1]) + qk1[2] * o[2]) + qk1[3] * o[3];
-          if constexpr (mt & 1) {
+          if constexpr (((s - TS) / PT) & 1) {
             t0 += __shfl_xor(t0, 16, kWave);
             t0 += __shfl_xor(t0, 32, kWave);
             t1 += __shfl_xor(t1, 16, kWave);
             t1 += __shfl_xor(t1, 32, kWave);
-            constexpr int hd = mt / 2;
+            const int hd = mt / 2;
             if (valid && g == hd) {
               double *al = palpha + 16 * std::size_t(p) + 4 * which + hd;
               al[0] = t0 * inv_avg;
@@ -1301,6 +1318,103 @@ k_filter_bwd_mfma(
       if (r < rc) {
         const double t = r / rc;
         grad += dfc * (-30.0 * t * t * (1.0 - t) * (1.0 - t) / rc);
+      }
+      dr[p] += grad;
+    }
+  }
+}
+
+// k_filter_bwd_mfma<false, false, true> for few pairs: eight wavefronts per 16
+// slots, one per filter and head, each with its head's two df chunks; the
+// spherical branch's silu' and E0^T are linear in the chunks' share of
+// E1^T df, so every wavefront takes its share through to dE/ds and dE/dr and
+// the shares are summed through LDS in wavefront order.
+__global__ __launch_bounds__(512) void k_filter_bwd_split(
+    const int *n_slots, const int *order, const int *pa, const double *pr, const double *ps,
+    const double *__restrict__ qkv, const double *__restrict__ psc, const double *__restrict__ pdfc, FilterMfma A,
+    double rc, double *ds, double *dr, const double *__restrict__ rtab, RadialDomain rd) {
+  SO3LR_EXP2_TABLE(A)
+  __shared__ double share[8][2][64];
+  const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
+  const int sub = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  const int wave = xcd_block_active((*n_slots + 15) / 16);
+  int p, ri;
+  bool inside;
+  v4d tp[2];
+  if (!rint_slots(n_slots, order, pr, rd, wave, j, g, p, ri, inside, tp)) return;  // the whole block
+  const bool valid = p >= 0;
+  const int pp = valid ? p : order[wave * 16];
+  const int a = pa[2 * pp], b = pa[2 * pp + 1];
+  const int which = sub >> 2, hd = sub & 3;
+  const int qoff = which ? 384 : 0, koff = which ? 512 : 128;
+  const double *ra = qkv + std::size_t(a) * 640 + 4 * g + 32 * hd, *rb = qkv + std::size_t(b) * 640 + 4 * g + 32 * hd;
+  const double *slopes = rtab + (std::size_t(ri) * 2 + which) * 16 * 256;
+  const double *e1t = which ? A.e1tp[1] : A.e1tp[0], *e0t = which ? A.e0tp[1] : A.e0tp[0];
+  const double *eb0 = which ? A.eb0p[1] : A.eb0p[0], *e0k = which ? A.e0pk[1] : A.e0pk[0];
+  auto row = [](const double *r) { return *reinterpret_cast<const v4d *>(r); };
+  v4d rows[2][4], fr[2][4];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    rows[t][0] = row(ra + qoff + 16 * t);
+    rows[t][1] = row(rb + koff + 16 * t);
+    rows[t][2] = row(rb + qoff + 16 * t);
+    rows[t][3] = row(ra + koff + 16 * t);
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      fr[t][q] = wload(e1t, 8, q, 2 * hd + t, lane);
+      fr[t][2 + q] = wload(slopes, 8, q, 2 * hd + t, lane);
+    }
+  }
+  const v4d rec = row(psc + 16 * std::size_t(pp) + 4 * hd);
+  const double s_in = which ? rec[2] : rec[0], s_out = which ? rec[3] : rec[1];
+  const double sg = ps[4 * std::size_t(pp) + g];
+  v4d pre[2] = {tile_load(eb0, 0, lane), tile_load(eb0, 1, lane)};
+  const v4d w0 = row(e0k + 4 * lane), t0 = wload(e0t, 2, 0, 0, lane), t1 = wload(e0t, 2, 0, 1, lane);
+  const v4d zero = v4d{0.0, 0.0, 0.0, 0.0};
+  v4d dh[2] = {zero, zero}, acc[2] = {zero, zero};
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const v4d df = s_in * (rows[t][0] * rows[t][1]) + s_out * (rows[t][2] * rows[t][3]);
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      dh[q] = mfma4(fr[t][q], df, dh[q]);
+      acc[q] = mfma4(fr[t][2 + q], df, acc[q]);
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    pre[q] = mfma(w0[q], sg, pre[q]);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) dh[q][r] *= silu_prime_tab_wide(pre[q][r], exp2_lds);
+  }
+  const v4d dsa = mfma4(t1, dh[1], mfma4(t0, dh[0], zero));
+  double part = 0.0;
+#pragma unroll
+  for (int m = 0; m < 2; ++m)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) part += acc[m][r] * tp[m][r];
+  share[sub][0][lane] = dsa[0];
+  share[sub][1][lane] = part;
+  __syncthreads();
+  if (sub != 0) return;
+  double ds_acc = 0.0;
+  part = 0.0;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    ds_acc += share[q][0][lane];
+    part += share[q][1][lane];
+  }
+  part = inside ? part : 0.0;
+  part += __shfl_xor(part, 16, kWave);
+  part += __shfl_xor(part, 32, kWave);
+  if (valid) {
+    ds[4 * std::size_t(p) + g] = ds_acc;
+    if (g == 0) {
+      const double r = pr[p];
+      double grad = part;
+      if (r < rc) {
+        const double t = r / rc;
+        grad += pdfc[p] * (-30.0 * t * t * (1.0 - t) * (1.0 - t) / rc);
       }
       dr[p] += grad;
     }
@@ -2818,7 +2932,8 @@ Evaluator::Evaluator(std::shared_ptr<Model> model, int device) : model_(std::mov
   HIP_CHECK(hipSetDevice(device));
   HIP_CHECK(hipStreamCreateWithFlags(&own_stream_, hipStreamNonBlocking));
   if (const char *nv = std::getenv("SO3LR_NAIVE_FILTERS")) naive_filters_ = nv[0] == '1';
-  if (const char *sp = std::getenv("SO3LR_SCALAR_FILTER_PAIRS")) scalar_pairs_max_ = std::atoll(sp);
+  if (const char *sp = std::getenv("SO3LR_SCALAR_FILTER_PAIRS"))
+    scalar_pairs_max_ = std::max(0LL, std::atoll(sp));
   // SO3LR_NO_GRAPH=1: always launch the kernels one by one (no graph replay)
   if (const char *ng = std::getenv("SO3LR_NO_GRAPH")) use_graphs_ = ng[0] != '1';
   if (const char *nc = std::getenv("SO3LR_NO_CLASS_TABLES")) class_tables_ = nc[0] != '1';
@@ -3381,7 +3496,7 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
     HIP_CHECK(hipMemcpyAsync(&total, cnt + nblk + 1, sizeof(int), hipMemcpyDeviceToHost, s));
     HIP_CHECK(hipStreamSynchronize(s));
     act_cap_ = std::min<std::int64_t>(P, std::int64_t(total) + total / 8 + 256);
-    scalar_now_ = std::int64_t(total) <= scalar_pairs_max_;
+    scalar_now_ = std::int64_t(total) <= (scalar_pairs_max_ >= 0 ? scalar_pairs_max_ : radial_blocks_ ? 0 : 256);
   }
   if (P == 0) scalar_now_ = false;
   const bool scalar = naive_filters_ || scalar_now_;
@@ -3746,6 +3861,8 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
   // slots of the bucket order: every bucket padded by fewer than 16
   const int rslots_max = PA + 16 * rkeys;
   const unsigned gR = unsigned(ceil_div(rslots_max, 64));  // 16 slots per wavefront
+  const unsigned gR16 = unsigned(ceil_div(rslots_max, 16));  // 16 slots per block (few pairs)
+  const bool few = PA < kFewPairs;
 
   // --- interaction blocks, forward ---
   for (int b = 0; b < L; ++b) {
@@ -3824,8 +3941,9 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
         hipLaunchKernelGGL(k_filter_fwd_mfma<true>, dim3(gP64), dim3(256), 0, s, nact, pa, pr, evb, qb, inv_avg, FM,
                            psb, pfb, pab);
       else if (use_rt)  // rows and logits in bucket order, the radial branches from the tables
-        hipLaunchKernelGGL(k_radial_fwd_rows, dim3(gR), dim3(256), 0, s, rslots, rord, pa, pr, evb, qb, B.rrow,
-                           rbl_dom_, inv_avg, FM, psb, pfb, pab);
+        hipLaunchKernelGGL(few ? k_radial_fwd_rows<true> : k_radial_fwd_rows<false>, dim3(few ? gR16 : gR),
+                           dim3(few ? 512 : 256), 0, s, rslots, rord, pa, pr, evb, qb, B.rrow, rbl_dom_, inv_avg, FM,
+                           psb, pfb, pab);
       else
         hipLaunchKernelGGL(k_filter_fwd_mfma<false>, dim3(gP64), dim3(256), 0, s, nact, pa, pr, evb, qb, inv_avg, FM,
                            psb, pfb, pab);
@@ -3955,6 +4073,9 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
                      qb, gainv, gaev, psc, dfc, inv_avg, FM, rc_, ds, dr, dY)
           if (b == 0 && first) SO3LR_FILTER_BWD(true, true);
           else if (b == 0) SO3LR_FILTER_BWD(true, false);
+          else if (use_rt && few)
+            hipLaunchKernelGGL(k_filter_bwd_split, dim3(gR16), dim3(512), 0, s, rslots, rord, pa, pr, psb, qb, psc, dfc,
+                               FM, rc_, ds, dr, B.rdr, rbl_dom_);
           else if (use_rt)  // in interval order, the radial branches' dE/dr from the slope tables
             hipLaunchKernelGGL((k_filter_bwd_mfma<false, false, true>), dim3(gR), dim3(256), 0, s, nact, pa, pr, psb,
                                pfc, pY, pab, qb, gainv, gaev, psc, dfc, inv_avg, FM, rc_, ds, dr, dY, rslots, rord,

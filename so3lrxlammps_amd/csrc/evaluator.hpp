@@ -275,12 +275,15 @@ class Evaluator {
   };
   bool timing_ = false;
   bool naive_filters_ = false;  // SO3LR_NAIVE_FILTERS=1: scalar filter kernels (cross-check)
-  // Small systems run the scalar filter kernels: with a few hundred active
-  // pairs the fully unrolled MFMA filters are bound by fetching their code
-  // into a cold instruction cache (30-40 us per launch).  Decided when a
-  // topology's active pairs are counted: at most scalar_pairs_max_ of them
-  // (SO3LR_SCALAR_FILTER_PAIRS; 0 never).
-  std::int64_t scalar_pairs_max_ = 256;
+  // Where the blocks after 0 have no radial tables, small systems run the
+  // scalar filter kernels: with a few hundred active pairs the fully unrolled
+  // MFMA filters are bound by fetching their code into a cold instruction
+  // cache (30-40 us per launch).  With the tables the split kernels for few
+  // pairs are the faster ones (22 atoms: 286 against 412 us per evaluation).
+  // Decided when a topology's active pairs are counted: at most
+  // scalar_pairs_max_ of them (SO3LR_SCALAR_FILTER_PAIRS; 0 never; -1, the
+  // default: 256 without the tables, none with them).
+  std::int64_t scalar_pairs_max_ = -1;
   bool scalar_now_ = false;
   // Block 0 through element-pair tables (k_filter_fwd_class and
   // k_filter_bwd_class): a one-image system of at most 16 elements, whose

@@ -39,6 +39,24 @@ def test_node_shares(orc, model, n):  # noqa: F811
     _both_paths(z, x, 0.0, m, orc, model)
 
 
+@pytest.mark.parametrize("limit", ["0", "1000000"])
+@pytest.mark.parametrize("n", [2, 3, 17, 65])
+def test_few_pairs(monkeypatch, n, limit):
+    """A pair or a handful per interval bucket (mostly padding slots) up to
+    several buckets of 16, on the kernels for few pairs and on the scalar ones."""
+    monkeypatch.setenv("SO3LR_SCALAR_FILTER_PAIRS", limit)
+    z, x, m = _cluster(n)
+    _both_paths(z, x, 0.0, m, Oracle(support.MODEL), support.MODEL)
+
+
+@pytest.mark.parametrize("n", [285, 296, 302, 320])
+def test_few_pairs_line(orc, model, n):  # noqa: F811
+    """Pair counts below, at and above the line between the kernels for few
+    pairs and those for many (the line is on 9/8 of the pairs plus 256)."""
+    z, x, m = _cluster(n)
+    _both_paths(z, x, 0.0, m, orc, model)
+
+
 @pytest.mark.parametrize("width", [129, 200])
 def test_head_width_remainder(tmp_path, width):
     """Energy and charge heads whose width is no multiple of 16 (the generic
