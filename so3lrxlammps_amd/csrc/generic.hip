@@ -119,7 +119,7 @@ __device__ __forceinline__ int g_xcd_block(int active) {
 // node n receives from each incident pair's partner o the invariant message
 // fc alpha v_o and the equivariant fc alpha_ev Y (parity of the direction),
 // then the residual and the first normalisation.  ev null: zero (block 0).
-// NodeShare: wavefronts per node.
+// W wavefronts per node.
 template <int W>
 __global__ __launch_bounds__(NodeShare<W>::kBlock) void g_attn_msg(GDims d, int N, const int *__restrict__ inc_off,
                                                   const int *__restrict__ iact, const int *__restrict__ iother,
@@ -199,11 +199,12 @@ __global__ __launch_bounds__(NodeShare<W>::kBlock) void g_attn_msg(GDims d, int 
 }
 
 // The attention reverse's node gathers (kokkos_attention_scatter_reverse.cpp:280-500):
-// dq at the receiver, dk and dv at the sender of each direction.  One
-// wavefront per node and 64 channels (F / 64 wavefronts per node, in one
-// workgroup): a lane holds one channel's five sums, so a wavefront needs
-// few registers and many are in flight to cover the entries' loads.
-__global__ __launch_bounds__(256) void g_attn_bwd_node(GDims d, int N, const int *__restrict__ inc_off,
+// dq at the receiver, dk and dv at the sender of each direction.  W wavefronts
+// per node and 64 channels: a lane holds one channel's five sums, so a
+// wavefront needs few registers and many are in flight to cover the entries'
+// loads.
+template <int W>
+__global__ __launch_bounds__(NodeShare<W>::kBlock) void g_attn_bwd_node(GDims d, int N, const int *__restrict__ inc_off,
                                                        const int *__restrict__ iact, const int *__restrict__ iother,
                                                        const double *__restrict__ qkv, const double *__restrict__ pf,
                                                        const double *__restrict__ pfc,
@@ -212,12 +213,12 @@ __global__ __launch_bounds__(256) void g_attn_bwd_node(GDims d, int N, const int
                                                        const double *__restrict__ gainv, double *__restrict__ gqkv) {
   const int lane = threadIdx.x & 63;
   const int F = d.F, NH = d.NH, NQ = F >> 6;
-  const int blk = g_xcd_block((N * NQ + 3) / 4);
-  if (blk < 0) return;
-  const int wq = blk * 4 + (threadIdx.x >> 6), n = wq / NQ;
-  if (n >= N) return;
-  const int c = 64 * (wq % NQ) + lane, h = c >> 5;
-  double gq = 0.0, gk = 0.0, gv = 0.0, gqe = 0.0, gke = 0.0;
+  __shared__ double lds[W > 1 ? NodeShare<W>::kBlock * 5 : 1];
+  const NodeShare<W> S(N, inc_off, NQ);
+  const int n = S.n;
+  if (W == 1 && !S.on) return;
+  const int c = 64 * S.c + lane, h = c >> 5;
+  double sum[5] = {0, 0, 0, 0, 0};  // d q, k, v, q_ev, k_ev
   // per entry: n receives along direction sn from o and sends along
   // so = 1 - sn to o
   struct Terms {
@@ -246,23 +247,22 @@ __global__ __launch_bounds__(256) void g_attn_bwd_node(GDims d, int N, const int
     return T;
   };
   auto add = [&](const Terms &T) {
-    gq += T.si * T.ko * T.fi;
-    gqe += T.sie * T.keo * T.fe;
-    gk += T.so * T.qo * T.fi;
-    gv += T.fc * T.ao * T.go;
-    gke += T.soe * T.qeo * T.fe;
+    sum[0] += T.si * T.ko * T.fi;
+    sum[3] += T.sie * T.keo * T.fe;
+    sum[1] += T.so * T.qo * T.fi;
+    sum[2] += T.fc * T.ao * T.go;
+    sum[4] += T.soe * T.qeo * T.fe;
   };
-  for_active_pairs(inc_off[n], inc_off[n + 1], iact, iother, lane, [&](int e1, int o1, int e2, int o2, bool two) {
+  for_active_pairs(S.beg, S.end, iact, iother, lane, [&](int e1, int o1, int e2, int o2, bool two) {
     const Terms A = load(e1, o1), B = load(e2, o2);
     add(A);
     if (two) add(B);
   });
+  share_sum<W>(lds, sum);
+  if (!S.on || !S.first) return;
   double *g = gqkv + std::size_t(n) * 5 * F + c;
-  g[0] = gq;
-  g[F] = gk;
-  g[2 * F] = gv;
-  g[3 * F] = gqe;
-  g[4 * F] = gke;
+#pragma unroll
+  for (int k = 0; k < 5; ++k) g[k * F] = sum[k];
 }
 
 // gev = ga + sum over incident pairs of 2 (ev_n - ev_o) cg ds[slot]: the
@@ -1336,7 +1336,8 @@ void launch_b0(hipStream_t s, int F, int R, std::size_t slots, const B0Args &A) 
 // per output tile the interval's coefficient tile (two K chunks against the
 // pairs' powers of t, in place of the W0 and W1 chains), the E1 chunks and
 // the endpoint rows; the rows go to pf and the logits to palpha as in
-// g_filt_fwd.
+// g_filt_fwd.  SPLIT: FT wavefronts per 16 slots, one per filter and head
+// (launch_rows).
 struct GRadArgs {
   const int *slots, *order, *pa;
   const double *pr, *ps, *qkv, *rtab;
@@ -1351,15 +1352,18 @@ struct GRadArgs {
   double *ds, *dr;
 };
 
-template <int FT>
-__global__ __launch_bounds__(256) void g_radial_fwd_rows(GRadArgs A) {
+template <int FT, bool SPLIT>
+__global__ __launch_bounds__(SPLIT ? 64 * FT : 256) void g_radial_fwd_rows(GRadArgs A) {
   constexpr int FHT = FT / 4, NH = FT / 2, HT = FT + FHT, F = 16 * FT, NE = 6 + FHT;
+  constexpr int NT = SPLIT ? 2 : FT;  // output tiles of a wavefront
   __shared__ double tab[256];
-  tab[threadIdx.x] = A.exp2_256[threadIdx.x];
+  if (!SPLIT || threadIdx.x < 256) tab[threadIdx.x & 255] = A.exp2_256[threadIdx.x & 255];
   __syncthreads();
   const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
-  const int blk = g_xcd_block((*A.slots + 63) / 64);
-  const int wave = blk < 0 ? -1 : blk * 4 + int(threadIdx.x >> 6);
+  const int blk = g_xcd_block((*A.slots + (SPLIT ? 15 : 63)) / (SPLIT ? 16 : 64));
+  const int sub = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  const int wave = blk < 0 ? -1 : (SPLIT ? blk : blk * 4 + sub);
+  const int w0 = SPLIT ? sub / NH : 0, mt0 = SPLIT ? 2 * (sub % NH) : 0;
   int p, ri;
   bool inside;
   v4d tp[2];
@@ -1374,34 +1378,48 @@ __global__ __launch_bounds__(256) void g_radial_fwd_rows(GRadArgs A) {
 #pragma unroll
   for (int v = 0; v < 4; ++v) sv[v] = g + 4 * v < NH ? A.ps[std::size_t(pp) * NH + g + 4 * v] : 0.0;
   const v4d zero = v4d{0.0, 0.0, 0.0, 0.0};
-  static_for<2>([&](auto wi) {
-    constexpr int w = decltype(wi)::value;
+  static_for<SPLIT ? 1 : 2>([&](auto wi) {
+    const int w = w0 + decltype(wi)::value;
+    const double *e0p = w ? A.e0p[1] : A.e0p[0], *eb0a = w ? A.eb0a[1] : A.eb0a[0], *wcp = w ? A.wcp[1] : A.wcp[0];
     v4d he[FHT];
+    auto hidden = [&](int t) {
+      const v4d e0 = frag_load(e0p, t, lane);
+      v4d h = mfma(e0[0], sv[0], frag_load(eb0a, t, lane));
+      if constexpr (NH > 4) h = mfma(e0[1], sv[1], h);
 #pragma unroll
-    for (int t = 0; t < FHT; ++t) {
-      const v4d e0 = frag_load(A.e0p[w], t, lane);
-      he[t] = mfma(e0[0], sv[0], frag_load(A.eb0a[w], t, lane));
-      if constexpr (NH > 4) he[t] = mfma(e0[1], sv[1], he[t]);
+      for (int r = 0; r < 4; ++r) h[r] = silu_tab_wide(h[r], tab);
+      return h;
+    };
+    if constexpr (!SPLIT) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) he[t][r] = silu_tab_wide(he[t][r], tab);
+      for (int t = 0; t < FHT; ++t) he[t] = hidden(t);
     }
     const double *coef = A.rtab + (std::size_t(ri) * 2 + w) * FT * 2 * 256;
-    constexpr int qo = w ? 3 * F : 0, ko = w ? 4 * F : F;  // q, k or q_ev, k_ev
+    const int qo = w ? 3 * F : 0, ko = w ? 4 * F : F;  // q, k or q_ev, k_ev
     auto ld = [&](auto si) -> v4d {
-      constexpr int S = decltype(si)::value, mt = S / NE, u = S % NE;
+      constexpr int S = decltype(si)::value, u = S % NE;
+      const int mt = mt0 + S / NE;
       if constexpr (u < 2) return frag_load(coef, mt * 2 + u, lane);
-      else if constexpr (u < 2 + FHT) return frag_load(A.wcp[w], mt * HT + FT + u - 2, lane);
+      else if constexpr (u < 2 + FHT) return frag_load(wcp, mt * HT + FT + u - 2, lane);
       else if constexpr (u == 2 + FHT) return *reinterpret_cast<const v4d *>(ra + qo + 16 * mt);
       else if constexpr (u == 3 + FHT) return *reinterpret_cast<const v4d *>(rr + ko + 16 * mt);
       else if constexpr (u == 4 + FHT) return *reinterpret_cast<const v4d *>(rr + qo + 16 * mt);
       else return *reinterpret_cast<const v4d *>(ra + ko + 16 * mt);
     };
-    Stream<FT * NE, 6, decltype(ld)> st(ld);
+    Stream<NT * NE, 6, decltype(ld)> st(ld);
     st.prime();
+    if constexpr (SPLIT) {  // the filters' hidden tiles, each formed by one wavefront
+      __shared__ v4d hid[2][FHT][64];
+      if (sub % NH < FHT) hid[w][sub % NH][lane] = hidden(sub % NH);
+      __syncthreads();
+#pragma unroll
+      for (int t = 0; t < FHT; ++t) he[t] = hid[w][t][lane];
+    }
     v4d o, qv, qk0, qk1;
     double t0 = 0.0, t1 = 0.0;
     st.run([&](auto si, const v4d &wv) {
-      constexpr int S = decltype(si)::value, mt = S / NE, u = S % NE;
+      constexpr int S = decltype(si)::value, u = S % NE;
+      const int mt = mt0 + S / NE;
       if constexpr (u == 0) {
         o = mfma4(wv, tp[0], zero);
       } else if constexpr (u == 1) {
@@ -1420,7 +1438,7 @@ __global__ __launch_bounds__(256) void g_radial_fwd_rows(GRadArgs A) {
           t0 += qk0[r] * o[r];
           t1 += qk1[r] * o[r];
         }
-        if constexpr (mt & 1) {  // head mt / 2 complete: sum over the lane groups
+        if constexpr ((S / NE) & 1) {  // head mt / 2 complete: sum over the lane groups
           t0 += __shfl_xor(t0, 16, 64);
           t0 += __shfl_xor(t0, 32, 64);
           t1 += __shfl_xor(t1, 16, 64);
@@ -1443,15 +1461,19 @@ __global__ __launch_bounds__(256) void g_radial_fwd_rows(GRadArgs A) {
 // adjoint (E1^T chunks) and the slope tiles against df, whose sum over the
 // powers of t is the radial branches' dE/dr; the spherical branch goes on
 // through silu' and E0^T to dE/ds.  No W1^T, no layer-0 recompute.
-template <int FT>
-__global__ __launch_bounds__(256) void g_radial_bwd_rows(GRadArgs A) {
+template <int FT, bool SPLIT>
+__global__ __launch_bounds__(SPLIT ? 64 * FT : 256) void g_radial_bwd_rows(GRadArgs A) {
   constexpr int FHT = FT / 4, NH = FT / 2, F = 16 * FT, NE = 4 + FHT + 2;
-  __shared__ double tab[256];
-  tab[threadIdx.x] = A.exp2_256[threadIdx.x];
+  constexpr int NT = SPLIT ? 2 : FT, NR = (NH + 3) / 4;
+  __shared__ double tab[256], share[SPLIT ? FT : 1][NR + 1][64];
+  __shared__ v4d prime[2][SPLIT ? FHT : 1][64];  // SPLIT: silu' of the hidden tiles, each formed by one wavefront
+  if (!SPLIT || threadIdx.x < 256) tab[threadIdx.x & 255] = A.exp2_256[threadIdx.x & 255];
   __syncthreads();
   const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
-  const int blk = g_xcd_block((*A.slots + 63) / 64);
-  const int wave = blk < 0 ? -1 : blk * 4 + int(threadIdx.x >> 6);
+  const int blk = g_xcd_block((*A.slots + (SPLIT ? 15 : 63)) / (SPLIT ? 16 : 64));
+  const int sub = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  const int wave = blk < 0 ? -1 : (SPLIT ? blk : blk * 4 + sub);
+  const int w0 = SPLIT ? sub / NH : 0, mt0 = SPLIT ? 2 * (sub % NH) : 0;
   int p, ri;
   bool inside;
   v4d tp[2];
@@ -1466,37 +1488,50 @@ __global__ __launch_bounds__(256) void g_radial_bwd_rows(GRadArgs A) {
   for (int v = 0; v < 4; ++v) sv[v] = g + 4 * v < NH ? A.ps[std::size_t(pp) * NH + g + 4 * v] : 0.0;
   const v4d zero = v4d{0.0, 0.0, 0.0, 0.0};
   v4d dsa = zero, accdr[2] = {zero, zero};
-  static_for<2>([&](auto wi) {
-    constexpr int w = decltype(wi)::value;
-    constexpr int qo = w ? 3 * F : 0, ko = w ? 4 * F : F;
+  static_for<SPLIT ? 1 : 2>([&](auto wi) {
+    const int w = w0 + decltype(wi)::value;
+    const int qo = w ? 3 * F : 0, ko = w ? 4 * F : F;
+    const double *e0p = w ? A.e0p[1] : A.e0p[0], *eb0a = w ? A.eb0a[1] : A.eb0a[0];
+    const double *e0tp = w ? A.e0tp[1] : A.e0tp[0], *wctp = w ? A.wctp[1] : A.wctp[0];
     const double *slope = A.rtab + (std::size_t(ri) * 2 + w) * 2 * FT * 256;
     v4d dh[FHT];
 #pragma unroll
     for (int t = 0; t < FHT; ++t) dh[t] = zero;
+    auto slope_of = [&](int t) {
+      const v4d e0 = frag_load(e0p, t, lane);
+      v4d pre = mfma(e0[0], sv[0], frag_load(eb0a, t, lane));
+      if constexpr (NH > 4) pre = mfma(e0[1], sv[1], pre);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) pre[r] = silu_prime_tab_wide(pre[r], tab);
+      return pre;
+    };
     auto ld = [&](auto si) -> v4d {
-      constexpr int S = decltype(si)::value, mt = S / NE, u = S % NE;
+      constexpr int S = decltype(si)::value, u = S % NE;
+      const int mt = mt0 + S / NE;
       if constexpr (u < 4) {
         const double *row = (u == 0 ? ra + qo : (u == 1 ? rr + ko : (u == 2 ? rr + qo : ra + ko))) + 16 * mt;
         return *reinterpret_cast<const v4d *>(row);
       } else if constexpr (u < 4 + FHT) {
-        return frag_load(A.wctp[w], (FT + u - 4) * FT + mt, lane);
+        return frag_load(wctp, (FT + u - 4) * FT + mt, lane);
       } else {
         return frag_load(slope, (u - 4 - FHT) * FT + mt, lane);
       }
     };
-    double c0 = ps[w * NH], c1 = ps[2 * NH + w * NH];  // head 0
+    double c0 = ps[w * NH + (mt0 >> 1)], c1 = ps[2 * NH + w * NH + (mt0 >> 1)];  // the first head
     v4d qv, df;
-    Stream<NE * FT, 6, decltype(ld)> st(ld);
+    Stream<NE * NT, 6, decltype(ld)> st(ld);
     st.prime();
+    if (SPLIT && sub % NH < FHT) prime[w][sub % NH][lane] = slope_of(sub % NH);
     st.run([&](auto si, const v4d &wv) {
-      constexpr int S = decltype(si)::value, mt = S / NE, u = S % NE;
+      constexpr int S = decltype(si)::value, u = S % NE;
+      const int mt = mt0 + S / NE;
       if constexpr (u == 0 || u == 2) {
         qv = wv;
       } else if constexpr (u == 1) {
         df = c0 * (qv * wv);
       } else if constexpr (u == 3) {
         df += c1 * (qv * wv);
-        const int hn = min(mt + 1, FT - 1) >> 1;  // the next tile's head
+        const int hn = min(mt + 1, mt0 + NT - 1) >> 1;  // the next tile's head
         c0 = ps[w * NH + hn];
         c1 = ps[2 * NH + w * NH + hn];
       } else if constexpr (u < 4 + FHT) {
@@ -1506,27 +1541,37 @@ __global__ __launch_bounds__(256) void g_radial_bwd_rows(GRadArgs A) {
       }
     });
     // the spherical branch: pre again, d hidden *= silu'(pre), E0^T
+    if constexpr (SPLIT) __syncthreads();
 #pragma unroll
     for (int t = 0; t < FHT; ++t) {
-      const v4d e0 = frag_load(A.e0p[w], t, lane);
-      v4d pre = mfma(e0[0], sv[0], frag_load(A.eb0a[w], t, lane));
-      if constexpr (NH > 4) pre = mfma(e0[1], sv[1], pre);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) dh[t][r] *= silu_prime_tab_wide(pre[r], tab);
-      dsa = mfma4(frag_load(A.e0tp[w], t, lane), dh[t], dsa);
+      dh[t] *= SPLIT ? prime[w][t][lane] : slope_of(t);
+      dsa = mfma4(frag_load(e0tp, t, lane), dh[t], dsa);
     }
   });
-  if (valid) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      if (g + 4 * r < NH) A.ds[std::size_t(pp) * NH + g + 4 * r] = dsa[r];
-  }
   // dE/dr: the radial branches' (powers 16 m + g + 4 r), plus the cutoff's
   double part = 0.0;
 #pragma unroll
   for (int m = 0; m < 2; ++m)
 #pragma unroll
     for (int r = 0; r < 4; ++r) part += accdr[m][r] * tp[m][r];
+  if constexpr (SPLIT) {  // the filters' and heads' shares, summed in wavefront order
+#pragma unroll
+    for (int r = 0; r < NR; ++r) share[sub][r][lane] = dsa[r];
+    share[sub][NR][lane] = part;
+    __syncthreads();
+    if (sub != 0) return;
+#pragma unroll
+    for (int q = 1; q < FT; ++q) {
+#pragma unroll
+      for (int r = 0; r < NR; ++r) dsa[r] += share[q][r][lane];
+      part += share[q][NR][lane];
+    }
+  }
+  if (valid) {
+#pragma unroll
+    for (int r = 0; r < NR; ++r)
+      if (g + 4 * r < NH) A.ds[std::size_t(pp) * NH + g + 4 * r] = dsa[r];
+  }
   if (!inside) part = 0.0;
   part += __shfl_xor(part, 16, 64);
   part += __shfl_xor(part, 32, 64);
@@ -1539,6 +1584,31 @@ __global__ __launch_bounds__(256) void g_radial_bwd_rows(GRadArgs A) {
     }
     A.dr[pp] += grad;
   }
+}
+
+// g_radial_fwd_rows / g_radial_bwd_rows at F = 128 or 256; below kFewRows
+// pairs their split forms, a wavefront per filter and head of 16 slots (see
+// k_radial_fwd_rows); their hidden tiles and its slopes are formed once per
+// block and pass through LDS, else 16 wavefronts form them each (632 against
+// 615 us per evaluation of 22 atoms at F = 256).  Whole evaluations at F = 256
+// without / with them (us, by pairs with their margin): 22 atoms 696 / 615,
+// 2,200 pairs 784 / 682, 4,700 822 / 792, 6,200 840 / 810, 10,300 889 / 944,
+// 11,200 901 / 959.
+constexpr int kFewRows = 7500;
+template <bool FWD>
+void launch_rows(hipStream_t s, int F, const GContext &c, const GRadArgs &A) {
+  auto go = [&](auto ft, auto split) {
+    constexpr int FT = decltype(ft)::value;
+    constexpr bool SPLIT = decltype(split)::value;
+    hipLaunchKernelGGL((FWD ? g_radial_fwd_rows<FT, SPLIT> : g_radial_bwd_rows<FT, SPLIT>),
+                       dim3(blocks_for(std::size_t(std::max(c.rint_max, 1)), SPLIT ? 16 : 64)),
+                       dim3(SPLIT ? 64 * FT : 256), 0, s, A);
+  };
+  const bool few = c.cap < kFewRows;
+  if (F == 128 && few) go(std::integral_constant<int, 8>{}, std::true_type{});
+  else if (F == 128) go(std::integral_constant<int, 8>{}, std::false_type{});
+  else if (few) go(std::integral_constant<int, 16>{}, std::true_type{});
+  else go(std::integral_constant<int, 16>{}, std::false_type{});
 }
 
 // g_radial_fwd / g_radial_bwd at NH = 4 or 8 heads over cap pairs
@@ -2028,11 +2098,7 @@ void GenericPath::forward(const GContext &c) {
       // the radial tables, in bucket order
       GRadArgs R{c.rint_slots, c.rint_order, c.pa, c.pr, psb, qb, B.rrow, rbl_dom_, {B.eb0a[0], B.eb0a[1]},
                  {B.e0p[0], B.e0p[1]}, {B.wcp[0], B.wcp[1]}, hw_.exp2_256, c.inv_avg, pfb, pab};
-      const dim3 grid(blocks_for(std::size_t(std::max(c.rint_max, 1)), 64));
-      section(c, "generic_filter_fwd_radial", [&] {
-        if (F == 128) hipLaunchKernelGGL(g_radial_fwd_rows<8>, grid, dim3(256), 0, s, R);
-        else hipLaunchKernelGGL(g_radial_fwd_rows<16>, grid, dim3(256), 0, s, R);
-      });
+      section(c, "generic_filter_fwd_radial", [&] { launch_rows<true>(s, F, c, R); });
     } else {
     // both filters' rows f = [W1 | E1] [silu(W0 rbf + b0) | silu(E0 s + e0)]
     // + b1 + e1 and the attention logits from them, fused
@@ -2121,8 +2187,12 @@ void GenericPath::reverse(const GContext &c) {
                          b == layers_ - 1 ? 1 : 0, b_[PSC], c.dY, b_[DFC]);
     });
     if (b > 0)
-      hipLaunchKernelGGL(g_attn_bwd_node, dim3((blocks_for(n * (F / 64), 4) + 7) / 8 * 8), dim3(256), 0, s, d, N, c.inc_off, c.iact, c.iother, qb, pfb,
-                         c.pfc, pab, b_[PSC], b_[GAINV], b_[GQKV]);
+      by_node_share(N, [&](auto w) {
+        constexpr int W = decltype(w)::value;
+        hipLaunchKernelGGL(g_attn_bwd_node<W>, dim3(blocks_for(n * (F / 64), NodeShare<W>::kNodes)),
+                           dim3(NodeShare<W>::kBlock), 0, s, d, N, c.inc_off, c.iact, c.iother, qb, pfb, c.pfc, pab,
+                           b_[PSC], b_[GAINV], b_[GQKV]);
+      });
     // filter reverse (kokkos_block2_attention_input_reverse.cpp:198-336)
     if (tables && c.rad_tab) {
       // block 0 through the radial tables: the logits' adjoints times the
@@ -2148,11 +2218,7 @@ void GenericPath::reverse(const GContext &c) {
       GRadArgs Rg{c.rint_slots, c.rint_order, c.pa, c.pr, psb, qb, B.rdr, rbl_dom_, {B.eb0a[0], B.eb0a[1]},
                   {B.e0p[0], B.e0p[1]}, {nullptr, nullptr}, hw_.exp2_256, c.inv_avg, nullptr, nullptr,
                   {B.e0tp[0], B.e0tp[1]}, {B.wctp[0], B.wctp[1]}, b_[PSC], b_[DFC], c.rc, b_[DS], c.dr};
-      const dim3 grid(blocks_for(std::size_t(std::max(c.rint_max, 1)), 64));
-      section(c, "generic_filter_bwd_radial", [&] {
-        if (F == 128) hipLaunchKernelGGL(g_radial_bwd_rows<8>, grid, dim3(256), 0, s, Rg);
-        else hipLaunchKernelGGL(g_radial_bwd_rows<16>, grid, dim3(256), 0, s, Rg);
-      });
+      section(c, "generic_filter_bwd_radial", [&] { launch_rows<false>(s, F, c, Rg); });
     } else {
       // both filters fused: d hidden = [W1 | E1]^T df (df from the logits'
       // adjoints psc), (.) silu'(pre), through W0^T and E0^T to dE/dr and

@@ -65,11 +65,14 @@ void by_node_share(int N, Launch &&launch) {
 template <int W>
 struct NodeShare {
   static constexpr int kBlock = W > 4 ? 64 * W : 256, kNodes = kBlock / 64 / W;
-  int n, beg, end;
+  int n, c, beg, end;
   bool on, first;  // n < N; this wavefront writes the node's results
-  __device__ __forceinline__ NodeShare(int N, const int *__restrict__ off) {
-    const int wv = threadIdx.x >> 6, part = wv % W;
-    n = xcd_block() * kNodes + wv / W;
+  // `cut`: a node's channels in that many slices, each with W wavefronts of
+  // its own (c: this wavefront's slice; kNodes slices per block)
+  __device__ __forceinline__ NodeShare(int N, const int *__restrict__ off, int cut = 1) {
+    const int wv = threadIdx.x >> 6, part = wv % W, u = xcd_block() * kNodes + wv / W;
+    n = u / cut;
+    c = u % cut;
     on = n < N;
     first = part == 0;
     if (on) {
