@@ -76,8 +76,8 @@ _FILTER_BWD_RT_ISSUED = 2 * 2 * _mac((32, 128), (32, 128), (4, 32))   # 33,280: 
 KERNEL_WORK = {
     # name: (kernel symbol, bound, algorithmic per unit, issued per unit, unit)
     # (bound "hbm": bytes per unit; "mfma": flop per unit)
-    "filter_fwd_radial": ("k_radial_fwd_rows", "hbm", _FILTER_RT_BYTES, _FILTER_RT_BYTES, "pair"),
-    "filter_bwd_radial": ("k_filter_bwd_mfma<false, false, true>", "mfma", _FILTER_BWD_RT, _FILTER_BWD_RT_ISSUED,
+    "filter_fwd_radial": ("k_rows_fwd", "hbm", _FILTER_RT_BYTES, _FILTER_RT_BYTES, "pair"),
+    "filter_bwd_radial": ("k_rows_bwd", "mfma", _FILTER_BWD_RT, _FILTER_BWD_RT_ISSUED,
                           "pair"),
     "filter_fwd": ("k_filter_fwd_mfma<false>", "mfma", _FILTER, _FILTER, "pair"),
     "filter_fwd_block0": ("k_filter_fwd_mfma<true>", "mfma", _FILTER_B0, _FILTER_B0, "pair"),
@@ -147,11 +147,11 @@ def kernel_work(widths, elements=0):
     # doubles written per pair with the 4 NH logits and NH invariants (the
     # invariants are read back), r and the endpoints read
     rt_bytes = 8 * (2 * F + 4 * NH + NH) + 16
-    work["generic_filter_fwd_radial"] = ("g_radial_fwd_rows", "hbm", rt_bytes, rt_bytes, "pair")
+    work["generic_filter_fwd_radial"] = ("k_rows_fwd", "hbm", rt_bytes, rt_bytes, "pair")
     # and the reverse: df against the slope polynomials (14 powers per
     # channel at the accuracy of degree 13; 32 issued), E1^T, E0^T
     rt_bwd = 2 * 2 * (14 * F + FH * F + NH * FH)
-    work["generic_filter_bwd_radial"] = ("g_radial_bwd_rows", "mfma", rt_bwd, 2 * 2 * (32 * F + FH * F + NH * FH),
+    work["generic_filter_bwd_radial"] = ("k_rows_bwd", "mfma", rt_bwd, 2 * 2 * (32 * F + FH * F + NH * FH),
                                          "pair")
     if elements:
         tab = 2 * 2 * (R * F + 2 * NH * F)

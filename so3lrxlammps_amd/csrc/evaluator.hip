@@ -12,7 +12,7 @@
 // (-1)^l Y(v/r).  Node sums are gathers over a CSR incidence list.
 #include "evaluator.hpp"
 #include "mfma_ops.hpp"
-#include "node_chain.hpp"
+#include "radial_rows.hpp"
 #include "radial_table.hpp"
 
 #include <algorithm>
@@ -343,16 +343,6 @@ __global__ __launch_bounds__(256) void k_sr_compact(
   }
 }
 
-// xcd_block for a grid sized for an upper bound of the work: only the first A
-// logical blocks have work (A <= gridDim.x, known on the device only), and
-// they are spread evenly over the XCDs; -1 for a block with none.
-__device__ __forceinline__ int xcd_block_active(int A) {
-  const int b = blockIdx.x;
-  const int per = A >> 3, rem = A & 7, xcd = b & 7, i = b >> 3;
-  if (i >= per + (xcd < rem ? 1 : 0)) return -1;
-  return xcd * per + (xcd < rem ? xcd : rem) + i;
-}
-
 // ---------------------------------------------------------------- filters
 // Per active pair: Bernstein basis and PhysNet cutoff of r, the equivariant
 // invariant s_l = sum_{m in l} (ev_a - ev_b)^2 cg, and both filters
@@ -591,14 +581,6 @@ __device__ __forceinline__ void rbf8(double r, int g, const FilterMfma &A, const
 // Both filters of one block for 16 pairs per wavefront, 4 wavefronts per block.
 // Per filter the stream holds 96 weight fragments: W0 (s < 16: tile s % 8,
 // K chunk s / 8), W1 (16 <= s < 80) and E1 (80 <= s < 96), tile-minor.
-// The RT reverse (blocks after 0 on their radial tables, in interval order):
-// operand-stream depth and wavefronts per SIMD.
-#ifndef SO3LR_RT_BWD_PF
-#define SO3LR_RT_BWD_PF 6
-#endif
-#ifndef SO3LR_RT_BWD_WAVES
-#define SO3LR_RT_BWD_WAVES 2
-#endif
 template <bool EV0>
 __global__ __launch_bounds__(256) FILTER_FWD_OCCUPANCY void k_filter_fwd_mfma(const int *n_active, const int *pa,
                                                                      const double *pr, const double *ev,
@@ -766,144 +748,6 @@ __global__ __launch_bounds__(256) FILTER_FWD_OCCUPANCY void k_filter_fwd_mfma(co
   });
 }
 
-// The forward filters of the blocks after 0 on their radial tables, in
-// bucket order (16 slots of one bucket, spatial block and interval, per
-// wavefront; -1 in the padding).  Per filter the stream holds the spherical
-// layer-0 biases and operand (3), then per output tile the interval's
-// coefficient tile (128 channels x 32 powers: two K chunks, against the
-// pairs' powers of t in place of the W0 and W1 chains), the endpoint rows
-// q_a, k_b, q_b, k_a of its channels (from L2: a spatial block's buckets
-// run together on one XCD) and the 2 E1 chunks.  The rows go to pf and the
-// logits of both directions to palpha as in k_filter_fwd_mfma.  Measured
-// as two passes (the rows in bucket order, the logits in pair order) it
-// took 0.79 against 0.70 ms.
-//
-// SPLIT, below kFewPairs pairs: eight wavefronts per 16 slots, one per filter
-// and head (two output tiles each, the spherical hidden layer formed by
-// each).  One wavefront walks 134 dependent operands for its 16 pairs, and
-// few pairs leave most SIMDs without one; with more, the hidden layer's
-// seven further copies cost more than the shorter walk gives.  Whole
-// evaluations without / with this kernel and k_filter_bwd_split (us, by pairs
-// with their margin): 22 atoms 316 / 284, 2,200 pairs 372 / 323, 4,700 394 /
-// 366, 6,200 396 / 374, 6,900 451 / 430, 10,300 420 / 431, 11,200 428 / 443.
-constexpr int kFewPairs = 8500;
-#ifndef SO3LR_RT_FWD_PF
-#define SO3LR_RT_FWD_PF 6
-#endif
-template <bool SPLIT>
-__global__ __launch_bounds__(SPLIT ? 512 : 256) FILTER_FWD_OCCUPANCY void k_radial_fwd_rows(
-    const int *n_slots, const int *order, const int *pa, const double *pr, const double *__restrict__ ev,
-    const double *__restrict__ qkv, const double *__restrict__ rtab, RadialDomain rd, double inv_avg, FilterMfma A,
-    double *ps, double *pf, double *palpha) {
-  SO3LR_EXP2_TABLE(A)
-  const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
-  const int blk = xcd_block_active(SPLIT ? (*n_slots + 15) / 16 : (*n_slots + 63) / 64);
-  const int sub = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
-  const int wave = blk < 0 ? -1 : (SPLIT ? blk : blk * 4 + sub);
-  const int which0 = SPLIT ? sub >> 2 : 0, mt0 = SPLIT ? 2 * (sub & 3) : 0;
-  int p, ri;
-  bool inside;
-  v4d tp[2];
-  if (!rint_slots(n_slots, order, pr, rd, wave, j, g, p, ri, inside, tp)) return;
-  const bool valid = p >= 0;
-  const int pp = valid ? p : order[wave * 16];
-  const int a = pa[2 * pp], b = pa[2 * pp + 1];
-  const double *qa = qkv + std::size_t(a) * 640 + 4 * g, *qb = qkv + std::size_t(b) * 640 + 4 * g;
-  const double *coef = rtab + std::size_t(ri) * 2 * 16 * 256;
-  constexpr int TS = 3, PT = 8, NF = TS + (SPLIT ? 2 : 8) * PT;
-  auto load = [&](auto si) -> v4d {
-    constexpr int S = decltype(si)::value, s = S % NF;
-    const int which = which0 + S / NF;
-    if constexpr (s < 2) return tile_load(which ? A.eb0p[1] : A.eb0p[0], s, lane);
-    else if constexpr (s == 2) return tile_load(which ? A.e0pk[1] : A.e0pk[0], 0, lane);
-    else {
-      constexpr int u = (s - TS) % PT;
-      const int mt = mt0 + (s - TS) / PT;
-      const int qoff = which ? 384 : 0, koff = which ? 512 : 128;
-      if constexpr (u < 2) return wload(coef + which * 16 * 256, 2, mt, u, lane);
-      else if constexpr (u == 2) return *reinterpret_cast<const v4d *>(qa + qoff + 16 * mt);
-      else if constexpr (u == 3) return *reinterpret_cast<const v4d *>(qb + koff + 16 * mt);
-      else if constexpr (u == 4) return *reinterpret_cast<const v4d *>(qb + qoff + 16 * mt);
-      else if constexpr (u == 5) return *reinterpret_cast<const v4d *>(qa + koff + 16 * mt);
-      else return wload(which ? A.e1p[1] : A.e1p[0], 2, mt, u - 6, lane);
-    }
-  };
-  Stream<(SPLIT ? 1 : 2) * NF, SO3LR_RT_FWD_PF, decltype(load)> st(load);
-  st.prime();
-  // equivariant invariant of degree slot g, all loads in flight at once
-  double sg = 0.0;
-  {
-    const int lo = g == 0 ? 0 : (g == 1 ? 3 : (g == 2 ? 8 : 15)), n = 2 * g + 3;
-    const double *ea = ev + std::size_t(a) * kE, *eb = ev + std::size_t(b) * kE;
-    double va[9], vb[9];
-#pragma unroll
-    for (int k = 0; k < 9; ++k) {
-      const int m = min(lo + k, kE - 1);
-      va[k] = ea[m];
-      vb[k] = eb[m];
-    }
-#pragma unroll
-    for (int k = 0; k < 9; ++k) {
-      const double d = va[k] - vb[k];
-      sg += k < n ? d * d * A.att_cg[lo + k] : 0.0;
-    }
-    if (valid && (!SPLIT || sub == 0)) ps[4 * std::size_t(p) + g] = sg;
-  }
-  v4d *const rowv = reinterpret_cast<v4d *>(pf + 256 * std::size_t(pp) + 4 * g);
-  const v4d zero = v4d{0.0, 0.0, 0.0, 0.0};
-  v4d h2[2], o, qv, qk0, qk1;
-  double t0 = 0.0, t1 = 0.0;
-  st.run([&](auto si, const v4d &w) {
-    constexpr int S = decltype(si)::value, s = S % NF;
-    const int which = which0 + S / NF;
-    if constexpr (s < 2) {
-      h2[s] = w;
-    } else if constexpr (s == 2) {
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        h2[t] = mfma(w[t], sg, h2[t]);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) h2[t][r] = silu_tab_wide(h2[t][r], exp2_lds);
-      }
-    } else {
-      constexpr int u = (s - TS) % PT;
-      const int mt = mt0 + (s - TS) / PT;
-      if constexpr (u == 0) {
-        o = mfma4(w, tp[0], zero);
-      } else if constexpr (u == 1) {
-        o = mfma4(w, tp[1], o);
-      } else if constexpr (u == 2 || u == 4) {
-        qv = w;
-      } else if constexpr (u == 3) {
-        qk0 = qv * w;  // q_a k_b: edge b -> a
-      } else if constexpr (u == 5) {
-        qk1 = qv * w;  // q_b k_a: edge a -> b
-      } else {
-        o = mfma4(w, h2[u - 6], o);
-        if constexpr (u == PT - 1) {
-          if (valid) __builtin_nontemporal_store(o, rowv + which * 32 + 4 * mt);
-          t0 += ((qk0[0] * o[0] + qk0[1] * o[1]) + qk0[2] * o[2]) + qk0[3] * o[3];
-          t1 += ((qk1[0] * o[0] + qk1[1] * o[1]) + qk1[2] * o[2]) + qk1[3] * o[3];
-          if constexpr (((s - TS) / PT) & 1) {
-            t0 += __shfl_xor(t0, 16, kWave);
-            t0 += __shfl_xor(t0, 32, kWave);
-            t1 += __shfl_xor(t1, 16, kWave);
-            t1 += __shfl_xor(t1, 32, kWave);
-            const int hd = mt / 2;
-            if (valid && g == hd) {
-              double *al = palpha + 16 * std::size_t(p) + 4 * which + hd;
-              al[0] = t0 * inv_avg;
-              al[8] = t1 * inv_avg;
-            }
-            t0 = 0.0;
-            t1 = 0.0;
-          }
-        }
-      }
-    }
-  });
-}
-
 // Operand schedule of the reverse filter's first section (per filter).
 // Entry kinds: P, a term of the invariant head scalars (q = 0..3: gainv_a,
 // v_b, gainv_b, v_a of chunk T, head h; `last` completes the head); R, a row
@@ -982,8 +826,7 @@ constexpr bool bwd_schedule_ok() {
     if (m_seen[T] != NM || rows_seen[T] != 4) return false;
   return true;
 }
-static_assert(bwd_schedule_ok<10, 1>() && bwd_schedule_ok<8, 0>() && bwd_schedule_ok<8, 2>() &&
-                  bwd_schedule_ok<4, 1>(),
+static_assert(bwd_schedule_ok<10, 1>() && bwd_schedule_ok<8, 0>() && bwd_schedule_ok<8, 2>(),
               "reverse-filter operand schedule out of order");
 
 // Reverse of the attention's pair terms, of both filters, of the Bernstein
@@ -1021,45 +864,24 @@ static_assert(bwd_schedule_ok<10, 1>() && bwd_schedule_ok<8, 0>() && bwd_schedul
 // EV0 (block 0, ev = 0): the spherical branch is a constant (folded into the
 // output bias by the forward kernel) and s has no adjoint to give, so its
 // entries are left out.
-// RT (blocks after 0 on their radial tables): pairs in bucket order as in
-// k_radial_fwd_rows; the first section keeps E1^T (2 entries per chunk) and takes
-// the interval's slope tile against each chunk's df (third entry), whose
-// sum over the powers of t is the radial branches' dE/dr; the layer-0
-// recompute, W0^T and the Bernstein basis are left out.
-template <bool EV0, bool FIRST, bool RT = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT ? SO3LR_RT_BWD_WAVES : SO3LR_FILTER_WAVES,
-                                                                     RT ? SO3LR_RT_BWD_WAVES : SO3LR_FILTER_WAVES))) void
-k_filter_bwd_mfma(
+template <bool EV0, bool FIRST>
+__global__ __launch_bounds__(256) FILTER_OCCUPANCY void k_filter_bwd_mfma(
     const int *n_active, const int *pa, const double *pr, const double *ps, const double *pfc, const double *pY,
     const double *palpha, const double *__restrict__ qkv, const double *__restrict__ gainv,
     const double *__restrict__ gaev, const double *__restrict__ psc, const double *__restrict__ pdfc, double inv_avg,
-    FilterMfma A, double rc, double *ds, double *dr, double *dY, const int *n_slots = nullptr,
-    const int *order = nullptr, const double *__restrict__ rtab = nullptr, RadialDomain rd = {}) {
-  static_assert(!(EV0 && RT), "block 0 has its own tables");
+    FilterMfma A, double rc, double *ds, double *dr, double *dY) {
   SO3LR_EXP2_TABLE(A)
   const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
-  int p, pp, ri = 0;
-  bool valid, inside = false;
-  v4d tp[2];
-  if constexpr (RT) {
-    // consecutive slots on one XCD: a spatial block's buckets share its L2
-    const int blk = xcd_block_active((*n_slots + 63) / 64);
-    const int wave = blk < 0 ? -1 : blk * 4 + (threadIdx.x >> 6);
-    if (!rint_slots(n_slots, order, pr, rd, wave, j, g, p, ri, inside, tp)) return;
-    valid = p >= 0;
-    pp = valid ? p : order[wave * 16];
-  } else {
-    const int nact = *n_active;
-    // consecutive pairs on one XCD: the node rows they gather are spatial
-    // neighbours, so they share that XCD's L2
-    const int blk = xcd_block_active((nact + 63) / 64);
-    if (blk < 0) return;
-    const int wave = blk * 4 + (threadIdx.x >> 6);
-    if (wave * 16 >= nact) return;
-    p = wave * 16 + j;
-    valid = p < nact;
-    pp = valid ? p : nact - 1;
-  }
+  const int nact = *n_active;
+  // consecutive pairs on one XCD: the node rows they gather are spatial
+  // neighbours, so they share that XCD's L2
+  const int blk = xcd_block_active((nact + 63) / 64);
+  if (blk < 0) return;
+  const int wave = blk * 4 + (threadIdx.x >> 6);
+  if (wave * 16 >= nact) return;
+  const int p = wave * 16 + j;
+  const bool valid = p < nact;
+  const int pp = valid ? p : nact - 1;
   const int a = pa[2 * pp], b = pa[2 * pp + 1];
   // node rows, tile-transposed: chunk T of this lane at +16 T
   const double *ra = qkv + std::size_t(a) * 640 + 4 * g, *rb = qkv + std::size_t(b) * 640 + 4 * g;
@@ -1068,10 +890,10 @@ k_filter_bwd_mfma(
 
   // head scalars: block 0 forms them here (SRC 0 and 2), later blocks read
   // the node-major reverse's record (SRC 1)
-  constexpr int NM = RT ? 4 : (EV0 ? 8 : 10), SRC0 = EV0 ? 0 : 1, SRC1 = EV0 ? 2 : 1;
+  constexpr int NM = EV0 ? 8 : 10, SRC0 = EV0 ? 0 : 1, SRC1 = EV0 ? 2 : 1;
   constexpr int A_END0 = bwd_section_len<NM, SRC0>(), A_END1 = bwd_section_len<NM, SRC1>();
   const double *rec = psc + 16 * std::size_t(pp);
-  constexpr int B_LEN = RT ? 0 : 24, C_LEN = EV0 ? 0 : 3, D_LEN = RT ? 0 : 16, E_LEN = EV0 ? 0 : 2;
+  constexpr int B_LEN = 24, C_LEN = EV0 ? 0 : 3, D_LEN = 16, E_LEN = EV0 ? 0 : 2;
   constexpr int TAIL = B_LEN + C_LEN + D_LEN + E_LEN;
   constexpr int NB0 = A_END0 + TAIL, NB1 = A_END1 + TAIL;
   auto load = [&](auto si) -> v4d {
@@ -1093,9 +915,7 @@ k_filter_bwd_mfma(
         else if constexpr (e.q == 2) return row(rb, qoff + 16 * e.T);
         else return row(ra, koff + 16 * e.T);
       } else {
-        if constexpr (RT && e.q >= 2) return wload(rtab + (std::size_t(ri) * 2 + which) * 16 * 256, 8, e.q - 2, e.T, lane);
-        else if constexpr (RT) return wload(A.e1tp[which], 8, e.q, e.T, lane);
-        else if constexpr (e.q < 8) return wload(A.w1tp[which], 8, e.q, e.T, lane);
+        if constexpr (e.q < 8) return wload(A.w1tp[which], 8, e.q, e.T, lane);
         else return wload(A.e1tp[which], 8, e.q - 8, e.T, lane);
       }
     } else if constexpr (s < A_END + B_LEN) {
@@ -1113,7 +933,7 @@ k_filter_bwd_mfma(
       return wload(A.e0tp[which], 2, 0, s - A_END - B_LEN - C_LEN - D_LEN, lane);
     }
   };
-  Stream<NB0 + NB1, RT ? SO3LR_RT_BWD_PF : SO3LR_FILTER_BWD_PF, decltype(load)> st(load);
+  Stream<NB0 + NB1, SO3LR_FILTER_BWD_PF, decltype(load)> st(load);
   st.prime();
 
   const double r = pr[pp];
@@ -1163,7 +983,7 @@ k_filter_bwd_mfma(
   // d rbf and d s of one filter, folded into scalars at the end of their
   // sections (dE/dr is linear in d rbf), so neither is held through the next
   // filter's df section
-  v4d drb[2], dsa, accdr[2];
+  v4d drb[2], dsa;
   double part = 0.0, ds_acc = 0.0;
   double ci = 0.0, co = 0.0, s_in = 0.0, s_out = 0.0;
 
@@ -1176,10 +996,6 @@ k_filter_bwd_mfma(
       for (int mt = 0; mt < 8; ++mt) dh[mt] = zero;
       dh2[0] = zero;
       dh2[1] = zero;
-      if constexpr (RT && which == 0) {
-        accdr[0] = zero;
-        accdr[1] = zero;
-      }
     }
     if constexpr (s < A_END) {
       constexpr BwdEntry e = bwd_entry<NM, which ? SRC1 : SRC0>(s);
@@ -1227,10 +1043,7 @@ k_filter_bwd_mfma(
         }
       } else {
         if constexpr (e.q == 0) bT = bTn;
-        if constexpr (RT) {
-          if constexpr (e.q < 2) dh2[e.q] = mfma4(w, bT, dh2[e.q]);
-          else accdr[e.q - 2] = mfma4(w, bT, accdr[e.q - 2]);  // slopes . df, rows = powers of t
-        } else if constexpr (e.q < 8) {
+        if constexpr (e.q < 8) {
           dh[e.q] = mfma4(w, bT, dh[e.q]);
         } else {
           dh2[e.q - 8] = mfma4(w, bT, dh2[e.q - 8]);
@@ -1291,22 +1104,12 @@ k_filter_bwd_mfma(
       }
     }
     // the last tile's silu' (it is needed from the last two W0^T steps on)
-    if constexpr (!RT && s == B_END) {
+    if constexpr (s == B_END) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) dh[7][q] *= silu_prime_tab(prev[q], exp2_lds);
     }
   });
 
-  // RT: the radial branches' dE/dr, sum over the powers of t (tile m, row
-  // g + 4 r: power 16 m + g + 4 r)
-  if constexpr (RT) {
-    double sum = 0.0;
-#pragma unroll
-    for (int m = 0; m < 2; ++m)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) sum += accdr[m][r] * tp[m][r];
-    part = inside ? sum : 0.0;
-  }
   // dE/dr: the Bernstein part of both filters + the cutoff
   part += __shfl_xor(part, 16, kWave);
   part += __shfl_xor(part, 32, kWave);
@@ -1318,103 +1121,6 @@ k_filter_bwd_mfma(
       if (r < rc) {
         const double t = r / rc;
         grad += dfc * (-30.0 * t * t * (1.0 - t) * (1.0 - t) / rc);
-      }
-      dr[p] += grad;
-    }
-  }
-}
-
-// k_filter_bwd_mfma<false, false, true> for few pairs: eight wavefronts per 16
-// slots, one per filter and head, each with its head's two df chunks; the
-// spherical branch's silu' and E0^T are linear in the chunks' share of
-// E1^T df, so every wavefront takes its share through to dE/ds and dE/dr and
-// the shares are summed through LDS in wavefront order.
-__global__ __launch_bounds__(512) void k_filter_bwd_split(
-    const int *n_slots, const int *order, const int *pa, const double *pr, const double *ps,
-    const double *__restrict__ qkv, const double *__restrict__ psc, const double *__restrict__ pdfc, FilterMfma A,
-    double rc, double *ds, double *dr, const double *__restrict__ rtab, RadialDomain rd) {
-  SO3LR_EXP2_TABLE(A)
-  __shared__ double share[8][2][64];
-  const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
-  const int sub = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
-  const int wave = xcd_block_active((*n_slots + 15) / 16);
-  int p, ri;
-  bool inside;
-  v4d tp[2];
-  if (!rint_slots(n_slots, order, pr, rd, wave, j, g, p, ri, inside, tp)) return;  // the whole block
-  const bool valid = p >= 0;
-  const int pp = valid ? p : order[wave * 16];
-  const int a = pa[2 * pp], b = pa[2 * pp + 1];
-  const int which = sub >> 2, hd = sub & 3;
-  const int qoff = which ? 384 : 0, koff = which ? 512 : 128;
-  const double *ra = qkv + std::size_t(a) * 640 + 4 * g + 32 * hd, *rb = qkv + std::size_t(b) * 640 + 4 * g + 32 * hd;
-  const double *slopes = rtab + (std::size_t(ri) * 2 + which) * 16 * 256;
-  const double *e1t = which ? A.e1tp[1] : A.e1tp[0], *e0t = which ? A.e0tp[1] : A.e0tp[0];
-  const double *eb0 = which ? A.eb0p[1] : A.eb0p[0], *e0k = which ? A.e0pk[1] : A.e0pk[0];
-  auto row = [](const double *r) { return *reinterpret_cast<const v4d *>(r); };
-  v4d rows[2][4], fr[2][4];
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    rows[t][0] = row(ra + qoff + 16 * t);
-    rows[t][1] = row(rb + koff + 16 * t);
-    rows[t][2] = row(rb + qoff + 16 * t);
-    rows[t][3] = row(ra + koff + 16 * t);
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      fr[t][q] = wload(e1t, 8, q, 2 * hd + t, lane);
-      fr[t][2 + q] = wload(slopes, 8, q, 2 * hd + t, lane);
-    }
-  }
-  const v4d rec = row(psc + 16 * std::size_t(pp) + 4 * hd);
-  const double s_in = which ? rec[2] : rec[0], s_out = which ? rec[3] : rec[1];
-  const double sg = ps[4 * std::size_t(pp) + g];
-  v4d pre[2] = {tile_load(eb0, 0, lane), tile_load(eb0, 1, lane)};
-  const v4d w0 = row(e0k + 4 * lane), t0 = wload(e0t, 2, 0, 0, lane), t1 = wload(e0t, 2, 0, 1, lane);
-  const v4d zero = v4d{0.0, 0.0, 0.0, 0.0};
-  v4d dh[2] = {zero, zero}, acc[2] = {zero, zero};
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const v4d df = s_in * (rows[t][0] * rows[t][1]) + s_out * (rows[t][2] * rows[t][3]);
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      dh[q] = mfma4(fr[t][q], df, dh[q]);
-      acc[q] = mfma4(fr[t][2 + q], df, acc[q]);
-    }
-  }
-#pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    pre[q] = mfma(w0[q], sg, pre[q]);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) dh[q][r] *= silu_prime_tab_wide(pre[q][r], exp2_lds);
-  }
-  const v4d dsa = mfma4(t1, dh[1], mfma4(t0, dh[0], zero));
-  double part = 0.0;
-#pragma unroll
-  for (int m = 0; m < 2; ++m)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) part += acc[m][r] * tp[m][r];
-  share[sub][0][lane] = dsa[0];
-  share[sub][1][lane] = part;
-  __syncthreads();
-  if (sub != 0) return;
-  double ds_acc = 0.0;
-  part = 0.0;
-#pragma unroll
-  for (int q = 0; q < 8; ++q) {
-    ds_acc += share[q][0][lane];
-    part += share[q][1][lane];
-  }
-  part = inside ? part : 0.0;
-  part += __shfl_xor(part, 16, kWave);
-  part += __shfl_xor(part, 32, kWave);
-  if (valid) {
-    ds[4 * std::size_t(p) + g] = ds_acc;
-    if (g == 0) {
-      const double r = pr[p];
-      double grad = part;
-      if (r < rc) {
-        const double t = r / rc;
-        grad += pdfc[p] * (-30.0 * t * t * (1.0 - t) * (1.0 - t) / rc);
       }
       dr[p] += grad;
     }
@@ -2894,6 +2600,21 @@ std::vector<double> tile_order(const std::vector<double> &v) {
   return t;
 }
 
+// The rows of w (M x K, M channels in heads of 32) in the order of the table
+// kernels' output tiles: row 16 (2 h + e) + j is channel 32 h + 2 j + e of the
+// node rows; `transposed`: rows in the tile-transposed order, whose place
+// 16 T + 4 g + r holds feature 16 T + g + 4 r.
+std::vector<double> head_pairs(const std::vector<double> &w, std::size_t M, std::size_t K, bool transposed) {
+  std::vector<double> p(w.size());
+  for (std::size_t o = 0; o < M; ++o) {
+    const std::size_t h = o / 32, e = o / 16 % 2, j = o % 16, at = 32 * h + 2 * j + e;
+    const std::size_t src = transposed ? 16 * (at / 16) + at % 16 / 4 + 4 * (at % 4) : at;
+    std::copy(w.begin() + std::ptrdiff_t(src * K), w.begin() + std::ptrdiff_t((src + 1) * K),
+              p.begin() + std::ptrdiff_t(o * K));
+  }
+  return p;
+}
+
 std::vector<double> permute_mfma(const std::vector<double> &w, std::size_t M, std::size_t K) {
   const std::size_t MT = (M + 15) / 16;
   if (K == 4) {
@@ -3018,6 +2739,7 @@ Evaluator::Evaluator(std::shared_ptr<Model> model, int device) : model_(std::mov
       B.w1p[k] = up(permute_mfma(w1, F, F));
       B.e0p[k] = up(permute_mfma(e0, FH, 4));
       B.e1p[k] = up(permute_mfma(e1, F, FH));
+      B.e1h[k] = up(permute_mfma(head_pairs(e1, F, FH, true), F, FH));
       B.w1tp[k] = up(permute_mfma(transpose(w1, F, F), F, F));
       B.w0tp[k] = up(permute_mfma(transpose(w0, F, R), R, F));
       B.e1tp[k] = up(permute_mfma(transpose(e1, F, FH), FH, F));
@@ -3131,7 +2853,7 @@ Evaluator::Evaluator(std::shared_ptr<Model> model, int device) : model_(std::mov
               cv[c * n + kk] = ft.value[(std::size_t(i) * n + kk) * F + c];
               st[kk * F + c] = ft.slope[(std::size_t(i) * n + kk) * F + c];
             }
-          const auto pr = permute_mfma(cv, F, n), pd = permute_mfma(st, n, F);
+          const auto pr = permute_mfma(head_pairs(cv, F, n, true), F, n), pd = permute_mfma(st, n, F);
           rows[std::size_t(b)].insert(rows[std::size_t(b)].end(), pr.begin(), pr.end());
           drs[std::size_t(b)].insert(drs[std::size_t(b)].end(), pd.begin(), pd.end());
         }
@@ -3561,10 +3283,10 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
   const bool use_cls = !gen_ && !scalar && class_tables_ && n_cls_ > 0;
   // and with the radial tables (k_radial_fwd, k_radial_bwd)
   const bool use_rad = use_cls && radial_ok_;
-  // the blocks after 0 on their radial tables (k_radial_fwd_rows,
-  // k_filter_bwd_mfma<false, false, true>)
+  // the blocks after 0 on their radial tables (k_rows_fwd,
+  // k_rows_bwd)
   const bool use_rt = !gen_ && !scalar && radial_blocks_ && L > 1;
-  // and the generic path's (g_radial_fwd_rows)
+  // and the generic path's (the same kernels)
   const bool use_grt = gen_ && gen_->radial_blocks_ok() && L > 1;
   int *rord = nullptr, *rhist = nullptr;
   // buckets of the blocks after 0: (spatial block of kRintAtoms nodes, interval)
@@ -3860,9 +3582,12 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
   const unsigned gP16 = unsigned(std::max(1, ceil_div(PA, 16)));  // 16 pairs per radial-table block
   // slots of the bucket order: every bucket padded by fewer than 16
   const int rslots_max = PA + 16 * rkeys;
-  const unsigned gR = unsigned(ceil_div(rslots_max, 64));  // 16 slots per wavefront
-  const unsigned gR16 = unsigned(ceil_div(rslots_max, 16));  // 16 slots per block (few pairs)
-  const bool few = PA < kFewPairs;
+  // the table kernels of the blocks after 0 (reverse: rtab and e1 its own)
+  auto rows_args = [&](const BlockWeights &B, double *psb, double *pfb, double *pab) {
+    return RowsArgs{rslots, rord, pa, pr, nullptr, B.rrow, rbl_dom_, {B.e0pk[0], B.e0pk[1]}, {B.eb0p[0], B.eb0p[1]},
+                    {B.e1h[0], B.e1h[1]}, {B.e0tp[0], B.e0tp[1]}, hw_.exp2_256, psb, nullptr, B.att_cg, inv_avg, pfb,
+                    pab, psc, dfc, rc_, ds, dr};
+  };
 
   // --- interaction blocks, forward ---
   for (int b = 0; b < L; ++b) {
@@ -3941,9 +3666,12 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
         hipLaunchKernelGGL(k_filter_fwd_mfma<true>, dim3(gP64), dim3(256), 0, s, nact, pa, pr, evb, qb, inv_avg, FM,
                            psb, pfb, pab);
       else if (use_rt)  // rows and logits in bucket order, the radial branches from the tables
-        hipLaunchKernelGGL(few ? k_radial_fwd_rows<true> : k_radial_fwd_rows<false>, dim3(few ? gR16 : gR),
-                           dim3(few ? 512 : 256), 0, s, rslots, rord, pa, pr, evb, qb, B.rrow, rbl_dom_, inv_avg, FM,
-                           psb, pfb, pab);
+      {
+        RowsArgs R = rows_args(B, psb, pfb, pab);
+        R.qkv = qb;
+        R.ev = evb;
+        launch_rows<8, true, true>(s, rslots_max, int(PA), R);
+      }
       else
         hipLaunchKernelGGL(k_filter_fwd_mfma<false>, dim3(gP64), dim3(256), 0, s, nact, pa, pr, evb, qb, inv_avg, FM,
                            psb, pfb, pab);
@@ -4073,14 +3801,13 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
                      qb, gainv, gaev, psc, dfc, inv_avg, FM, rc_, ds, dr, dY)
           if (b == 0 && first) SO3LR_FILTER_BWD(true, true);
           else if (b == 0) SO3LR_FILTER_BWD(true, false);
-          else if (use_rt && few)
-            hipLaunchKernelGGL(k_filter_bwd_split, dim3(gR16), dim3(512), 0, s, rslots, rord, pa, pr, psb, qb, psc, dfc,
-                               FM, rc_, ds, dr, B.rdr, rbl_dom_);
-          else if (use_rt)  // in interval order, the radial branches' dE/dr from the slope tables
-            hipLaunchKernelGGL((k_filter_bwd_mfma<false, false, true>), dim3(gR), dim3(256), 0, s, nact, pa, pr, psb,
-                               pfc, pY, pab, qb, gainv, gaev, psc, dfc, inv_avg, FM, rc_, ds, dr, dY, rslots, rord,
-                               B.rdr, rbl_dom_);
-          else SO3LR_FILTER_BWD(false, false);  // dE/dY of blocks after 0: the node-major reverse
+          else if (use_rt) {  // in bucket order, the radial branches' dE/dr from the slope tables
+            RowsArgs R = rows_args(B, psb, nullptr, nullptr);
+            R.rtab = B.rdr;
+            R.qkv = qb;
+            for (int k = 0; k < 2; ++k) R.e1[k] = B.e1tp[k];
+            launch_rows<8, true, false>(s, rslots_max, int(PA), R);
+          } else SO3LR_FILTER_BWD(false, false);  // dE/dY of blocks after 0: the node-major reverse
 #undef SO3LR_FILTER_BWD
         });
       }

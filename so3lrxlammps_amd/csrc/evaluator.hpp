@@ -47,6 +47,7 @@ struct TopologyError : std::runtime_error {
 std::vector<double> transpose(const std::vector<double> &w, std::size_t rows, std::size_t cols);
 std::vector<double> bias_acc(const std::vector<double> &b, std::size_t M);
 std::vector<double> permute_mfma(const std::vector<double> &w, std::size_t M, std::size_t K);
+std::vector<double> head_pairs(const std::vector<double> &w, std::size_t M, std::size_t K, bool transposed);
 std::vector<double> tile_order(const std::vector<double> &v);
 
 // Device weight pointers for one interaction block.
@@ -62,12 +63,13 @@ struct BlockWeights {
   const double *ln1w, *ln1b, *ln2w, *ln2b;  // (128) in the tile-transposed order of the node rows
   // MFMA operand order of the filter weights (see permute_mfma in evaluator.hip)
   const double *w0p[2], *w1p[2], *e0p[2], *e1p[2];     // forward
+  const double *e1h[2];                                // E1 with its rows in head-pair order (radial_rows.hpp)
   const double *w1tp[2], *w0tp[2], *e1tp[2], *e0tp[2];  // reverse (transposes)
   const double *b0p[2], *eb0p[2], *ob1p[2];             // biases in accumulator order
   const double *ob1p0[2];                               // ob1p with the ev = 0 spherical branch folded in (block 0) (ob1 = b1 + eb1)
   const double *ob10[2];                                // the same output bias in natural order (block 0's tables)
   const double *e0pk[2];                                // spherical layer 0, one v4d per lane
-  // radial tables of the blocks after 0 (the RT filter kernels): per
+  // radial tables of the blocks after 0 (radial_rows.hpp): per
   // interval and filter, the radial branch W1 silu(W0 rbf + b0) + ob1 as
   // 16 powers of t (an MFMA A operand of 128 x 16) and its r-derivative
   // (16 x 128); null without the tables

@@ -14,7 +14,7 @@
 #include "generic.hpp"
 #include "evaluator.hpp"
 #include "mfma_ops.hpp"
-#include "node_chain.hpp"
+#include "radial_rows.hpp"
 
 #include <algorithm>
 #include <array>
@@ -102,18 +102,6 @@ struct SlotsG {
   __device__ __forceinline__ int off(int s) const { return d.off[s]; }
   __device__ __forceinline__ int slot(int m) const { return d.slot[m]; }
 };
-
-// Dispatch block b (round-robin over the 8 XCDs) to logical block: each XCD
-// takes a contiguous run of the `active` blocks, so consecutive pairs or
-// nodes (spatially sorted: they share endpoints and partners) share that
-// XCD's L2.  -1: beyond the active blocks.  The grid is a multiple of 8 and
-// holds at least `active` blocks.
-__device__ __forceinline__ int g_xcd_block(int active) {
-  const int b = blockIdx.x;
-  const int per = active >> 3, rem = active & 7, xcd = b & 7, i = b >> 3;
-  if (i >= per + (xcd < rem ? 1 : 0)) return -1;
-  return xcd * per + (xcd < rem ? xcd : rem) + i;
-}
 
 // Attention messages, node-major (kokkos_integrated_block0.cpp:330-385):
 // node n receives from each incident pair's partner o the invariant message
@@ -395,7 +383,7 @@ __global__ __launch_bounds__(256) void g_attn_bwd_pairs(GDims d, const int *nact
   __shared__ double lte[4][2][kGMaxE];  // per wavefront: gaev_r Y' per direction and channel
   __shared__ double lps[4][32];         // per wavefront: psc of the pair
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int blk = g_xcd_block((min(*nact, cap) + 3) / 4);
+  const int blk = xcd_block_active((min(*nact, cap) + 3) / 4);
   if (blk < 0) return;
   const int p = blk * 4 + wv;
   if (p >= min(*nact, cap)) return;
@@ -915,7 +903,7 @@ struct FiltArgs {
 // false: the wavefront has no pair
 __device__ __forceinline__ bool filt_pair(const FiltArgs &A, int j, int &pp, bool &valid) {
   const int nact = min(*A.nact, A.cap);
-  const int blk = g_xcd_block((nact + 63) / 64);
+  const int blk = xcd_block_active((nact + 63) / 64);
   if (blk < 0) return false;
   const int wave = blk * 4 + int(threadIdx.x >> 6);
   if (wave * 16 >= nact) return false;
@@ -1329,286 +1317,10 @@ void launch_b0(hipStream_t s, int F, int R, std::size_t slots, const B0Args &A) 
   throw std::logic_error("SO3LR: block 0's table kernels at widths other than F = 128, 256 and R = 32, 64");
 }
 
-// The forward filters of the blocks after 0 on their radial tables (the
-// algebra of evaluator.hip's k_radial_fwd_rows at generic widths): the pairs
-// in bucket order (16 slots of one bucket, spatial block and interval, per
-// wavefront), per filter the spherical hidden tiles silu(E0 s + e0), then
-// per output tile the interval's coefficient tile (two K chunks against the
-// pairs' powers of t, in place of the W0 and W1 chains), the E1 chunks and
-// the endpoint rows; the rows go to pf and the logits to palpha as in
-// g_filt_fwd.  SPLIT: FT wavefronts per 16 slots, one per filter and head
-// (launch_rows).
-struct GRadArgs {
-  const int *slots, *order, *pa;
-  const double *pr, *ps, *qkv, *rtab;
-  RadialDomain d;
-  const double *eb0a[2], *e0p[2], *wcp[2];
-  const double *exp2_256;
-  double inv_avg;
-  double *pf, *palpha;
-  // reverse (g_radial_bwd_rows): rtab holds the slope tiles
-  const double *e0tp[2], *wctp[2], *psc, *dfc;
-  double rc;
-  double *ds, *dr;
-};
-
-template <int FT, bool SPLIT>
-__global__ __launch_bounds__(SPLIT ? 64 * FT : 256) void g_radial_fwd_rows(GRadArgs A) {
-  constexpr int FHT = FT / 4, NH = FT / 2, HT = FT + FHT, F = 16 * FT, NE = 6 + FHT;
-  constexpr int NT = SPLIT ? 2 : FT;  // output tiles of a wavefront
-  __shared__ double tab[256];
-  if (!SPLIT || threadIdx.x < 256) tab[threadIdx.x & 255] = A.exp2_256[threadIdx.x & 255];
-  __syncthreads();
-  const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
-  const int blk = g_xcd_block((*A.slots + (SPLIT ? 15 : 63)) / (SPLIT ? 16 : 64));
-  const int sub = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
-  const int wave = blk < 0 ? -1 : (SPLIT ? blk : blk * 4 + sub);
-  const int w0 = SPLIT ? sub / NH : 0, mt0 = SPLIT ? 2 * (sub % NH) : 0;
-  int p, ri;
-  bool inside;
-  v4d tp[2];
-  if (!rint_slots(A.slots, A.order, A.pr, A.d, wave, j, g, p, ri, inside, tp)) return;
-  const bool valid = p >= 0;
-  const int pp = valid ? p : A.order[wave * 16];
-  const int a = A.pa[2 * pp], b = A.pa[2 * pp + 1];
-  const double *ra = A.qkv + std::size_t(a) * 5 * F + 4 * g, *rr = A.qkv + std::size_t(b) * 5 * F + 4 * g;
-  double *frow = A.pf + std::size_t(pp) * 2 * F + 4 * g;
-  double *al = A.palpha + std::size_t(pp) * 4 * NH;
-  v4d sv;
-#pragma unroll
-  for (int v = 0; v < 4; ++v) sv[v] = g + 4 * v < NH ? A.ps[std::size_t(pp) * NH + g + 4 * v] : 0.0;
-  const v4d zero = v4d{0.0, 0.0, 0.0, 0.0};
-  static_for<SPLIT ? 1 : 2>([&](auto wi) {
-    const int w = w0 + decltype(wi)::value;
-    const double *e0p = w ? A.e0p[1] : A.e0p[0], *eb0a = w ? A.eb0a[1] : A.eb0a[0], *wcp = w ? A.wcp[1] : A.wcp[0];
-    v4d he[FHT];
-    auto hidden = [&](int t) {
-      const v4d e0 = frag_load(e0p, t, lane);
-      v4d h = mfma(e0[0], sv[0], frag_load(eb0a, t, lane));
-      if constexpr (NH > 4) h = mfma(e0[1], sv[1], h);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) h[r] = silu_tab_wide(h[r], tab);
-      return h;
-    };
-    if constexpr (!SPLIT) {
-#pragma unroll
-      for (int t = 0; t < FHT; ++t) he[t] = hidden(t);
-    }
-    const double *coef = A.rtab + (std::size_t(ri) * 2 + w) * FT * 2 * 256;
-    const int qo = w ? 3 * F : 0, ko = w ? 4 * F : F;  // q, k or q_ev, k_ev
-    auto ld = [&](auto si) -> v4d {
-      constexpr int S = decltype(si)::value, u = S % NE;
-      const int mt = mt0 + S / NE;
-      if constexpr (u < 2) return frag_load(coef, mt * 2 + u, lane);
-      else if constexpr (u < 2 + FHT) return frag_load(wcp, mt * HT + FT + u - 2, lane);
-      else if constexpr (u == 2 + FHT) return *reinterpret_cast<const v4d *>(ra + qo + 16 * mt);
-      else if constexpr (u == 3 + FHT) return *reinterpret_cast<const v4d *>(rr + ko + 16 * mt);
-      else if constexpr (u == 4 + FHT) return *reinterpret_cast<const v4d *>(rr + qo + 16 * mt);
-      else return *reinterpret_cast<const v4d *>(ra + ko + 16 * mt);
-    };
-    Stream<NT * NE, 6, decltype(ld)> st(ld);
-    st.prime();
-    if constexpr (SPLIT) {  // the filters' hidden tiles, each formed by one wavefront
-      __shared__ v4d hid[2][FHT][64];
-      if (sub % NH < FHT) hid[w][sub % NH][lane] = hidden(sub % NH);
-      __syncthreads();
-#pragma unroll
-      for (int t = 0; t < FHT; ++t) he[t] = hid[w][t][lane];
-    }
-    v4d o, qv, qk0, qk1;
-    double t0 = 0.0, t1 = 0.0;
-    st.run([&](auto si, const v4d &wv) {
-      constexpr int S = decltype(si)::value, u = S % NE;
-      const int mt = mt0 + S / NE;
-      if constexpr (u == 0) {
-        o = mfma4(wv, tp[0], zero);
-      } else if constexpr (u == 1) {
-        o = mfma4(wv, tp[1], o);
-      } else if constexpr (u < 2 + FHT) {
-        o = mfma4(wv, he[u - 2], o);
-      } else if constexpr (u == 2 + FHT || u == 4 + FHT) {
-        qv = wv;
-      } else if constexpr (u == 3 + FHT) {
-        qk0 = qv * wv;  // q_a k_b: edge b -> a
-      } else {
-        qk1 = qv * wv;  // q_b k_a: edge a -> b
-        if (valid) *reinterpret_cast<v4d *>(frow + w * F + 16 * mt) = o;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          t0 += qk0[r] * o[r];
-          t1 += qk1[r] * o[r];
-        }
-        if constexpr ((S / NE) & 1) {  // head mt / 2 complete: sum over the lane groups
-          t0 += __shfl_xor(t0, 16, 64);
-          t0 += __shfl_xor(t0, 32, 64);
-          t1 += __shfl_xor(t1, 16, 64);
-          t1 += __shfl_xor(t1, 32, 64);
-          if (valid && g == 0) {
-            al[w * NH + (mt >> 1)] = t0 * A.inv_avg;
-            al[2 * NH + w * NH + (mt >> 1)] = t1 * A.inv_avg;
-          }
-          t0 = 0.0;
-          t1 = 0.0;
-        }
-      }
-    });
-  });
-}
-
-// The reverse filters of the blocks after 0 on their radial tables, in
-// bucket order: per filter and output tile mt, df from the logits' adjoints
-// and the endpoint rows as in g_filt_bwd, then the spherical hidden row's
-// adjoint (E1^T chunks) and the slope tiles against df, whose sum over the
-// powers of t is the radial branches' dE/dr; the spherical branch goes on
-// through silu' and E0^T to dE/ds.  No W1^T, no layer-0 recompute.
-template <int FT, bool SPLIT>
-__global__ __launch_bounds__(SPLIT ? 64 * FT : 256) void g_radial_bwd_rows(GRadArgs A) {
-  constexpr int FHT = FT / 4, NH = FT / 2, F = 16 * FT, NE = 4 + FHT + 2;
-  constexpr int NT = SPLIT ? 2 : FT, NR = (NH + 3) / 4;
-  __shared__ double tab[256], share[SPLIT ? FT : 1][NR + 1][64];
-  __shared__ v4d prime[2][SPLIT ? FHT : 1][64];  // SPLIT: silu' of the hidden tiles, each formed by one wavefront
-  if (!SPLIT || threadIdx.x < 256) tab[threadIdx.x & 255] = A.exp2_256[threadIdx.x & 255];
-  __syncthreads();
-  const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
-  const int blk = g_xcd_block((*A.slots + (SPLIT ? 15 : 63)) / (SPLIT ? 16 : 64));
-  const int sub = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
-  const int wave = blk < 0 ? -1 : (SPLIT ? blk : blk * 4 + sub);
-  const int w0 = SPLIT ? sub / NH : 0, mt0 = SPLIT ? 2 * (sub % NH) : 0;
-  int p, ri;
-  bool inside;
-  v4d tp[2];
-  if (!rint_slots(A.slots, A.order, A.pr, A.d, wave, j, g, p, ri, inside, tp)) return;
-  const bool valid = p >= 0;
-  const int pp = valid ? p : A.order[wave * 16];
-  const int a = A.pa[2 * pp], b = A.pa[2 * pp + 1];
-  const double *ra = A.qkv + std::size_t(a) * 5 * F + 4 * g, *rr = A.qkv + std::size_t(b) * 5 * F + 4 * g;
-  const double *ps = A.psc + std::size_t(pp) * 4 * NH;
-  v4d sv;
-#pragma unroll
-  for (int v = 0; v < 4; ++v) sv[v] = g + 4 * v < NH ? A.ps[std::size_t(pp) * NH + g + 4 * v] : 0.0;
-  const v4d zero = v4d{0.0, 0.0, 0.0, 0.0};
-  v4d dsa = zero, accdr[2] = {zero, zero};
-  static_for<SPLIT ? 1 : 2>([&](auto wi) {
-    const int w = w0 + decltype(wi)::value;
-    const int qo = w ? 3 * F : 0, ko = w ? 4 * F : F;
-    const double *e0p = w ? A.e0p[1] : A.e0p[0], *eb0a = w ? A.eb0a[1] : A.eb0a[0];
-    const double *e0tp = w ? A.e0tp[1] : A.e0tp[0], *wctp = w ? A.wctp[1] : A.wctp[0];
-    const double *slope = A.rtab + (std::size_t(ri) * 2 + w) * 2 * FT * 256;
-    v4d dh[FHT];
-#pragma unroll
-    for (int t = 0; t < FHT; ++t) dh[t] = zero;
-    auto slope_of = [&](int t) {
-      const v4d e0 = frag_load(e0p, t, lane);
-      v4d pre = mfma(e0[0], sv[0], frag_load(eb0a, t, lane));
-      if constexpr (NH > 4) pre = mfma(e0[1], sv[1], pre);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) pre[r] = silu_prime_tab_wide(pre[r], tab);
-      return pre;
-    };
-    auto ld = [&](auto si) -> v4d {
-      constexpr int S = decltype(si)::value, u = S % NE;
-      const int mt = mt0 + S / NE;
-      if constexpr (u < 4) {
-        const double *row = (u == 0 ? ra + qo : (u == 1 ? rr + ko : (u == 2 ? rr + qo : ra + ko))) + 16 * mt;
-        return *reinterpret_cast<const v4d *>(row);
-      } else if constexpr (u < 4 + FHT) {
-        return frag_load(wctp, (FT + u - 4) * FT + mt, lane);
-      } else {
-        return frag_load(slope, (u - 4 - FHT) * FT + mt, lane);
-      }
-    };
-    double c0 = ps[w * NH + (mt0 >> 1)], c1 = ps[2 * NH + w * NH + (mt0 >> 1)];  // the first head
-    v4d qv, df;
-    Stream<NE * NT, 6, decltype(ld)> st(ld);
-    st.prime();
-    if (SPLIT && sub % NH < FHT) prime[w][sub % NH][lane] = slope_of(sub % NH);
-    st.run([&](auto si, const v4d &wv) {
-      constexpr int S = decltype(si)::value, u = S % NE;
-      const int mt = mt0 + S / NE;
-      if constexpr (u == 0 || u == 2) {
-        qv = wv;
-      } else if constexpr (u == 1) {
-        df = c0 * (qv * wv);
-      } else if constexpr (u == 3) {
-        df += c1 * (qv * wv);
-        const int hn = min(mt + 1, mt0 + NT - 1) >> 1;  // the next tile's head
-        c0 = ps[w * NH + hn];
-        c1 = ps[2 * NH + w * NH + hn];
-      } else if constexpr (u < 4 + FHT) {
-        dh[u - 4] = mfma4(wv, df, dh[u - 4]);
-      } else {
-        accdr[u - 4 - FHT] = mfma4(wv, df, accdr[u - 4 - FHT]);
-      }
-    });
-    // the spherical branch: pre again, d hidden *= silu'(pre), E0^T
-    if constexpr (SPLIT) __syncthreads();
-#pragma unroll
-    for (int t = 0; t < FHT; ++t) {
-      dh[t] *= SPLIT ? prime[w][t][lane] : slope_of(t);
-      dsa = mfma4(frag_load(e0tp, t, lane), dh[t], dsa);
-    }
-  });
-  // dE/dr: the radial branches' (powers 16 m + g + 4 r), plus the cutoff's
-  double part = 0.0;
-#pragma unroll
-  for (int m = 0; m < 2; ++m)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) part += accdr[m][r] * tp[m][r];
-  if constexpr (SPLIT) {  // the filters' and heads' shares, summed in wavefront order
-#pragma unroll
-    for (int r = 0; r < NR; ++r) share[sub][r][lane] = dsa[r];
-    share[sub][NR][lane] = part;
-    __syncthreads();
-    if (sub != 0) return;
-#pragma unroll
-    for (int q = 1; q < FT; ++q) {
-#pragma unroll
-      for (int r = 0; r < NR; ++r) dsa[r] += share[q][r][lane];
-      part += share[q][NR][lane];
-    }
-  }
-  if (valid) {
-#pragma unroll
-    for (int r = 0; r < NR; ++r)
-      if (g + 4 * r < NH) A.ds[std::size_t(pp) * NH + g + 4 * r] = dsa[r];
-  }
-  if (!inside) part = 0.0;
-  part += __shfl_xor(part, 16, 64);
-  part += __shfl_xor(part, 32, 64);
-  if (valid && g == 0) {
-    const double r = A.pr[pp];
-    double grad = part;
-    if (r < A.rc) {
-      const double t = r / A.rc;
-      grad += A.dfc[pp] * (-30.0 * t * t * (1.0 - t) * (1.0 - t) / A.rc);
-    }
-    A.dr[pp] += grad;
-  }
-}
-
-// g_radial_fwd_rows / g_radial_bwd_rows at F = 128 or 256; below kFewRows
-// pairs their split forms, a wavefront per filter and head of 16 slots (see
-// k_radial_fwd_rows); their hidden tiles and its slopes are formed once per
-// block and pass through LDS, else 16 wavefronts form them each (632 against
-// 615 us per evaluation of 22 atoms at F = 256).  Whole evaluations at F = 256
-// without / with them (us, by pairs with their margin): 22 atoms 696 / 615,
-// 2,200 pairs 784 / 682, 4,700 822 / 792, 6,200 840 / 810, 10,300 889 / 944,
-// 11,200 901 / 959.
-constexpr int kFewRows = 7500;
 template <bool FWD>
-void launch_rows(hipStream_t s, int F, const GContext &c, const GRadArgs &A) {
-  auto go = [&](auto ft, auto split) {
-    constexpr int FT = decltype(ft)::value;
-    constexpr bool SPLIT = decltype(split)::value;
-    hipLaunchKernelGGL((FWD ? g_radial_fwd_rows<FT, SPLIT> : g_radial_bwd_rows<FT, SPLIT>),
-                       dim3(blocks_for(std::size_t(std::max(c.rint_max, 1)), SPLIT ? 16 : 64)),
-                       dim3(SPLIT ? 64 * FT : 256), 0, s, A);
-  };
-  const bool few = c.cap < kFewRows;
-  if (F == 128 && few) go(std::integral_constant<int, 8>{}, std::true_type{});
-  else if (F == 128) go(std::integral_constant<int, 8>{}, std::false_type{});
-  else if (few) go(std::integral_constant<int, 16>{}, std::true_type{});
-  else go(std::integral_constant<int, 16>{}, std::false_type{});
+void rows_launch(hipStream_t s, int F, const GContext &c, const RowsArgs &A) {
+  if (F == 128) launch_rows<8, false, FWD>(s, std::max(c.rint_max, 1), c.cap, A);
+  else launch_rows<16, false, FWD>(s, std::max(c.rint_max, 1), c.cap, A);
 }
 
 // g_radial_fwd / g_radial_bwd at NH = 4 or 8 heads over cap pairs
@@ -1632,7 +1344,7 @@ void launch_radial(hipStream_t s, int NH, const GContext &c, const double *tab, 
 }
 
 // g_filt_fwd / g_filt_bwd at F = 16 FT, R = 16 RT over cap pairs (one
-// wavefront per 16, the grid a multiple of 8: g_xcd_block)
+// wavefront per 16, the grid a multiple of 8: xcd_block_active)
 template <bool FWD>
 void launch_filt(hipStream_t s, int F, int R, std::size_t cap, const FiltArgs &A) {
   const dim3 grid((blocks_for(cap, 64) + 7) / 8 * 8);
@@ -1842,6 +1554,7 @@ GenericPath::GenericPath(const Model &m, const std::function<const double *(cons
           bcr[o] = bc[src];
         }
         B.wcp[k] = up(permute_mfma(wcr, F, F + FH));
+        if (F % 32 == 0 && FH % 16 == 0) B.e1h[k] = up(permute_mfma(head_pairs(e1, F, FH, false), F, FH));
         B.bca[k] = up(bias_acc(bcr, F));
         B.wctp[k] = up(permute_mfma_kc(transpose(wc, F, F + FH), F + FH, F));
       }
@@ -1984,11 +1697,9 @@ GenericPath::GenericPath(const Model &m, const std::function<const double *(cons
         for (int k = 0; k < 2; ++k) {
           const RadialFit &ft = fits[std::size_t(k)];
           std::vector<double> cv(F * n);
-          for (std::size_t o = 0; o < F; ++o) {
-            const std::size_t src = 16 * (o / 16) + 4 * (o % 4) + (o % 16) / 4;
-            for (std::size_t kk = 0; kk < n; ++kk) cv[o * n + kk] = ft.value[(std::size_t(i) * n + kk) * F + src];
-          }
-          const auto pr = permute_mfma(cv, F, n);
+          for (std::size_t o = 0; o < F; ++o)
+            for (std::size_t kk = 0; kk < n; ++kk) cv[o * n + kk] = ft.value[(std::size_t(i) * n + kk) * F + o];
+          const auto pr = permute_mfma(head_pairs(cv, F, n, false), F, n);
           rows[std::size_t(b)].insert(rows[std::size_t(b)].end(), pr.begin(), pr.end());
           // the slopes transposed, channels in natural order (the reverse's df)
           std::vector<double> st(n * F);
@@ -2096,9 +1807,10 @@ void GenericPath::forward(const GContext &c) {
                        B.att_cg, psb);
     if (b > 0 && c.rint_order) {
       // the radial tables, in bucket order
-      GRadArgs R{c.rint_slots, c.rint_order, c.pa, c.pr, psb, qb, B.rrow, rbl_dom_, {B.eb0a[0], B.eb0a[1]},
-                 {B.e0p[0], B.e0p[1]}, {B.wcp[0], B.wcp[1]}, hw_.exp2_256, c.inv_avg, pfb, pab};
-      section(c, "generic_filter_fwd_radial", [&] { launch_rows<true>(s, F, c, R); });
+      const RowsArgs R{c.rint_slots, c.rint_order, c.pa, c.pr, qb, B.rrow, rbl_dom_, {B.e0p[0], B.e0p[1]},
+                       {B.eb0a[0], B.eb0a[1]}, {B.e1h[0], B.e1h[1]}, {nullptr, nullptr}, hw_.exp2_256, psb, nullptr,
+                       nullptr, c.inv_avg, pfb, pab, nullptr, nullptr, c.rc, nullptr, nullptr};
+      section(c, "generic_filter_fwd_radial", [&] { rows_launch<true>(s, F, c, R); });
     } else {
     // both filters' rows f = [W1 | E1] [silu(W0 rbf + b0) | silu(E0 s + e0)]
     // + b1 + e1 and the attention logits from them, fused
@@ -2215,10 +1927,12 @@ void GenericPath::reverse(const GContext &c) {
     } else if (b > 0 && c.rint_order) {
       // the radial tables, in bucket order: df against the slope tiles to
       // dE/dr, the spherical branch to dE/ds
-      GRadArgs Rg{c.rint_slots, c.rint_order, c.pa, c.pr, psb, qb, B.rdr, rbl_dom_, {B.eb0a[0], B.eb0a[1]},
-                  {B.e0p[0], B.e0p[1]}, {nullptr, nullptr}, hw_.exp2_256, c.inv_avg, nullptr, nullptr,
-                  {B.e0tp[0], B.e0tp[1]}, {B.wctp[0], B.wctp[1]}, b_[PSC], b_[DFC], c.rc, b_[DS], c.dr};
-      section(c, "generic_filter_bwd_radial", [&] { launch_rows<false>(s, F, c, Rg); });
+      const std::size_t e1t = std::size_t(F) * F;  // [W1 | E1]^T: past W1's rows
+      const RowsArgs Rg{c.rint_slots, c.rint_order, c.pa, c.pr, qb, B.rdr, rbl_dom_, {B.e0p[0], B.e0p[1]},
+                        {B.eb0a[0], B.eb0a[1]}, {B.wctp[0] + e1t, B.wctp[1] + e1t}, {B.e0tp[0], B.e0tp[1]},
+                        hw_.exp2_256, psb, nullptr, nullptr, c.inv_avg, nullptr, nullptr, b_[PSC], b_[DFC], c.rc,
+                        b_[DS], c.dr};
+      section(c, "generic_filter_bwd_radial", [&] { rows_launch<false>(s, F, c, Rg); });
     } else {
       // both filters fused: d hidden = [W1 | E1]^T df (df from the logits'
       // adjoints psc), (.) silu'(pre), through W0^T and E0^T to dE/dr and

@@ -56,10 +56,11 @@ struct GBlock {
   // bias_acc): W0 (F x R), E0 (FH x NH, K padded to 16), [W1 | E1], and their
   // transposes; b0, e0, b1 + e1
   const double *w0p[2], *e0p[2], *wcp[2], *w0tp[2], *e0tp[2], *wctp[2];
+  const double *e1h[2];  // E1 with its rows in head-pair order (radial_rows.hpp)
   const double *b0a[2], *eb0a[2], *bca[2];
   // blocks after 0 on their radial tables: per interval and filter the radial
   // branch W1 silu(W0 rbf + b0) + b1 + e1 as F x 32 powers of t (rows
-  // permuted within each tile as wcp's), MFMA A operands; null without them
+  // in head-pair order), MFMA A operands; null without them
   const double *rrow;
   // and their slopes transposed, 32 powers x F (permute_mfma_kc, as wctp)
   const double *rdr;

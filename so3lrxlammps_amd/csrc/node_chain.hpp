@@ -47,6 +47,16 @@ __device__ __forceinline__ int xcd_block() {
   const int per = G >> 3, rem = G & 7, xcd = b & 7, i = b >> 3;
   return xcd * per + (xcd < rem ? xcd : rem) + i;
 }
+// xcd_block for a grid sized for an upper bound of the work: only the first A
+// logical blocks have work (A <= gridDim.x, known on the device only), and
+// they are spread evenly over the XCDs; -1 for a block with none.
+__device__ __forceinline__ int xcd_block_active(int A) {
+  const int b = blockIdx.x;
+  const int per = A >> 3, rem = A & 7, xcd = b & 7, i = b >> 3;
+  if (i >= per + (xcd < rem ? 1 : 0)) return -1;
+  return xcd * per + (xcd < rem ? xcd : rem) + i;
+}
+
 // A node's wavefronts in the node-major kernels: W wavefronts share a node's
 // incidence list in W runs, and the first adds the others' sums in run order.
 // One wavefront per node reads its list serially (about 1 us per pair of
