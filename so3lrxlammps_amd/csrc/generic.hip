@@ -103,6 +103,16 @@ struct SlotsG {
   __device__ __forceinline__ int slot(int m) const { return d.slot[m]; }
 };
 
+// A pair's value for this lane's head, of the two heads a wavefront's 64
+// channels span: q is the same in every lane, so both come through the scalar
+// cache.  As vector loads the reverse's five values of an entry took about as
+// many L1 accesses as the seven rows it reads.  Evaluations at F = 256, vector
+// loads / this (us): 3,000 atoms 2,067 / 1,924, 24,000 atoms 14,565 / 13,132.
+__device__ __forceinline__ double head_pair(const double *__restrict__ q, int lane) {
+  const double a = q[0], b = q[1];
+  return lane < 32 ? a : b;
+}
+
 // Attention messages, node-major (kokkos_integrated_block0.cpp:330-385):
 // node n receives from each incident pair's partner o the invariant message
 // fc alpha v_o and the equivariant fc alpha_ev Y (parity of the direction),
@@ -149,7 +159,7 @@ __global__ __launch_bounds__(NodeShare<W>::kBlock) void g_attn_msg(GDims d, int 
     for (int j = 0; j < 4; ++j) {
       const int c = lane + 64 * (j < J ? j : 0);
       T.v[j] = vo[c];
-      T.a[j] = al[c >> 5];
+      T.a[j] = head_pair(al + 2 * (j < J ? j : 0), lane);
     }
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
@@ -205,7 +215,7 @@ __global__ __launch_bounds__(NodeShare<W>::kBlock) void g_attn_bwd_node(GDims d,
   const NodeShare<W> S(N, inc_off, NQ);
   const int n = S.n;
   if (W == 1 && !S.on) return;
-  const int c = 64 * S.c + lane, h = c >> 5;
+  const int c = 64 * S.c + lane, h = 2 * S.c;
   double sum[5] = {0, 0, 0, 0, 0};  // d q, k, v, q_ev, k_ev
   // per entry: n receives along direction sn from o and sends along
   // so = 1 - sn to o
@@ -220,11 +230,11 @@ __global__ __launch_bounds__(NodeShare<W>::kBlock) void g_attn_bwd_node(GDims d,
     const double *al = palpha + std::size_t(p) * 4 * NH;
     const double *fi = pf + std::size_t(p) * 2 * F;
     const double *qo = qkv + std::size_t(o) * 5 * F;
-    T.si = sc[sn * 2 * NH + h];
-    T.sie = sc[sn * 2 * NH + NH + h];
-    T.so = sc[so * 2 * NH + h];
-    T.soe = sc[so * 2 * NH + NH + h];
-    T.ao = al[so * 2 * NH + h];
+    T.si = head_pair(sc + sn * 2 * NH + h, lane);
+    T.sie = head_pair(sc + sn * 2 * NH + NH + h, lane);
+    T.so = head_pair(sc + so * 2 * NH + h, lane);
+    T.soe = head_pair(sc + so * 2 * NH + NH + h, lane);
+    T.ao = head_pair(al + so * 2 * NH + h, lane);
     T.fi = fi[c];
     T.fe = fi[F + c];
     T.qo = qo[c];

@@ -80,7 +80,8 @@ struct NodeShare {
   // `cut`: a node's channels in that many slices, each with W wavefronts of
   // its own (c: this wavefront's slice; kNodes slices per block)
   __device__ __forceinline__ NodeShare(int N, const int *__restrict__ off, int cut = 1) {
-    const int wv = threadIdx.x >> 6, part = wv % W, u = xcd_block() * kNodes + wv / W;
+    // the same in every lane: the node's offsets and rows are addressed by scalars
+    const int wv = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6), part = wv % W, u = xcd_block() * kNodes + wv / W;
     n = u / cut;
     c = u % cut;
     on = n < N;
