@@ -382,4 +382,32 @@ __device__ __forceinline__ void for_active_pairs(int beg, int end, const int *__
   }
 }
 
+// The same walk four entries at a time: body(e, o, count), the entries past
+// count repeating the last; o is row(partner), found for 64 entries at once.
+template <class Row, class Body>
+__device__ __forceinline__ void for_active_quads(int beg, int end, const int *__restrict__ iact,
+                                                 const int *__restrict__ iother, int lane, Row &&row,
+                                                 Body &&body) {
+  for (int k0 = beg; k0 < end; k0 += 64) {
+    const int k = k0 + lane;
+    const int ent = k < end ? iact[k] : -1;
+    const int oth = ent >= 0 ? row(iother[k]) : 0;
+    unsigned long long mask = __ballot(ent >= 0);
+    while (mask) {
+      int e[4], o[4], l = 0, count = 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (mask) {
+          l = __ffsll(mask) - 1;
+          mask &= mask - 1;
+          ++count;
+        }
+        e[i] = __builtin_amdgcn_readlane(ent, l);
+        o[i] = __builtin_amdgcn_readlane(oth, l);
+      }
+      body(e, o, count);
+    }
+  }
+}
+
 }  // namespace so3lr_amd

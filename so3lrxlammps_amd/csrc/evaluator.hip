@@ -73,7 +73,7 @@ constexpr int kPrefixBlocks = 1024;
 
 // DPP lane permute of a double within the 16-lane rows of a wavefront (two
 // 32-bit moves).  CTRL: 0xB1 quad_perm(1,0,3,2), 0x4E quad_perm(2,3,0,1),
-// 0x141 row_half_mirror, 0x140 row_mirror.
+// 0x141 row_half_mirror, 0x140 row_mirror, 0x150 + n row_newbcast (lane n).
 template <int CTRL>
 __device__ __forceinline__ double dpp_f64(double v) {
   const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
@@ -98,6 +98,35 @@ __device__ __forceinline__ double group_sum(double v) {
   v += dpp_f64<0x140>(v);
   return v;
 }
+
+// An incidence entry's harmonics and attention weights in one load, for the
+// lane layout of the node-major kernels (row h of 16 lanes, t the lane in it):
+// lanes t < 12 hold channel m's harmonic of the pair (channel 0 beyond the
+// row's 2 h + 3), lanes 12 to 15 head h's weights of the entry's own direction
+// (invariant, equivariant) and of the other one, which weight<k> spreads over
+// the row.  A load of 8 bytes a lane costs about 16 L1 accesses however few of
+// its addresses differ (counters: 77 per entry in k_attn_msg, 16 of them for
+// the partner's row), so the weights' own loads cost as much as whole rows.
+// The direction is in the address: chosen after the load it is a branch, and
+// an entry's loads no longer overlap the next one's.
+// 24,000 / 3,000 atoms, separate loads / this one (us): k_attn_bwd_nodes 776 /
+// 738 and 109 / 102.
+struct EntryScalars {
+  const double *base;
+  unsigned c;
+  bool y;
+  __device__ __forceinline__ EntryScalars(const double *pY, const double *palpha, int h, int t, int m)
+      : base(t < 12 ? pY : palpha), c(t < 12 ? m : 4 * (t - 12) + h), y(t < 12) {}
+  // pair p = e / 2 < 2^27 (its filter rows alone are 2 KiB)
+  __device__ __forceinline__ double load(int e) const {
+    const unsigned p = unsigned(e) >> 1, side = e & 1;
+    return base[y ? 24u * p + c : 16u * p + (c ^ (8u * side))];
+  }
+  template <int K>
+  static __device__ __forceinline__ double weight(double v) {
+    return dpp_f64<0x150 + 12 + K>(v);
+  }
+};
 // Sum over the wavefront: row sums combined in row order (uniform result).
 __device__ __forceinline__ double wave_sum(double v) {
   v = group_sum(v);
@@ -1927,22 +1956,28 @@ __global__ __launch_bounds__(NodeShare<W>::kBlock) void k_attn_msg(int N, const 
   const int m = evv ? ev_offset(h) + t : 0;
   const double par = slot_parity(h);
   double acc[3] = {0.0, 0.0, 0.0};
-  struct Terms { double d0, d1, de; };
-  auto terms = [&](int e, int o) {
-    const int p = e >> 1, side = e & 1;
-    // block 0 on the table path: qkv holds one row per element class
-    const double2 vv = ld2(qkv + std::size_t(cls ? cls[z[o]] : o) * 640 + 256 + p0);
-    const double *al = palpha + 16 * std::size_t(p) + 8 * side;
-    const double ai = al[h], ae = al[4 + h];
-    const double fc = pfc[p];
-    const double y = pY[kE * std::size_t(p) + m] * (side == 0 ? 1.0 : par);
-    return Terms{fc * ai * vv.x, fc * ai * vv.y, fc * ae * y};
-  };
-  for_active_pairs(S.beg, S.end, iact, iother, lane, [&](int e1, int o1, int e2, int o2, bool two) {
-    const Terms A = terms(e1, o1);
-    const Terms B = terms(e2, o2);
-    acc[0] += A.d0; acc[1] += A.d1; acc[2] += A.de;
-    if (two) { acc[0] += B.d0; acc[1] += B.d1; acc[2] += B.de; }
+  const EntryScalars es(pY, palpha, h, t, m);
+  // Bound by its loads: L1 accesses with many nodes, latency with few.  With
+  // the weights in the harmonics' load and four entries in flight 24,000 atoms
+  // take 107 us for 175, 3,000 atoms 17.0 for 20.7.
+  // Block 0 on the table path: qkv holds one row per element class.
+  auto row = [&](int o) { return cls ? cls[z[o]] : o; };
+  for_active_quads(S.beg, S.end, iact, iother, lane, row, [&](const int (&e)[4], const int (&o)[4], int count) {
+    double2 v[4];
+    double s[4], fc[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      v[i] = ld2(qkv + std::size_t(o[i]) * 640 + 256 + p0);
+      s[i] = es.load(e[i]);
+      fc[i] = pfc[e[i] >> 1];
+    }
+    __builtin_amdgcn_sched_barrier(0);  // all loads before the first use
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const double ai = es.weight<0>(s[i]), ae = es.weight<1>(s[i]);
+      const double y = s[i] * ((e[i] & 1) == 0 ? 1.0 : par);
+      if (i < count) { acc[0] += fc[i] * ai * v[i].x; acc[1] += fc[i] * ai * v[i].y; acc[2] += fc[i] * ae * y; }
+    }
   });
   share_sum<W>(lds, acc);
   if (!S.on || !S.first) return;
@@ -2302,6 +2337,7 @@ __global__ __launch_bounds__(NodeShare<W>::kBlock) void k_attn_bwd_nodes(int N, 
   const double2 mgv = ld2(gainv + std::size_t(n) * kF + p0);
   const double mge = evv ? gaev[std::size_t(n) * kE + m] : 0.0;
   double d[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};  // dq, dk, dv, dq_ev, dk_ev, two channels each
+  const EntryScalars es(pY, palpha, h, t, m);
   auto visit = [&](int e, int o) {
     const int p = e >> 1, side = e & 1;
     const double *ot = qkv + std::size_t(o) * 640;
@@ -2313,9 +2349,8 @@ __global__ __launch_bounds__(NodeShare<W>::kBlock) void k_attn_bwd_nodes(int N, 
     const v2d fiv = __builtin_nontemporal_load(reinterpret_cast<const v2d *>(fp + p0));
     const v2d fev = __builtin_nontemporal_load(reinterpret_cast<const v2d *>(fp + 128 + p0));
     const double fc = pfc[p];
-    const double y_ld = pY[kE * std::size_t(p) + m];
-    const double *al = palpha + 16 * std::size_t(p);
-    const double aout_i = al[8 * (1 - side) + h];
+    const double y_ld = es.load(e);
+    const double aout_i = es.weight<2>(y_ld);
     const double oge = evv ? oge_ld : 0.0;
     const double y = evv ? y_ld : 0.0;
     const double y_n = side == 0 ? y : par * y;  // harmonics of edge o -> n
@@ -2334,7 +2369,7 @@ __global__ __launch_bounds__(NodeShare<W>::kBlock) void k_attn_bwd_nodes(int N, 
     // the pair's terms, once per pair (its side-0 endpoint; side is uniform
     // across the wavefront): every head's sums appear in that head's 16 lanes
     if (side == 0) {
-      const double ain_i = al[h], ain_e = al[4 + h], aout_e = al[12 + h];
+      const double ain_i = es.weight<0>(y_ld), ain_e = es.weight<1>(y_ld), aout_e = es.weight<3>(y_ld);
       const double part = ain_i * ci + ain_e * ce + aout_i * co + aout_e * coe;
       const double fcg = lane_read(part, 0) + lane_read(part, 16) + lane_read(part, 32) + lane_read(part, 48);
       if (t == 0) *reinterpret_cast<v4d *>(psc + 16 * std::size_t(p) + 4 * h) = v4d{sin_, sout, sine, soute};
@@ -2367,18 +2402,30 @@ __global__ __launch_bounds__(NodeShare<W>::kBlock) void k_ev_bwd(int N, const in
   const NodeShare<W> S(N, inc_off);
   const int n = S.n;
   if (W == 1 && !S.on) return;
-  const int c = lane < kE ? lane : 0;
-  const int slot = degree_slot(c);
+  const int h = lane >> 4, t = lane & 15;
+  const bool evv = t < 2 * h + 3;
+  const int c = evv ? ev_offset(h) + t : 0;
+  // one load an entry: the partner's channel c, and in lane 12 of a row the
+  // slot's ds; four entries in flight (24,000 atoms: 44 us, 67 with two loads
+  // an entry and two entries)
+  const double *base = t < 12 ? ev + c : ds + h;
   const double en = ev[std::size_t(n) * kE + c];
   double acc[1] = {S.first ? gaev[std::size_t(n) * kE + c] : 0.0};
-  auto term = [&](int e, int o) { return 2.0 * (en - ev[std::size_t(o) * kE + c]) * cg[c] * ds[4 * std::size_t(e >> 1) + slot]; };
-  for_active_pairs(S.beg, S.end, iact, iother, lane, [&](int e1, int o1, int e2, int o2, bool two) {
-    const double a = term(e1, o1), b = term(e2, o2);
-    acc[0] += a;
-    if (two) acc[0] += b;
+  const double w = cg[c];
+  auto row = [](int o) { return o; };
+  for_active_quads(S.beg, S.end, iact, iother, lane, row, [&](const int (&e)[4], const int (&o)[4], int count) {
+    double v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = base[t < 12 ? kE * unsigned(o[i]) : 4u * (unsigned(e[i]) >> 1)];
+    __builtin_amdgcn_sched_barrier(0);  // all loads before the first use
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const double a = 2.0 * (en - v[i]) * w * dpp_f64<0x150 + 12>(v[i]);
+      if (i < count) acc[0] += a;
+    }
   });
   share_sum<W>(lds, acc);
-  if (S.on && S.first && lane < kE) gev[std::size_t(n) * kE + lane] = acc[0];
+  if (S.on && S.first && evv) gev[std::size_t(n) * kE + c] = acc[0];
 }
 
 // ---------------------------------------------------------------- geometry

@@ -39,6 +39,19 @@ def test_node_shares(orc, model, n):  # noqa: F811
     _both_paths(z, x, 0.0, m, orc, model)
 
 
+@pytest.mark.parametrize("copies", [17, 86])
+def test_partner_counts(orc, model, copies):  # noqa: F811
+    """Separate groups of 1 to 7 atoms: nodes with 0 to 6 active partners, the
+    remainders of the four entries the node-major sums read at a time, with
+    the list shared by 8 wavefronts (476 atoms) and read by one (2,408)."""
+    parts = [_cluster(1 + k % 7, seed=k) for k in range(7 * copies)]
+    g = int(np.ceil(len(parts) ** (1 / 3) - 1e-9))
+    at = 9.0 * np.array([[k // (g * g), k // g % g, k % g] for k in range(len(parts))], float)
+    z = np.concatenate([p[0] for p in parts])
+    x = np.concatenate([p[1] + o for p, o in zip(parts, at)])
+    _both_paths(z, x, 0.0, 1.0 + float((z == 1).sum() % 2), orc, model)
+
+
 @pytest.mark.parametrize("limit", ["0", "1000000"])
 @pytest.mark.parametrize("n", [2, 3, 17, 65])
 def test_few_pairs(monkeypatch, n, limit):
