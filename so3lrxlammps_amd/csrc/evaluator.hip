@@ -99,23 +99,6 @@ __device__ __forceinline__ double group_sum(double v) {
   return v;
 }
 
-// The sums of v[0..4) over the 16-lane row, every lane ending with all four:
-// half of the values go to the partner at each of the first two steps, 5
-// exchanges and 4 broadcasts where 4 separate sums take 16.  All 64 lanes must
-// be active.
-__device__ __forceinline__ void group_sum4(double (&v)[4], int t) {
-  const bool b3 = t & 8, b2 = t & 4;
-  const double u0 = (b3 ? v[2] : v[0]) + dpp_f64<0x140>(b3 ? v[0] : v[2]);
-  const double u1 = (b3 ? v[3] : v[1]) + dpp_f64<0x140>(b3 ? v[1] : v[3]);
-  double x = (b2 ? u1 : u0) + dpp_f64<0x141>(b2 ? u0 : u1);
-  x += dpp_f64<0x4E>(x);
-  x += dpp_f64<0xB1>(x);
-  v[0] = dpp_f64<0x150>(x);
-  v[1] = dpp_f64<0x150 + 4>(x);
-  v[2] = dpp_f64<0x150 + 8>(x);
-  v[3] = dpp_f64<0x150 + 12>(x);
-}
-
 // An incidence entry's harmonics and attention weights in one load, for the
 // lane layout of the node-major kernels (row h of 16 lanes, t the lane in it):
 // lanes t < 12 hold channel m's harmonic of the pair (channel 0 beyond the
@@ -2372,9 +2355,10 @@ __global__ __launch_bounds__(NodeShare<W>::kBlock) void k_attn_bwd_nodes(int N, 
     const double y = evv ? y_ld : 0.0;
     const double y_n = side == 0 ? y : par * y;  // harmonics of edge o -> n
     const double y_o = side == 0 ? par * y : y;  // harmonics of edge n -> o
-    double c4[4] = {mgv.x * ovv.x + mgv.y * ovv.y, ogv.x * mvv.x + ogv.y * mvv.y, mge * y_n, oge * y_o};
-    group_sum4(c4, t);
-    const double ci = c4[0], co = c4[1], ce = c4[2], coe = c4[3];
+    const double ci = group_sum(mgv.x * ovv.x + mgv.y * ovv.y);
+    const double ce = group_sum(mge * y_n);
+    const double co = group_sum(ogv.x * mvv.x + ogv.y * mvv.y);
+    const double coe = group_sum(oge * y_o);
     const double sin_ = fc * ci * inv_avg, sine = fc * ce * inv_avg;
     const double sout = fc * co * inv_avg, soute = fc * coe * inv_avg;
     d[0] += sin_ * okv.x * fiv.x; d[1] += sin_ * okv.y * fiv.y;
