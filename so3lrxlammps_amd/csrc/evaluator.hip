@@ -3887,7 +3887,7 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
   };  // enqueue
 
   const GraphKey key{x_in, fo, etot, flags, {box_len_[0], box_len_[1], box_len_[2]}, s, topo_version_,
-                     alloc_epoch_};
+                     alloc_epoch_, PA};
   if (from_scratch) {
     enqueue();  // instantiating a graph allocates: never here
   } else if (timing_ || !use_graphs_) {

@@ -326,10 +326,14 @@ class Evaluator {
     double box[3] = {0, 0, 0};
     hipStream_t stream = nullptr;
     std::uint64_t topology = 0, epoch = 0;
+    // capacity of the active-pair buffers: the launches' grids, clamps and
+    // per-block offsets hold it by value, and it can grow without any buffer
+    // growing (buffers keep the capacity of an earlier, larger topology)
+    std::int64_t pairs = 0;
     bool operator==(const GraphKey &o) const {
       return x == o.x && f == o.f && eatom == o.eatom && flags == o.flags && box[0] == o.box[0] &&
              box[1] == o.box[1] && box[2] == o.box[2] && stream == o.stream && topology == o.topology &&
-             epoch == o.epoch;
+             epoch == o.epoch && pairs == o.pairs;
     }
   };
   bool use_graphs_ = true;  // SO3LR_NO_GRAPH=1 turns replay off

@@ -645,6 +645,58 @@ def test_active_pair_capacity_overflow_reevaluates():
     b.close()
 
 
+@pytest.mark.parametrize("route", ["host", "device"])
+def test_capacity_overflow_after_larger_topology(route):
+    """The capacity grows, but no buffer does: the context held a topology
+    with more pairs before.  The call that overflows comes after the same call
+    was captured for replay; what was captured holds the old capacity and must
+    not be replayed (pairs beyond it would be left out without a sign).
+    Against a context that counted at that geometry, bit for bit; then further
+    calls, which replay what the grown capacity captured."""
+    import torch
+    from so3lrxlammps_amd import Context, Lists
+    ref, z, pos, box = support.load_golden("water3000")
+    lists = Lists(pos, np.zeros(3), box, (1, 1, 1))
+    rows = [np.ascontiguousarray(lists.rows_positions(pos) * s) for s in (1.0, 0.94)]
+
+    def caller(c):
+        if route == "host":
+            return lambda k: c.compute(rows[k])
+        dev = torch.device("cuda:0")
+        xt = torch.empty(rows[0].shape, dtype=torch.float64, device=dev)
+        f = torch.empty((len(z), 3), dtype=torch.float64, device=dev)
+        e = torch.empty(len(z), dtype=torch.float64, device=dev)
+
+        def call(k):
+            xt.copy_(torch.from_numpy(rows[k]))
+            torch.cuda.synchronize()
+            energy, w = c.compute_device(xt, f, e)
+            return energy, f.cpu().numpy(), e.cpu().numpy(), w
+        return call
+
+    print("case water3000", route, flush=True)
+    b = Context(support.MODEL, 0)
+    b.set_system(z, 0, 1)
+    b.set_topology(lists)
+    want = caller(b)(1)
+    b.close()
+    a = Context(support.MODEL, 0)
+    a.set_system(z, 0, 1)
+    call = caller(a)
+    a.set_topology(lists)
+    call(1)  # the buffers get the compressed geometry's size
+    n1 = a.graph_stats()[0]
+    a.set_topology(lists)
+    for _ in range(3):  # counted at the smaller number; captured, replayed
+        call(0)
+    n0 = a.graph_stats()[0]
+    assert n1 > n0 + n0 // 8 + 256  # the compressed geometry overflows the capacity
+    for k in range(4):
+        e, f, ea, w = call(1)
+        assert e == want[0] and np.array_equal(f, want[1]) and np.array_equal(ea, want[2]) and np.array_equal(w, want[3]), k
+    a.close()
+
+
 def test_refused_first_evaluation_leaves_context_usable():
     """The first evaluation of a single system's LAMMPS-list topology puts its
     nodes in spatial order and sorts the incidence there.  A first evaluation
