@@ -222,7 +222,11 @@ __device__ __forceinline__ bool sr_active(const Pos &pos, int c, double rc2, dou
 
 // Active candidates per block of kCompactPerBlock; in the same launch, what
 // the evaluation needs before its first pair: positions gathered into node
-// order (xn, with perm) and the bucket counters cleared.
+// order (xn, with perm) and the bucket counters cleared.  The grid covers the
+// candidates, and with fewer of them than that needs (a gas) up to
+// kGatherBlocks blocks of it as well: 64,000 atoms with one close pair, 569 us
+// on the one block of candidates, 9 on the wider grid.
+constexpr int kGatherBlocks = 1024;
 struct CountExtras {
   int n3, nkeys;       // 3 N values of xn (0: none); counters
   const double *xin;
@@ -242,7 +246,7 @@ __global__ __launch_bounds__(256) void k_sr_count(int P, Pos pos, double rc2, in
   const unsigned long long m = __ballot(in);
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = __popcll(m);
   __syncthreads();
-  if (threadIdx.x == 0) blk_count[blockIdx.x] = (part[0] + part[1]) + (part[2] + part[3]);
+  if (threadIdx.x == 0 && c < P) blk_count[blockIdx.x] = (part[0] + part[1]) + (part[2] + part[3]);
 }
 
 // exclusive scan of per-block counts in place (one block, a run of counts per
@@ -3505,7 +3509,9 @@ void Evaluator::compute_impl(const double *x, int flags, double *f_out, double *
     using CountPos = decltype(count_pos);
     using Pos = decltype(pos);
     const CountExtras X{gather_pos ? int(3 * N) : 0, buckets ? rkeys : 0, x_in, perm, const_cast<double *>(x), rhist};
-    hipLaunchKernelGGL(k_sr_count<CountPos>, dim3(nblk), dim3(256), 0, s, int(P), count_pos, rc2, blk, X);
+    const int extra = ceil_div(std::max(X.n3, X.nkeys), 256);
+    hipLaunchKernelGGL(k_sr_count<CountPos>, dim3(unsigned(std::max(nblk, std::min(extra, kGatherBlocks)))), dim3(256),
+                       0, s, int(P), count_pos, rc2, blk, X);
 #define SO3LR_COMPACT(PREFIX)                                                                                       \
   hipLaunchKernelGGL((k_sr_compact<Pos, PREFIX>), dim3(nblk), dim3(256), 0, s, int(P), pos, sr_nodes, rc2, blk, cap, \
                      z, zbl_, c2a, pa, pv, pr, pY, pfc, pzbl, dr, nact, nact + 1, bdom, buckets ? rhist : nullptr)

@@ -52,6 +52,20 @@ def test_partner_counts(orc, model, copies):  # noqa: F811
     _both_paths(z, x, 0.0, 1.0 + float((z == 1).sum() % 2), orc, model)
 
 
+@pytest.mark.parametrize("n", [85, 86, 1000])
+def test_few_candidates(orc, model, n):  # noqa: F811
+    """One candidate pair and the other atoms on a 7 A lattice without any:
+    the launch that counts the candidates gathers 3 n coordinates beside it
+    (255 and 258, on both sides of its blocks of 256, and many blocks)."""
+    g = int(np.ceil(n ** (1 / 3) - 1e-9))
+    sites = np.array([[i, j, k] for i in range(g) for j in range(g) for k in range(g)], float)[:n]
+    x = 7.0 * sites + np.random.default_rng(n).uniform(-0.2, 0.2, (n, 3))
+    x[1] = x[0] + [1.0, 0.3, -0.2]
+    z = np.full(n, 8)
+    z[:2] = 1
+    _both_paths(z, x, 0.0, 1.0, orc, model)
+
+
 @pytest.mark.parametrize("limit", ["0", "1000000"])
 @pytest.mark.parametrize("n", [2, 3, 17, 65])
 def test_few_pairs(monkeypatch, n, limit):
