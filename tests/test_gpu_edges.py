@@ -7,8 +7,8 @@ charge and multiplicity (a bare proton, an open-shell H atom, triplet O).
 Both the LAMMPS-rows path and the HBM-resident device path are checked at the
 bars of the other parity tests: energy 1e-10 relative, forces and virial
 1e-9 eV/A; each case runs on the shipped model (with the filter kernels
-the library picks for these sizes, and with the fused MFMA ones forced) and
-on an F = 256 model (generic kernels).
+the library picks for these sizes, with the scalar ones ruled out, and with
+the scalar ones forced) and on an F = 256 model (generic kernels).
 """
 import os
 
@@ -21,18 +21,18 @@ from oracle.oracle import Oracle
 pytestmark = pytest.mark.gpu
 
 
-@pytest.fixture(scope="module", params=["v1", "v1_mfma", "generic"])
+@pytest.fixture(scope="module", params=["v1", "v1_mfma", "v1_scalar", "generic"])
 def model(request, tmp_path_factory):
-    """The shipped model (v1 kernels: these systems are small enough for the
-    scalar filter kernels), the same with the fused MFMA filters forced
-    (SO3LR_SCALAR_FILTER_PAIRS=0 while its tests create their contexts), and
-    a perturbed F = 256, R = 64 lift with duplicated degrees (generic
-    kernels)."""
+    """The shipped model (v1 kernels; its radial tables hold, so by default no
+    size runs the scalar filter kernels), the same with the scalar filters
+    ruled out and with them forced at every size (SO3LR_SCALAR_FILTER_PAIRS=0
+    and 1000000 while its tests create their contexts), and a perturbed
+    F = 256, R = 64 lift with duplicated degrees (generic kernels)."""
     if request.param == "v1":
         yield support.MODEL
-    elif request.param == "v1_mfma":
+    elif request.param in ("v1_mfma", "v1_scalar"):
         old = os.environ.get("SO3LR_SCALAR_FILTER_PAIRS")
-        os.environ["SO3LR_SCALAR_FILTER_PAIRS"] = "0"
+        os.environ["SO3LR_SCALAR_FILTER_PAIRS"] = "0" if request.param == "v1_mfma" else "1000000"
         yield support.MODEL
         if old is None:
             del os.environ["SO3LR_SCALAR_FILTER_PAIRS"]

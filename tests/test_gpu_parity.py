@@ -71,17 +71,18 @@ def test_molecule_matches_oracle(ctx, orc, name):
     _check(out, e, f, ea, w, terms)
 
 
-def test_molecules_mfma_filters_match_oracle(orc, monkeypatch):
-    """Molecules this small run the scalar filter kernels by default (at most
-    SO3LR_SCALAR_FILTER_PAIRS active pairs); the same molecules with the fused
-    MFMA filters forced, against the oracle at the same bars."""
+@pytest.mark.parametrize("limit", ["0", "1000000"])
+def test_molecules_mfma_filters_match_oracle(orc, monkeypatch, limit):
+    """The molecules on the MFMA filters (SO3LR_SCALAR_FILTER_PAIRS=0, what the
+    shipped model runs by default) and on the scalar filter kernels (1000000),
+    against the oracle at the same bars."""
     from so3lrxlammps_amd import Context
-    monkeypatch.setenv("SO3LR_SCALAR_FILTER_PAIRS", "0")
+    monkeypatch.setenv("SO3LR_SCALAR_FILTER_PAIRS", limit)
     c = Context(support.MODEL, 0)
     for name in MOLECULES:
         ref, z, pos, box = support.load_golden(name)
         q, m = ref.get("charge", 0), ref.get("multiplicity", 1)
-        print("case", name, "(MFMA filters)", flush=True)
+        print("case", name, "(scalar filters up to %s pairs)" % limit, flush=True)
         e, f, ea, w, terms = _hip_single_point(c, z, pos, box, q, m)
         out = orc.evaluate(z, *support.build_graphs(pos, box), charge=q, multiplicity=m)
         _check(out, e, f, ea, w, terms)
@@ -89,9 +90,11 @@ def test_molecules_mfma_filters_match_oracle(orc, monkeypatch):
 
 
 def test_small_system_filter_paths_agree(monkeypatch):
-    """The filter path switches with the active-pair count; both paths on the
-    same molecule agree to rounding (the scalar kernels use the library exp
-    and division, the MFMA ones the lean activations)."""
+    """The filter path can switch with the active-pair count
+    (SO3LR_SCALAR_FILTER_PAIRS, and by default in models without radial
+    tables); both paths on the same molecule agree to rounding (the scalar
+    kernels use the library exp and division, the MFMA ones the lean
+    activations)."""
     from so3lrxlammps_amd import Context
     ref, z, pos, box = support.load_golden("alanine_cation")
     res = []

@@ -1,6 +1,6 @@
 """HIP path vs the CPU oracle at the sizes where the kernels' work is cut: atom
-counts at and beside the edges of their 16-atom tiles, on the scalar and the
-fused filter kernels of the shipped model and on the generic widths; head
+counts at and beside the edges of their 16-atom tiles, on the fused and the
+scalar filter kernels of the shipped model and on the generic widths; head
 widths that leave a part of a 16-unit tile.  Bars as in test_gpu_edges.py:
 energy 1e-10 relative, forces and virial 1e-9.
 """
