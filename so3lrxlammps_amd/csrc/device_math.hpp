@@ -356,6 +356,19 @@ __device__ __forceinline__ bool lr_pair_terms(const LrParams &P, const double *_
   return true;
 }
 
+// DPP lane permute of a double within the 16-lane rows of a wavefront (two
+// 32-bit moves).  CTRL: 0xB1 quad_perm(1,0,3,2), 0x4E quad_perm(2,3,0,1),
+// 0x141 row_half_mirror, 0x140 row_mirror, 0x150 + n row_newbcast (lane n):
+// each names a lane for every lane, so BOUND (0 where there is none) changes
+// no value, only how the compiler may place the moves.
+template <int CTRL, bool BOUND = false>
+__device__ __forceinline__ double dpp_f64(double v) {
+  const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+  const unsigned lo = unsigned(__builtin_amdgcn_update_dpp(0, int(unsigned(b)), CTRL, 0xF, 0xF, BOUND));
+  const unsigned hi = unsigned(__builtin_amdgcn_update_dpp(0, int(unsigned(b >> 32)), CTRL, 0xF, 0xF, BOUND));
+  return __builtin_bit_cast(double, (unsigned long long)lo | ((unsigned long long)hi << 32));
+}
+
 // Walks the active incidence entries of a node, [beg, end), in list order:
 // 64 entries per coalesced load of iact / iother, then the active ones two at
 // a time as uniform values, body(e1, o1, e2, o2, two) (when one is left the

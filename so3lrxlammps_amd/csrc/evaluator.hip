@@ -71,16 +71,6 @@ constexpr int kCompactPerBlock = 256;  // candidates per compaction block, one p
 // own; more go through k_scan_counts
 constexpr int kPrefixBlocks = 1024;
 
-// DPP lane permute of a double within the 16-lane rows of a wavefront (two
-// 32-bit moves).  CTRL: 0xB1 quad_perm(1,0,3,2), 0x4E quad_perm(2,3,0,1),
-// 0x141 row_half_mirror, 0x140 row_mirror, 0x150 + n row_newbcast (lane n).
-template <int CTRL>
-__device__ __forceinline__ double dpp_f64(double v) {
-  const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
-  const unsigned lo = unsigned(__builtin_amdgcn_update_dpp(0, int(unsigned(b)), CTRL, 0xF, 0xF, false));
-  const unsigned hi = unsigned(__builtin_amdgcn_update_dpp(0, int(unsigned(b >> 32)), CTRL, 0xF, 0xF, false));
-  return __builtin_bit_cast(double, (unsigned long long)lo | ((unsigned long long)hi << 32));
-}
 // value of v in lane l (uniform)
 __device__ __forceinline__ double lane_read(double v, int l) {
   const unsigned long long b = __builtin_bit_cast(unsigned long long, v);

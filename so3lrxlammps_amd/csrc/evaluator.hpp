@@ -71,8 +71,8 @@ struct BlockWeights {
   const double *e0pk[2];                                // spherical layer 0, one v4d per lane
   // radial tables of the blocks after 0 (radial_rows.hpp): per
   // interval and filter, the radial branch W1 silu(W0 rbf + b0) + ob1 as
-  // 16 powers of t (an MFMA A operand of 128 x 16) and its r-derivative
-  // (16 x 128); null without the tables
+  // 32 powers of t (128 x 32, the rows in head-pair order as e1h's) and its
+  // r-derivative (32 x 128), MFMA operands; null without the tables
   const double *rrow, *rdr;
   // MFMA operand order of the node layers: forward and reverse (transpose)
   const double *qkvp, *qkvtp;           // per head (160 x 32) and (32 x 160)
@@ -281,7 +281,9 @@ class Evaluator {
   // scalar filter kernels: with a few hundred active pairs the fully unrolled
   // MFMA filters are bound by fetching their code into a cold instruction
   // cache (30-40 us per launch).  With the tables the split kernels for few
-  // pairs are the faster ones (22 atoms: 286 against 412 us per evaluation).
+  // pairs are the faster ones, also for packed images, whose block 0 has no
+  // tables (us per evaluation, scalar / split: one molecule of 22 atoms 412 /
+  // 283, two of 12 atoms 382 / 345, two water molecules 326 / 312).
   // Decided when a topology's active pairs are counted: at most
   // scalar_pairs_max_ of them (SO3LR_SCALAR_FILTER_PAIRS; 0 never; -1, the
   // default: 256 without the tables, none with them).

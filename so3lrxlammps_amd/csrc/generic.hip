@@ -33,10 +33,6 @@ namespace so3lr_amd {
 namespace {
 
 __device__ __forceinline__ double gsilu(double x) { return x / (1.0 + exp(-x)); }
-__device__ __forceinline__ double gsilu_prime(double x) {
-  const double s = 1.0 / (1.0 + exp(-x));
-  return s * (1.0 + x * (1.0 - s));
-}
 // Sum over the 64 lanes of a wavefront, the same value in every lane (lane
 // 0's butterfly result, broadcast).  All lanes must be active.
 __device__ __forceinline__ double wsum(double v) {
@@ -1676,8 +1672,8 @@ GenericPath::GenericPath(const Model &m, const std::function<const double *(cons
   }
   // the blocks after 0: each filter's radial branch W1 h(r) + b1 + e1 as
   // piecewise polynomials (32 intervals of degree 31, the same bound), per
-  // interval and filter an F x 32 coefficient tile with the output rows
-  // permuted within each tile as wcp's (g_filt_fwd's channel order)
+  // interval and filter an F x 32 coefficient tile, its output rows in
+  // head-pair order (head_pairs, as e1h)
   if (fit_radial && layers_ > 1) {
     const auto bb = m.f64("model.radial_embedding.radial_basis_fn.b", {R});
     bool ok = true;

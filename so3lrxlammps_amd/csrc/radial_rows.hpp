@@ -51,16 +51,6 @@ struct RowsArgs {
 template <int FT>
 constexpr int kFewRows = FT == 8 ? 7500 : 3700;
 
-// v of the lane that row_mirror (0x140), row_half_mirror (0x141) or a quad
-// permutation names
-template <int CTRL>
-__device__ __forceinline__ double dpp(double v) {
-  typedef int v2i __attribute__((ext_vector_type(2)));
-  v2i x = __builtin_bit_cast(v2i, v);
-  x[0] = __builtin_amdgcn_update_dpp(0, x[0], CTRL, 0xf, 0xf, true);
-  x[1] = __builtin_amdgcn_update_dpp(0, x[1], CTRL, 0xf, 0xf, true);
-  return __builtin_bit_cast(double, x);
-}
 // The sums of v[0..8) over the 16 lanes of a group: lane j ends with that of
 // v[4 b3 + 2 b2 + b1], b its index's bits.  Half of the values go to the
 // partner at each step: 8 exchanges where 8 separate sums take 32.
@@ -68,11 +58,11 @@ __device__ __forceinline__ double spread_sum8(const double (&v)[8], int j) {
   const bool b3 = j & 8, b2 = j & 4, b1 = j & 2;
   double u[4], w[2];
 #pragma unroll
-  for (int k = 0; k < 4; ++k) u[k] = (b3 ? v[k + 4] : v[k]) + dpp<0x140>(b3 ? v[k] : v[k + 4]);
+  for (int k = 0; k < 4; ++k) u[k] = (b3 ? v[k + 4] : v[k]) + dpp_f64<0x140, true>(b3 ? v[k] : v[k + 4]);
 #pragma unroll
-  for (int k = 0; k < 2; ++k) w[k] = (b2 ? u[k + 2] : u[k]) + dpp<0x141>(b2 ? u[k] : u[k + 2]);
-  const double x = (b1 ? w[1] : w[0]) + dpp<0x4E>(b1 ? w[0] : w[1]);
-  return x + dpp<0xB1>(x);
+  for (int k = 0; k < 2; ++k) w[k] = (b2 ? u[k + 2] : u[k]) + dpp_f64<0x141, true>(b2 ? u[k] : u[k + 2]);
+  const double x = (b1 ? w[1] : w[0]) + dpp_f64<0x4E, true>(b1 ? w[0] : w[1]);
+  return x + dpp_f64<0xB1, true>(x);
 }
 // LDS values of one wavefront's lanes to its other lanes
 __device__ __forceinline__ void wave_lds() {
