@@ -147,12 +147,12 @@ def kernel_work(widths, elements=0):
     # doubles written per pair with the 4 NH logits and NH invariants (the
     # invariants are read back), r and the endpoints read
     rt_bytes = 8 * (2 * F + 4 * NH + NH) + 16
-    work["generic_filter_fwd_radial"] = ("k_rows_fwd", "hbm", rt_bytes, rt_bytes, "pair")
+    work["generic_filter_fwd_radial"] = ("k_rows_fwd<%d>" % (F // 16), "hbm", rt_bytes, rt_bytes, "pair")
     # and the reverse: df against the slope polynomials (14 powers per
     # channel at the accuracy of degree 13; 32 issued), E1^T, E0^T
     rt_bwd = 2 * 2 * (14 * F + FH * F + NH * FH)
-    work["generic_filter_bwd_radial"] = ("k_rows_bwd", "mfma", rt_bwd, 2 * 2 * (32 * F + FH * F + NH * FH),
-                                         "pair")
+    work["generic_filter_bwd_radial"] = ("k_rows_bwd<%d>" % (F // 16), "mfma", rt_bwd,
+                                         2 * 2 * (32 * F + FH * F + NH * FH), "pair")
     if elements:
         tab = 2 * 2 * (R * F + 2 * NH * F)
         work["generic_filter_fwd_block0_tables"] = ("g_b0_fwd: block 0's fused table filters", "mfma", tab,

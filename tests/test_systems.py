@@ -66,3 +66,19 @@ def test_water_configs_density_and_overlap():
     a = np.sort(np.minimum(lr[0], lr[1]) * len(z) + np.maximum(lr[0], lr[1]))
     b2 = np.sort(np.minimum(lr2[0], lr2[1]) * len(z) + np.maximum(lr2[0], lr2[1]))
     assert np.array_equal(a, b2)
+
+
+def test_bench_traffic_covers_the_kernels_of_the_default_workload():
+    """The bench line's `traffic` of the table kernels comes from the committed
+    counter summary, by kernel name; another model's kernels of the same
+    template are not in it."""
+    import bench
+    for section in ("filter_fwd_radial", "filter_bwd_radial"):
+        symbol, _, algorithmic, _, _ = bench.KERNEL_WORK[section]
+        traffic, source = bench.traffic_per_launch(symbol, 3, 1000)
+        assert traffic is not None and "pmc_traffic_config3" in source, symbol
+        if section == "filter_fwd_radial":
+            assert traffic > 1000 * algorithmic  # never below what the kernel must move
+    widths = {"invariant_features": 256, "radial_basis_features": 64, "degree_slots": [1, 1, 2, 2, 3, 3, 4, 4]}
+    wide = bench.kernel_work(widths)
+    assert bench.traffic_per_launch(wide["generic_filter_fwd_radial"][0], 3, 1000) == (None, None)
