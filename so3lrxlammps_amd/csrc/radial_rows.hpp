@@ -9,11 +9,13 @@
 // 64 accesses; with 16 lanes along one row it takes 16.  So the rows are
 // loaded and stored with lane j of a group of 16 on channels 2 j and 2 j + 1
 // of a head and the pairs g + 4 r (r = 0..3) one after the other.  24,000
-// atoms, 537,000 pairs (us, pairs on the lanes / this layout): forward 697 /
-// 515, reverse 528 / 416; F = 256 1,887 / 1,208 and 1,396 / 1,035.  The L1's
-// accesses alone were 605, 496, 1,240 and 1,240 us of that; now the matrix
-// pipe (500,000 to 570,000 of 980,000 clocks a SIMD) with the other vector
-// instructions, which share its issue, bound both.
+// atoms, 476,500 pairs (us, pairs on the lanes / this layout): forward 697 /
+// 515, reverse 528 / 416; F = 256 1,887 / 1,208 and 1,396 / 1,035.  By the
+// counters the L1's accesses alone were 0.93, 0.91, 0.69 and 0.91 of the time
+// before and are 0.55, 0.59, 0.55 and 0.61 now.  No unit is busy all the time:
+// the matrix pipe 0.44, 0.55, 0.57 and 0.70, the other vector instructions,
+// none of which runs beside an MFMA, up to 0.18, 0.11, 0.14 and 0.08; the rest
+// is waits, two wavefronts a SIMD not covering every operand from L2.
 #pragma once
 
 #include "node_chain.hpp"
