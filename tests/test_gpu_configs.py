@@ -186,7 +186,7 @@ def test_config4_memory_ceiling_properties(orc):
 def test_config4_full_size(orc):
     """The 150,000-atom memory-ceiling water, all atoms, device path against
     the oracle (about 60 GB of host memory for the oracle's per-edge
-    buffers and a few tens of seconds on the GPU box's cores)."""
+    buffers and a few tens of seconds on 16 cores)."""
     import resource
     import time
     from so3lrxlammps_amd import Context, Lists, systems
